@@ -18,17 +18,19 @@ N = 70                                                         # tokens of the p
 class Model:
     """A two-layer model file and its float64 pass.  part: "attention" or "ffn", what the first layer adds to the residual."""
 
-    def __init__(self, lib, part, wtype, dim, hidden, heads, kv_heads, gain, seed=3, zero=True):
+    def __init__(self, lib, part, wtype, dim, hidden, heads, kv_heads, gain, seed=3, also=None):
         self.lib, self.dim, self.hidden, self.heads, self.kv_heads, self.w = lib, dim, hidden, heads, kv_heads, {}
         off = {"attention": "ffn_down", "ffn": "attn_output"}[part]
 
         def hook(name, dims, t, data):
-            if zero and name == "blk.0.%s.weight" % off:
+            if name == "blk.0.%s.weight" % off:
                 data = np.zeros_like(data)
-            if zero and name.startswith("token_embd"):         # the residual is the operator's result and next to nothing else
+            if name.startswith("token_embd"):         # the residual is the operator's result and next to nothing else
                 data = (data.view(np.float32) * np.float32(1e-6)).view(np.uint8)
             if name.endswith("_norm.weight") and name.startswith("blk.0"):
                 data = (data.view(np.float32) * np.float32(gain)).view(np.uint8)
+            if also:
+                dims, t, data = also(name, dims, t, data)
             self.w[name] = (dims, t, data)
             return dims, t, data
 
@@ -121,3 +123,30 @@ def test_error_with_small_activations(backend, oracle_lib, shape, wtype, gain):
     _, first, second = errors(backend, m)
     assert first < BAR[0], first
     assert gain < 0.05 or second < BAR[1], second
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("kv_f16", [False, True])
+@pytest.mark.parametrize("gain", [1.0, 0.05, 0.01])
+def test_error_of_attention(backend, oracle_lib, shape, kv_f16, gain):
+    """Queries, keys and values of every size.  An f16 cache rounds what it holds to 2^-11 (2.1e-4 of the values' 2-norm)."""
+    m = Model(oracle_lib, "attention", Q8_0, *SHAPES[shape], gain)
+    _, first, second = errors(backend, m, kv_f16)
+    assert first < (2.5e-4 if kv_f16 else BAR[0]) and second < (6e-4 if kv_f16 else BAR[1]), (first, second)
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("kv_f16", [False, True])
+def test_error_of_sharp_attention(backend, oracle_lib, shape, kv_f16):
+    """Queries of 2e-3 against keys of 6e2 and the other way round: the scores are ordinary ones, the pairs are not."""
+    for up in ("attn_q", "attn_k"):
+        def hook(name, dims, t, data, up=up):
+            if name.startswith("blk.0.attn_q.") or name.startswith("blk.0.attn_k."):
+                data = data.copy()
+                d = data.reshape(-1, 34)[:, :2].copy().view(np.float16) * np.float16(2.0 ** 9 if up in name else 2.0 ** -9)
+                data.reshape(-1, 34)[:, :2] = d.view(np.uint8)
+            return dims, t, data
+
+        m = Model(oracle_lib, "attention", Q8_0, *SHAPES[shape], 1.0, also=hook)
+        keys, _, second = errors(backend, m, kv_f16)
+        assert second < (6e-4 if kv_f16 else 2 * BAR[1]), (up, keys, second)
