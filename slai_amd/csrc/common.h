@@ -75,6 +75,7 @@ struct slai_ctx {
     int prompt_split_f16 = 1;           // SLAI_PROMPT_SPLIT_F16: 0 = prompt-chunk GEMMs in fp32 MFMA, 1 = the models' on the f16 matrix cores (f16 head + remainder), 2 = slai_matmul_quant_columns too
     int *split_flag = nullptr;          // device word the kernels that write split activations set when a value is beyond f16
     bool prompt_gemm = true;            // SLAI_PROMPT_GEMM=0: prompt chunks never take the matrix-core kernels
+    size_t prompt_copy_bytes = (size_t)1 << 30;   // SLAI_PROMPT_COPY_MB (1024): most a model's padded copies for the wide prompt pass may take
     // tuning knobs (environment overridable, see runtime.cpp)
     int gemv_rows_per_wg = 8;
     int gemv_max_threads = 1024;

@@ -150,35 +150,39 @@ struct WidePass {
 };
 
 // The matrices the wide pass reads: a model's own where they lie in tiles, padded copies in tiles of Q8_0 / Q4_0 ones whose
-// rows are no multiple of 256 (small models: a copy is a few megabytes).
+// rows are no multiple of 256.  The copies are memory for speed (a token read in a pass of 64 costs a tenth of one in the
+// token loop), so a model has none where they would take more than ctx->prompt_copy_bytes (1 GiB) or an eighth of what is free,
+// where they cannot be allocated, and in a context that keeps every matrix in rows.  6 MB for the 15 M parameter Llama.
 struct WideMats {
     std::vector<slai_qmat *> copies;                           // (their memory is one block)
     uint8_t *block = nullptr;
     // m itself, a copy (its memory is assigned by `make`), or null where neither is possible
-    slai_qmat *take(slai_qmat *m) {
+    slai_qmat *take(const slai_ctx *ctx, slai_qmat *m) {
         if (wide_gemm_supports(m)) return m;
-        if (m->tiled || (m->type != T_Q8_0 && m->type != T_Q4_0)) return nullptr;
+        if (!ctx->tiled_layout || m->tiled || (m->type != T_Q8_0 && m->type != T_Q4_0)) return nullptr;
         const TiledGeom g = tiled_geom(m->type, m->nrows, (m->ncols + 255) / 256 * 256, 4u);
         slai_qmat *c = new slai_qmat();
-        c->type = m->type; c->nrows = m->nrows; c->ncols = m->ncols; c->nb = m->nb; c->tiled = true; c->wbound = m->wbound;
-        c->rows_log2 = g.rows_log2; c->ncb = g.ncb; c->ngroups = g.ngroups; c->ntiles = g.ntiles; c->unit_bytes = g.unit_bytes; c->bytes = tiled_bytes(g);
         copies.push_back(c);
         sources.push_back(m);
-        return c;
+        c->type = m->type; c->nrows = m->nrows; c->ncols = m->ncols; c->nb = m->nb; c->tiled = true; c->wbound = m->wbound;
+        c->rows_log2 = g.rows_log2; c->ncb = g.ncb; c->ngroups = g.ngroups; c->ntiles = g.ntiles; c->unit_bytes = g.unit_bytes; c->bytes = tiled_bytes(g);
+        return wide_gemm_supports(c) ? c : nullptr;
     }
-    int make(slai_ctx *ctx) {
-        size_t total = 0;
+    // false: the model does without
+    bool make(const slai_ctx *ctx) {
+        size_t total = 0, free_bytes = 0, all_bytes = 0;
         for (const slai_qmat *c : copies) total += (c->bytes + 255) / 256 * 256;
-        if (!total) return SLAI_OK;
-        SLAI_HIP_TRY(ctx, hipMalloc((void **)&block, total));
-        SLAI_HIP_TRY(ctx, hipMemsetAsync(block, 0, total, ctx->stream));
+        if (!total) return true;
+        if (total > ctx->prompt_copy_bytes || hipMemGetInfo(&free_bytes, &all_bytes) != hipSuccess || total > free_bytes / 8) return false;
+        if (hipMalloc((void **)&block, total) != hipSuccess) { block = nullptr; (void)hipGetLastError(); return false; }
+        bool ok = hipMemsetAsync(block, 0, total, ctx->stream) == hipSuccess;
         size_t at = 0;
-        for (size_t i = 0; i < copies.size(); ++i) {
+        for (size_t i = 0; i < copies.size() && ok; ++i) {
             copies[i]->dptr = block + at;
             at += (copies[i]->bytes + 255) / 256 * 256;
-            SLAI_HIP_TRY(ctx, launch_rows_to_tiles(ctx->stream, sources[i], copies[i]));
+            ok = launch_rows_to_tiles(ctx->stream, sources[i], copies[i]) == hipSuccess;
         }
-        return SLAI_OK;
+        return ok;
     }
     void drop() {
         for (slai_qmat *c : copies) delete c;
@@ -310,7 +314,7 @@ struct slai_llama2 {
     struct WideLayer { slai_qmat *q, *k, *v, *o, *gate, *up, *down; };
     std::vector<WideLayer> wide_layers;  // empty: the model has no wide pass (kernels_prompt_wide.hip)
     WideMats wide_mats;
-    int wide_setup();
+    void wide_setup();
     int enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev);   // n <= wide::MAX_TOKENS, activations as f16 pairs
     // q / k / v given as nparts partial sums, 32 rows apart; out_quads: the result goes to xn, quad-major, instead of xb
     int chunk_attention(uint32_t l, uint32_t pos0, uint32_t n, uint32_t nparts = 1, bool out_quads = false, int *split_flag = nullptr);
@@ -455,7 +459,7 @@ int slai_llama2::load(const slai_gguf *gg) {
     TRY(ensure_attn_scratch(ctx, attention_scratch_floats(config.n_q_heads, head_size(), attn_splits)));
     TRY(loop_init(ctx, loop, config.seq_len + 1));
     TRY(persistent_setup());
-    TRY(wide_setup());
+    wide_setup();
     // (said only to a caller who asked for the form by name: most models simply have other shapes)
     const char *asked = getenv("SLAI_PERSISTENT");
     if (asked && ctx->persistent && !persistent.ready)
@@ -992,23 +996,21 @@ int slai_llama2::enqueue_chunk_gemm(uint32_t pos0, uint32_t n, const int *tokens
     return SLAI_OK;
 }
 
-int slai_llama2::wide_setup() {
+void slai_llama2::wide_setup() {
     const uint32_t hs = head_size();
-    if ((hs != 48 && hs != 64 && hs != 128) || kv_dim() % 8 || config.dim > 16384 || !ctx->prompt_gemm) return SLAI_OK;
+    if ((hs != 48 && hs != 64 && hs != 128) || kv_dim() % 8 || config.dim > 16384 || !ctx->prompt_gemm) return;
     std::vector<WideLayer> layers;
     bool ok = true;
     for (const Llama2LayerWeights &w : weights.layers) {
-        const WideLayer l{wide_mats.take(w.attn_q), wide_mats.take(w.attn_k), wide_mats.take(w.attn_v), wide_mats.take(w.attn_output), wide_mats.take(w.ffn_gate),
-                          wide_mats.take(w.ffn_up), wide_mats.take(w.ffn_down)};
+        const auto take = [&](slai_qmat *m) { return wide_mats.take(ctx, m); };
+        const WideLayer l{take(w.attn_q), take(w.attn_k), take(w.attn_v), take(w.attn_output), take(w.ffn_gate), take(w.ffn_up), take(w.ffn_down)};
         for (const slai_qmat *m : {l.q, l.k, l.v, l.o, l.gate, l.up, l.down}) ok = ok && m && m->wbound < 255.0f;
         if (!ok) break;
         ok = l.gate->type == l.up->type && l.gate->rows_log2 == l.up->rows_log2 && !(hs == 48 && (l.o->type == T_Q4_K || l.o->type == T_Q5_K));
         layers.push_back(l);
     }
-    if (!ok) { wide_mats.drop(); return SLAI_OK; }
-    TRY(wide_mats.make(ctx));
-    wide_layers = std::move(layers);
-    return SLAI_OK;
+    if (ok && wide_mats.make(ctx)) wide_layers = std::move(layers);
+    else wide_mats.drop();
 }
 
 // The layer loop (transformer.rs:316-381) for up to 1024 tokens at once: per layer the residual brought up to date and its

@@ -88,6 +88,7 @@ SLAI_EXPORT int slai_ctx_create(int device, slai_ctx **out) {
     }
     ctx->gemv_max_wgs = env_int("SLAI_GEMV_MAX_WGS", 512);
     ctx->tiled_layout = env_int("SLAI_TILED", 1) != 0;
+    ctx->prompt_copy_bytes = (size_t)std::max(0, env_int("SLAI_PROMPT_COPY_MB", 1024)) << 20;
     ctx->rowtile_gemv = env_int("SLAI_ROWTILE", 1) != 0;
     ctx->fuse_qkv_attention = env_int("SLAI_FUSE_QKV_ATTN", 1) != 0;
     ctx->persistent = env_int("SLAI_PERSISTENT", 1) != 0;

@@ -93,3 +93,24 @@ def test_wide_rows_that_are_no_multiple_of_256(backend, n, kv_f16, wtype, hidden
     """Rows of 288 and heads of 48: the pass reads padded copies in tiles (the model's own matrices keep the row layout)."""
     data = gw.tiny_llama_gguf(seed=99, std=0.1, norm_random=True, vocab=4096, wtype=wtype, hidden_dim=hidden)
     check_prefill(backend, data, prompt_of(n, 4096), 8, [0], kv_f16, expect_path=0)
+
+
+@pytest.mark.parametrize("setting,copies", [(None, True), (("SLAI_TILED", "0"), False), (("SLAI_PROMPT_COPY_MB", "1"), False)], ids=["default", "rows asked for", "too little memory allowed"])
+def test_padded_copies_are_bounded(monkeypatch, setting, copies):
+    """Padded copies (6 MB here) are made only where tiles are allowed and within the bound; without them the prompt goes
+    through the token loop, to the bit."""
+    from slai_amd.runtime import Backend, Gguf, Llama2
+    from test_gpu_prefill import read_cache
+    if setting:
+        monkeypatch.setenv(*setting)
+    b = Backend(0)
+    gg = Gguf(gw.tiny_llama_gguf(seed=99, std=0.1, norm_random=True, vocab=4096))
+    prompt = prompt_of(41, 4096).astype(np.int32)
+    caches = []
+    for loop in (True, False):
+        m = Llama2(b, gg, _ffi.MODEL_LLAMA, _ffi.KV_F32)
+        m.generate(prompt, 40) if loop else m.prefill(prompt[:40])
+        caches.append(np.concatenate([a for l in range(6) for a in read_cache(b, m, l, 40 * 288 * 4)]))
+        m.destroy()
+    gg.close(); b.close()
+    assert np.array_equal(*caches) == (not copies)
