@@ -7,6 +7,7 @@
 #include <utility>
 #include <vector>
 
+#include "once_per_device.h"
 #include "slai_hip.h"
 
 #define SLAI_EXPORT extern "C" __attribute__((visibility("default")))
@@ -102,6 +103,13 @@ namespace slai {
 
 int set_error(slai_ctx *ctx, int code, const std::string &msg);
 int hip_fail(slai_ctx *ctx, hipError_t e, const char *what);
+
+// The limit of a kernel's dynamic LDS on the current device (`once`: one object per kernel)
+inline hipError_t allow_lds(const void *kernel, uint32_t bytes, OncePerDevice &once) {
+    int device = 0;
+    if (const hipError_t e = hipGetDevice(&device)) return e;
+    return once(device, [&] { return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes); });
+}
 
 #define SLAI_HIP_TRY(ctx, call)                                         \
     do {                                                                \
