@@ -282,17 +282,20 @@ struct WideGemmParams {
     uint32_t ksplit = 1;          // WIDE_ROWS: the columns in ranges of whole super-blocks, each its own workgroups and result
     uint8_t *pairs_out = nullptr; // WIDE_GATED, WIDE_GELU: super-blocks per token out_ncb
     uint32_t out_ncb = 0;
+    bool out_sums = false;        // their sums of 32 too
     int *flag = nullptr;          // set when an output is beyond f16
     uint32_t token_blocks = 0, row_units = 0, out_c8 = 0;   // filled by the launcher
 };
 bool wide_gemm_supports(const slai_qmat *m);
+bool wide_reads_sums(const slai_qmat *m);   // whether its input needs the sums of 32 (offsets per sub-block)
 // Form and number of column ranges for nseg matrices over one input (splits: ranges are possible, WIDE_ROWS)
 struct WidePlan { bool large; uint32_t ksplit; };
 WidePlan wide_plan(const uint32_t *nrows, int nseg, uint32_t ntokens, uint32_t ncb, bool splits);
 hipError_t launch_wide_gemm(hipStream_t st, WideGemmParams p, int mode);
-// x += its nparts partial results (parts + s * part_stride, rows of n), then RMSNorm (b null) or LayerNorm as pairs
+// x += its nparts partial results (parts + s * part_stride, rows of n), then RMSNorm (b null) or LayerNorm as pairs (with
+// `sums` also their sums of 32)
 hipError_t launch_norm_pairs(hipStream_t st, uint8_t *out, float *x, const float *parts, uint32_t nparts, uint32_t part_stride, const float *w, const float *b, uint32_t n,
-                             uint32_t ntokens, float eps, int *flag);
+                             uint32_t ntokens, float eps, bool sums, int *flag);
 
 // Causal attention of n queries (token i at position pos0 + i, rotated, rows of q_stride floats) over the caches, which
 // already hold their keys and values; the result as pairs (kernels_prompt_attention.hip).  Head sizes 48 (no sums of 32: not
@@ -303,6 +306,7 @@ struct PromptAttention {
     uint32_t q_stride = 0, kv_dim = 0, n_heads = 0, kv_mul = 1, pos0 = 0, n = 0;
     uint8_t *out = nullptr;
     uint32_t out_ncb = 0;
+    bool sums = false;            // the sums of 32 too
     int *flag = nullptr;
 };
 hipError_t launch_prompt_attention(hipStream_t st, const PromptAttention &p, uint32_t head_size, bool kv_f16);

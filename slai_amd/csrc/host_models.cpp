@@ -1039,7 +1039,8 @@ int slai_llama2::enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev) 
         const Llama2LayerWeights &wl = weights.layers[l];
         const WideLayer &wm = wide_layers[l];
         const bool last = l + 1 == config.n_layers;
-        SLAI_HIP_TRY(ctx, launch_norm_pairs(ctx->stream, pairs, x, parts, nparts, n * dim, (const float *)wl.attn_norm.buf->dptr, nullptr, dim, n, config.rms_norm_eps, flag));
+        SLAI_HIP_TRY(ctx, launch_norm_pairs(ctx->stream, pairs, x, parts, nparts, n * dim, (const float *)wl.attn_norm.buf->dptr, nullptr, dim, n, config.rms_norm_eps,
+                                             wide_reads_sums(wm.q) || wide_reads_sums(wm.k) || wide_reads_sums(wm.v), flag));
         const WideGemmSeg qkv[3] = {wide_seg(wm.v, v, kvd, n * kvd), wide_seg(wm.k, k, kvd, n * kvd), wide_seg(wm.q, q, dim, n * dim)};
         TRY(wide_rows(ctx, last ? 2 : 3, qkv, pairs, ncb, n, p_qkv, "llama2 qkv (prompt)"));
         AttnLaunch a{};
@@ -1054,14 +1055,15 @@ int slai_llama2::enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev) 
         if (last) break;
         PromptAttention pa;
         pa.q = q; pa.q_stride = dim; pa.kcache = a.kcache; pa.vcache = a.vcache; pa.kv_dim = kvd; pa.n_heads = a.n_heads; pa.kv_mul = a.kv_mul;
-        pa.pos0 = pos0; pa.n = n; pa.out = pairs; pa.out_ncb = ncb; pa.flag = flag;
+        pa.pos0 = pos0; pa.n = n; pa.out = pairs; pa.out_ncb = ncb; pa.sums = wide_reads_sums(wm.o); pa.flag = flag;
         SLAI_HIP_TRY(ctx, launch_prompt_attention(ctx->stream, pa, hs, a.kv_f16 != 0));
         const WideGemmSeg o = wide_seg(wm.o, parts, dim, n * dim);
         TRY(wide_rows(ctx, 1, &o, pairs, ncb, n, p_o, "llama2 attn_output (prompt)"));
-        SLAI_HIP_TRY(ctx, launch_norm_pairs(ctx->stream, pairs, x, parts, ks_o, n * dim, (const float *)wl.ffn_norm.buf->dptr, nullptr, dim, n, config.rms_norm_eps, flag));
+        SLAI_HIP_TRY(ctx, launch_norm_pairs(ctx->stream, pairs, x, parts, ks_o, n * dim, (const float *)wl.ffn_norm.buf->dptr, nullptr, dim, n, config.rms_norm_eps,
+                                             wide_reads_sums(wm.gate), flag));
         WideGemmParams g;
         g.nseg = 2; g.seg[0] = wide_seg(wm.gate, nullptr, 0, 0); g.seg[1] = wide_seg(wm.up, nullptr, 0, 0);
-        g.x = pairs; g.ncb = ncb; g.ntokens = n; g.pairs_out = hidden; g.out_ncb = hcb; g.flag = flag; g.large = wide_plan(r_ffn, 2, n, ncb, false).large;
+        g.x = pairs; g.ncb = ncb; g.ntokens = n; g.pairs_out = hidden; g.out_ncb = hcb; g.out_sums = wide_reads_sums(wm.down); g.flag = flag; g.large = wide_plan(r_ffn, 2, n, ncb, false).large;
         TRY(wide_call(ctx, g, WIDE_GATED, "llama2 ffn gate/up (prompt)"));
         const WideGemmSeg d = wide_seg(wm.down, parts, dim, n * dim);
         TRY(wide_rows(ctx, 1, &d, hidden, hcb, n, p_d, "llama2 ffn_down (prompt)"));
@@ -1723,7 +1725,8 @@ int slai_gpt2::enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev) {
     for (uint32_t l = 0; l < params.n_layer; ++l) {
         Gpt2Layer &w = layers[l];
         const bool last = l + 1 == params.n_layer;
-        SLAI_HIP_TRY(ctx, launch_norm_pairs(ctx->stream, pairs, x, parts, nparts, n * E, (const float *)w.ln_1_g.buf->dptr, (const float *)w.ln_1_b.buf->dptr, E, n, eps, flag));
+        SLAI_HIP_TRY(ctx, launch_norm_pairs(ctx->stream, pairs, x, parts, nparts, n * E, (const float *)w.ln_1_g.buf->dptr, (const float *)w.ln_1_b.buf->dptr, E, n, eps,
+                                             wide_reads_sums(w.c_attn_attn_w), flag));
         const WideGemmSeg sq = wide_seg(w.c_attn_attn_w, qkv, 3 * E, n * 3 * E, &w.c_attn_attn_b);
         TRY(wide_rows(ctx, 1, &sq, pairs, ncb, n, p_qkv, "gpt2 qkv (prompt)"));
         AttnLaunch a{};
@@ -1735,14 +1738,15 @@ int slai_gpt2::enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev) {
         if (last) break;
         PromptAttention pa;
         pa.q = qkv; pa.q_stride = 3 * E; pa.kcache = a.kcache; pa.vcache = a.vcache; pa.kv_dim = E; pa.n_heads = params.n_head; pa.kv_mul = 1;
-        pa.pos0 = pos0; pa.n = n; pa.out = pairs; pa.out_ncb = ncb; pa.flag = flag;
+        pa.pos0 = pos0; pa.n = n; pa.out = pairs; pa.out_ncb = ncb; pa.sums = wide_reads_sums(w.c_attn_proj_w); pa.flag = flag;
         SLAI_HIP_TRY(ctx, launch_prompt_attention(ctx->stream, pa, hs, a.kv_f16 != 0));
         const WideGemmSeg so = wide_seg(w.c_attn_proj_w, parts, E, n * E, &w.c_attn_proj_b);
         TRY(wide_rows(ctx, 1, &so, pairs, ncb, n, p_o, "gpt2 attn proj (prompt)"));
-        SLAI_HIP_TRY(ctx, launch_norm_pairs(ctx->stream, pairs, x, parts, ks_o, n * E, (const float *)w.ln_2_g.buf->dptr, (const float *)w.ln_2_b.buf->dptr, E, n, eps, flag));
+        SLAI_HIP_TRY(ctx, launch_norm_pairs(ctx->stream, pairs, x, parts, ks_o, n * E, (const float *)w.ln_2_g.buf->dptr, (const float *)w.ln_2_b.buf->dptr, E, n, eps,
+                                             wide_reads_sums(w.c_mlp_fc_w), flag));
         WideGemmParams g;
         g.nseg = 1; g.seg[0] = wide_seg(w.c_mlp_fc_w, nullptr, 0, 0, &w.c_mlp_fc_b);
-        g.x = pairs; g.ncb = ncb; g.ntokens = n; g.pairs_out = hidden; g.out_ncb = fcb; g.flag = flag; g.large = wide_plan(&F, 1, n, ncb, false).large;
+        g.x = pairs; g.ncb = ncb; g.ntokens = n; g.pairs_out = hidden; g.out_ncb = fcb; g.out_sums = wide_reads_sums(w.c_mlp_proj_w); g.flag = flag; g.large = wide_plan(&F, 1, n, ncb, false).large;
         TRY(wide_call(ctx, g, WIDE_GELU, "gpt2 mlp fc (prompt)"));
         const WideGemmSeg sd = wide_seg(w.c_mlp_proj_w, parts, E, n * E, &w.c_mlp_proj_b);
         TRY(wide_rows(ctx, 1, &sd, hidden, fcb, n, p_d, "gpt2 mlp proj (prompt)"));

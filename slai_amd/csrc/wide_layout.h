@@ -4,8 +4,8 @@
 // Tokens in tiles of 32, columns in super-blocks of 256 of sixteen chunks.  Chunk c of super-block cb of token tile tt is
 // 2048 bytes: [head | 2^11 remainder][columns 0-7 | 8-15 of the chunk][32 tokens][8 columns, in the order 0, 2, 1, 3, 4, 6, 5, 7],
 // so that a lane (token = lane % 32, half = lane / 32) finds its operand at lane * 16.  Behind the sixteen chunks lie the sums of
-// 32 consecutive activations as their pairs hold them, which the formats with an offset per sub-block multiply with their mins:
-// [head | 2^11 remainder][32 tokens][8 sub-blocks, same order], 1024 bytes.
+// 32 consecutive activations as their pairs hold them, which the formats with an offset per sub-block multiply with their mins, divided
+// by 32 (written only where such a format reads them): [head | 2^11 remainder][32 tokens][8 sub-blocks, same order], 1024 bytes.
 #pragma once
 #include <stdint.h>
 

@@ -150,3 +150,24 @@ def test_error_of_sharp_attention(backend, oracle_lib, shape, kv_f16):
         m = Model(oracle_lib, "attention", Q8_0, *SHAPES[shape], 1.0, also=hook)
         keys, _, second = errors(backend, m, kv_f16)
         assert second < (6e-4 if kv_f16 else 2 * BAR[1]), (up, keys, second)
+
+
+@pytest.mark.parametrize("wtype,block", [(Q8_0, 34), (Q4_K, 144)], ids=["q8_0", "q4_k"])
+def test_aligned_activations_are_read_once(backend, oracle_lib, wtype, block):
+    """Normalised rows of about 3000 of one sign: each fits f16, the sum of 32 does not.  Such a prompt needs no fp32 repeat
+    (`errors` looks), whether the format reads the sums or not."""
+    def hook(name, dims, t, data):
+        if name.startswith("token_embd"):
+            data = (1 + 0.1 * np.random.Generator(np.random.PCG64(1)).standard_normal(data.size // 4)).astype(np.float32).view(np.uint8)
+        if name in ("blk.0.ffn_gate.weight", "blk.0.ffn_up.weight"):        # hidden values of about 5
+            data = data.copy().reshape(-1, block)
+            scales = 2 if t == Q8_0 else 4
+            data[:, :scales] = (data[:, :scales].copy().view(np.float16) * np.float16(2.0 ** -10)).view(np.uint8)
+            data = data.reshape(-1)
+        return dims, t, data
+
+    m = Model(oracle_lib, "ffn", wtype, *SHAPES["heads of 128"], 3000.0, also=hook)
+    _, first, second = errors(backend, m)
+    # (Q4_K: the sums of m and of sc over activations of one sign are 26 times the result they leave)
+    up = 1 if wtype == Q8_0 else 26
+    assert first < up * BAR[0] and second < up * BAR[1], (first, second)
