@@ -168,6 +168,6 @@ def test_aligned_activations_are_read_once(backend, oracle_lib, wtype, block):
 
     m = Model(oracle_lib, "ffn", wtype, *SHAPES["heads of 128"], 3000.0, also=hook)
     _, first, second = errors(backend, m)
-    # (Q4_K: the sums of m and of sc over activations of one sign are 26 times the result they leave)
-    up = 1 if wtype == Q8_0 else 26
-    assert first < up * BAR[0] and second < up * BAR[1], (first, second)
+    # Q4_K multiplies q - 8, on average half a step below zero: over 256 activations of one sign its partial sums reach 0.5 * 256
+    # steps against a result of sqrt(256) * 4.6, 1.7 times as much, and round accordingly
+    assert first < 2 * BAR[0] and second < 2 * BAR[1], (first, second)
