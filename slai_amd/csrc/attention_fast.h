@@ -270,6 +270,10 @@ __device__ __forceinline__ void attn_fast_body(const AttnLaunch &a, uint32_t h, 
             const float pw = __shfl(pr, KL * (u * PW + vgl), 64);      // 0 for positions past the end
             float vv[8];
             Vec8<F16>::decode(vv0[u], vv);
+            if (own_new && t0 == pos) {                        // (uniform) lanes without a position had no row but the one being written: a NaN it held would survive the factor 0
+#pragma unroll
+                for (int q = 0; q < 8; ++q) vv[q] = 0.0f;
+            }
             if (own_new && tv == pos) {
 #pragma unroll
                 for (int q = 0; q < 8; ++q) vv[q] = sv[ve + q];

@@ -316,3 +316,36 @@ def test_time_steps_names_every_launch_of_a_token(backend):
     assert all(s[1] > 0.0 and s[3] > 0.0 for s in steps), steps
     assert np.array_equal(m.forward_logits(8, int(toks[7])), ref)
     m.destroy(); g.close()
+
+
+@pytest.mark.parametrize("kv_f16", [False, True])
+@pytest.mark.parametrize("heads", [48, 64, 128, "resident", "gpt2"])
+def test_what_the_caches_held_before_does_not_matter(backend, heads, kv_f16):
+    """A conversation that starts over writes over caches that may hold anything, NaN included (a pass whose values were beyond
+    f16 leaves them): rows at and behind the current position must not be looked at."""
+    from slai_amd.runtime import Gguf, Gpt2, Llama2
+    kv = _ffi.KV_F16 if kv_f16 else _ffi.KV_F32
+    if heads == "gpt2":
+        data = gw.gpt2_gguf(n_layer=2, seed=61, std=0.05, vocab=1000, n_seq=64)
+    elif heads == 48:
+        data = gw.tiny_llama_gguf(seed=61, std=0.1, vocab=1000, seq_len=64)
+    elif heads == "resident":                                  # the whole token in one launch: width 1024, heads of 128, no grouped queries
+        data = gw.llama_gguf(dim=1024, hidden_dim=2816, n_layers=2, n_heads=8, n_kv_heads=8, vocab=1000, seq_len=64, wtype=12, seed=61, std=0.05)
+    else:
+        data = gw.llama_gguf(dim=512, hidden_dim=1024, n_layers=2, n_heads=512 // heads, n_kv_heads=256 // heads, vocab=1000, seq_len=64, wtype=12, seed=61, std=0.05)
+    gg = Gguf(data)
+    prompt = np.array([5, 6, 7], np.int32)
+    got = []
+    for stale in (False, True):
+        m = Gpt2(backend, gg, kv) if heads == "gpt2" else Llama2(backend, gg, _ffi.MODEL_LLAMA, kv)
+        if stale and heads == "gpt2":                          # (its caches are not shown: a first answer with values beyond them)
+            m.generate(prompt, 40)
+        elif stale:
+            nan = np.full(m.config.seq_len * m.config.dim // m.config.n_q_heads * m.config.n_kv_heads, np.nan, np.float16 if kv_f16 else np.float32)
+            for layer in range(m.config.n_layers):
+                for b in m.kv_buffers(layer):
+                    backend.check(backend.L.slai_write_buffer(backend.h, b, 0, nan.ctypes.data, nan.nbytes))
+        got.append((m.generate(prompt, 20)[0], m.forward_logits(20, 3)))
+        m.destroy()
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
+    gg.close()

@@ -114,3 +114,32 @@ def test_padded_copies_are_bounded(monkeypatch, setting, copies):
         m.destroy()
     gg.close(); b.close()
     assert np.array_equal(*caches) == (not copies)
+
+
+@pytest.mark.parametrize("scale,repeats", [(1.0, 0), (5.0e4, 1)])
+def test_wide_padded_copies_repeat_in_the_token_loop(backend, scale, repeats):
+    """Values beyond f16 in a model whose pass reads padded copies: the repeat is the token loop, whose caches it leaves."""
+    data = gw.tiny_llama_gguf(seed=98, std=0.1, norm_random=True, vocab=4096, ffn_norm_scale=scale)
+    check_prefill(backend, data, prompt_of(50, 4096), 8, [0], False, expect_path=0, expect_repeats=repeats)
+
+
+@pytest.mark.parametrize("scale,repeats", [(1.0, 0), (5.0e4, 1)])
+def test_wide_gpt2_values_beyond_f16_repeat_in_fp32(backend, scale, repeats):
+    from helpers import OracleGguf
+    from slai_amd.runtime import Gguf, Gpt2
+    data = gw.gpt2_gguf(n_layer=2, seed=53, std=0.05, vocab=2000, n_seq=256, ffn_norm_scale=scale)
+    g = OracleGguf(data); L = g.L
+    om = L.slo_gpt2_from_gguf(g.h, 0)
+    n, n_gen = 70, 6
+    prompt = prompt_of(n, 2000, 54).astype(np.int32)
+    steps = n - 1 + n_gen
+    ref, ref_logits = np.zeros(steps, np.int32), np.zeros((steps, 2000), np.float32)
+    assert L.slo_gpt2_generate(om, prompt.ctypes.data, n, 0, steps, -1, ref.ctypes.data, ref_logits.ctypes.data) == steps
+    gg = Gguf(data)
+    m = Gpt2(backend, gg, _ffi.KV_F32)
+    assert m.prefill(prompt[:-1], 0) > 0
+    assert m.prefill_fp32_repeats() == repeats
+    assert rel_err(m.forward_logits(n - 1, int(prompt[-1])), ref_logits[n - 1]) < 1e-2
+    got, _ = m.generate(prompt, n_gen, start_pos=n - 1)
+    assert np.array_equal(got, ref[n - 1:])
+    m.destroy(); gg.close(); L.slo_gpt2_free(om); g.close()
