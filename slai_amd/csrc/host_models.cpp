@@ -1389,7 +1389,13 @@ SLAI_EXPORT int slai_llama2_prefill(slai_llama2 *m, const int32_t *tokens, uint3
         if (!beyond) break;
         ++m->prefill_fp32_repeats;
         split = false;
-        if (!gemm) return one_by_one();
+        if (!gemm) {                                           // (the time of the pass that is repeated counts too)
+            float first = 0.0f;
+            SLAI_HIP_TRY(ctx, hipEventElapsedTime(&first, m->loop.ev0, m->loop.ev1));
+            const int rc = one_by_one();
+            if (elapsed_ms) *elapsed_ms += first;
+            return rc;
+        }
         TRY(m->chunk_reserve(chunk));
     }
     if (elapsed_ms) SLAI_HIP_TRY(ctx, hipEventElapsedTime(elapsed_ms, m->loop.ev0, m->loop.ev1));
