@@ -68,7 +68,7 @@ struct slai_ctx {
     // per-workgroup activation slots of the row-tile GEMV (grown on demand, never inside a capture)
     float *gemv_scratch = nullptr;
     size_t gemv_scratch_floats = 0;
-    float *sampler_scratch = nullptr;   // probabilities of the device sampler (one float per vocabulary entry)
+    float *sampler_scratch = nullptr;   // of the device sampler: sample_scratch_floats (about three floats per vocabulary entry)
     size_t sampler_scratch_floats = 0;
     uint32_t *handoff_counters = nullptr;   // q/k/v + attention in one launch: one 128-byte line per head, then a timeout flag
     uint32_t handoff_heads = 0;
@@ -405,7 +405,9 @@ hipError_t launch_argmax(hipStream_t s, const float *v, uint32_t n, int *out_ind
 // `scratch`: sample_scratch_floats(n) floats of device memory, or at least sample_scratch_least(n): then one slower launch
 size_t sample_scratch_floats(uint32_t n);
 size_t sample_scratch_least(uint32_t n);
-hipError_t launch_sample(hipStream_t s, const float *v, uint32_t n, float temperature, float topp, float coin, float *scratch, size_t scratch_floats, int *out_index,
+// `scan`: sample_scans() of the temperature and top-p that the pick will have
+bool sample_scans(float temperature, float topp);
+hipError_t launch_sample(hipStream_t s, const float *v, uint32_t n, float temperature, float topp, float coin, float *scratch, size_t scratch_floats, bool scan, int *out_index,
                          DecodeState *decode, const int *prompt, int *out_tokens);
 
 // ---- attention ---------------------------------------------------------------------

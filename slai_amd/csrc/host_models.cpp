@@ -108,7 +108,7 @@ struct DeviceLoop {           // device-resident state of the greedy loop
     slai_buffer *prompt = nullptr;      // int32[capacity]
     slai_buffer *out_tokens = nullptr;  // int32[capacity]
     uint32_t capacity = 0;
-    slai_graph *graph[3][2] = {{nullptr, nullptr}, {nullptr, nullptr}, {nullptr, nullptr}};   // one token, [launch form][greedy pick | temperature / top-p pick]
+    slai_graph *graph[3][3] = {};       // one token, [launch form][greedy | temperature and top-p | plain temperature pick]
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
 };
 int loop_init(slai_ctx *ctx, DeviceLoop &L, uint32_t capacity) {
@@ -285,7 +285,7 @@ struct slai_llama2 {
 
     int load(const slai_gguf *g);
     int launch(LlmContext &ctxt, const slai_attn_params &attn_params, uint32_t pos);   // transformer.rs:316-381
-    int enqueue_fused(int sampler, int form = 0);   // sampler 0: stop at the logits, 1: greedy pick + loop state, 2: temperature / top-p pick + loop state; form 1: the resident launch
+    int enqueue_fused(int sampler, int form = 0);   // sampler 0: stop at the logits, 1: greedy pick + loop state, 2: temperature / top-p pick + loop state, 3: the same without a top-p cut; form 1: the resident launch
     int form_at(uint32_t pos) const;               // the launch form of the token at `pos`
 
     // The layer stack as ONE resident launch per token (kernels_decode_persistent.hip), for the models it covers.
@@ -562,8 +562,8 @@ int slai_llama2::enqueue_persistent(int sampler, bool far) {
     if (sampler == 1)
         SLAI_HIP_TRY(ctx, launch_argmax(ctx->stream, (const float *)s.logits.buf->dptr, config.vocab_size, nullptr, ds,
                                         (const int *)loop.prompt->dptr, (int *)loop.out_tokens->dptr));
-    else if (sampler == 2)
-        SLAI_HIP_TRY(ctx, launch_sample(ctx->stream, (const float *)s.logits.buf->dptr, config.vocab_size, 0.0f, 0.0f, 0.0f, ctx->sampler_scratch, ctx->sampler_scratch_floats, nullptr, ds,
+    else if (sampler)
+        SLAI_HIP_TRY(ctx, launch_sample(ctx->stream, (const float *)s.logits.buf->dptr, config.vocab_size, 0.0f, 0.0f, 0.0f, ctx->sampler_scratch, ctx->sampler_scratch_floats, sampler == 2, nullptr, ds,
                                         (const int *)loop.prompt->dptr, (int *)loop.out_tokens->dptr));
     return SLAI_OK;
 }
@@ -755,8 +755,8 @@ int slai_llama2::enqueue_fused(int sampler, int form) {
     if (sampler == 1)
         SLAI_HIP_TRY(ctx, launch_argmax(ctx->stream, (const float *)s.logits.buf->dptr, config.vocab_size, nullptr, ds,
                                         (const int *)loop.prompt->dptr, (int *)loop.out_tokens->dptr));
-    else if (sampler == 2)
-        SLAI_HIP_TRY(ctx, launch_sample(ctx->stream, (const float *)s.logits.buf->dptr, config.vocab_size, 0.0f, 0.0f, 0.0f, ctx->sampler_scratch, ctx->sampler_scratch_floats, nullptr, ds,
+    else if (sampler)
+        SLAI_HIP_TRY(ctx, launch_sample(ctx->stream, (const float *)s.logits.buf->dptr, config.vocab_size, 0.0f, 0.0f, 0.0f, ctx->sampler_scratch, ctx->sampler_scratch_floats, sampler == 2, nullptr, ds,
                                         (const int *)loop.prompt->dptr, (int *)loop.out_tokens->dptr));
     return SLAI_OK;
 }
@@ -1268,7 +1268,7 @@ template <class Model>
 static int generate_impl(Model *m, slai_ctx *ctx, DeviceLoop &L, uint32_t seq_len, uint32_t vocab, const int32_t *prompt, uint32_t n_prompt,
                          uint32_t start_pos, uint32_t n_steps, int32_t *out_tokens, float *elapsed_ms, const SamplingParams *sampling = nullptr) {
     if (sampling && !(sampling->temperature >= 0.0f)) return set_error(ctx, SLAI_E_ARG, "generate: the temperature must not be negative");
-    const int mode = sampling ? 2 : 1;
+    const int mode = !sampling ? 1 : sample_scans(sampling->temperature, sampling->topp) ? 2 : 3;
     if (sampling) TRY(sampler_scratch_reserve(ctx, sample_scratch_floats(vocab)));
     if (!prompt || !out_tokens || n_prompt == 0 || start_pos >= n_prompt) return set_error(ctx, SLAI_E_ARG, "generate: bad prompt / start position");
     if (n_steps == 0) return SLAI_OK;
@@ -1291,7 +1291,7 @@ static int generate_impl(Model *m, slai_ctx *ctx, DeviceLoop &L, uint32_t seq_le
     }
     // one captured token per launch form the run needs (the form depends on the position: Model::form_at)
     for (uint32_t i = 0; i < n_steps; ++i) {
-        slai_graph *&graph = L.graph[m->form_at(start_pos + i)][sampling ? 1 : 0];
+        slai_graph *&graph = L.graph[m->form_at(start_pos + i)][mode - 1];
         if (graph) continue;
         TRY(slai_graph_begin_capture(ctx));
         int rc = m->enqueue_fused(mode, m->form_at(start_pos + i));
@@ -1302,7 +1302,7 @@ static int generate_impl(Model *m, slai_ctx *ctx, DeviceLoop &L, uint32_t seq_le
         graph = g;
     }
     SLAI_HIP_TRY(ctx, hipEventRecord(L.ev0, ctx->stream));
-    for (uint32_t i = 0; i < n_steps; ++i) TRY(slai_graph_launch(ctx, L.graph[m->form_at(start_pos + i)][sampling ? 1 : 0]));   // chat_llama2.rs:109 loop
+    for (uint32_t i = 0; i < n_steps; ++i) TRY(slai_graph_launch(ctx, L.graph[m->form_at(start_pos + i)][mode - 1]));   // chat_llama2.rs:109 loop
     SLAI_HIP_TRY(ctx, hipEventRecord(L.ev1, ctx->stream));
     TRY(slai_synchronize(ctx));
     TRY(handoff_check(ctx));
@@ -1441,7 +1441,7 @@ struct slai_gpt2 {
     uint32_t attn_splits = 1;
 
     int load(const slai_gguf *g);
-    int enqueue_fused(int sampler, int form = 0);   // 0: stop at the logits, 1: greedy pick + loop state, 2: temperature / top-p pick + loop state (one form only)
+    int enqueue_fused(int sampler, int form = 0);   // 0: stop at the logits, 1: greedy pick + loop state, 2: temperature / top-p pick + loop state, 3: the same without a top-p cut (one form only)
     int form_at(uint32_t) const { return 0; }
 
     // Prompt tokens in chunks of up to 32 on the matrix cores (see slai_llama2::enqueue_chunk_gemm); row-major x and qkv,
@@ -1621,8 +1621,8 @@ int slai_gpt2::enqueue_fused(int sampler, int) {
     }
     if (sampler == 1)
         SLAI_HIP_TRY(ctx, launch_argmax(ctx->stream, logits, params.n_vocab, nullptr, ds, (const int *)loop.prompt->dptr, (int *)loop.out_tokens->dptr));
-    else if (sampler == 2)
-        SLAI_HIP_TRY(ctx, launch_sample(ctx->stream, logits, params.n_vocab, 0.0f, 0.0f, 0.0f, ctx->sampler_scratch, ctx->sampler_scratch_floats, nullptr, ds, (const int *)loop.prompt->dptr,
+    else if (sampler)
+        SLAI_HIP_TRY(ctx, launch_sample(ctx->stream, logits, params.n_vocab, 0.0f, 0.0f, 0.0f, ctx->sampler_scratch, ctx->sampler_scratch_floats, sampler == 2, nullptr, ds, (const int *)loop.prompt->dptr,
                                         (int *)loop.out_tokens->dptr));
     return SLAI_OK;
 }

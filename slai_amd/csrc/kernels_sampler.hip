@@ -667,6 +667,8 @@ picked:
 
 // Vocabularies that take the scan first: a single compute unit reads 32000 entries slowly enough for two launches to win
 // (n = 32000: 33 -> 20.5 us with both launches, 50257: 51 -> 22, 152064: 110 -> 26); a few thousand it takes in one.
+// Plain sampling (no top-p cut) needs every entry and takes the one launch at any size.
+bool sample_scans(float temperature, float topp) { return temperature == 0.0f || (topp > 0.0f && topp < 1.0f); }
 static bool scanned(uint32_t n) { return n > 4 * SCAN && scan_slices(n) <= SCAN_SLICES; }
 
 // floats of scratch a launch over n logits needs at least: above 32768 the probabilities and the packed candidates
@@ -681,10 +683,10 @@ size_t sample_scratch_floats(uint32_t n) {
     return least > scan ? least : scan;
 }
 
-hipError_t launch_sample(hipStream_t s, const float *v, uint32_t n, float temperature, float topp, float coin, float *scratch, size_t scratch_floats, int *out_index,
+hipError_t launch_sample(hipStream_t s, const float *v, uint32_t n, float temperature, float topp, float coin, float *scratch, size_t scratch_floats, bool scan, int *out_index,
                          DecodeState *decode, const int *prompt, int *out_tokens) {
     const bool small = n <= NW * 64 * 32;
-    if (scanned(n) && scratch_floats >= sample_scratch_floats(n)) {
+    if (scan && scanned(n) && scratch_floats >= sample_scratch_floats(n)) {
         sample_scan_kernel<<<scan_slices(n), SCAN_NT, 0, s>>>(v, n, temperature, topp, scratch, decode);
         if (small) sample_kernel<32, true><<<1, NT, 0, s>>>(v, n, temperature, topp, coin, scratch, out_index, decode, prompt, out_tokens);
         else sample_kernel<0, true><<<1, NT, 0, s>>>(v, n, temperature, topp, coin, scratch, out_index, decode, prompt, out_tokens);

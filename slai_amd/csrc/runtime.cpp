@@ -908,7 +908,7 @@ SLAI_EXPORT int slai_sample(slai_ctx *ctx, slai_view logits, float temperature, 
     if (!(temperature >= 0.0f) || !(coin >= 0.0f && coin < 1.0f)) return set_error(ctx, SLAI_E_ARG, "slai_sample: temperature must be >= 0 and the draw in [0, 1)");
     // (under capture nothing can grow: the one-launch form needs less)
     if (int rc = sampler_scratch_reserve(ctx, ctx->capturing ? sample_scratch_least(vl.n) : sample_scratch_floats(vl.n))) return rc;
-    SLAI_HIP_TRY(ctx, launch_sample(ctx->stream, vl.p, vl.n, temperature, topp, coin, ctx->sampler_scratch, ctx->sampler_scratch_floats, (int *)out_index->dptr, nullptr, nullptr,
+    SLAI_HIP_TRY(ctx, launch_sample(ctx->stream, vl.p, vl.n, temperature, topp, coin, ctx->sampler_scratch, ctx->sampler_scratch_floats, sample_scans(temperature, topp), (int *)out_index->dptr, nullptr, nullptr,
                                     nullptr));
     return SLAI_OK;
 }

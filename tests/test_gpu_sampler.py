@@ -174,3 +174,23 @@ def test_coin_stream_is_uniform():
     assert coins.min() >= 0.0 and coins.max() < 1.0
     assert abs(coins.mean() - 0.5) < 0.02 and abs(np.mean(coins < 0.25) - 0.25) < 0.03
     assert len(set(coins.tolist())) > 3990
+
+
+def test_generate_sampled_kinds_in_turn(backend):
+    """One model, a vocabulary that is scanned first: a top-p cut, none (its own captured form, without the scan), greedy, in
+    turn; each token is the operator's pick from the same logits."""
+    data = gw.llama_gguf(dim=128, hidden_dim=256, n_layers=1, n_heads=4, n_kv_heads=2, vocab=10240, seq_len=32, wtype=8, seed=78, std=0.3, norm_random=True)
+    gg = Gguf(data)
+    m = Llama2(backend, gg, _ffi.MODEL_LLAMA, _ffi.KV_F32)
+    ctxt, gout = LlmContext(backend), GpuTensor(backend, 1, 1, _ffi.DT_I32)
+    prompt, seed = np.array([5, 100], np.int32), 99
+    for temperature, topp in ((0.7, 0.95), (0.7, 0.0), (0.7, 1.0), (0.0, 1.0), (0.7, 0.95), (1.1, 2.0)):
+        got, _ = m.generate_sampled(prompt, 10, temperature, topp, seed)
+        tok = int(prompt[0])
+        for pos in range(10):
+            g = GpuTensor.vector(backend, m.forward_logits(pos, tok))
+            pick = device_sample(backend, ctxt, g, gout, temperature, topp, sampler_coin(seed, pos))
+            g.destroy()
+            tok = int(prompt[pos + 1]) if pos + 1 < prompt.size else pick
+            assert tok == int(got[pos]), (temperature, topp, pos)
+    m.destroy(); gout.destroy(); gg.close()
