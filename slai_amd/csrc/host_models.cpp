@@ -88,12 +88,15 @@ int check_vector(const Gguf &g, const std::string &name, bool required, uint64_t
 // What every form of the prompt pass needs on the device: room for the token ids and the positions 0, 1, 2, ... (token b of
 // a pass at pos0 reads its position from positions + pos0 + b).
 int prompt_ids_reserve(slai_ctx *ctx, uint32_t seq_len, slai_buffer **positions, slai_buffer **tokens) {
-    if (*positions && *tokens) return SLAI_OK;
-    TRY(slai_buffer_create(ctx, (size_t)seq_len * 4, SLAI_DT_I32, STORAGE | COPY_DST, tokens));
-    TRY(slai_buffer_create(ctx, (size_t)seq_len * 4, SLAI_DT_I32, STORAGE | COPY_DST, positions));
+    if (!*tokens) TRY(slai_buffer_create(ctx, (size_t)seq_len * 4, SLAI_DT_I32, STORAGE | COPY_DST, tokens));
+    if (*positions) return SLAI_OK;                            // (set only once they are written)
+    slai_buffer *b = nullptr;
+    TRY(slai_buffer_create(ctx, (size_t)seq_len * 4, SLAI_DT_I32, STORAGE | COPY_DST, &b));
     std::vector<uint32_t> iota(seq_len);
     for (uint32_t i = 0; i < seq_len; ++i) iota[i] = i;
-    return slai_write_buffer(ctx, *positions, 0, iota.data(), iota.size() * 4);
+    if (const int rc = slai_write_buffer(ctx, b, 0, iota.data(), iota.size() * 4)) { slai_buffer_destroy(ctx, b); return rc; }
+    *positions = b;
+    return SLAI_OK;
 }
 
 // Two matrices over the same input can share a GEMV launch: any formats in 64-row tiles, otherwise one format and layout.
