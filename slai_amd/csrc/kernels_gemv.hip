@@ -345,9 +345,13 @@ template <int T, bool DUAL> hipError_t launch_short(slai_ctx *ctx, GemvParams &p
     const uint32_t k = (nchunks + lanes - 1) / lanes;
     uint32_t waves = 0;
     for (int i = 0; i < p.nseg; ++i) waves += (p.seg[i].nrows + 64 / lanes - 1) / (64 / lanes);
-    // few rows: one wave per workgroup, spread over all compute units; many: four row groups per wave
-    const bool many = waves >= 2048;
-    const uint32_t nt = waves <= 1024 ? 64 : 256, rows = nt / lanes * (many ? 4 : 1);
+    // Few rows: one wave per workgroup, spread over all compute units; from 3072 waves on four row groups per wave, whose x
+    // and norm are then fetched and computed once.  us a launch in a chain, one
+    // group / four, by waves (Q8_0 rows of 288, of 768, Q4_K rows of 512, of 2048): 1024: 2.7 / 4.1, 2.9 / 4.3, 3.3 / 5.9, - ;
+    // 2048: 3.4 / 4.1, 3.6 / 4.3, 5.4 / 5.9, 5.7 / 6.1; 3072: 4.4 / 4.1, 4.6 / 4.3, 7.4 / 6.0, - ; 4096: 5.1 / 4.1, 5.5 / 4.3, 9.4 / 6.0,
+    // 9.9 / 6.2; 16384: 15.8 / 14.2, 16.5 / 15.6, 34.3 / 21.4, 35.4 / 22.2.  One group in workgroups of 256 was never ahead.
+    const bool many = waves >= 3072;
+    const uint32_t nt = many ? 256 : 64, rows = nt / lanes * (many ? 4 : 1);
     uint32_t grid = 0;
     for (int i = 0; i < p.nseg; ++i) grid += p.seg[i].nblocks = (p.seg[i].nrows + rows - 1) / rows;
     hipStream_t st = ctx->stream;

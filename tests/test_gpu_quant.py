@@ -401,7 +401,7 @@ SHORT = {0: (4, 128, 132, 256), 1: (8, 256, 264, 512), 2: (32, 512, 544, 1056, 2
 
 
 @pytest.mark.parametrize("t, ncols", [(t, n) for t, ns in SHORT.items() for n in ns], ids=lambda v: str(v))
-@pytest.mark.parametrize("nrows", [1, 37, 17000])
+@pytest.mark.parametrize("nrows", [1, 37, 17000, 24700])     # (24700: four groups of rows per wave at every width below 600)
 def test_short_rows(backend, oracle_lib, t, ncols, nrows):
     """Rows of few chunks (several per wave): plain, RMSNorm before, gate / up + SiLU and accumulating, against 64 bits."""
     from slai_amd.runtime import GpuQuantMatrix, GpuTensor, LlmContext
