@@ -334,17 +334,20 @@ int slai_llama2_generate_sampled(slai_llama2 *m, const int32_t *prompt, uint32_t
  * prompt position but the last (chat_llama2.rs:105-158 with the forced-token rule, slai-chat/src/sampler.rs:100-105);
  * this fills the caches for positions start_pos .. start_pos+n_tokens-1 with `chunk` tokens per pass over the
  * weights and computes no logits (chunk: 0 = the path's default, 1 = token by token, at most 64).  Generation then
- * continues with slai_llama2_generate(prompt, n_prompt, n_prompt - 1, ...).  slai_llama2_prefill_supported() says which
- * path a model takes: 2 = matrix-core GEMM over the dequantised tiles (every format with a tiled layout), at most
- * 32 tokens per pass: on the half-precision units with every weight and activation split into an f16 head and an f16
- * remainder (about 22 bits of each, fp32 accumulation), repeated with fp32 MFMA when an activation turns out to be beyond
- * the f16 range (slai_llama2_prefill_fp32_repeats counts those calls), in fp32 MFMA from the start when the context was
- * created with SLAI_PROMPT_SPLIT_F16=0 or when the block scales of a layer matrix allow a weight of 255 or more in
- * magnitude (the pair form holds 256 * w in f16; trained models are orders of magnitude below); 1 = the GEMV kernels with
- * one workgroup per token and tile sharing the weights through L2 (the same layouts when the context was created with
- * SLAI_PROMPT_GEMM=0); 0 = layouts without chunked kernels: token by token with the same result when `chunk` says so or the
- * format has no tiles, over padded copies of the matrices in tiles otherwise (Q8_0, Q4_0).  With chunk 0 (and, over 32 tokens,
- * with larger chunks) a model whose matrices have tiles or such copies reads up to 1024 tokens per pass in the pair form. */
+ * continues with slai_llama2_generate(prompt, n_prompt, n_prompt - 1, ...).
+ * Chunks of more than 32 tokens (chunk 0: passes of up to 1024) of a model whose layer matrices lie in tiles, with heads of 48, 64
+ * or 128 elements (the sizes the pass's attention is built for), are multiplied on the half-precision matrix cores: the
+ * quantised integers as they are, activations as an f16 head and an f16 remainder (about 23 bits down to 2^-14, fp32
+ * accumulation).  Models of Q8_0 / Q4_0 in rows that are no multiple of 256 do so with chunk 0 from 4 tokens on, over copies in
+ * tiles made at load (at most SLAI_PROMPT_COPY_MB = 1024 of them and an eighth of the free memory, none with SLAI_TILED=0).
+ * slai_llama2_prefill_supported() says what any other prompt takes: 2 = matrix-core GEMM over the dequantised tiles (every
+ * format with a tiled layout), at most 32 tokens per pass, weights and activations as f16 pairs (about 22 bits); 1 = the GEMV kernels with one
+ * workgroup per token and tile sharing the weights through L2 (the same layouts when the context was created with
+ * SLAI_PROMPT_GEMM=0); 0 = the ordinary loop (no tiles).
+ * A call in pairs is repeated when an activation turns out to be beyond the f16 range (slai_llama2_prefill_fp32_repeats counts
+ * those calls), with fp32 MFMA, or in the ordinary loop where there are no tiles; it takes those from the start when the context
+ * was created with SLAI_PROMPT_SPLIT_F16=0 or when the block scales of a layer matrix allow a weight of 255 or more in
+ * magnitude (the pair form of the weights holds 256 * w in f16; trained models are orders of magnitude below). */
 int slai_llama2_prefill(slai_llama2 *m, const int32_t *tokens, uint32_t n_tokens, uint32_t start_pos, uint32_t chunk,
                         float *elapsed_ms);
 int slai_llama2_prefill_supported(const slai_llama2 *m);
@@ -390,8 +393,8 @@ int slai_gpt2_generate(slai_gpt2 *m, const int32_t *prompt, uint32_t n_prompt, u
 int slai_gpt2_generate_sampled(slai_gpt2 *m, const int32_t *prompt, uint32_t n_prompt, uint32_t start_pos,
                                uint32_t n_steps, float temperature, float topp, uint64_t seed, int32_t *out_tokens,
                                float *elapsed_ms);
-/* slai_llama2_prefill for GPT-2 (gpt2/cpu.rs:225-383 for a chunk of tokens; no counterpart in the reference): 32 tokens
- * per pass over the weights on the matrix cores where every layer matrix has a tiled layout
+/* slai_llama2_prefill for GPT-2 (gpt2/cpu.rs:225-383 for a chunk of tokens; no counterpart in the reference): passes of up to
+ * 1024 tokens, or 32 and fewer, on the matrix cores as there where every layer matrix has a tiled layout
  * (slai_gpt2_prefill_supported() == 2; f16 head + remainder pairs with the fp32 repeat of slai_llama2_prefill, counted by
  * slai_gpt2_prefill_fp32_repeats), token by token with the same result otherwise (0). */
 int slai_gpt2_prefill(slai_gpt2 *m, const int32_t *tokens, uint32_t n_tokens, uint32_t start_pos, uint32_t chunk,

@@ -18,6 +18,14 @@ template <int BYTES> __device__ __forceinline__ void touch_kernel_arguments() {
     asm volatile("" : : "s"(w));
 }
 
+// Workgroup barrier that orders LDS traffic only.  __syncthreads() also fences global memory, which on this target means
+// waiting for every outstanding global load (vmcnt(0)) -- it would serialise the weight stream behind each reduction step.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // A lane-broadcast word as an unsigned value (the builtin returns `int`; see join_words in resident_plan.h).
 __device__ __forceinline__ uint32_t uniform_word(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
 

@@ -3,18 +3,11 @@
 // issues a unit's 16-byte weight pieces on request of the dot products in quant_tiled.h, and small reductions.
 #pragma once
 #include "common.h"
+#include "device_util.h"
 #include "quant_tiled.h"
 
 namespace slai {
 namespace lanes {
-
-// Workgroup barrier that orders LDS traffic only.  __syncthreads() also fences global memory, which on this target means
-// waiting for every outstanding global load (vmcnt(0)) -- it would serialise the weight stream behind each reduction step.
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
 
 __device__ __forceinline__ float gelu_f(float x) {
     const float GELU_COEF_A = 0.044715f, SQRT_2_OVER_PI = 0.7978846f;   // ops/unary.rs:81-85

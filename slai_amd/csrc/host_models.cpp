@@ -1329,7 +1329,7 @@ SLAI_EXPORT int slai_llama2_generate_sampled(slai_llama2 *m, const int32_t *prom
     return generate_impl(m, m->ctx, m->loop, m->config.seq_len, m->config.vocab_size, prompt, n_prompt, start_pos, n_steps, out_tokens, elapsed_ms, &sp);
 }
 
-// 0: the ordinary loop, 1: per-token workgroups over shared weights, 2: matrix cores
+// 0: the ordinary loop, 1: per-token workgroups over shared weights, 2: matrix cores (of prompts that take no wide pass)
 SLAI_EXPORT int slai_llama2_prefill_supported(const slai_llama2 *m) {
     if (!m) return 0;
     if (m->ctx->prompt_gemm && m->chunk_gemm_supported()) return 2;
@@ -1350,8 +1350,9 @@ SLAI_EXPORT int slai_llama2_prefill(slai_llama2 *m, const int32_t *tokens, uint3
     for (uint32_t i = 0; i < n_tokens; ++i)
         if (tokens[i] < 0 || (uint32_t)tokens[i] >= m->config.vocab_size) return set_error(ctx, SLAI_E_ARG, "slai_llama2_prefill: token out of range");
     if (chunk > 64) return set_error(ctx, SLAI_E_ARG, "slai_llama2_prefill: at most 64 tokens per chunk");
-    // K-quants in the tiled layouts: matrix cores, 32 tokens per pass; other tiled formats: one workgroup per token and
-    // tile over shared weights; anything else: the ordinary loop
+    // tiled layouts: matrix cores, up to 32 tokens per pass (kernels_gemm_chunk.hip), or one workgroup per token and tile over
+    // shared weights; more tokens, and any more than three over padded copies: up to 1024 per pass (kernels_prompt_wide.hip);
+    // anything else: the ordinary loop
     const bool gemm = ctx->prompt_gemm && m->chunk_gemm_supported();
     const bool shared = !gemm && m->chunk_supported();
     const uint32_t wide_tokens = std::min(chunk ? chunk : wide_pass_tokens(n_tokens), n_tokens);
