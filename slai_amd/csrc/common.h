@@ -272,6 +272,7 @@ struct WideGemmSeg {
     float *out = nullptr;         // WIDE_ROWS: token t at out + t * out_stride; range s of ksplit s * part_stride floats on
     uint32_t out_stride = 0, part_stride = 0;
     const float *bias = nullptr;  // optional (WIDE_ROWS: added to range 0's result); WIDE_GELU: required
+    float down = 1.0f;            // WIDE_ROWS: factor of the result (undoes what its input was scaled by)
 };
 struct WideGemmParams {
     WideGemmSeg seg[3];           // WIDE_GATED: gate, up
@@ -283,6 +284,7 @@ struct WideGemmParams {
     uint8_t *pairs_out = nullptr; // WIDE_GATED, WIDE_GELU: super-blocks per token out_ncb
     uint32_t out_ncb = 0;
     bool out_sums = false;        // their sums of 32 too
+    float up = 1.0f;              // WIDE_GATED: factor of the output, a power of two
     int *flag = nullptr;          // set when an output is beyond f16
     uint32_t token_blocks = 0, row_units = 0, out_c8 = 0;   // filled by the launcher
 };

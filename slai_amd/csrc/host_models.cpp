@@ -34,7 +34,8 @@ const uint32_t STORAGE = SLAI_USAGE_STORAGE, UNIFORM = SLAI_USAGE_UNIFORM, COPY_
 // `gguf.tensors[name].data().as_f32().unwrap()` + `GpuTensor::vector` (transformer.rs:250-263)
 // The kernels index these vectors by the model's widths, so a tensor of any other length is refused here, before
 // anything is launched (`expected` elements: the width the readers assume).
-int f32_vector_from_gguf(slai_ctx *ctx, const Gguf &g, const std::string &name, bool required, uint32_t expected, GpuTensor *out) {
+int f32_vector_from_gguf(slai_ctx *ctx, const Gguf &g, const std::string &name, bool required, uint32_t expected, GpuTensor *out,
+                         float *largest = nullptr /* magnitude */) {
     const GgufTensorInfo *t = g.find(name);
     if (!t) return required ? set_error(ctx, SLAI_E_MISSING, "missing tensor '" + name + "'") : SLAI_OK;
     if (t->type != 0) return set_error(ctx, SLAI_E_TYPE, "tensor '" + name + "' must be F32");
@@ -44,6 +45,14 @@ int f32_vector_from_gguf(slai_ctx *ctx, const Gguf &g, const std::string &name, 
     }
     if (n != expected)
         return set_error(ctx, SLAI_E_SHAPE, "tensor '" + name + "' has " + std::to_string(n) + " elements, the model needs " + std::to_string(expected));
+    if (largest) {
+        *largest = 0.0f;
+        for (uint64_t i = 0; i < n; ++i) {
+            float v;
+            memcpy(&v, g.bytes + t->offset + 4 * i, 4);
+            if (!(fabsf(v) <= *largest)) *largest = fabsf(v);  // (a NaN stays)
+        }
+    }
     return GpuTensor::vector_from(ctx, reinterpret_cast<const float *>(g.bytes + t->offset), (uint32_t)n, STORAGE, out);
 }
 int qmat_from_gguf(slai_ctx *ctx, const slai_gguf *g, const std::string &name, slai_qmat **out, int layout = SLAI_LAYOUT_AUTO) {
@@ -198,6 +207,18 @@ private:
     std::vector<const slai_qmat *> sources;
 };
 
+// What a gated layer's hidden values are multiplied by on their way into pairs (a power of two, taken out behind the down
+// projection).  A normalised row is at most sqrt(dim) times the largest gain long and a row of weights sqrt(dim) times their bound,
+// so |silu(gate) * up| <= gate * up <= the product below: where that is far below f16's largest, hidden values are too, and
+// small gains (0.001: hidden values of 5e-7) would leave them among f16's subnormals.
+float wide_hidden_up(float gate_bound, float up_bound, float gain, uint32_t dim) {
+    const double row = (double)gain * dim, bound = (double)gate_bound * up_bound * row * row;
+    if (!(bound < 16384.0)) return 1.0f;                       // (NaN and infinite gains too)
+    int up = 0;
+    while (up < 60 && bound * (double)(2ull << up) <= 16384.0) ++up;
+    return (float)(1ull << up);
+}
+
 // Tokens of each pass of a prompt of n: equal passes of whole 64-token blocks
 uint32_t wide_pass_tokens(uint32_t n) {
     const uint32_t passes = (n + wide::MAX_TOKENS - 1) / wide::MAX_TOKENS;
@@ -244,6 +265,7 @@ struct Llama2LayerWeights {          // transformer.rs:179-192
     GpuTensor attn_k_bias, attn_q_bias, attn_v_bias;   // optional
     slai_qmat *ffn_down = nullptr, *ffn_gate = nullptr;
     GpuTensor ffn_norm;
+    float ffn_norm_largest = 0.0f;
     slai_qmat *ffn_up = nullptr, *attn_output = nullptr;
 };
 struct Llama2Weights {               // transformer.rs:194-199
@@ -314,7 +336,7 @@ struct slai_llama2 {
     uint32_t prefill_fp32_repeats = 0;   // prefill calls repeated in fp32 because an activation was beyond the f16 range
     int enqueue_chunk_gemm(uint32_t pos0, uint32_t n, const int *tokens_dev, bool split_f16);   // the same on the matrix cores, n <= 32
     WidePass wide;
-    struct WideLayer { slai_qmat *q, *k, *v, *o, *gate, *up, *down; };
+    struct WideLayer { slai_qmat *q, *k, *v, *o, *gate, *up, *down; float hidden_up; };   // hidden_up: see wide_hidden_up
     std::vector<WideLayer> wide_layers;  // empty: the model has no wide pass (kernels_prompt_wide.hip)
     WideMats wide_mats;
     void wide_setup();
@@ -410,7 +432,7 @@ int slai_llama2::load(const slai_gguf *gg) {
         TRY(qmat_from_gguf(ctx, gg, p + "ffn_down.weight", &w.ffn_down, SLAI_LAYOUT_TILE16));
         TRY(qmat_from_gguf(ctx, gg, p + "ffn_gate.weight", &w.ffn_gate, SLAI_LAYOUT_TILE64));
         TRY(qmat_from_gguf(ctx, gg, p + "ffn_up.weight", &w.ffn_up, SLAI_LAYOUT_TILE64));
-        TRY(f32_vector_from_gguf(ctx, g, p + "ffn_norm.weight", true, dim, &w.ffn_norm));
+        TRY(f32_vector_from_gguf(ctx, g, p + "ffn_norm.weight", true, dim, &w.ffn_norm, &w.ffn_norm_largest));
         TRY(f32_vector_from_gguf(ctx, g, p + "attn_norm.weight", true, dim, &w.attn_norm));
         struct { slai_qmat *m; uint32_t r, c; } chk[] = {{w.attn_q, dim, dim}, {w.attn_k, kvd, dim}, {w.attn_v, kvd, dim},
             {w.attn_output, dim, dim}, {w.ffn_down, dim, config.hidden_dim}, {w.ffn_gate, config.hidden_dim, dim}, {w.ffn_up, config.hidden_dim, dim}};
@@ -1006,7 +1028,8 @@ void slai_llama2::wide_setup() {
     bool ok = true;
     for (const Llama2LayerWeights &w : weights.layers) {
         const auto take = [&](slai_qmat *m) { return wide_mats.take(ctx, m); };
-        const WideLayer l{take(w.attn_q), take(w.attn_k), take(w.attn_v), take(w.attn_output), take(w.ffn_gate), take(w.ffn_up), take(w.ffn_down)};
+        const WideLayer l{take(w.attn_q), take(w.attn_k), take(w.attn_v), take(w.attn_output), take(w.ffn_gate), take(w.ffn_up), take(w.ffn_down),
+                          wide_hidden_up(w.ffn_gate->wbound, w.ffn_up->wbound, w.ffn_norm_largest, config.dim)};
         for (const slai_qmat *m : {l.q, l.k, l.v, l.o, l.gate, l.up, l.down}) ok = ok && m && m->wbound < 255.0f;
         if (!ok) break;
         ok = l.gate->type == l.up->type && l.gate->rows_log2 == l.up->rows_log2 && !(hs == 48 && (l.o->type == T_Q4_K || l.o->type == T_Q5_K));
@@ -1066,9 +1089,10 @@ int slai_llama2::enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev) 
                                              wide_reads_sums(wm.gate), flag));
         WideGemmParams g;
         g.nseg = 2; g.seg[0] = wide_seg(wm.gate, nullptr, 0, 0); g.seg[1] = wide_seg(wm.up, nullptr, 0, 0);
-        g.x = pairs; g.ncb = ncb; g.ntokens = n; g.pairs_out = hidden; g.out_ncb = hcb; g.out_sums = wide_reads_sums(wm.down); g.flag = flag; g.large = wide_plan(r_ffn, 2, n, ncb, false).large;
+        g.x = pairs; g.ncb = ncb; g.ntokens = n; g.pairs_out = hidden; g.out_ncb = hcb; g.out_sums = wide_reads_sums(wm.down); g.up = wm.hidden_up; g.flag = flag; g.large = wide_plan(r_ffn, 2, n, ncb, false).large;
         TRY(wide_call(ctx, g, WIDE_GATED, "llama2 ffn gate/up (prompt)"));
-        const WideGemmSeg d = wide_seg(wm.down, parts, dim, n * dim);
+        WideGemmSeg d = wide_seg(wm.down, parts, dim, n * dim);
+        d.down = 1.0f / wm.hidden_up;
         TRY(wide_rows(ctx, 1, &d, hidden, hcb, n, p_d, "llama2 ffn_down (prompt)"));
         nparts = ks_d;
     }

@@ -116,13 +116,12 @@ def test_error_of_formats_with_offsets(backend, oracle_lib, part, wtype):
 @pytest.mark.parametrize("wtype", [Q8_0, Q4_0, Q4_K, Q6_K], ids=["q8_0", "q4_0", "q4_k", "q6_k"])
 @pytest.mark.parametrize("gain", [1.0, 0.05, 0.001])
 def test_error_with_small_activations(backend, oracle_lib, shape, wtype, gain):
-    """Normalised rows of every size (the first layer's values), and hidden values (the second's) down to about 2e-3."""
+    """Normalised rows of every size (the first layer's values), and hidden values (the second's) down to about 5e-7."""
     if SHAPES[shape][0] % 256 and wtype not in (Q8_0, Q4_0):
         pytest.skip("blocks of 256 do not divide the rows")
     m = Model(oracle_lib, "ffn", wtype, *SHAPES[shape], gain)
     _, first, second = errors(backend, m)
-    assert first < BAR[0], first
-    assert gain < 0.05 or second < BAR[1], second
+    assert first < BAR[0] and second < BAR[1], (first, second)
 
 
 @pytest.mark.parametrize("shape", SHAPES)
