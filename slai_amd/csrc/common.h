@@ -279,7 +279,7 @@ struct WideGemmParams {
     int nseg = 1;
     const uint8_t *x = nullptr;
     uint32_t ncb = 0, ntokens = 0;
-    bool large = true;            // the form (wide_plan)
+    int form = 0;                 // wide_plan
     uint32_t ksplit = 1;          // WIDE_ROWS: the columns in ranges of whole super-blocks, each its own workgroups and result
     uint8_t *pairs_out = nullptr; // WIDE_GATED, WIDE_GELU: super-blocks per token out_ncb
     uint32_t out_ncb = 0;
@@ -291,7 +291,8 @@ struct WideGemmParams {
 bool wide_gemm_supports(const slai_qmat *m);
 bool wide_reads_sums(const slai_qmat *m);   // whether its input needs the sums of 32 (offsets per sub-block)
 // Form and number of column ranges for nseg matrices over one input (splits: ranges are possible, WIDE_ROWS)
-struct WidePlan { bool large; uint32_t ksplit; };
+enum { WIDE_LARGE = 0, WIDE_SMALL, WIDE_SLIM4, WIDE_SLIM8 };
+struct WidePlan { int form; uint32_t ksplit; };
 WidePlan wide_plan(const uint32_t *nrows, int nseg, uint32_t ntokens, uint32_t ncb, bool splits);
 hipError_t launch_wide_gemm(hipStream_t st, WideGemmParams p, int mode);
 // x += its nparts partial results (parts + s * part_stride, rows of n), then RMSNorm (b null) or LayerNorm as pairs (with

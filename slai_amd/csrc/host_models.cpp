@@ -244,7 +244,7 @@ int wide_rows(slai_ctx *ctx, int nseg, const WideGemmSeg *segs, const uint8_t *x
     for (int i = 0; i < nseg; ++i) {
         if (done[i]) continue;
         WideGemmParams p;
-        p.nseg = 0; p.x = x; p.ncb = ncb; p.ntokens = ntokens; p.ksplit = plan.ksplit; p.large = plan.large;
+        p.nseg = 0; p.x = x; p.ncb = ncb; p.ntokens = ntokens; p.ksplit = plan.ksplit; p.form = plan.form;
         for (int j = i; j < nseg; ++j) {
             if (done[j] || (segs[j].type != segs[i].type && !(kq(segs[j].type) && kq(segs[i].type)))) continue;
             p.seg[p.nseg++] = segs[j];
@@ -1089,7 +1089,7 @@ int slai_llama2::enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev) 
                                              wide_reads_sums(wm.gate), flag));
         WideGemmParams g;
         g.nseg = 2; g.seg[0] = wide_seg(wm.gate, nullptr, 0, 0); g.seg[1] = wide_seg(wm.up, nullptr, 0, 0);
-        g.x = pairs; g.ncb = ncb; g.ntokens = n; g.pairs_out = hidden; g.out_ncb = hcb; g.out_sums = wide_reads_sums(wm.down); g.up = wm.hidden_up; g.flag = flag; g.large = wide_plan(r_ffn, 2, n, ncb, false).large;
+        g.x = pairs; g.ncb = ncb; g.ntokens = n; g.pairs_out = hidden; g.out_ncb = hcb; g.out_sums = wide_reads_sums(wm.down); g.up = wm.hidden_up; g.flag = flag; g.form = wide_plan(r_ffn, 2, n, ncb, false).form;
         TRY(wide_call(ctx, g, WIDE_GATED, "llama2 ffn gate/up (prompt)"));
         WideGemmSeg d = wide_seg(wm.down, parts, dim, n * dim);
         d.down = 1.0f / wm.hidden_up;
@@ -1380,8 +1380,9 @@ SLAI_EXPORT int slai_llama2_prefill(slai_llama2 *m, const int32_t *tokens, uint3
     const bool gemm = ctx->prompt_gemm && m->chunk_gemm_supported();
     const bool shared = !gemm && m->chunk_supported();
     const uint32_t wide_tokens = std::min(chunk ? chunk : wide_pass_tokens(n_tokens), n_tokens);
-    // (a wide pass costs what 32 tokens cost in the kernels for up to 32, or about three in the ordinary loop)
-    const bool wide = !m->wide_layers.empty() && ctx->prompt_split_f16 != 0 && ctx->split_flag && (gemm || (chunk == 0 && !shared)) && wide_tokens > (gemm ? 32u : 3u);
+    // (7B shape Q4_K: 9 tokens 3283 us in the kernels for up to 32 and 3112 in a wide pass, 32: 3610 and 3171; a pass over padded copies costs about three
+    // tokens of the ordinary loop; chunks that a caller asks for stay what they were)
+    const bool wide = !m->wide_layers.empty() && ctx->prompt_split_f16 != 0 && ctx->split_flag && (gemm || (chunk == 0 && !shared)) && wide_tokens > (gemm ? chunk == 0 ? 7u : 32u : 3u);
     const auto one_by_one = [&]() {
         // one token per pass, picks discarded
         std::vector<int32_t> prompt((size_t)start_pos + n_tokens, 0), picks(n_tokens);
@@ -1780,7 +1781,7 @@ int slai_gpt2::enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev) {
                                              wide_reads_sums(w.c_mlp_fc_w), flag));
         WideGemmParams g;
         g.nseg = 1; g.seg[0] = wide_seg(w.c_mlp_fc_w, nullptr, 0, 0, &w.c_mlp_fc_b);
-        g.x = pairs; g.ncb = ncb; g.ntokens = n; g.pairs_out = hidden; g.out_ncb = fcb; g.out_sums = wide_reads_sums(w.c_mlp_proj_w); g.flag = flag; g.large = wide_plan(&F, 1, n, ncb, false).large;
+        g.x = pairs; g.ncb = ncb; g.ntokens = n; g.pairs_out = hidden; g.out_ncb = fcb; g.out_sums = wide_reads_sums(w.c_mlp_proj_w); g.flag = flag; g.form = wide_plan(&F, 1, n, ncb, false).form;
         TRY(wide_call(ctx, g, WIDE_GELU, "gpt2 mlp fc (prompt)"));
         const WideGemmSeg sd = wide_seg(w.c_mlp_proj_w, parts, E, n * E, &w.c_mlp_proj_b);
         TRY(wide_rows(ctx, 1, &sd, hidden, fcb, n, p_d, "gpt2 mlp proj (prompt)"));
@@ -1878,7 +1879,7 @@ SLAI_EXPORT int slai_gpt2_prefill(slai_gpt2 *m, const int32_t *tokens, uint32_t 
     // on the half-precision matrix cores first, repeated in fp32 when an activation was beyond f16 (see slai_llama2_prefill)
     bool split = ctx->prompt_split_f16 != 0 && ctx->split_flag && m->chunk_split_ok();
     const uint32_t wide_tokens = std::min(chunk ? chunk : wide_pass_tokens(n_tokens), n_tokens);
-    const bool wide = split && wide_tokens > 32 && m->wide_supported();
+    const bool wide = split && wide_tokens > (chunk == 0 ? 7u : 32u) && m->wide_supported();   // (GPT-2 small: 9 tokens 714 us in the kernels for up to 32, 550 in a wide pass)
     if (chunk == 0 || chunk > 32) chunk = 32;
     if (!wide) TRY(m->chunk_reserve());
     SLAI_HIP_TRY(ctx, hipEventRecord(m->loop.ev0, ctx->stream));

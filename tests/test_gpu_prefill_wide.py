@@ -35,6 +35,17 @@ def test_wide_formats_and_tile_heights(backend, wtype, dims):
     check_prefill(backend, data, prompt_of(71, 512), 6, [0], True)
 
 
+@pytest.mark.parametrize("n", [9, 10, 32, 33, 34])             # n - 1 tokens: the fewest of a pass, and around one token tile
+@pytest.mark.parametrize("wtype", [12, 13, 14, 8, 2], ids=["q4_k", "q5_k", "q6_k", "q8_0", "q4_0"])
+@pytest.mark.parametrize("dims", [(256, 768, 4), (1024, 3072, 8)], ids=["fewer super-blocks than waves", "several super-blocks a wave"])
+def test_wide_few_tokens(backend, wtype, dims, n):
+    """The form for few tokens, in which the waves of a workgroup share the super-blocks out: some without one, some with several."""
+    dim, hidden, heads = dims
+    data = gw.llama_gguf(dim=dim, hidden_dim=hidden, n_layers=2, n_heads=heads, n_kv_heads=heads // 2, vocab=512, seq_len=64, wtype=wtype, seed=26, std=0.05,
+                         norm_random=True)
+    check_prefill(backend, data, prompt_of(n, 512), 6, [0], n % 2 == 0)
+
+
 def test_wide_bias_neox_grouped_queries_continued(backend):
     """Qwen2 form: biases, NeoX pairs, seven query heads per cache head; a second pass on top of 45 cached positions."""
     data = gw.llama_gguf(dim=1792, hidden_dim=2048, n_layers=2, n_heads=14, n_kv_heads=2, vocab=512, seq_len=192, wtype=12, v_type=14, seed=23, std=0.05,
