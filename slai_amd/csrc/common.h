@@ -91,6 +91,7 @@ struct slai_ctx {
     hipEvent_t timer0 = nullptr, timer1 = nullptr;
     // the one-launch-per-token form of the Llama-2 layer stack where a model's shapes allow it (SLAI_PERSISTENT=0 switches it off)
     bool persistent = true;
+    uint32_t small_spins = 1u << 17;        // SLAI_SMALL_SPINS: see SmallParams::spin_limit
     uint32_t resident_max_pos = 2048;   // tokens at positions below this take the resident launch (where the model has one): SLAI_RESIDENT_MAX_POS
     // When set, every launch of a decode step is followed by an event recorded under the step's name
     // (slai_llama2_time_steps); null otherwise.
@@ -365,11 +366,15 @@ QMatDev qmat_dev(const slai_qmat *m);
 // A copy of a Q8_0 / Q4_0 matrix in the row layout as 16-row tiles, rows padded with zeros to whole super-blocks: what the wide
 // prompt pass reads where rows are no multiple of 256.  `tiles`: its geometry, dptr zeroed.
 hipError_t launch_rows_to_tiles(hipStream_t s, const slai_qmat *rows, const slai_qmat *tiles);
+// The other way round: a tiled Q8_0 / Q4_0 matrix as rows (`rows`: its geometry and memory)
+hipError_t launch_tiles_to_rows(hipStream_t s, const slai_qmat *tiles, const slai_qmat *rows);
 hipError_t launch_repack(hipStream_t s, const slai_qmat *m, const uint8_t *src_gguf_rows);
 // rows [row0,row0+nrows) to f32, out[r*out_stride + c]
 hipError_t launch_dequant_rows(hipStream_t s, const slai_qmat *m, uint32_t row0, uint32_t nrows, float *out, size_t out_stride);
 // out[c] = deq(A[row_a][c]) (+ deq(B[row_b][c]) when B != null); row indices read from device memory
-hipError_t launch_embed(hipStream_t s, const slai_qmat *a, const int *row_a, const slai_qmat *b, const int *row_b, uint32_t ncols, float *out);
+// (zero: nzero words cleared by the same launch)
+hipError_t launch_embed(hipStream_t s, const slai_qmat *a, const int *row_a, const slai_qmat *b, const int *row_b, uint32_t ncols, float *out, uint32_t *zero = nullptr,
+                        uint32_t nzero = 0);
 
 // ---- element-wise / normalisation ops -------------------------------------------------
 struct VecView { float *p; uint32_t n; uint32_t stride; };  // element i at p[i*stride]
@@ -465,6 +470,31 @@ int attention_describe(slai_ctx *ctx, const char *fn, const slai_attn_params *pa
 // slai_attention_static (called by slai_ctx_create).
 hipError_t attention_static_setup(int device);
 
+
+// ---- the layers of a small model's token in one resident launch on one die (kernels_decode_small.hip) ----------------------
+constexpr uint32_t SMALL_WGS = 32, SMALL_STEPS = 5;            // workgroups that work; counters (a 128-byte line each) of a layer
+constexpr uint32_t small_pad(uint32_t floats) { return (floats + 31) & ~31u; }   // hand-over vectors start on lines of their own
+struct SmallLayer {                                            // packed rows (row layout); biases are optional
+    const uint8_t *q, *k, *v, *o, *gate, *up, *down;
+    const float *norm1, *norm2, *qb, *kb, *vb;
+    void *kcache, *vcache;
+};
+struct SmallParams {
+    const SmallLayer *layers = nullptr;
+    float *work = nullptr;                                     // work_stride floats per layer: q | k | v, attention, x, hidden, x
+    uint32_t *counters = nullptr, *abort_flag = nullptr;       // SMALL_STEPS * 32 words per layer, zero at the start of a launch
+    float *x = nullptr;                                        // the embedding row in, the last layer's residual out
+    const uint32_t *pos_ptr = nullptr;
+    const float *rope_theta = nullptr;
+    uint32_t work_stride = 0, n_layers = 0, dim = 0, kvd = 0, hidden = 0, n_heads = 0, kv_mul = 1, head_size = 0, seq_len = 0;
+    uint32_t stride_e = 0, stride_h = 0;                       // bytes of a packed row of dim / hidden columns
+    int type = 0, kv_f16 = 0, rope_variant = -1;
+    float eps = 0.0f, rope_base = 0.0f;
+    uint32_t die = 0;                                          // workgroups i with i mod 8 == die
+    uint32_t spin_limit = 1u << 17;                            // looks at a counter before a workgroup gives up (about 0.1 s)
+};
+bool small_shape_ok(const SmallParams &p);
+hipError_t launch_decode_small(hipStream_t s, const SmallParams &p);
 
 // ---- the whole layer stack of a Llama-2 token in one resident launch (kernels_decode_persistent.hip) ----------------------
 // A matrix, vector or cache as the kernel sees it: address and size in bytes.  Every access of the kernel to it goes

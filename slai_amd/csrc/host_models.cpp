@@ -12,6 +12,8 @@
 #include "wide_layout.h"
 
 #include <algorithm>
+#include <array>
+#include <atomic>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -120,7 +122,7 @@ struct DeviceLoop {           // device-resident state of the greedy loop
     slai_buffer *prompt = nullptr;      // int32[capacity]
     slai_buffer *out_tokens = nullptr;  // int32[capacity]
     uint32_t capacity = 0;
-    slai_graph *graph[3][3] = {};       // one token, [launch form][greedy | temperature and top-p | plain temperature pick]
+    slai_graph *graph[4][3] = {};       // one token, [launch form][greedy | temperature and top-p | plain temperature pick]
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
 };
 int loop_init(slai_ctx *ctx, DeviceLoop &L, uint32_t capacity) {
@@ -254,6 +256,86 @@ int wide_rows(slai_ctx *ctx, int nseg, const WideGemmSeg *segs, const uint8_t *x
     }
     return SLAI_OK;
 }
+
+// The layers of a token as one resident launch on one die (kernels_decode_small.hip), for the models whose shapes and formats it covers.  It
+// reads packed rows: matrices in tiles get copies as rows (one block of memory, bounded like WideMats).
+struct SmallForm {
+    bool ready = false;
+    SmallParams params;
+    slai_buffer *layers = nullptr, *work = nullptr, *counters = nullptr;
+    std::vector<slai_qmat *> copies;
+    std::vector<const slai_qmat *> sources;
+    uint8_t *block = nullptr;
+
+    uint32_t counter_words() const { return params.n_layers * SMALL_STEPS * 32; }
+    // What the kernel reads of m: m itself, or its copy as rows (memory assigned by `make`)
+    slai_qmat *take(slai_qmat *m) {
+        if (!m->tiled) return m;
+        slai_qmat *c = new slai_qmat();
+        copies.push_back(c);
+        sources.push_back(m);
+        c->type = m->type; c->nrows = m->nrows; c->ncols = m->ncols; c->nb = m->nb;
+        c->row_stride = device_row_stride(m->type, m->ncols); c->bytes = c->row_stride * m->nrows;
+        return c;
+    }
+    // false: the model keeps one launch per step
+    bool make(slai_ctx *ctx) {
+        size_t total = 0, free_bytes = 0, all_bytes = 0;
+        for (const slai_qmat *c : copies) total += (c->bytes + 255) / 256 * 256;
+        if (!total) return true;
+        if (total > ctx->prompt_copy_bytes || hipMemGetInfo(&free_bytes, &all_bytes) != hipSuccess || total > free_bytes / 8) return false;
+        if (hipMalloc((void **)&block, total) != hipSuccess) { block = nullptr; (void)hipGetLastError(); return false; }
+        size_t at = 0;
+        for (size_t i = 0; i < copies.size(); ++i) {
+            copies[i]->dptr = block + at;
+            at += (copies[i]->bytes + 255) / 256 * 256;
+            if (launch_tiles_to_rows(ctx->stream, sources[i], copies[i]) != hipSuccess) return false;
+        }
+        return true;
+    }
+    // `params` but for the buffers, and the layers' vectors and caches; mats(l): its seven matrices (q, k, v, o, gate, up, down)
+    template <class Mats> int setup(slai_ctx *ctx, std::vector<SmallLayer> &host, Mats &&mats) {
+        SmallParams &p = params;
+        if (!ctx->persistent || !ctx->fuse_qkv_attention || !ctx->handoff_counters || !small_shape_ok(p)) return SLAI_OK;
+        p.stride_e = (uint32_t)device_row_stride(p.type, p.dim); p.stride_h = (uint32_t)device_row_stride(p.type, p.hidden);
+        std::vector<std::array<slai_qmat *, 7>> rows(host.size());
+        for (size_t l = 0; l < host.size(); ++l) {
+            rows[l] = mats(l);
+            for (slai_qmat *&m : rows[l]) {
+                if (m->type != p.type) { drop(ctx); return SLAI_OK; }
+                m = take(m);
+            }
+        }
+        if (!make(ctx)) { drop(ctx); return SLAI_OK; }
+        for (size_t l = 0; l < host.size(); ++l) {
+            const auto &r = rows[l];
+            SmallLayer &d = host[l];
+            d.q = r[0]->dptr; d.k = r[1]->dptr; d.v = r[2]->dptr; d.o = r[3]->dptr; d.gate = r[4]->dptr; d.up = r[5]->dptr; d.down = r[6]->dptr;
+        }
+        p.work_stride = small_pad(p.dim + 2 * p.kvd) + 3 * small_pad(p.dim) + small_pad(p.hidden);
+        TRY(slai_buffer_create(ctx, host.size() * sizeof(SmallLayer), SLAI_DT_U8, STORAGE | COPY_DST, &layers));
+        TRY(slai_write_buffer(ctx, layers, 0, host.data(), host.size() * sizeof(SmallLayer)));
+        TRY(slai_buffer_create(ctx, host.size() * p.work_stride * sizeof(float), SLAI_DT_F32, STORAGE, &work));
+        TRY(slai_buffer_create(ctx, (size_t)counter_words() * 4, SLAI_DT_U8, STORAGE, &counters));
+        p.layers = (const SmallLayer *)layers->dptr; p.work = (float *)work->dptr; p.counters = (uint32_t *)counters->dptr;
+        p.abort_flag = ctx->handoff_counters + (size_t)ctx->handoff_heads * 32;
+        // (contexts that run at the same time take different dies: a die keeps the workgroups of one launch resident)
+        static std::atomic<uint32_t> next_die{0};
+        p.die = next_die.fetch_add(1) & 7u;
+        p.spin_limit = ctx->small_spins;
+        ready = true;
+        return SLAI_OK;
+    }
+    void drop(slai_ctx *ctx) {
+        ready = false;
+        for (slai_qmat *c : copies) delete c;
+        copies.clear(); sources.clear();
+        if (block) (void)hipFree(block);
+        block = nullptr;
+        for (slai_buffer **b : {&layers, &work, &counters})
+            if (*b) { slai_buffer_destroy(ctx, *b); *b = nullptr; }
+    }
+};
 }  // namespace
 
 // =================================================================================================
@@ -322,6 +404,11 @@ struct slai_llama2 {
         slai_buffer *layers = nullptr, *flow = nullptr, *slots = nullptr;
         size_t flow_bytes = 0;
     } persistent;
+    SmallForm small;                              // form 3
+    int small_setup();
+    int enqueue_small(int sampler);
+    bool drop_small() { const bool was = small.ready; small.ready = false; return was; }   // from now on one launch per step
+    int enqueue_output(const float *prepared, int sampler);   // the output matrix and the pick
     bool persistent_supported() const;
     int persistent_setup();
     int enqueue_persistent(int sampler, bool far);
@@ -484,6 +571,7 @@ int slai_llama2::load(const slai_gguf *gg) {
     TRY(ensure_attn_scratch(ctx, attention_scratch_floats(config.n_q_heads, head_size(), attn_splits)));
     TRY(loop_init(ctx, loop, config.seq_len + 1));
     TRY(persistent_setup());
+    TRY(small_setup());
     wide_setup();
     // (said only to a caller who asked for the form by name: most models simply have other shapes)
     const char *asked = getenv("SLAI_PERSISTENT");
@@ -642,11 +730,42 @@ int slai_llama2::launch(LlmContext &ctxt, const slai_attn_params &attn_params, u
 // rows beyond the ones the attention asks for ahead into the die's L2 -- a kernel of its own, so that the short contexts do
 // not carry that code.)
 int slai_llama2::form_at(uint32_t pos) const {
+    if (small.ready) return 3;
     if (!persistent.ready || pos >= ctx->resident_max_pos) return 0;
     return pos > resident_far_from(kv_dtype == SLAI_KV_F16) ? 2 : 1;
 }
 
+int slai_llama2::small_setup() {
+    if (persistent.ready || weights.layers.empty()) return SLAI_OK;
+    SmallParams &p = small.params;
+    p.n_layers = config.n_layers; p.dim = config.dim; p.kvd = kv_dim(); p.hidden = config.hidden_dim; p.n_heads = config.n_q_heads; p.kv_mul = config.n_q_heads / config.n_kv_heads;
+    p.head_size = head_size(); p.seq_len = config.seq_len; p.type = weights.layers[0].attn_q->type; p.kv_f16 = kv_dtype == SLAI_KV_F16;
+    p.rope_variant = rope_variant(); p.rope_base = config.rope_base_freq; p.rope_theta = (const float *)state.rope_theta.buf->dptr; p.eps = config.rms_norm_eps;
+    p.x = (float *)state.x.buf->dptr; p.pos_ptr = (const uint32_t *)&((DecodeState *)loop.state->dptr)->pos;
+    std::vector<SmallLayer> host(config.n_layers);
+    const auto vec = [](const GpuTensor &t) { return t.buf ? (const float *)t.buf->dptr : nullptr; };
+    for (uint32_t l = 0; l < config.n_layers; ++l) {
+        const Llama2LayerWeights &w = weights.layers[l];
+        SmallLayer &d = host[l];
+        d.norm1 = vec(w.attn_norm); d.norm2 = vec(w.ffn_norm); d.qb = vec(w.attn_q_bias); d.kb = vec(w.attn_k_bias); d.vb = vec(w.attn_v_bias);
+        d.kcache = state.key_cache[l].buf->dptr; d.vcache = state.value_cache[l].buf->dptr;
+    }
+    return small.setup(ctx, host, [&](size_t l) {
+        const Llama2LayerWeights &w = weights.layers[l];
+        return std::array<slai_qmat *, 7>{w.attn_q, w.attn_k, w.attn_v, w.attn_output, w.ffn_gate, w.ffn_up, w.ffn_down};
+    });
+}
+
+// embedding row and counters cleared | the layers | output matrix | pick
+int slai_llama2::enqueue_small(int sampler) {
+    DecodeState *ds = (DecodeState *)loop.state->dptr;
+    SLAI_HIP_TRY(ctx, launch_embed(ctx->stream, weights.token_embd, &ds->token, nullptr, nullptr, config.dim, (float *)state.x.buf->dptr, small.params.counters, small.counter_words()));
+    SLAI_HIP_TRY(ctx, launch_decode_small(ctx->stream, small.params));
+    return enqueue_output(nullptr, sampler);
+}
+
 int slai_llama2::enqueue_fused(int sampler, int form) {
+    if (form == 3) return small.ready ? enqueue_small(sampler) : set_error(ctx, SLAI_E_STATE, "this model does not take the launch on one die");
     if (form != 0) return persistent.ready ? enqueue_persistent(sampler, form == 2) : set_error(ctx, SLAI_E_STATE, "this model does not take the resident launch");
     Llama2State &s = state;
     DecodeState *ds = (DecodeState *)loop.state->dptr;
@@ -770,6 +889,13 @@ int slai_llama2::enqueue_fused(int sampler, int form) {
             TRY(gemv_call(ctx, c, "llama2 ffn_down"));
         }
     }
+    return enqueue_output(prepared, sampler);
+}
+
+int slai_llama2::enqueue_output(const float *prepared, int sampler) {
+    Llama2State &s = state;
+    DecodeState *ds = (DecodeState *)loop.state->dptr;
+    const float *x = (const float *)s.x.buf->dptr;
     {
         GemvCall c;
         c.m[0] = weights.output; c.out[0] = (float *)s.logits.buf->dptr; c.x = x;
@@ -1135,6 +1261,7 @@ SLAI_EXPORT void slai_llama2_destroy(slai_llama2 *m) {
     for (slai_buffer *b : {pc.positions, pc.tokens}) if (b) slai_buffer_destroy(ctx, b);
     m->wide.destroy(ctx);
     m->wide_mats.drop();
+    m->small.drop(ctx);
     delete m;
 }
 
@@ -1284,7 +1411,10 @@ SLAI_EXPORT int slai_llama2_forward_logits(slai_llama2 *m, uint32_t pos, uint32_
         TRY(m->enqueue_fused(0, m->form_at(pos)));
     }
     TRY(slai_synchronize(ctx));                                          // :219
-    TRY(handoff_check(ctx));
+    if (const int rc = handoff_check(ctx)) {
+        if (!fused || !m->drop_small()) return rc;
+        return slai_llama2_forward_logits(m, pos, token, fused, logits_out);
+    }
     if (logits_out) TRY(slai_read_buffer(ctx, s.logits.buf, 0, logits_out, (size_t)m->config.vocab_size * 4));   // :225-227
     return SLAI_OK;
 }
@@ -1305,6 +1435,11 @@ static int generate_impl(Model *m, slai_ctx *ctx, DeviceLoop &L, uint32_t seq_le
         if (prompt[i] < 0 || (uint32_t)prompt[i] >= vocab) return set_error(ctx, SLAI_E_ARG, "generate: prompt token out of range");
     DecodeState ds{(int)start_pos, prompt[start_pos], (int)n_prompt, 0, 0.0f, 0.0f, 0, 0};     // chat_llama2.rs:105
     if (sampling) { ds.temperature = sampling->temperature; ds.topp = sampling->topp; ds.seed_lo = (uint32_t)sampling->seed; ds.seed_hi = (uint32_t)(sampling->seed >> 32); }
+    // a launch on one die that did not get its die to itself gave up: the same call once more, with one launch per step from now on
+    const auto again = [&](int rc) {
+        if (!m->drop_small()) return rc;
+        return generate_impl(m, ctx, L, seq_len, vocab, prompt, n_prompt, start_pos, n_steps, out_tokens, elapsed_ms, sampling);
+    };
     TRY(slai_write_buffer(ctx, L.state, 0, &ds, sizeof ds));
     TRY(slai_write_buffer(ctx, L.prompt, 0, prompt, (size_t)n_prompt * 4));
     if (!ctx->use_graph) {
@@ -1312,7 +1447,7 @@ static int generate_impl(Model *m, slai_ctx *ctx, DeviceLoop &L, uint32_t seq_le
         for (uint32_t i = 0; i < n_steps; ++i) TRY(m->enqueue_fused(mode, m->form_at(start_pos + i)));
         SLAI_HIP_TRY(ctx, hipEventRecord(L.ev1, ctx->stream));
         TRY(slai_synchronize(ctx));
-        TRY(handoff_check(ctx));
+        if (const int rc = handoff_check(ctx)) return again(rc);
         if (elapsed_ms) SLAI_HIP_TRY(ctx, hipEventElapsedTime(elapsed_ms, L.ev0, L.ev1));
         return slai_read_buffer(ctx, L.out_tokens, 0, out_tokens, (size_t)n_steps * 4);
     }
@@ -1332,7 +1467,7 @@ static int generate_impl(Model *m, slai_ctx *ctx, DeviceLoop &L, uint32_t seq_le
     for (uint32_t i = 0; i < n_steps; ++i) TRY(slai_graph_launch(ctx, L.graph[m->form_at(start_pos + i)][mode - 1]));   // chat_llama2.rs:109 loop
     SLAI_HIP_TRY(ctx, hipEventRecord(L.ev1, ctx->stream));
     TRY(slai_synchronize(ctx));
-    TRY(handoff_check(ctx));
+    if (const int rc = handoff_check(ctx)) return again(rc);
     if (elapsed_ms) SLAI_HIP_TRY(ctx, hipEventElapsedTime(elapsed_ms, L.ev0, L.ev1));
     return slai_read_buffer(ctx, L.out_tokens, 0, out_tokens, (size_t)n_steps * 4);
 }
@@ -1472,6 +1607,7 @@ struct slai_gpt2 {
     int load(const slai_gguf *g);
     int enqueue_fused(int sampler, int form = 0);   // 0: stop at the logits, 1: greedy pick + loop state, 2: temperature / top-p pick + loop state, 3: the same without a top-p cut (one form only)
     int form_at(uint32_t) const { return 0; }
+    bool drop_small() { return false; }
 
     // Prompt tokens in chunks of up to 32 on the matrix cores (see slai_llama2::enqueue_chunk_gemm); row-major x and qkv,
     // quad-major xn (normalised rows, then the attention output) and h.

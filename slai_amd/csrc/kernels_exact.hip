@@ -56,6 +56,19 @@ __global__ void rows_to_tiles_kernel(QMatDev rows, QMatDev tiles, uint8_t *dst) 
     }
 }
 
+// The same block back
+__global__ void tiles_to_rows_kernel(QMatDev tiles, QMatDev rows, uint8_t *dst) {
+    const size_t total = (size_t)rows.nrows * rows.nb;
+    const TiledGeom g = geom_of(tiles);
+    const uint32_t qbytes = rows.type == T_Q8_0 ? 32u : 16u;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (size_t)gridDim.x * blockDim.x) {
+        const uint32_t r = (uint32_t)(i / rows.nb), b = (uint32_t)(i % rows.nb), cb = b / 8, bi = b % 8;
+        uint8_t *row = dst + (size_t)r * rows.row_stride, *q = row + b * qbytes, *d = row + rows.nb * qbytes + b * 2u;
+        for (uint32_t k = 0; k < qbytes; ++k) q[k] = tiles.dptr[tiled_byte_offset(g, r, cb, qbytes * bi + k)];
+        for (uint32_t k = 0; k < 2; ++k) d[k] = tiles.dptr[tiled_byte_offset(g, r, cb, qbytes * 8 + 2 * bi + k)];
+    }
+}
+
 // f32 / f16 rows: plain copy with the padded device stride
 __global__ void copy_rows_kernel(const uint8_t *src, uint8_t *dst, uint32_t nrows, size_t gguf_row, size_t dev_row) {
     const size_t words = gguf_row / 2;  // rows are multiples of 2 bytes
@@ -74,8 +87,9 @@ __global__ void dequant_rows_kernel(QMatDev m, uint32_t row0, uint32_t nrows, fl
     }
 }
 
-__global__ void embed_kernel(QMatDev a, const int *row_a, QMatDev b, const int *row_b, int has_b, uint32_t ncols, float *out) {
+__global__ void embed_kernel(QMatDev a, const int *row_a, QMatDev b, const int *row_b, int has_b, uint32_t ncols, float *out, uint32_t *zero, uint32_t nzero) {
     const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
+    for (uint32_t i = c; i < nzero; i += gridDim.x * blockDim.x) zero[i] = 0u;
     if (c >= ncols) return;
     float v = qmat_elem(a, (uint32_t)*row_a, c);
     // gpt2/cpu.rs:227-228: token embedding first, then += position embedding
@@ -112,6 +126,14 @@ hipError_t launch_rows_to_tiles(hipStream_t s, const slai_qmat *rows, const slai
     return hipGetLastError();
 }
 
+hipError_t launch_tiles_to_rows(hipStream_t s, const slai_qmat *tiles, const slai_qmat *rows) {
+    if (rows->tiled || !tiles->tiled || (rows->type != T_Q8_0 && rows->type != T_Q4_0) || tiles->type != rows->type || tiles->nrows != rows->nrows || tiles->ncols != rows->ncols)
+        return hipErrorInvalidValue;
+    const size_t total = (size_t)rows->nrows * rows->nb;
+    tiles_to_rows_kernel<<<(uint32_t)std::min<size_t>((total + 255) / 256, 2048), 256, 0, s>>>(qmat_dev(tiles), qmat_dev(rows), rows->dptr);
+    return hipGetLastError();
+}
+
 hipError_t launch_dequant_rows(hipStream_t s, const slai_qmat *m, uint32_t row0, uint32_t nrows, float *out, size_t out_stride) {
     size_t total = (size_t)nrows * m->ncols;
     uint32_t grid = (uint32_t)((total + 255) / 256);
@@ -121,8 +143,9 @@ hipError_t launch_dequant_rows(hipStream_t s, const slai_qmat *m, uint32_t row0,
     return hipGetLastError();
 }
 
-hipError_t launch_embed(hipStream_t s, const slai_qmat *a, const int *row_a, const slai_qmat *b, const int *row_b, uint32_t ncols, float *out) {
-    embed_kernel<<<(ncols + 255) / 256, 256, 0, s>>>(qmat_dev(a), row_a, qmat_dev(b), row_b, b ? 1 : 0, ncols, out);
+hipError_t launch_embed(hipStream_t s, const slai_qmat *a, const int *row_a, const slai_qmat *b, const int *row_b, uint32_t ncols, float *out, uint32_t *zero,
+                        uint32_t nzero) {
+    embed_kernel<<<(ncols + 255) / 256, 256, 0, s>>>(qmat_dev(a), row_a, qmat_dev(b), row_b, b ? 1 : 0, ncols, out, zero, zero ? nzero : 0u);
     return hipGetLastError();
 }
 

@@ -1,0 +1,82 @@
+"""The layers of a small model's token as one launch on one die (kernels_decode_small.hip): shapes at the edges of what it covers (two
+rows per wave, heads of 8 to 64, grouped queries, biases and NeoX pairs), both formats and cache types, positions past one and two passes of
+its attention (120 positions each), against the oracle; a launch that gives up; several models taking turns on one context."""
+import numpy as np
+import pytest
+
+from gpu_common import backend, rel_err  # noqa: F401
+from slai_amd import _ffi
+from slai_amd import gguf_writer as gw
+from slai_amd.runtime import Backend, Gguf, Llama2
+from test_gpu_models import check_llama
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = {                                 # dim, hidden, heads, kv heads
+    "15 M parameters": (288, 768, 6, 6),
+    "widest": (480, 960, 15, 3),           # 15 rows a workgroup, 30 gated pairs
+    "heads of 64": (256, 1024 - 64, 4, 4),
+    "heads of 8, fewer rows than waves": (64, 96, 8, 2),
+    "one head": (32, 32, 1, 1),
+}
+
+
+def model(shape, wtype, seq, seed=31, **kw):
+    dim, hidden, heads, kv = SHAPES[shape]
+    return gw.llama_gguf(dim=dim, hidden_dim=hidden, n_layers=3, n_heads=heads, n_kv_heads=kv, vocab=500, seq_len=seq, wtype=wtype, seed=seed, std=0.08,
+                         norm_random=True, **kw)
+
+
+@pytest.mark.parametrize("kv_f16", [False, True])
+@pytest.mark.parametrize("wtype", [8, 2], ids=["q8_0", "q4_0"])
+@pytest.mark.parametrize("shape", sorted(SHAPES))
+def test_small_shapes(backend, shape, wtype, kv_f16):
+    prompt = np.random.Generator(np.random.PCG64(3)).integers(0, 500, 9)
+    check_llama(backend, model(shape, wtype, 64), prompt, 40, kv_f16=kv_f16)
+
+
+def test_small_bias_neox(backend):
+    data = model("widest", 8, 64, arch="qwen2", bias=True, rope_base=1000000.0, rms_eps=1e-6)
+    check_llama(backend, data, [5, 400, 17], 30, model_type=_ffi.MODEL_QWEN2, neox=1, name=b"qwen2")
+
+
+@pytest.mark.parametrize("kv_f16", [False, True])
+def test_small_positions_beyond_one_pass(backend, kv_f16):
+    prompt = np.random.Generator(np.random.PCG64(4)).integers(0, 500, 230)
+    check_llama(backend, model("15 M parameters", 8, 256), prompt, 252, kv_f16=kv_f16, check_logit_steps=125)
+
+
+def test_small_gives_up_and_the_call_is_repeated(monkeypatch):
+    """One look at a counter is never enough: every wait gives up at once, and the calls come back from launches per step."""
+    data = model("15 M parameters", 8, 64)
+    prompt = np.array([3, 77, 410, 8], np.int32)
+    results = []
+    for spins in ("131072", "1"):
+        monkeypatch.setenv("SLAI_SMALL_SPINS", spins)
+        b = Backend(0)
+        g = Gguf(data)
+        m = Llama2(b, g, _ffi.MODEL_LLAMA, _ffi.KV_F32)
+        ids, _ = m.generate(prompt, 20)
+        first = Llama2(b, g, _ffi.MODEL_LLAMA, _ffi.KV_F32)
+        results.append((ids, m.forward_logits(20, int(ids[-1])), first.forward_logits(0, 3)))
+        first.destroy(); m.destroy(); g.close(); b.close()
+    assert np.array_equal(results[0][0], results[1][0])
+    assert rel_err(results[1][1], results[0][1]) < 1e-5 and rel_err(results[1][2], results[0][2]) < 1e-5
+
+
+def test_small_models_in_turn(backend):
+    data = [model(s, 8, 64, seed=40 + i) for i, s in enumerate(("15 M parameters", "heads of 64"))]
+    gs = [Gguf(d) for d in data]
+    ms = [Llama2(backend, g, _ffi.MODEL_LLAMA, _ffi.KV_F16) for g in gs]
+    alone = [m.generate(np.array([9, 2], np.int32), 24)[0] for m in ms]
+    mixed = [[], []]
+    for i in range(24):
+        for k, m in enumerate(ms):
+            seq = np.concatenate([[9, 2], alone[k][1:i + 1]]).astype(np.int32)[:max(i + 1, 2)]
+            mixed[k].append(int(m.generate(seq, 1, start_pos=i)[0][0]))
+    for k in range(2):
+        assert mixed[k] == alone[k].tolist()
+    for m in ms:
+        m.destroy()
+    for g in gs:
+        g.close()
