@@ -22,9 +22,12 @@ using namespace lanes;
 // One workgroup = `ngroups` waves; wave w owns column group w of every tile the workgroup visits.  The
 // workgroup walks its tiles with a stride of the segment's workgroup count; the next tile's weights
 // are requested before the current tile is consumed.
+// G = 2: wave w owns the column groups w and w + waves (those of the launch), one after the other: matrices of more than sixteen
+// groups in one launch instead of one for every sixteen, the second adding to what the first wrote (18944 columns x 3584 rows of
+// Q4_K, the down projection of the Qwen2-7B shape: 7.9 + 7.9 us as two launches; a token at position 1210 1838 -> 1755 us, Q8_0 2217 -> 2143).
 // `vec`: which input vector of a batched launch (0 otherwise) and its strides (see GemvBatch).
 struct TiledVec { size_t x_off, emit_off, out0, out1, out2; };
-template <int T, bool DUAL, int LD>
+template <int T, bool DUAL, int LD, int G>
 __device__ __forceinline__ void tiled_body(const GemvTiledParams &p, uint32_t blk, float *smem, const TiledVec vec) {
     using F = Tiled<T>;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, NW = blockDim.x >> 6;
@@ -50,13 +53,22 @@ __device__ __forceinline__ void tiled_body(const GemvTiledParams &p, uint32_t bl
     const uint32_t step = seg.nblocks;
 
     // ---- requests first: activations (small, cache resident), then the first tile's weights --------
-    const uint32_t g = p.group0 + wave;                      // column group owned by this wave
+    const uint32_t g = p.group0 + wave;                      // column group owned by this wave (the first of them)
     const uint32_t cb = g * KQ + kq;
     const bool valid = cb < p.ncb;
     const size_t xoff = (size_t)(valid ? cb : 0) * 256 + lane16;
     DevX X;
 #pragma unroll
     for (int i = 0; i < 16; ++i) X.x[i] = p.x[vec.x_off + xoff + 16 * i];
+    const bool second = G == 2 && (uint32_t)(wave + NW) < p.launch_groups;      // (uniform over the wave)
+    DevX X2;
+    if constexpr (G == 2) {
+        const uint32_t cb2 = (g + NW) * KQ + kq;
+        const bool valid2 = second && cb2 < p.ncb;
+        const size_t xoff2 = (size_t)(valid2 ? cb2 : 0) * 256 + lane16;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) { const float v = p.x[vec.x_off + xoff2 + 16 * i]; X2.x[i] = valid2 ? v : 0.0f; }
+    }
     float nw[16], nb[16];
     if (p.prologue != PRO_NONE) {
 #pragma unroll
@@ -72,7 +84,7 @@ __device__ __forceinline__ void tiled_body(const GemvTiledParams &p, uint32_t bl
     typename F::Data d, e;                                   // e: second matrix of a gated pair
     uint16_t dt = 0, et = 0;
     UnitLoader<T, NM, LD> ld;
-    auto point = [&](uint32_t t) {
+    auto point = [&](uint32_t t, uint32_t g) {
         const size_t off = ((size_t)t * p.ngroups + g) * p.unit_bytes;
         ld.unit[0] = seg.W + off + lane * 16; ld.tailp[0] = seg.W + off + (size_t)F::PT * 1024 + lane * 2; ld.d[0] = &d; ld.t[0] = &dt;
         if constexpr (DUAL) { ld.unit[1] = seg.W2 + off + lane * 16; ld.tailp[1] = seg.W2 + off + (size_t)F::PT * 1024 + lane * 2; ld.d[1] = &e; ld.t[1] = &et; }
@@ -91,11 +103,11 @@ __device__ __forceinline__ void tiled_body(const GemvTiledParams &p, uint32_t bl
     };
     uint32_t tile = blk;
     float old = 0.0f, bias = 0.0f, ew = 0.0f;
-    if (tile < ntiles) { epi_request(tile, old, bias, ew); point(tile); F::lead(ld); }
+    if (tile < ntiles) { epi_request(tile, old, bias, ew); point(tile, g); F::lead(ld); }
 #pragma unroll
     for (int i = 0; i < 16; ++i) X.x[i] = valid ? X.x[i] : 0.0f;
 
-    if (p.prologue != PRO_NONE) {
+    if (G == 1 && p.prologue != PRO_NONE) {
         // every activation is held by ROWS/16 DPP rows; count it once
         const bool counted = valid && (lane & (ROWS - 1)) < 16;
         const float n = (float)p.ncols;
@@ -132,14 +144,18 @@ __device__ __forceinline__ void tiled_body(const GemvTiledParams &p, uint32_t bl
             X.x[i] = valid ? v : 0.0f;
         }
     }
-    if constexpr (T == T_Q6_K) {
+    const auto sums = [](DevX &v) {
+        if constexpr (T == T_Q6_K) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) X.s[i] = row16_sum(X.x[i]);
-    } else {
-        // Q4_K and Q8_0 only use sums over 32 consecutive activations: reduce pairs, keep the odd slots 0
+            for (int i = 0; i < 16; ++i) v.s[i] = row16_sum(v.x[i]);
+        } else {
+            // Q4_K and Q8_0 only use sums over 32 consecutive activations: reduce pairs, keep the odd slots 0
 #pragma unroll
-        for (int i = 0; i < 16; i += 2) { X.s[i] = row16_sum(X.x[i] + X.x[i + 1]); X.s[i + 1] = 0.0f; }
-    }
+            for (int i = 0; i < 16; i += 2) { v.s[i] = row16_sum(v.x[i] + v.x[i + 1]); v.s[i + 1] = 0.0f; }
+        }
+    };
+    sums(X);
+    if constexpr (G == 2) sums(X2);
 
     // ---- tiles ------------------------------------------------------------------------------------------
     while (tile < ntiles) {
@@ -149,9 +165,20 @@ __device__ __forceinline__ void tiled_body(const GemvTiledParams &p, uint32_t bl
         dp[0] = &d; tails[0] = dt;
         if constexpr (DUAL) { dp[1] = &e; tails[1] = et; }
         F::template dotn<NM>(dp, tails, X, o2, ld);
+        if constexpr (G == 2) {
+            static_assert(!DUAL, "two groups per wave: one matrix");
+            if (second) {
+                const float first = o2[0];
+                point(tile, g + NW);
+                F::lead(ld);
+                tails[0] = dt;
+                F::template dotn<NM>(dp, tails, X2, o2, ld);
+                o2[0] += first;
+            }
+        }
         const uint32_t next = tile + step;
         const float old_c = old, bias_c = bias, ew_c = ew;
-        if (next < ntiles) { epi_request(next, old, bias, ew); point(next); F::lead(ld); }
+        if (next < ntiles) { epi_request(next, old, bias, ew); point(next, g); F::lead(ld); }
         float v = o2[0];
         for (int m = ROWS; m < 64; m <<= 1) v += __shfl_xor(v, m, 64);     // across the KQ super-blocks of the wave
         if (lane < ROWS) partial[wave * 64 + lane] = v;
@@ -195,18 +222,18 @@ __device__ __forceinline__ void tiled_body(const GemvTiledParams &p, uint32_t bl
 // with more than two, and so do the narrow ones with six or eight.
 constexpr int lead_stages(int maxt) { return maxt <= 256 ? 4 : 2; }
 
-template <int T, bool DUAL, int MAXT>
+template <int T, bool DUAL, int MAXT, int G>
 __global__ void __launch_bounds__(MAXT) gemv_tiled_kernel(const GemvTiledParams p) {
     extern __shared__ float smem[];
     touch_kernel_arguments<sizeof(GemvTiledParams)>();
-    tiled_body<T, DUAL, lead_stages(MAXT)>(p, blockIdx.x, smem, TiledVec{0, 0, 0, 0, 0});
+    tiled_body<T, DUAL, lead_stages(MAXT), G>(p, blockIdx.x, smem, TiledVec{0, 0, 0, 0, 0});
 }
 
 // The same for several input vectors (a chunk of prompt tokens).  Workgroup i runs on XCD i % 8 and workgroups are
 // dispatched in index order: the bt.n workgroups that walk the same tiles get consecutive indices on ONE XCD,
 // i = ((blk / 8) * bt.n + b) * 8 + blk % 8, so the first request for a piece of a tile brings it from memory and the
 // others find it in that XCD's L2.
-template <int T, bool DUAL, int MAXT>
+template <int T, bool DUAL, int MAXT, int G>
 __global__ void __launch_bounds__(MAXT) gemv_tiled_batch_kernel(const GemvTiledParams p, const GemvBatch bt, uint32_t total_blocks) {
     extern __shared__ float smem[];
     touch_kernel_arguments<((sizeof(GemvTiledParams) + 63) / 64 + 1) * 64>();
@@ -215,37 +242,38 @@ __global__ void __launch_bounds__(MAXT) gemv_tiled_batch_kernel(const GemvTiledP
     if (blk >= total_blocks) return;                            // (uniform) the block count rounded up to the eight XCDs
     const TiledVec vec{(size_t)b * bt.x_stride, (size_t)b * bt.emit_stride,
                        (size_t)b * bt.out_stride[0], (size_t)b * bt.out_stride[1], (size_t)b * bt.out_stride[2]};
-    tiled_body<T, DUAL, lead_stages(MAXT)>(p, blk, smem, vec);
+    tiled_body<T, DUAL, lead_stages(MAXT), G>(p, blk, smem, vec);
 }
 
-template <int T, bool DUAL>
+template <int T, bool DUAL, int G>
 hipError_t go(hipStream_t s, const GemvTiledParams &p, dim3 grid, int NT, size_t smem, const GemvBatch *bt) {
+    // the bound decides the register budget: 256/512 threads leave 256, 768 leave 168, 1024 leave 128 per lane (two groups per wave: nine waves or more)
     if (bt && bt->n > 1) {
         const uint32_t total = grid.x;
         const dim3 g((total + 7) / 8 * 8 * bt->n);
-        if (NT <= 256) gemv_tiled_batch_kernel<T, DUAL, 256><<<g, NT, smem, s>>>(p, *bt, total);
-        else if (NT <= 512) gemv_tiled_batch_kernel<T, DUAL, 512><<<g, NT, smem, s>>>(p, *bt, total);
-        else if (NT <= 768) gemv_tiled_batch_kernel<T, DUAL, 768><<<g, NT, smem, s>>>(p, *bt, total);
-        else gemv_tiled_batch_kernel<T, DUAL, 1024><<<g, NT, smem, s>>>(p, *bt, total);
+        if (G == 1 && NT <= 256) gemv_tiled_batch_kernel<T, DUAL, G == 1 ? 256 : 768, G><<<g, NT, smem, s>>>(p, *bt, total);
+        else if (G == 1 && NT <= 512) gemv_tiled_batch_kernel<T, DUAL, G == 1 ? 512 : 768, G><<<g, NT, smem, s>>>(p, *bt, total);
+        else if (NT <= 768) gemv_tiled_batch_kernel<T, DUAL, 768, G><<<g, NT, smem, s>>>(p, *bt, total);
+        else gemv_tiled_batch_kernel<T, DUAL, 1024, G><<<g, NT, smem, s>>>(p, *bt, total);
         return hipGetLastError();
     }
-    // the bound decides the register budget: 256/512 threads leave 256, 768 leave 168, 1024 leave 128 per lane
-    if (NT <= 256) gemv_tiled_kernel<T, DUAL, 256><<<grid, NT, smem, s>>>(p);
-    else if (NT <= 512) gemv_tiled_kernel<T, DUAL, 512><<<grid, NT, smem, s>>>(p);
-    else if (NT <= 768) gemv_tiled_kernel<T, DUAL, 768><<<grid, NT, smem, s>>>(p);
-    else gemv_tiled_kernel<T, DUAL, 1024><<<grid, NT, smem, s>>>(p);
+    if (G == 1 && NT <= 256) gemv_tiled_kernel<T, DUAL, G == 1 ? 256 : 768, G><<<grid, NT, smem, s>>>(p);
+    else if (G == 1 && NT <= 512) gemv_tiled_kernel<T, DUAL, G == 1 ? 512 : 768, G><<<grid, NT, smem, s>>>(p);
+    else if (NT <= 768) gemv_tiled_kernel<T, DUAL, 768, G><<<grid, NT, smem, s>>>(p);
+    else gemv_tiled_kernel<T, DUAL, 1024, G><<<grid, NT, smem, s>>>(p);
     return hipGetLastError();
 }
 
 template <int T> hipError_t launch_t(slai_ctx *ctx, GemvTiledParams &p, const GemvBatch *bt) {
     if (p.launch_groups == 0) p.launch_groups = p.ngroups;
-    if (p.ngroups == 0 || p.launch_groups > 16 || p.group0 + p.launch_groups > p.ngroups) return hipErrorInvalidValue;
+    if (p.ngroups == 0 || p.launch_groups > GEMV_TILED_LAUNCH_GROUPS || p.group0 + p.launch_groups > p.ngroups) return hipErrorInvalidValue;
     // a partial launch cannot normalise its input (that needs every column) or apply a non-linear epilogue
     if (p.launch_groups != p.ngroups && p.prologue != PRO_NONE) return hipErrorInvalidValue;
     for (int i = 0; i < p.nseg; ++i)
         if ((p.seg[i].flags & GEMV_EMIT) && (i != 0 || !p.emit_w || !p.emit_out || p.seg[i].nrows % 16 || (p.seg[i].flags & GEMV_SILU_GATE)))
             return hipErrorInvalidValue;
-    const int NT = (int)p.launch_groups * 64;
+    const bool two = p.launch_groups > 16;                   // groups per wave
+    const int NT = (int)(two ? (p.launch_groups + 1) / 2 : p.launch_groups) * 64;
     const uint32_t rows = 1u << p.rows_log2;
     bool dual = false;
     uint32_t total_tiles = 0;
@@ -268,8 +296,9 @@ template <int T> hipError_t launch_t(slai_ctx *ctx, GemvTiledParams &p, const Ge
     const int NW = NT / 64;
     const size_t smem = ((size_t)(dual ? 2 : 1) * NW * 64 + NW) * sizeof(float);
     dim3 grid(total);
-    if (dual) return go<T, true>(ctx->stream, p, grid, NT, smem, bt);
-    return go<T, false>(ctx->stream, p, grid, NT, smem, bt);
+    if (two) return dual || p.prologue != PRO_NONE ? hipErrorInvalidValue : go<T, false, 2>(ctx->stream, p, grid, NT, smem, bt);
+    if (dual) return go<T, true, 1>(ctx->stream, p, grid, NT, smem, bt);
+    return go<T, false, 1>(ctx->stream, p, grid, NT, smem, bt);
 }
 
 }  // namespace

@@ -574,12 +574,12 @@ static int gemv_call_impl(slai_ctx *ctx, const GemvCall &c, const char *who, con
         if (m0->ngroups <= 16) {
             e = launch_gemv_tiled(ctx, m0->type, p, batch);
         } else {
-            // wide matrix: balanced slices of at most 16 column groups, one launch each; the first writes (or adds to
-            // the residual), the others accumulate, the last one emits
+            // wide matrix: balanced slices of as many column groups as a launch takes (two per wave), one launch each; the first
+            // writes (or adds to the residual), the others accumulate, the last one emits
             if (c.prologue != PRO_NONE) return set_error(ctx, SLAI_E_SHAPE, std::string(who) + ": no normalisation prologue over more than 16384 columns in 16-row tiles");
             for (int i = 0; i < c.nseg; ++i)
                 if (c.flags[i] & (GEMV_GELU | GEMV_SILU_GATE)) return set_error(ctx, SLAI_E_SHAPE, std::string(who) + ": no non-linear epilogue over more than 16384 columns in 16-row tiles");
-            const uint32_t nchunks = (m0->ngroups + 15) / 16, per = (m0->ngroups + nchunks - 1) / nchunks;
+            const uint32_t nchunks = (m0->ngroups + GEMV_TILED_LAUNCH_GROUPS - 1) / GEMV_TILED_LAUNCH_GROUPS, per = (m0->ngroups + nchunks - 1) / nchunks;
             e = hipSuccess;
             for (uint32_t k = 0; k < nchunks && e == hipSuccess; ++k) {
                 GemvTiledParams q = p;
