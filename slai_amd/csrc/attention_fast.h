@@ -334,8 +334,14 @@ __device__ __forceinline__ void attn_fast_body(const AttnLaunch &a, uint32_t h, 
             }
         } else {
             float *po = a.scratch + ((size_t)h * a.n_splits + split) * (hs + 2);
-            po[tid] = r;
-            if (tid == 0) { po[hs] = (t1 > t0) ? M : -FLT_MAX; po[hs + 1] = (t1 > t0) ? l : 0.0f; }
+            const float pm = (t1 > t0) ? M : -FLT_MAX, pl = (t1 > t0) ? l : 0.0f;
+            if (a.combine_far) {
+                flow_store(po + tid, r);
+                if (tid == 0) { flow_store(po + hs, pm); flow_store(po + hs + 1, pl); }
+            } else {
+                po[tid] = r;
+                if (tid == 0) { po[hs] = pm; po[hs + 1] = pl; }
+            }
         }
     }
 }

@@ -439,6 +439,7 @@ struct AttnLaunch {
     // who have verified that workgroup i of a launch runs on die i mod 8 (slai_ctx::fuse_qkv_attention): the partial
     // results of a head's splits then meet in that die's L2.
     uint32_t *combine_counters;
+    int combine_far;         // (launch_attention) the splits of a head run on several dies: the partial results and the count go through memory
 };
 hipError_t launch_attention(hipStream_t s, const AttnLaunch &a);
 // A chunk of `n` consecutive tokens whose keys and values are already in the caches: token b attends from q + b * q_stride

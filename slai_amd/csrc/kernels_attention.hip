@@ -177,6 +177,7 @@ __global__ void __launch_bounds__(ATT_THREADS) attn_kernel(AttnLaunch a, uint32_
 // a die's workgroups share its L2, so the workgroups of one (kv head, split) are given indices 8 apart: they run at the
 // same time on one die, the rows come from memory once, and the other kv_mul - 1 workgroups find them in that L2.
 //   b = (key mod 8) + 8 * (j + kv_mul * (key / 8)),  key = kv head + n_kv_heads * split,  j = query head within the group
+template <bool FAR>
 __device__ __forceinline__ void combine_head(const float *scratch, float *out, uint32_t hs, uint32_t n_splits, uint32_t h, uint32_t tid, uint32_t nthreads, float *sw);
 
 template <bool F16, int NT, int HS, bool SINGLE, bool PADDED>
@@ -205,13 +206,23 @@ __global__ void __launch_bounds__(NT) attn_fast_kernel(AttnLaunch a, uint32_t ma
             if (threadIdx.x == 0) {
                 uint32_t *counter = a.combine_counters + (size_t)h * 32;
                 uint32_t seen;
-                const uint32_t one = 1;
-                asm volatile("global_atomic_add %0, %1, %2, off sc0\n\ts_waitcnt vmcnt(0)" : "=&v"(seen) : "v"(counter), "v"(one) : "memory");
+                if (a.combine_far) {
+                    seen = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                } else {
+                    const uint32_t one = 1;
+                    asm volatile("global_atomic_add %0, %1, %2, off sc0\n\ts_waitcnt vmcnt(0)" : "=&v"(seen) : "v"(counter), "v"(one) : "memory");
+                }
                 last = seen + 1 == a.n_splits ? 1u : 0u;
-                if (last) *counter = 0u;                               // for the next launch; nobody else touches it any more
+                if (last) {                                            // for the next launch; nobody else touches it any more
+                    if (a.combine_far) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    else *counter = 0u;
+                }
             }
             __syncthreads();
-            if (last) combine_head(a.scratch, a.out, PADDED ? a.head_size : HS, a.n_splits, h, threadIdx.x, NT, sw);
+            if (last) {
+                if (a.combine_far) combine_head<true>(a.scratch, a.out, PADDED ? a.head_size : HS, a.n_splits, h, threadIdx.x, NT, sw);
+                else combine_head<false>(a.scratch, a.out, PADDED ? a.head_size : HS, a.n_splits, h, threadIdx.x, NT, sw);
+            }
         }
     }
 }
@@ -291,12 +302,15 @@ __global__ void rope_theta_kernel(float *out, uint32_t hs, float base) {
 // grid = n_heads, block = 128: merge the per-split (max, sum, unnormalised output) triples.
 // n_splits <= 64: one lane per split computes its weight exp(m_s - M) / L, then every thread
 // accumulates its output elements with independent loads.
+// FAR: the partial results come from other dies of this very launch.
+template <bool FAR>
 __device__ __forceinline__ void combine_head(const float *scratch, float *out, uint32_t hs, uint32_t n_splits, uint32_t h, uint32_t tid, uint32_t nthreads, float *sw /* [64], LDS */) {
+    const auto get = [](const float *q) { if constexpr (FAR) return flow_load(q); else return *q; };
     const float *base = scratch + (size_t)h * n_splits * (hs + 2);
     if (tid < 64) {
         const bool on = tid < n_splits;
-        const float ms = on ? base[(size_t)tid * (hs + 2) + hs] : -FLT_MAX;
-        const float ls = on ? base[(size_t)tid * (hs + 2) + hs + 1] : 0.0f;
+        const float ms = on ? get(base + (size_t)tid * (hs + 2) + hs) : -FLT_MAX;
+        const float ls = on ? get(base + (size_t)tid * (hs + 2) + hs + 1) : 0.0f;
         const float M = wave_max(ms);
         const float w = ls > 0.0f ? expf(ms - M) : 0.0f;
         const float L = wave_sum(w * ls);
@@ -306,13 +320,13 @@ __device__ __forceinline__ void combine_head(const float *scratch, float *out, u
     for (uint32_t e = tid; e < hs; e += nthreads) {
         float acc = 0.0f;
 #pragma unroll 8
-        for (uint32_t s = 0; s < n_splits; ++s) acc = fmaf(sw[s], base[(size_t)s * (hs + 2) + e], acc);
+        for (uint32_t s = 0; s < n_splits; ++s) acc = fmaf(sw[s], get(base + (size_t)s * (hs + 2) + e), acc);
         out[(size_t)h * hs + e] = acc;
     }
 }
 __global__ void __launch_bounds__(128) attn_combine_kernel(const float *scratch, float *out, uint32_t hs, uint32_t n_splits) {
     __shared__ float sw[64];
-    combine_head(scratch, out, hs, n_splits, blockIdx.x, threadIdx.x, blockDim.x, sw);
+    combine_head<false>(scratch, out, hs, n_splits, blockIdx.x, threadIdx.x, blockDim.x, sw);
 }
 
 }  // namespace
@@ -350,7 +364,8 @@ hipError_t launch_attention(hipStream_t s, const AttnLaunch &a_in) {
     // (head, split) of the two-dimensional grid has index head + n_heads * split, a (kv head, split) key of the grouped
     // grid lands on die (kv head + n_kv_heads * split) mod 8.
     const uint32_t per_die = grouped ? a.n_heads / a.kv_mul : a.n_heads;
-    if (a.n_splits <= 1 || !fast || per_die % 8 != 0) a.combine_counters = nullptr;
+    if (a.n_splits <= 1 || !fast) a.combine_counters = nullptr;
+    a.combine_far = a.combine_counters && per_die % 8 != 0 ? 1 : 0;
     const uint32_t max_split_len = (a.seq_len + a.n_splits - 1) / a.n_splits;
     dim3 grid(grouped ? grouped_grid(a) : a.n_heads, grouped ? 1u : a.n_splits);
     // the general kernel keeps its scores in LDS (heads that the fast form masks are refused at the same length)
