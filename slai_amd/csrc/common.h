@@ -373,9 +373,9 @@ hipError_t launch_repack(hipStream_t s, const slai_qmat *m, const uint8_t *src_g
 // rows [row0,row0+nrows) to f32, out[r*out_stride + c]
 hipError_t launch_dequant_rows(hipStream_t s, const slai_qmat *m, uint32_t row0, uint32_t nrows, float *out, size_t out_stride);
 // out[c] = deq(A[row_a][c]) (+ deq(B[row_b][c]) when B != null); row indices read from device memory
-// (zero: nzero words cleared by the same launch)
-hipError_t launch_embed(hipStream_t s, const slai_qmat *a, const int *row_a, const slai_qmat *b, const int *row_b, uint32_t ncols, float *out, uint32_t *zero = nullptr,
-                        uint32_t nzero = 0);
+// (also: n_also words set to also_value by the same launch)
+hipError_t launch_embed(hipStream_t s, const slai_qmat *a, const int *row_a, const slai_qmat *b, const int *row_b, uint32_t ncols, float *out, uint32_t *also = nullptr,
+                        uint32_t n_also = 0, uint32_t also_value = 0);
 
 // ---- element-wise / normalisation ops -------------------------------------------------
 struct VecView { float *p; uint32_t n; uint32_t stride; };  // element i at p[i*stride]
@@ -479,6 +479,7 @@ constexpr uint32_t small_pad(uint32_t floats) { return (floats + 31) & ~31u; }  
 struct SmallLayer {                                            // packed rows (row layout); biases are optional
     const uint8_t *q, *k, *v, *o, *gate, *up, *down;
     const float *norm1, *norm2, *qb, *kb, *vb;
+    const float *norm1b, *norm2b, *ob, *upb, *downb;          // GPT-2: LayerNorm offsets and the other biases (its first FFN matrix is `up`, q, k and v are thirds of one matrix)
     void *kcache, *vcache;
 };
 struct SmallParams {
@@ -497,6 +498,11 @@ struct SmallParams {
 };
 bool small_shape_ok(const SmallParams &p);
 hipError_t launch_decode_small(hipStream_t s, const SmallParams &p);
+// The same for GPT-2 over the whole device (kernels_decode_mid.hip); `work` holds FLOW_EMPTY at the start of a launch, no counters
+constexpr uint32_t MID_WGS = 256;
+bool mid_shape_ok(const SmallParams &p);
+hipError_t launch_decode_mid(hipStream_t s, const SmallParams &p);
+hipError_t mid_capacity(const SmallParams &p, int device, uint32_t *resident);
 
 // ---- the whole layer stack of a Llama-2 token in one resident launch (kernels_decode_persistent.hip) ----------------------
 // A matrix, vector or cache as the kernel sees it: address and size in bytes.  Every access of the kernel to it goes

@@ -257,8 +257,8 @@ int wide_rows(slai_ctx *ctx, int nseg, const WideGemmSeg *segs, const uint8_t *x
     return SLAI_OK;
 }
 
-// The layers of a token as one resident launch on one die (kernels_decode_small.hip), for the models whose shapes and formats it covers.  It
-// reads packed rows: matrices in tiles get copies as rows (one block of memory, bounded like WideMats).
+// The layers of a token as one resident launch, for the models whose shapes and formats it covers: small Llamas on one die
+// (kernels_decode_small.hip), GPT-2 over the whole device (kernels_decode_mid.hip).  It reads packed rows: matrices in tiles get copies as rows (one block of memory, bounded like WideMats).
 struct SmallForm {
     bool ready = false;
     SmallParams params;
@@ -268,6 +268,7 @@ struct SmallForm {
     uint8_t *block = nullptr;
 
     uint32_t counter_words() const { return params.n_layers * SMALL_STEPS * 32; }
+    uint32_t work_words() const { return params.n_layers * params.work_stride; }
     // What the kernel reads of m: m itself, or its copy as rows (memory assigned by `make`)
     slai_qmat *take(slai_qmat *m) {
         if (!m->tiled) return m;
@@ -293,15 +294,22 @@ struct SmallForm {
         }
         return true;
     }
-    // `params` but for the buffers, and the layers' vectors and caches; mats(l): its seven matrices (q, k, v, o, gate, up, down)
-    template <class Mats> int setup(slai_ctx *ctx, std::vector<SmallLayer> &host, Mats &&mats) {
+    // `params` but for the buffers, and the layers' vectors and caches; mats(l): its seven matrices (q, k, v, o, gate, up, down; null: none)
+    template <class Mats> int setup(slai_ctx *ctx, std::vector<SmallLayer> &host, bool one_die, Mats &&mats) {
         SmallParams &p = params;
-        if (!ctx->persistent || !ctx->fuse_qkv_attention || !ctx->handoff_counters || !small_shape_ok(p)) return SLAI_OK;
+        if (!ctx->persistent || !ctx->handoff_counters) return SLAI_OK;
+        if (one_die) {
+            if (!ctx->fuse_qkv_attention || !small_shape_ok(p)) return SLAI_OK;
+        } else {
+            uint32_t resident = 0;
+            if (!mid_shape_ok(p) || mid_capacity(p, ctx->device, &resident) != hipSuccess || resident < MID_WGS) return SLAI_OK;
+        }
         p.stride_e = (uint32_t)device_row_stride(p.type, p.dim); p.stride_h = (uint32_t)device_row_stride(p.type, p.hidden);
         std::vector<std::array<slai_qmat *, 7>> rows(host.size());
         for (size_t l = 0; l < host.size(); ++l) {
             rows[l] = mats(l);
             for (slai_qmat *&m : rows[l]) {
+                if (!m) continue;
                 if (m->type != p.type) { drop(ctx); return SLAI_OK; }
                 m = take(m);
             }
@@ -310,7 +318,8 @@ struct SmallForm {
         for (size_t l = 0; l < host.size(); ++l) {
             const auto &r = rows[l];
             SmallLayer &d = host[l];
-            d.q = r[0]->dptr; d.k = r[1]->dptr; d.v = r[2]->dptr; d.o = r[3]->dptr; d.gate = r[4]->dptr; d.up = r[5]->dptr; d.down = r[6]->dptr;
+            const uint8_t **at[7] = {&d.q, &d.k, &d.v, &d.o, &d.gate, &d.up, &d.down};
+            for (int i = 0; i < 7; ++i) *at[i] = r[i] ? r[i]->dptr : nullptr;
         }
         p.work_stride = small_pad(p.dim + 2 * p.kvd) + 3 * small_pad(p.dim) + small_pad(p.hidden);
         TRY(slai_buffer_create(ctx, host.size() * sizeof(SmallLayer), SLAI_DT_U8, STORAGE | COPY_DST, &layers));
@@ -750,7 +759,7 @@ int slai_llama2::small_setup() {
         d.norm1 = vec(w.attn_norm); d.norm2 = vec(w.ffn_norm); d.qb = vec(w.attn_q_bias); d.kb = vec(w.attn_k_bias); d.vb = vec(w.attn_v_bias);
         d.kcache = state.key_cache[l].buf->dptr; d.vcache = state.value_cache[l].buf->dptr;
     }
-    return small.setup(ctx, host, [&](size_t l) {
+    return small.setup(ctx, host, true, [&](size_t l) {
         const Llama2LayerWeights &w = weights.layers[l];
         return std::array<slai_qmat *, 7>{w.attn_q, w.attn_k, w.attn_v, w.attn_output, w.ffn_gate, w.ffn_up, w.ffn_down};
     });
@@ -1605,9 +1614,11 @@ struct slai_gpt2 {
     uint32_t attn_splits = 1;
 
     int load(const slai_gguf *g);
-    int enqueue_fused(int sampler, int form = 0);   // 0: stop at the logits, 1: greedy pick + loop state, 2: temperature / top-p pick + loop state, 3: the same without a top-p cut (one form only)
-    int form_at(uint32_t) const { return 0; }
-    bool drop_small() { return false; }
+    int enqueue_fused(int sampler, int form = 0);   // 0: stop at the logits, 1: greedy pick + loop state, 2: temperature / top-p pick + loop state, 3: the same without a top-p cut (form 3: the layers as one launch)
+    int form_at(uint32_t) const { return small.ready ? 3 : 0; }
+    SmallForm small;                              // form 3
+    int small_setup();
+    bool drop_small() { const bool was = small.ready; small.ready = false; return was; }   // from now on one launch per step
 
     // Prompt tokens in chunks of up to 32 on the matrix cores (see slai_llama2::enqueue_chunk_gemm); row-major x and qkv,
     // quad-major xn (normalised rows, then the attention output) and h.
@@ -1729,19 +1740,44 @@ int slai_gpt2::load(const slai_gguf *gg) {
     attn_splits = pick_attn_splits(ctx, params.n_head, params.n_seq);
     TRY(ensure_attn_scratch(ctx, attention_scratch_floats(params.n_head, E / params.n_head, attn_splits)));
     TRY(loop_init(ctx, loop, params.n_seq + 1));
+    TRY(small_setup());
     return slai_synchronize(ctx);
 }
 
+int slai_gpt2::small_setup() {
+    TRY(handoff_reserve(ctx, params.n_head));
+    if (layers.empty()) return SLAI_OK;
+    SmallParams &p = small.params;
+    p.n_layers = params.n_layer; p.dim = params.n_embd; p.kvd = params.n_embd; p.hidden = params.ff_len; p.n_heads = params.n_head; p.kv_mul = 1; p.head_size = params.n_embd / params.n_head;
+    p.seq_len = params.n_seq; p.type = layers[0].c_attn_attn_w->type; p.kv_f16 = kv_dtype == SLAI_KV_F16; p.rope_variant = -1; p.eps = 1.0e-5f;
+    p.x = (float *)layer_input.buf->dptr; p.pos_ptr = (const uint32_t *)&((DecodeState *)loop.state->dptr)->pos;
+    std::vector<SmallLayer> host(params.n_layer);
+    const auto vec = [](const GpuTensor &t) { return (const float *)t.buf->dptr; };
+    for (uint32_t l = 0; l < params.n_layer; ++l) {
+        const Gpt2Layer &w = layers[l];
+        SmallLayer &d = host[l];
+        d.norm1 = vec(w.ln_1_g); d.norm1b = vec(w.ln_1_b); d.norm2 = vec(w.ln_2_g); d.norm2b = vec(w.ln_2_b);
+        d.qb = vec(w.c_attn_attn_b); d.ob = vec(w.c_attn_proj_b); d.upb = vec(w.c_mlp_fc_b); d.downb = vec(w.c_mlp_proj_b);
+        d.kcache = w.key_cache.buf->dptr; d.vcache = w.value_cache.buf->dptr;
+    }
+    return small.setup(ctx, host, false, [&](size_t l) {
+        const Gpt2Layer &w = layers[l];
+        return std::array<slai_qmat *, 7>{w.c_attn_attn_w, nullptr, nullptr, w.c_attn_proj_w, nullptr, w.c_mlp_fc_w, w.c_mlp_proj_w};
+    });
+}
+
 // gpt2/cpu.rs:224-383 as fused kernels (LayerNorm eps 1e-5: ops/layernorm.rs:105)
-int slai_gpt2::enqueue_fused(int sampler, int) {
+int slai_gpt2::enqueue_fused(int sampler, int form) {
     DecodeState *ds = (DecodeState *)loop.state->dptr;
     const uint32_t E = params.n_embd;
     float *x = (float *)layer_input.buf->dptr, *att_out = (float *)curr_768.buf->dptr, *qkv = (float *)curr_2304.buf->dptr,
           *h = (float *)curr_3072.buf->dptr, *logits = (float *)curr_vocab.buf->dptr;
     const float eps = 1.0e-5f;
     // :227-228 wte[:,tok] + wpe[:,pos]
-    SLAI_HIP_TRY(ctx, launch_embed(ctx->stream, wte, &ds->token, wpe, &ds->pos, E, x));
-    for (uint32_t l = 0; l < params.n_layer; ++l) {
+    const bool one_launch = form == 3 && small.ready;
+    SLAI_HIP_TRY(ctx, launch_embed(ctx->stream, wte, &ds->token, wpe, &ds->pos, E, x, one_launch ? (uint32_t *)small.params.work : nullptr, one_launch ? small.work_words() : 0, 0xFFFFFFFFu));
+    if (one_launch) SLAI_HIP_TRY(ctx, launch_decode_mid(ctx->stream, small.params));
+    for (uint32_t l = 0; l < params.n_layer && !one_launch; ++l) {
         Gpt2Layer &w = layers[l];
         {   // :235-255 LayerNorm*g+b, qkv GEMV + bias
             GemvCall c;
@@ -1953,6 +1989,7 @@ SLAI_EXPORT void slai_gpt2_destroy(slai_gpt2 *m) {
     for (GpuTensor *t : {&m->chunk.x, &m->chunk.xn, &m->chunk.qkv, &m->chunk.h}) t->destroy(ctx);
     for (slai_buffer *b : {m->chunk.positions, m->chunk.tokens}) if (b) slai_buffer_destroy(ctx, b);
     m->wide.destroy(ctx);
+    m->small.drop(ctx);
     delete m;
 }
 
@@ -1969,8 +2006,12 @@ SLAI_EXPORT int slai_gpt2_forward_logits(slai_gpt2 *m, uint32_t pos, uint32_t to
     if (pos >= m->params.n_seq || token >= m->params.n_vocab) return set_error(ctx, SLAI_E_ARG, "slai_gpt2_forward_logits: position or token out of range");
     DecodeState ds{(int)pos, (int)token, 0, 0};
     TRY(slai_write_buffer(ctx, m->loop.state, 0, &ds, sizeof ds));
-    TRY(m->enqueue_fused(false));
+    TRY(m->enqueue_fused(0, m->form_at(pos)));
     TRY(slai_synchronize(ctx));
+    if (const int rc = handoff_check(ctx)) {
+        if (!m->drop_small()) return rc;
+        return slai_gpt2_forward_logits(m, pos, token, logits_out);
+    }
     if (logits_out) TRY(slai_read_buffer(ctx, m->curr_vocab.buf, 0, logits_out, (size_t)m->params.n_vocab * 4));
     return SLAI_OK;
 }

@@ -87,9 +87,10 @@ __global__ void dequant_rows_kernel(QMatDev m, uint32_t row0, uint32_t nrows, fl
     }
 }
 
-__global__ void embed_kernel(QMatDev a, const int *row_a, QMatDev b, const int *row_b, int has_b, uint32_t ncols, float *out, uint32_t *zero, uint32_t nzero) {
+__global__ void embed_kernel(QMatDev a, const int *row_a, QMatDev b, const int *row_b, int has_b, uint32_t ncols, float *out, uint32_t *also, uint32_t n_also,
+                             uint32_t also_value) {
     const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-    for (uint32_t i = c; i < nzero; i += gridDim.x * blockDim.x) zero[i] = 0u;
+    for (uint32_t i = c; i < n_also; i += gridDim.x * blockDim.x) also[i] = also_value;
     if (c >= ncols) return;
     float v = qmat_elem(a, (uint32_t)*row_a, c);
     // gpt2/cpu.rs:227-228: token embedding first, then += position embedding
@@ -143,9 +144,11 @@ hipError_t launch_dequant_rows(hipStream_t s, const slai_qmat *m, uint32_t row0,
     return hipGetLastError();
 }
 
-hipError_t launch_embed(hipStream_t s, const slai_qmat *a, const int *row_a, const slai_qmat *b, const int *row_b, uint32_t ncols, float *out, uint32_t *zero,
-                        uint32_t nzero) {
-    embed_kernel<<<(ncols + 255) / 256, 256, 0, s>>>(qmat_dev(a), row_a, qmat_dev(b), row_b, b ? 1 : 0, ncols, out, zero, zero ? nzero : 0u);
+hipError_t launch_embed(hipStream_t s, const slai_qmat *a, const int *row_a, const slai_qmat *b, const int *row_b, uint32_t ncols, float *out, uint32_t *also, uint32_t n_also,
+                        uint32_t also_value) {
+    if (!also) n_also = 0;
+    const uint32_t grid = std::max((ncols + 255) / 256, std::min((n_also + 1023) / 1024, 256u));
+    embed_kernel<<<grid, 256, 0, s>>>(qmat_dev(a), row_a, qmat_dev(b), row_b, b ? 1 : 0, ncols, out, also, n_also, also_value);
     return hipGetLastError();
 }
 

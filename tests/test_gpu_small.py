@@ -1,4 +1,4 @@
-"""The layers of a small model's token as one launch on one die (kernels_decode_small.hip): shapes at the edges of what it covers (two
+"""The layers of a small model's token as one launch, on one die (kernels_decode_small.hip) or over the device (kernels_decode_mid.hip): shapes at the edges of what it covers (two
 rows per wave, heads of 8 to 64, grouped queries, biases and NeoX pairs), both formats and cache types, positions past one and two passes of
 its attention (120 positions each), against the oracle; a launch that gives up; several models taking turns on one context."""
 import numpy as np
@@ -7,7 +7,8 @@ import pytest
 from gpu_common import backend, rel_err  # noqa: F401
 from slai_amd import _ffi
 from slai_amd import gguf_writer as gw
-from slai_amd.runtime import Backend, Gguf, Llama2
+from helpers import OracleGguf
+from slai_amd.runtime import Backend, Gguf, Gpt2, Llama2
 from test_gpu_models import check_llama
 
 pytestmark = pytest.mark.gpu
@@ -80,3 +81,62 @@ def test_small_models_in_turn(backend):
         m.destroy()
     for g in gs:
         g.close()
+
+
+# GPT-2 shapes: embedding, FFN, heads, context
+GPT2 = {
+    "small": (768, 3072, 12, 256),         # nine rows a workgroup, three waves a row of the FFN's width
+    "widest": (1024, 2560, 16, 64),        # twelve rows a workgroup
+    "heads of 8, most workgroups without a row": (96, 160, 12, 64),
+    "heads of 40": (320, 1056, 8, 64),     # rows end inside a chunk of 64
+}
+
+
+def check_gpt2(backend, data, kv_f16, n_prompt, steps, vocab):
+    g = OracleGguf(data); L = g.L
+    om = L.slo_gpt2_from_gguf(g.h, int(kv_f16))
+    prompt = np.random.Generator(np.random.PCG64(8)).integers(0, vocab, n_prompt).astype(np.int32)
+    ref, ref_logits = np.zeros(steps, np.int32), np.zeros((steps, vocab), np.float32)
+    assert L.slo_gpt2_generate(om, prompt.ctypes.data, n_prompt, 0, steps, -1, ref.ctypes.data, ref_logits.ctypes.data) == steps
+    gg = Gguf(data)
+    m = Gpt2(backend, gg, _ffi.KV_F16 if kv_f16 else _ffi.KV_F32)
+    tok = int(prompt[0])
+    for pos in range(steps):
+        assert rel_err(m.forward_logits(pos, tok), ref_logits[pos]) < 1e-2
+        tok = int(ref[pos])
+    m.destroy()
+    m = Gpt2(backend, gg, _ffi.KV_F16 if kv_f16 else _ffi.KV_F32)
+    got, _ = m.generate(prompt, steps)
+    assert np.array_equal(got, ref)
+    m.destroy(); gg.close(); L.slo_gpt2_free(om); g.close()
+
+
+@pytest.mark.parametrize("kv_f16", [False, True])
+@pytest.mark.parametrize("wtype", [8, 2], ids=["q8_0", "q4_0"])
+@pytest.mark.parametrize("shape", sorted(GPT2))
+def test_gpt2_in_one_launch(backend, shape, wtype, kv_f16):
+    dim, hidden, heads, seq = GPT2[shape]
+    data = gw.gpt2_gguf(n_embd=dim, n_layer=2, n_head=heads, ff_len=hidden, vocab=700, n_seq=seq, wtype=wtype, seed=61, std=0.05)
+    # ("small": positions past two passes of the attention)
+    check_gpt2(backend, data, kv_f16, seq - 30 if shape == "small" else 7, seq - 4 if shape == "small" else 30, 700)
+
+
+def test_gpt2_in_one_launch_single_layer(backend):
+    data = gw.gpt2_gguf(n_embd=64, n_layer=1, n_head=2, ff_len=128, vocab=700, n_seq=32, wtype=8, seed=62, std=0.08)
+    check_gpt2(backend, data, False, 4, 20, 700)
+
+
+def test_gpt2_gives_up_and_the_call_is_repeated(monkeypatch):
+    data = gw.gpt2_gguf(n_embd=768, n_layer=2, n_head=12, ff_len=3072, vocab=700, n_seq=64, wtype=8, seed=63, std=0.05)
+    results = []
+    for spins in ("131072", "1"):
+        monkeypatch.setenv("SLAI_SMALL_SPINS", spins)
+        b = Backend(0)
+        g = Gguf(data)
+        m = Gpt2(b, g, _ffi.KV_F32)
+        ids, _ = m.generate(np.array([3, 77], np.int32), 20)
+        first = Gpt2(b, g, _ffi.KV_F32)
+        results.append((ids, m.forward_logits(20, int(ids[-1])), first.forward_logits(0, 3)))
+        first.destroy(); m.destroy(); g.close(); b.close()
+    assert np.array_equal(results[0][0], results[1][0])
+    assert rel_err(results[1][1], results[0][1]) < 1e-5 and rel_err(results[1][2], results[0][2]) < 1e-5
