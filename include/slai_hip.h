@@ -335,7 +335,7 @@ int slai_llama2_generate_sampled(slai_llama2 *m, const int32_t *prompt, uint32_t
  * this fills the caches for positions start_pos .. start_pos+n_tokens-1 with `chunk` tokens per pass over the
  * weights and computes no logits (chunk: 0 = the path's default, 1 = token by token, at most 64).  Generation then
  * continues with slai_llama2_generate(prompt, n_prompt, n_prompt - 1, ...).
- * Chunks of more than 32 tokens (chunk 0: passes of up to 1024) of a model whose layer matrices lie in tiles, with heads of 48, 64
+ * Chunks of more than 32 tokens (chunk 0: passes of 8 to 1024) of a model whose layer matrices lie in tiles, with heads of 48, 64
  * or 128 elements (the sizes the pass's attention is built for), are multiplied on the half-precision matrix cores: the
  * quantised integers as they are, activations as an f16 head and an f16 remainder (about 23 bits down to 2^-14, fp32
  * accumulation).  Models of Q8_0 / Q4_0 in rows that are no multiple of 256 do so with chunk 0 from 4 tokens on, over copies in
@@ -353,7 +353,7 @@ int slai_llama2_prefill(slai_llama2 *m, const int32_t *tokens, uint32_t n_tokens
 int slai_llama2_prefill_supported(const slai_llama2 *m);
 uint32_t slai_llama2_prefill_fp32_repeats(const slai_llama2 *m);
 /* Which form the per-token loop of this model takes: 0 = one launch per step of `Llama2::launch` (transformer.rs:316-381;
- * four to five per layer), 1 = the whole layer stack and the output matrix in one resident launch per token (widths of
+ * four to five per layer; small Q8_0 / Q4_0 models up to 512 columns: their layers in one launch on one die, the rest per step), 1 = the whole layer stack and the output matrix in one resident launch per token (widths of
  * 1024 .. 4096 in steps of 1024, as many cache heads as query heads of size 128, Q4_K / Q5_K / Q6_K mixes, gate / up in
  * Q4_K; a context created with SLAI_PERSISTENT=0 in the environment never takes it).  The form is chosen per token: a model
  * of form 1 takes the resident launch at positions below SLAI_RESIDENT_MAX_POS (environment, default 2048) and one launch
@@ -393,8 +393,8 @@ int slai_gpt2_generate(slai_gpt2 *m, const int32_t *prompt, uint32_t n_prompt, u
 int slai_gpt2_generate_sampled(slai_gpt2 *m, const int32_t *prompt, uint32_t n_prompt, uint32_t start_pos,
                                uint32_t n_steps, float temperature, float topp, uint64_t seed, int32_t *out_tokens,
                                float *elapsed_ms);
-/* slai_llama2_prefill for GPT-2 (gpt2/cpu.rs:225-383 for a chunk of tokens; no counterpart in the reference): passes of up to
- * 1024 tokens, or 32 and fewer, on the matrix cores as there where every layer matrix has a tiled layout
+/* slai_llama2_prefill for GPT-2 (gpt2/cpu.rs:225-383 for a chunk of tokens; no counterpart in the reference): passes of 8
+ * to 1024 tokens (chunk 0), or 32 and fewer, on the matrix cores as there where every layer matrix has a tiled layout
  * (slai_gpt2_prefill_supported() == 2; f16 head + remainder pairs with the fp32 repeat of slai_llama2_prefill, counted by
  * slai_gpt2_prefill_fp32_repeats), token by token with the same result otherwise (0). */
 int slai_gpt2_prefill(slai_gpt2 *m, const int32_t *tokens, uint32_t n_tokens, uint32_t start_pos, uint32_t chunk,
