@@ -353,12 +353,15 @@ int slai_llama2_prefill(slai_llama2 *m, const int32_t *tokens, uint32_t n_tokens
 int slai_llama2_prefill_supported(const slai_llama2 *m);
 uint32_t slai_llama2_prefill_fp32_repeats(const slai_llama2 *m);
 /* Which form the per-token loop of this model takes: 0 = one launch per step of `Llama2::launch` (transformer.rs:316-381;
- * four to five per layer; small Q8_0 / Q4_0 models up to 512 columns: their layers in one launch on one die, the rest per step), 1 = the whole layer stack and the output matrix in one resident launch per token (widths of
+ * four to five per layer; or a small model's layers in one launch: slai_llama2_decode_form_at), 1 = the whole layer stack and the output matrix in one resident launch per token (widths of
  * 1024 .. 4096 in steps of 1024, as many cache heads as query heads of size 128, Q4_K / Q5_K / Q6_K mixes, gate / up in
  * Q4_K; a context created with SLAI_PERSISTENT=0 in the environment never takes it).  The form is chosen per token: a model
  * of form 1 takes the resident launch at positions below SLAI_RESIDENT_MAX_POS (environment, default 2048) and one launch
  * per step beyond, with the same caches and loop state.  Results are the same to within summation order. */
 int slai_llama2_decode_form(const slai_llama2 *m);
+/* The form that the next token at position `pos` takes (generate, and forward_logits with fused kernels): 0 = one launch per
+ * step, 1 = the resident launch, 2 = a small model's layers in one launch (embedding row, output matrix and pick per step). */
+int slai_llama2_decode_form_at(const slai_llama2 *m, uint32_t pos);
 /* Measurement aid without a reference counterpart (profilers see the resident launch as one kernel): runs one token at
  * (pos, token) with in-kernel time stamps and returns them, n_workgroups x stamps_per_workgroup 64-bit ticks of the
  * constant 100 MHz clock; per workgroup 16 per layer -- 4 per phase (q/k/v + attention, output projection, gate/up, down
@@ -393,6 +396,8 @@ int slai_gpt2_generate(slai_gpt2 *m, const int32_t *prompt, uint32_t n_prompt, u
 int slai_gpt2_generate_sampled(slai_gpt2 *m, const int32_t *prompt, uint32_t n_prompt, uint32_t start_pos,
                                uint32_t n_steps, float temperature, float topp, uint64_t seed, int32_t *out_tokens,
                                float *elapsed_ms);
+/* slai_llama2_decode_form_at for GPT-2: 0 or 2 */
+int slai_gpt2_decode_form_at(const slai_gpt2 *m, uint32_t pos);
 /* slai_llama2_prefill for GPT-2 (gpt2/cpu.rs:225-383 for a chunk of tokens; no counterpart in the reference): passes of 8
  * to 1024 tokens (chunk 0), or 32 and fewer, on the matrix cores as there where every layer matrix has a tiled layout
  * (slai_gpt2_prefill_supported() == 2; f16 head + remainder pairs with the fp32 repeat of slai_llama2_prefill, counted by

@@ -1276,6 +1276,10 @@ SLAI_EXPORT void slai_llama2_destroy(slai_llama2 *m) {
 
 SLAI_EXPORT int slai_llama2_decode_form(const slai_llama2 *m) { return m && m->persistent.ready ? 1 : 0; }
 
+// the forms of form_at as the header counts them (the resident launch for far positions is one of the two kernels of form 1)
+static int form_for_callers(int form) { return form == 3 ? 2 : form == 0 ? 0 : 1; }
+SLAI_EXPORT int slai_llama2_decode_form_at(const slai_llama2 *m, uint32_t pos) { return m ? form_for_callers(m->form_at(pos)) : 0; }
+
 // One token at (pos, token) through the resident launch with its time stamps switched on: per workgroup 16 stamps per
 // layer (four per phase: entered, input staged, multiplied, reduced) and 8 for the output matrix, in ticks of the
 // constant 100 MHz clock.  The caches are left as any forward pass at that position leaves them.
@@ -2015,6 +2019,8 @@ SLAI_EXPORT int slai_gpt2_forward_logits(slai_gpt2 *m, uint32_t pos, uint32_t to
     if (logits_out) TRY(slai_read_buffer(ctx, m->curr_vocab.buf, 0, logits_out, (size_t)m->params.n_vocab * 4));
     return SLAI_OK;
 }
+
+SLAI_EXPORT int slai_gpt2_decode_form_at(const slai_gpt2 *m, uint32_t pos) { return m ? form_for_callers(m->form_at(pos)) : 0; }
 
 SLAI_EXPORT int slai_gpt2_generate(slai_gpt2 *m, const int32_t *prompt, uint32_t n_prompt, uint32_t start_pos, uint32_t n_steps,
                                    int32_t *out_tokens, float *elapsed_ms) {

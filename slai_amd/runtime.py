@@ -537,6 +537,10 @@ class Llama2:
         """0: one launch per step of the layer loop, 1: the whole layer stack in one resident launch per token."""
         return int(self.b.L.slai_llama2_decode_form(self.h))
 
+    def decode_form_at(self, pos):
+        """The form of the next token at `pos` -- 0: one launch per step, 1: resident, 2: a small model's layers in one launch."""
+        return int(self.b.L.slai_llama2_decode_form_at(self.h, pos))
+
     def trace_token(self, pos, token):
         """In-kernel time stamps of one token through the resident launch: uint64 [workgroups, 16 * n_layers + 8], ticks of
         the 100 MHz clock (see slai_llama2_trace_token)."""
@@ -626,6 +630,10 @@ class Gpt2:
         self.b.check(self.b.L.slai_gpt2_generate_sampled(self.h, prompt.ctypes.data, prompt.size, start_pos, n_steps, temperature, topp,
                                                          seed, out.ctypes.data, C.byref(ms)))
         return out, ms.value
+
+    def decode_form_at(self, pos):
+        """The form of the next token at `pos` -- 0: one launch per step, 2: the layers in one launch."""
+        return int(self.b.L.slai_gpt2_decode_form_at(self.h, pos))
 
     def prefill_path(self):
         """2: matrix-core GEMM, 0: the token-by-token loop."""

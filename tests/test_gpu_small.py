@@ -12,6 +12,7 @@ from slai_amd.runtime import Backend, Gguf, Gpt2, Llama2
 from test_gpu_models import check_llama
 
 pytestmark = pytest.mark.gpu
+LAUNCHES, ONE_LAUNCH = 0, 2                # decode_form_at
 
 SHAPES = {                                 # dim, hidden, heads, kv heads
     "15 M parameters": (288, 768, 6, 6),
@@ -28,23 +29,48 @@ def model(shape, wtype, seq, seed=31, **kw):
                          norm_random=True, **kw)
 
 
+def llama_form(backend, data, pos=0, model_type=_ffi.MODEL_LLAMA):
+    g = Gguf(data)
+    m = Llama2(backend, g, model_type, _ffi.KV_F16)
+    form = m.decode_form_at(pos)
+    m.destroy(); g.close()
+    return form
+
+
 @pytest.mark.parametrize("kv_f16", [False, True])
 @pytest.mark.parametrize("wtype", [8, 2], ids=["q8_0", "q4_0"])
 @pytest.mark.parametrize("shape", sorted(SHAPES))
 def test_small_shapes(backend, shape, wtype, kv_f16):
     prompt = np.random.Generator(np.random.PCG64(3)).integers(0, 500, 9)
-    check_llama(backend, model(shape, wtype, 64), prompt, 40, kv_f16=kv_f16)
+    data = model(shape, wtype, 64)
+    assert llama_form(backend, data, 63) == ONE_LAUNCH
+    check_llama(backend, data, prompt, 40, kv_f16=kv_f16)
+
+
+@pytest.mark.parametrize("wtype", [8, 2], ids=["q8_0", "q4_0"])
+@pytest.mark.parametrize("shape", sorted(SHAPES))
+def test_small_shapes_in_launches(monkeypatch, shape, wtype):
+    """The form that a launch which gives up falls back to."""
+    monkeypatch.setenv("SLAI_PERSISTENT", "0")
+    b = Backend(0)
+    data = model(shape, wtype, 64)
+    assert llama_form(b, data) == LAUNCHES
+    check_llama(b, data, np.random.Generator(np.random.PCG64(3)).integers(0, 500, 9), 40, kv_f16=wtype == 2)
+    b.close()
 
 
 def test_small_bias_neox(backend):
     data = model("widest", 8, 64, arch="qwen2", bias=True, rope_base=1000000.0, rms_eps=1e-6)
+    assert llama_form(backend, data, model_type=_ffi.MODEL_QWEN2) == ONE_LAUNCH
     check_llama(backend, data, [5, 400, 17], 30, model_type=_ffi.MODEL_QWEN2, neox=1, name=b"qwen2")
 
 
 @pytest.mark.parametrize("kv_f16", [False, True])
 def test_small_positions_beyond_one_pass(backend, kv_f16):
     prompt = np.random.Generator(np.random.PCG64(4)).integers(0, 500, 230)
-    check_llama(backend, model("15 M parameters", 8, 256), prompt, 252, kv_f16=kv_f16, check_logit_steps=125)
+    data = model("15 M parameters", 8, 256)
+    assert llama_form(backend, data, 255) == ONE_LAUNCH
+    check_llama(backend, data, prompt, 252, kv_f16=kv_f16, check_logit_steps=125)
 
 
 def test_small_gives_up_and_the_call_is_repeated(monkeypatch):
@@ -57,7 +83,9 @@ def test_small_gives_up_and_the_call_is_repeated(monkeypatch):
         b = Backend(0)
         g = Gguf(data)
         m = Llama2(b, g, _ffi.MODEL_LLAMA, _ffi.KV_F32)
+        assert m.decode_form_at(0) == ONE_LAUNCH
         ids, _ = m.generate(prompt, 20)
+        assert m.decode_form_at(0) == (LAUNCHES if spins == "1" else ONE_LAUNCH)
         first = Llama2(b, g, _ffi.MODEL_LLAMA, _ffi.KV_F32)
         results.append((ids, m.forward_logits(20, int(ids[-1])), first.forward_logits(0, 3)))
         first.destroy(); m.destroy(); g.close(); b.close()
@@ -69,6 +97,7 @@ def test_small_models_in_turn(backend):
     data = [model(s, 8, 64, seed=40 + i) for i, s in enumerate(("15 M parameters", "heads of 64"))]
     gs = [Gguf(d) for d in data]
     ms = [Llama2(backend, g, _ffi.MODEL_LLAMA, _ffi.KV_F16) for g in gs]
+    assert [m.decode_form_at(0) for m in ms] == [ONE_LAUNCH] * 2
     alone = [m.generate(np.array([9, 2], np.int32), 24)[0] for m in ms]
     mixed = [[], []]
     for i in range(24):
@@ -92,7 +121,7 @@ GPT2 = {
 }
 
 
-def check_gpt2(backend, data, kv_f16, n_prompt, steps, vocab):
+def check_gpt2(backend, data, kv_f16, n_prompt, steps, vocab, form=ONE_LAUNCH):
     g = OracleGguf(data); L = g.L
     om = L.slo_gpt2_from_gguf(g.h, int(kv_f16))
     prompt = np.random.Generator(np.random.PCG64(8)).integers(0, vocab, n_prompt).astype(np.int32)
@@ -100,6 +129,7 @@ def check_gpt2(backend, data, kv_f16, n_prompt, steps, vocab):
     assert L.slo_gpt2_generate(om, prompt.ctypes.data, n_prompt, 0, steps, -1, ref.ctypes.data, ref_logits.ctypes.data) == steps
     gg = Gguf(data)
     m = Gpt2(backend, gg, _ffi.KV_F16 if kv_f16 else _ffi.KV_F32)
+    assert m.decode_form_at(0) == m.decode_form_at(steps - 1) == form
     tok = int(prompt[0])
     for pos in range(steps):
         assert rel_err(m.forward_logits(pos, tok), ref_logits[pos]) < 1e-2
@@ -121,6 +151,14 @@ def test_gpt2_in_one_launch(backend, shape, wtype, kv_f16):
     check_gpt2(backend, data, kv_f16, seq - 30 if shape == "small" else 7, seq - 4 if shape == "small" else 30, 700)
 
 
+@pytest.mark.parametrize("wtype", [8, 2], ids=["q8_0", "q4_0"])
+def test_gpt2_in_launches(monkeypatch, wtype):
+    monkeypatch.setenv("SLAI_PERSISTENT", "0")
+    b = Backend(0)
+    check_gpt2(b, gw.gpt2_gguf(n_embd=768, n_layer=2, n_head=12, ff_len=3072, vocab=700, n_seq=64, wtype=wtype, seed=61, std=0.05), wtype == 2, 7, 30, 700, LAUNCHES)
+    b.close()
+
+
 def test_gpt2_in_one_launch_single_layer(backend):
     data = gw.gpt2_gguf(n_embd=64, n_layer=1, n_head=2, ff_len=128, vocab=700, n_seq=32, wtype=8, seed=62, std=0.08)
     check_gpt2(backend, data, False, 4, 20, 700)
@@ -134,7 +172,9 @@ def test_gpt2_gives_up_and_the_call_is_repeated(monkeypatch):
         b = Backend(0)
         g = Gguf(data)
         m = Gpt2(b, g, _ffi.KV_F32)
+        assert m.decode_form_at(0) == ONE_LAUNCH
         ids, _ = m.generate(np.array([3, 77], np.int32), 20)
+        assert m.decode_form_at(0) == (LAUNCHES if spins == "1" else ONE_LAUNCH)
         first = Gpt2(b, g, _ffi.KV_F32)
         results.append((ids, m.forward_logits(20, int(ids[-1])), first.forward_logits(0, 3)))
         first.destroy(); m.destroy(); g.close(); b.close()
