@@ -92,6 +92,7 @@ struct slai_ctx {
     // the one-launch-per-token form of the Llama-2 layer stack where a model's shapes allow it (SLAI_PERSISTENT=0 switches it off)
     bool persistent = true;
     uint32_t small_spins = 1u << 17;        // SLAI_SMALL_SPINS: see SmallParams::spin_limit
+    uint32_t small_absent = 0;              // SLAI_SMALL_ABSENT: see SmallParams::absent
     uint32_t resident_max_pos = 2048;   // tokens at positions below this take the resident launch (where the model has one): SLAI_RESIDENT_MAX_POS
     // When set, every launch of a decode step is followed by an event recorded under the step's name
     // (slai_llama2_time_steps); null otherwise.
@@ -495,6 +496,7 @@ struct SmallParams {
     float eps = 0.0f, rope_base = 0.0f;
     uint32_t die = 0;                                          // workgroups i with i mod 8 == die
     uint32_t spin_limit = 1u << 17;                            // looks at a counter before a workgroup gives up (about 0.1 s)
+    uint32_t absent = 0;                                       // workgroups left out of the launch, which then gives up (for tests)
 };
 bool small_shape_ok(const SmallParams &p);
 hipError_t launch_decode_small(hipStream_t s, const SmallParams &p);

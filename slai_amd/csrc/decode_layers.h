@@ -28,6 +28,12 @@ __device__ __forceinline__ float max64(float v) {
                  fmaxf(__builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 32)), __builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 48))));
 }
 
+// The flag of a launch that gave up (the host clears it once it has seen it).  A launch looks at it once, as it starts: a call that cannot have its
+// compute units then pays one time limit and not one for every token queued.  (Looking every 64 rounds of a wait as well was 1 us a
+// token of 92, for the instructions around its rounds.)
+__device__ __forceinline__ void abort_launch(uint32_t *flag) { __hip_atomic_store(flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ bool aborted(const uint32_t *flag) { return __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0; }
+
 // The layer table through the scalar cache (it does not change while a kernel runs)
 typedef const SmallLayer __attribute__((address_space(4))) LayerEntry;
 __device__ __forceinline__ void touch_layers(const SmallLayer *layers, uint32_t n) {

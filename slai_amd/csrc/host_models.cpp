@@ -332,6 +332,7 @@ struct SmallForm {
         static std::atomic<uint32_t> next_die{0};
         p.die = next_die.fetch_add(1) & 7u;
         p.spin_limit = ctx->small_spins;
+        p.absent = std::min(ctx->small_absent, SMALL_WGS - 1);
         ready = true;
         return SLAI_OK;
     }

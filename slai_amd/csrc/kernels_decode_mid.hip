@@ -13,7 +13,8 @@
 // us a token in the loop, launches / this: Q8_0, f32 cache, position 16: 329 / 195, 100: 330 / 201, 900: 429 / 307; Q4_0, f16 cache, 100: 322 / 218.
 // A layer takes about 13 us: five hand-overs through memory of 1.5 us and their instructions; on one die (kernels_decode_small.hip) a token took 321 us,
 // bound by instructions.  Copies of the matrices as rows are 90 MB of memory.
-// Every wait is bounded: a workgroup that gives up sets a flag and waits no more; the host then repeats the call with launches.
+// Every wait is bounded: a workgroup that gives up sets a flag and waits no more, nor does any of a launch that finds the flag set; the host then
+// repeats the call with launches.
 #include "common.h"
 #include "decode_layers.h"
 
@@ -32,12 +33,12 @@ __device__ __forceinline__ bool empty4(u32x4b v) { return v.x == FLOW_EMPTY || v
 struct Waits {
     uint32_t *abort_flag;
     uint32_t spin_limit;
-    bool dead = false;
+    bool dead;
     // whether to look again (`missing`: this lane saw an empty word); the same in every lane
     __device__ __forceinline__ bool again(bool missing, uint32_t &looks) {
         if (dead || __builtin_amdgcn_ballot_w64(missing) == 0) return false;
         if (++looks < spin_limit) return true;
-        *abort_flag = 1u;
+        abort_launch(abort_flag);
         dead = true;
         return false;
     }
@@ -158,7 +159,7 @@ __global__ void __launch_bounds__(NT) decode_mid_kernel(const SmallParams p) {
     const bool has_head = wg < p.n_heads;
     touch_layers(p.layers, p.n_layers);
     if (wave == 0) {
-        Waits waits{p.abort_flag, p.spin_limit};
+        Waits waits{p.abort_flag, p.spin_limit, aborted(p.abort_flag)};
         const float *x = p.x;
         for (uint32_t l = 0; l < p.n_layers; ++l) {
             const LayerEntry *L = (const LayerEntry *)(uintptr_t)p.layers + l;
@@ -258,13 +259,13 @@ hipError_t mid_capacity(const SmallParams &p, int device, uint32_t *resident) {
 }
 
 hipError_t launch_decode_mid(hipStream_t s, const SmallParams &p) {
-    if (!mid_shape_ok(p) || !p.layers || !p.work || !p.abort_flag || !p.x || !p.pos_ptr || p.rope_variant >= 0) return hipErrorInvalidValue;
+    if (!mid_shape_ok(p) || p.absent >= NWG || !p.layers || !p.work || !p.abort_flag || !p.x || !p.pos_ptr || p.rope_variant >= 0) return hipErrorInvalidValue;
     if (p.type == T_Q8_0) {
-        if (p.kv_f16) decode_mid_kernel<T_Q8_0, true><<<NWG, NT, 0, s>>>(p);
-        else decode_mid_kernel<T_Q8_0, false><<<NWG, NT, 0, s>>>(p);
+        if (p.kv_f16) decode_mid_kernel<T_Q8_0, true><<<NWG - p.absent, NT, 0, s>>>(p);
+        else decode_mid_kernel<T_Q8_0, false><<<NWG - p.absent, NT, 0, s>>>(p);
     } else {
-        if (p.kv_f16) decode_mid_kernel<T_Q4_0, true><<<NWG, NT, 0, s>>>(p);
-        else decode_mid_kernel<T_Q4_0, false><<<NWG, NT, 0, s>>>(p);
+        if (p.kv_f16) decode_mid_kernel<T_Q4_0, true><<<NWG - p.absent, NT, 0, s>>>(p);
+        else decode_mid_kernel<T_Q4_0, false><<<NWG - p.absent, NT, 0, s>>>(p);
     }
     return hipGetLastError();
 }

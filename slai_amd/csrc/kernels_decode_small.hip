@@ -14,7 +14,8 @@
 //     512 times at once: 123 us a token.  A whole wave per row of 18 chunks: 102.)
 //   * vectors are handed over in memory of their own per layer and step: no line is read before it is complete, so plain loads do
 //     (a compute unit's cache cannot hold an older copy).
-//   * every wait is bounded: a workgroup that gives up sets a flag and waits no more.  The host then repeats the call with launches.
+//   * every wait is bounded: a workgroup that gives up sets a flag and waits no more, nor does any of a launch that finds the flag set.  The
+//     host then repeats the call with launches.
 // us a token in the loop, one launch per step / this: Q8_0, f32 cache, position 16: 130.6 / 92.9, 200: 139.6 / 101.3; Q4_0, f16 cache: 143.6 / 104.5.
 // A layer takes about 11 us: five hand-overs of 0.5 to 0.9 us from the last report to the first input, 0.2 us until that input is read, and
 // 0.3 to 0.6 us of instructions on each side of a step; nothing in it waits for a weight.  GPT-2 small in this form took 321 us a token
@@ -32,7 +33,7 @@ constexpr uint32_t NWG = SMALL_WGS;
 struct Steps {
     uint32_t *abort_flag;
     uint32_t tid, spin_limit;
-    bool dead = false;
+    bool dead;
     __device__ __forceinline__ void wait(uint32_t *counter, uint32_t target) {        // wave 0 only
         if (tid == 0 && !dead) {
             uint32_t seen = 0, spins = 0;
@@ -42,7 +43,7 @@ struct Steps {
                 asm volatile("global_atomic_add %0, %1, %2, off sc0\n\ts_waitcnt vmcnt(0)" : "=&v"(seen) : "v"(counter), "v"(zero) : "memory");
                 ++spins;
             } while (seen < target && spins < spin_limit);
-            if (seen < target) { *abort_flag = 1u; dead = true; }
+            if (seen < target) { abort_launch(abort_flag); dead = true; }
         }
         asm volatile("" ::: "memory");
     }
@@ -210,7 +211,7 @@ __global__ void __launch_bounds__(NT) decode_small_kernel(const SmallParams p) {
         return SmallLayer{le->q, le->k, le->v, le->o, le->gate, le->up, le->down, le->norm1, le->norm2, le->qb, le->kb, le->vb, nullptr, nullptr, nullptr, nullptr, nullptr, le->kcache, le->vcache};
     };
     if (wave == 0) {
-        Steps steps{p.abort_flag, tid, p.spin_limit};
+        Steps steps{p.abort_flag, tid, p.spin_limit, aborted(p.abort_flag)};
         float c = 1.0f, sn = 0.0f;                             // rope.slang:36-39: the angle depends on (2*i) mod head_size for both variants
         if (has_head && p.rope_variant >= 0 && lane < p.head_size / 2) sincosf((float)pos * p.rope_theta[lane], &sn, &c);
         const float *x = p.x;
@@ -275,8 +276,8 @@ bool small_shape_ok(const SmallParams &p) {
 }
 
 hipError_t launch_decode_small(hipStream_t s, const SmallParams &p) {
-    if (!small_shape_ok(p) || p.die > 7 || !p.layers || !p.work || !p.counters || !p.abort_flag || !p.x || !p.pos_ptr || (p.rope_variant >= 0 && !p.rope_theta)) return hipErrorInvalidValue;
-    const dim3 grid(NWG * 8);
+    if (!small_shape_ok(p) || p.die > 7 || p.absent >= NWG || !p.layers || !p.work || !p.counters || !p.abort_flag || !p.x || !p.pos_ptr || (p.rope_variant >= 0 && !p.rope_theta)) return hipErrorInvalidValue;
+    const dim3 grid((NWG - p.absent) * 8);
     if (p.type == T_Q8_0) {
         if (p.kv_f16) decode_small_kernel<T_Q8_0, true><<<grid, NT, 0, s>>>(p);
         else decode_small_kernel<T_Q8_0, false><<<grid, NT, 0, s>>>(p);

@@ -1,6 +1,8 @@
 """The layers of a small model's token as one launch, on one die (kernels_decode_small.hip) or over the device (kernels_decode_mid.hip): shapes at the edges of what it covers (two
 rows per wave, heads of 8 to 64, grouped queries, biases and NeoX pairs), both formats and cache types, positions past one and two passes of
 its attention (120 positions each), against the oracle; a launch that gives up; several models taking turns on one context."""
+import time
+
 import numpy as np
 import pytest
 
@@ -180,3 +182,30 @@ def test_gpt2_gives_up_and_the_call_is_repeated(monkeypatch):
         first.destroy(); m.destroy(); g.close(); b.close()
     assert np.array_equal(results[0][0], results[1][0])
     assert rel_err(results[1][1], results[0][1]) < 1e-5 and rel_err(results[1][2], results[0][2]) < 1e-5
+
+
+def small_and_gpt2():
+    return [(lambda b, g: Llama2(b, g, _ffi.MODEL_LLAMA, _ffi.KV_F32), model("15 M parameters", 8, 256)),
+            (lambda b, g: Gpt2(b, g, _ffi.KV_F32), gw.gpt2_gguf(n_embd=768, n_layer=2, n_head=12, ff_len=3072, vocab=700, n_seq=256, wtype=8, seed=63, std=0.05))]
+
+
+@pytest.mark.parametrize("which", [0, 1], ids=["llama", "gpt2"])
+def test_one_time_limit_for_all_queued_tokens(monkeypatch, which):
+    """A launch without one of its workgroups waits out its limit (32768 looks, at least 10 ms); the tokens queued behind it do not."""
+    monkeypatch.setenv("SLAI_SMALL_ABSENT", "1")
+    monkeypatch.setenv("SLAI_SMALL_SPINS", "32768")
+    make, data = small_and_gpt2()[which]
+    b = Backend(0)
+    g = Gguf(data)
+    m = make(b, g)
+    assert m.decode_form_at(0) == ONE_LAUNCH
+    t0 = time.perf_counter()
+    ids, _ = m.generate(np.array([3, 77], np.int32), 1)
+    one = time.perf_counter() - t0                             # a time limit, twice a capture and a token in launches
+    m.destroy()
+    m = make(b, g)
+    t0 = time.perf_counter()
+    m.generate(np.array([3, 77], np.int32), 200)
+    many = time.perf_counter() - t0
+    assert many < 5 * one + 0.2, (one, many)
+    m.destroy(); g.close(); b.close()
