@@ -92,6 +92,7 @@ struct slai_ctx {
     // the one-launch-per-token form of the Llama-2 layer stack where a model's shapes allow it (SLAI_PERSISTENT=0 switches it off)
     bool persistent = true;
     uint32_t small_spins = 1u << 17;        // SLAI_SMALL_SPINS: see SmallParams::spin_limit
+    int small_max_pos = -1;                 // SLAI_SMALL_MAX_POS: tokens at positions below this take a small model's one launch; -1: small_positions, mid_positions
     uint32_t small_absent = 0;              // SLAI_SMALL_ABSENT: see SmallParams::absent
     uint32_t resident_max_pos = 2048;   // tokens at positions below this take the resident launch (where the model has one): SLAI_RESIDENT_MAX_POS
     // When set, every launch of a decode step is followed by an event recorded under the step's name
@@ -499,10 +500,12 @@ struct SmallParams {
     uint32_t absent = 0;                                       // workgroups left out of the launch, which then gives up (for tests)
 };
 bool small_shape_ok(const SmallParams &p);
+uint32_t small_positions(const SmallParams &p);                // where a token in launches becomes the faster one
 hipError_t launch_decode_small(hipStream_t s, const SmallParams &p);
 // The same for GPT-2 over the whole device (kernels_decode_mid.hip); `work` holds FLOW_EMPTY at the start of a launch, no counters
 constexpr uint32_t MID_WGS = 256;
 bool mid_shape_ok(const SmallParams &p);
+uint32_t mid_positions(const SmallParams &p);
 hipError_t launch_decode_mid(hipStream_t s, const SmallParams &p);
 hipError_t mid_capacity(const SmallParams &p, int device, uint32_t *resident);
 

@@ -262,11 +262,13 @@ int wide_rows(slai_ctx *ctx, int nseg, const WideGemmSeg *segs, const uint8_t *x
 struct SmallForm {
     bool ready = false;
     SmallParams params;
+    uint32_t max_pos = 0;                                      // tokens at positions from here on take launches
     slai_buffer *layers = nullptr, *work = nullptr, *counters = nullptr;
     std::vector<slai_qmat *> copies;
     std::vector<const slai_qmat *> sources;
     uint8_t *block = nullptr;
 
+    bool at(uint32_t pos) const { return ready && pos < max_pos; }
     uint32_t counter_words() const { return params.n_layers * SMALL_STEPS * 32; }
     uint32_t work_words() const { return params.n_layers * params.work_stride; }
     // What the kernel reads of m: m itself, or its copy as rows (memory assigned by `make`)
@@ -333,6 +335,7 @@ struct SmallForm {
         p.die = next_die.fetch_add(1) & 7u;
         p.spin_limit = ctx->small_spins;
         p.absent = std::min(ctx->small_absent, SMALL_WGS - 1);
+        max_pos = ctx->small_max_pos >= 0 ? (uint32_t)ctx->small_max_pos : one_die ? small_positions(p) : mid_positions(p);
         ready = true;
         return SLAI_OK;
     }
@@ -740,7 +743,7 @@ int slai_llama2::launch(LlmContext &ctxt, const slai_attn_params &attn_params, u
 // rows beyond the ones the attention asks for ahead into the die's L2 -- a kernel of its own, so that the short contexts do
 // not carry that code.)
 int slai_llama2::form_at(uint32_t pos) const {
-    if (small.ready) return 3;
+    if (small.at(pos)) return 3;
     if (!persistent.ready || pos >= ctx->resident_max_pos) return 0;
     return pos > resident_far_from(kv_dtype == SLAI_KV_F16) ? 2 : 1;
 }
@@ -1620,7 +1623,7 @@ struct slai_gpt2 {
 
     int load(const slai_gguf *g);
     int enqueue_fused(int sampler, int form = 0);   // 0: stop at the logits, 1: greedy pick + loop state, 2: temperature / top-p pick + loop state, 3: the same without a top-p cut (form 3: the layers as one launch)
-    int form_at(uint32_t) const { return small.ready ? 3 : 0; }
+    int form_at(uint32_t pos) const { return small.at(pos) ? 3 : 0; }
     SmallForm small;                              // form 3
     int small_setup();
     bool drop_small() { const bool was = small.ready; small.ready = false; return was; }   // from now on one launch per step

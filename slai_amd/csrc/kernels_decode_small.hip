@@ -275,6 +275,11 @@ bool small_shape_ok(const SmallParams &p) {
     return most(p.dim + 2 * p.kvd) <= 2 * RW && most(p.dim) <= RW && most(p.hidden) <= 2 * RW;
 }
 
+// One workgroup per head walks the cache at 11 ns (f32) or 12 (f16) a position and layer; launches split a head over the device and grow by less than one.
+// us a token of six layers, launches / this, at positions 500, 700, 900 (the slowest format and cache type of each shape; Q4_0 with an f16 cache):
+//   288 wide 154 / 137, 156 / 153, 156 / 166;  480 wide 151 / 135, 151 / 151, 151 / 164;  128 wide 123 / 126, 123 / 140;  64 wide 122 / 126, 123 / 141
+uint32_t small_positions(const SmallParams &p) { return p.dim < 256 ? 448 : 672; }
+
 hipError_t launch_decode_small(hipStream_t s, const SmallParams &p) {
     if (!small_shape_ok(p) || p.die > 7 || p.absent >= NWG || !p.layers || !p.work || !p.counters || !p.abort_flag || !p.x || !p.pos_ptr || (p.rope_variant >= 0 && !p.rope_theta)) return hipErrorInvalidValue;
     const dim3 grid((NWG - p.absent) * 8);

@@ -131,7 +131,8 @@ def check_gpt2(backend, data, kv_f16, n_prompt, steps, vocab, form=ONE_LAUNCH):
     assert L.slo_gpt2_generate(om, prompt.ctypes.data, n_prompt, 0, steps, -1, ref.ctypes.data, ref_logits.ctypes.data) == steps
     gg = Gguf(data)
     m = Gpt2(backend, gg, _ffi.KV_F16 if kv_f16 else _ffi.KV_F32)
-    assert m.decode_form_at(0) == m.decode_form_at(steps - 1) == form
+    if form is not None:
+        assert m.decode_form_at(0) == m.decode_form_at(steps - 1) == form
     tok = int(prompt[0])
     for pos in range(steps):
         assert rel_err(m.forward_logits(pos, tok), ref_logits[pos]) < 1e-2
@@ -209,3 +210,25 @@ def test_one_time_limit_for_all_queued_tokens(monkeypatch, which):
     many = time.perf_counter() - t0
     assert many < 5 * one + 0.2, (one, many)
     m.destroy(); g.close(); b.close()
+
+
+def test_form_by_position(backend):
+    """Small models take one launch a token only as far as that is the faster one, and launches beyond."""
+    for dim, hidden, heads, kv, line in ((64, 96, 8, 2, 448), (288, 768, 6, 6, 672)):
+        g = Gguf(gw.llama_gguf(dim=dim, hidden_dim=hidden, n_layers=2, n_heads=heads, n_kv_heads=kv, vocab=500, seq_len=4096, wtype=8, seed=64, std=0.08))
+        m = Llama2(backend, g, _ffi.MODEL_LLAMA, _ffi.KV_F16)
+        assert [m.decode_form_at(p) for p in (0, line - 1, line, 4095)] == [ONE_LAUNCH, ONE_LAUNCH, LAUNCHES, LAUNCHES]
+        m.destroy(); g.close()
+    for dim, line in ((96, 153), (768, 1024)):
+        g = Gguf(gw.gpt2_gguf(n_embd=dim, n_layer=2, n_head=12, ff_len=4 * dim, vocab=700, n_seq=2048, wtype=8, seed=65, std=0.05))
+        m = Gpt2(backend, g, _ffi.KV_F32)
+        assert [m.decode_form_at(p) for p in (0, line - 1, line, 2047)] == [ONE_LAUNCH, ONE_LAUNCH, LAUNCHES, LAUNCHES]
+        m.destroy(); g.close()
+
+
+def test_tokens_across_the_line(backend):
+    """The caches are the same in both forms: a call that passes from one to the other, and one that begins beyond."""
+    prompt = np.random.Generator(np.random.PCG64(5)).integers(0, 500, 440)
+    check_llama(backend, gw.llama_gguf(dim=64, hidden_dim=96, n_layers=2, n_heads=8, n_kv_heads=2, vocab=500, seq_len=512, wtype=8, seed=66, std=0.08, norm_random=True),
+                prompt, 470, check_logit_steps=460)
+    check_gpt2(backend, gw.gpt2_gguf(n_embd=96, n_layer=2, n_head=12, ff_len=160, vocab=700, n_seq=192, wtype=8, seed=67, std=0.05), True, 140, 180, 700, None)
