@@ -1455,7 +1455,11 @@ static int generate_impl(Model *m, slai_ctx *ctx, DeviceLoop &L, uint32_t seq_le
     // a launch on one die that did not get its die to itself gave up: the same call once more, with one launch per step from now on
     const auto again = [&](int rc) {
         if (!m->drop_small()) return rc;
-        return generate_impl(m, ctx, L, seq_len, vocab, prompt, n_prompt, start_pos, n_steps, out_tokens, elapsed_ms, sampling);
+        float first = 0.0f;                                    // (its time counts too)
+        SLAI_HIP_TRY(ctx, hipEventElapsedTime(&first, L.ev0, L.ev1));
+        TRY(generate_impl(m, ctx, L, seq_len, vocab, prompt, n_prompt, start_pos, n_steps, out_tokens, elapsed_ms, sampling));
+        if (elapsed_ms) *elapsed_ms += first;
+        return SLAI_OK;
     };
     TRY(slai_write_buffer(ctx, L.state, 0, &ds, sizeof ds));
     TRY(slai_write_buffer(ctx, L.prompt, 0, prompt, (size_t)n_prompt * 4));

@@ -251,7 +251,7 @@ bool mid_shape_ok(const SmallParams &p) {
 // The same walk of the cache as on one die (small_positions), but the launches that it saves are the longer the wider the model is.  us a token of six
 // layers, launches / this (Q4_0, f16 cache, the slowest):
 //   96 wide, position 250: 132 / 130, 400: 132 / 139;  320, 500: 154 / 151, 700: 155 / 166;  384, 700: 164 / 162;  512, 900: 166 / 172;
-//   640, 1100: 189 / 191;  768, 900: 188 / 174, 1100: 188 / 192;  1024, 1000: 178 / 182, Q8_0 181 / 170
+//   640, 1100: 189 / 191;  768, 900: 188 / 174, 1100: 188 / 192;  1024, 1000: 178 / 182, Q8_0 181 / 172
 uint32_t mid_positions(const SmallParams &p) { return min(p.dim * 8 / 5, p.type == T_Q4_0 ? 960u : 1024u); }
 
 // Workgroups of the launch that the device keeps resident

@@ -232,3 +232,22 @@ def test_tokens_across_the_line(backend):
     check_llama(backend, gw.llama_gguf(dim=64, hidden_dim=96, n_layers=2, n_heads=8, n_kv_heads=2, vocab=500, seq_len=512, wtype=8, seed=66, std=0.08, norm_random=True),
                 prompt, 470, check_logit_steps=460)
     check_gpt2(backend, gw.gpt2_gguf(n_embd=96, n_layer=2, n_head=12, ff_len=160, vocab=700, n_seq=192, wtype=8, seed=67, std=0.05), True, 140, 180, 700, None)
+
+
+@pytest.mark.parametrize("which", [0, 1], ids=["llama", "gpt2"])
+def test_elapsed_time_of_a_repeated_call(monkeypatch, which):
+    """The time that a call reports has the launch that gave up in it: at least 65536 looks of 0.3 us, where eight tokens in launches take 1.2 ms."""
+    monkeypatch.setenv("SLAI_SMALL_ABSENT", "1")
+    monkeypatch.setenv("SLAI_SMALL_SPINS", "65536")
+    make, data = small_and_gpt2()[which]
+    b = Backend(0)
+    g = Gguf(data)
+    m = make(b, g)
+    assert m.decode_form_at(0) == ONE_LAUNCH
+    t0 = time.perf_counter()
+    ids, ms = m.generate(np.array([3, 77], np.int32), 8)
+    host = (time.perf_counter() - t0) * 1e3
+    again, ms_launches = m.generate(np.array([3, 77], np.int32), 8)
+    assert m.decode_form_at(0) == LAUNCHES and np.array_equal(ids, again)
+    assert ms_launches + 15.0 < ms < host, (ms, ms_launches, host)
+    m.destroy(); g.close(); b.close()
