@@ -268,7 +268,20 @@ struct SmallForm {
     std::vector<const slai_qmat *> sources;
     uint8_t *block = nullptr;
 
-    bool at(uint32_t pos) const { return ready && pos < max_pos; }
+    // After a launch that did not get its compute units (another process or context had them) the form rests for 64 calls, twice as many after each further one
+    // up to 65536: a limit of 0.1 s then costs a program that keeps colliding less and less, and one that collided once next to nothing.
+    uint32_t resting = 0, next_rest = 64;
+    struct Call {                                              // one of generate, forward_logits
+        SmallForm &form;
+        ~Call() { if (form.resting) --form.resting; }
+    };
+    bool gave_up() {                                           // (within a call, which is then repeated.)  false: it was not this form
+        if (!ready || resting) return false;
+        resting = next_rest + 2;
+        next_rest = std::min(2 * next_rest, 65536u);
+        return true;
+    }
+    bool at(uint32_t pos) const { return ready && !resting && pos < max_pos; }
     uint32_t counter_words() const { return params.n_layers * SMALL_STEPS * 32; }
     uint32_t work_words() const { return params.n_layers * params.work_stride; }
     // What the kernel reads of m: m itself, or its copy as rows (memory assigned by `make`)
@@ -420,7 +433,6 @@ struct slai_llama2 {
     SmallForm small;                              // form 3
     int small_setup();
     int enqueue_small(int sampler);
-    bool drop_small() { const bool was = small.ready; small.ready = false; return was; }   // from now on one launch per step
     int enqueue_output(const float *prepared, int sampler);   // the output matrix and the pick
     bool persistent_supported() const;
     int persistent_setup();
@@ -1408,6 +1420,7 @@ SLAI_EXPORT int slai_llama2_forward_logits(slai_llama2 *m, uint32_t pos, uint32_
     if (!m) return SLAI_E_ARG;
     slai_ctx *ctx = m->ctx;
     if (pos >= m->config.seq_len || token >= m->config.vocab_size) return set_error(ctx, SLAI_E_ARG, "slai_llama2_forward_logits: position or token out of range");
+    const SmallForm::Call call{m->small};
     Llama2State &s = m->state;
     if (!fused) {
         // chat_llama2.rs:176-189: per-token uniforms, then the embedding column into x
@@ -1429,7 +1442,7 @@ SLAI_EXPORT int slai_llama2_forward_logits(slai_llama2 *m, uint32_t pos, uint32_
     }
     TRY(slai_synchronize(ctx));                                          // :219
     if (const int rc = handoff_check(ctx)) {
-        if (!fused || !m->drop_small()) return rc;
+        if (!fused || !m->small.gave_up()) return rc;
         return slai_llama2_forward_logits(m, pos, token, fused, logits_out);
     }
     if (logits_out) TRY(slai_read_buffer(ctx, s.logits.buf, 0, logits_out, (size_t)m->config.vocab_size * 4));   // :225-227
@@ -1450,11 +1463,12 @@ static int generate_impl(Model *m, slai_ctx *ctx, DeviceLoop &L, uint32_t seq_le
     if (n_prompt > L.capacity || n_steps > L.capacity) return set_error(ctx, SLAI_E_SHAPE, "generate: prompt longer than the context length");
     for (uint32_t i = 0; i < n_prompt; ++i)
         if (prompt[i] < 0 || (uint32_t)prompt[i] >= vocab) return set_error(ctx, SLAI_E_ARG, "generate: prompt token out of range");
+    const SmallForm::Call call{m->small};
     DecodeState ds{(int)start_pos, prompt[start_pos], (int)n_prompt, 0, 0.0f, 0.0f, 0, 0};     // chat_llama2.rs:105
     if (sampling) { ds.temperature = sampling->temperature; ds.topp = sampling->topp; ds.seed_lo = (uint32_t)sampling->seed; ds.seed_hi = (uint32_t)(sampling->seed >> 32); }
-    // a launch on one die that did not get its die to itself gave up: the same call once more, with one launch per step from now on
+    // a small model's one launch that did not get its compute units gave up: the same call once more, in launches
     const auto again = [&](int rc) {
-        if (!m->drop_small()) return rc;
+        if (!m->small.gave_up()) return rc;
         float first = 0.0f;                                    // (its time counts too)
         SLAI_HIP_TRY(ctx, hipEventElapsedTime(&first, L.ev0, L.ev1));
         TRY(generate_impl(m, ctx, L, seq_len, vocab, prompt, n_prompt, start_pos, n_steps, out_tokens, elapsed_ms, sampling));
@@ -1630,7 +1644,6 @@ struct slai_gpt2 {
     int form_at(uint32_t pos) const { return small.at(pos) ? 3 : 0; }
     SmallForm small;                              // form 3
     int small_setup();
-    bool drop_small() { const bool was = small.ready; small.ready = false; return was; }   // from now on one launch per step
 
     // Prompt tokens in chunks of up to 32 on the matrix cores (see slai_llama2::enqueue_chunk_gemm); row-major x and qkv,
     // quad-major xn (normalised rows, then the attention output) and h.
@@ -2016,12 +2029,13 @@ SLAI_EXPORT int slai_gpt2_forward_logits(slai_gpt2 *m, uint32_t pos, uint32_t to
     if (!m) return SLAI_E_ARG;
     slai_ctx *ctx = m->ctx;
     if (pos >= m->params.n_seq || token >= m->params.n_vocab) return set_error(ctx, SLAI_E_ARG, "slai_gpt2_forward_logits: position or token out of range");
+    const SmallForm::Call call{m->small};
     DecodeState ds{(int)pos, (int)token, 0, 0};
     TRY(slai_write_buffer(ctx, m->loop.state, 0, &ds, sizeof ds));
     TRY(m->enqueue_fused(0, m->form_at(pos)));
     TRY(slai_synchronize(ctx));
     if (const int rc = handoff_check(ctx)) {
-        if (!m->drop_small()) return rc;
+        if (!m->small.gave_up()) return rc;
         return slai_gpt2_forward_logits(m, pos, token, logits_out);
     }
     if (logits_out) TRY(slai_read_buffer(ctx, m->curr_vocab.buf, 0, logits_out, (size_t)m->params.n_vocab * 4));

@@ -251,3 +251,25 @@ def test_elapsed_time_of_a_repeated_call(monkeypatch, which):
     assert m.decode_form_at(0) == LAUNCHES and np.array_equal(ids, again)
     assert ms_launches + 15.0 < ms < host, (ms, ms_launches, host)
     m.destroy(); g.close(); b.close()
+
+
+@pytest.mark.parametrize("which", [0, 1], ids=["llama", "gpt2"])
+def test_the_form_comes_back(monkeypatch, which):
+    """A model whose launch gave up takes launches for 64 calls and then tries again; it rests twice as long after the second failure."""
+    monkeypatch.setenv("SLAI_SMALL_SPINS", "1")
+    make, data = small_and_gpt2()[which]
+    b = Backend(0)
+    g = Gguf(data)
+    m = make(b, g)
+    prompt = np.array([3, 77], np.int32)
+    ref, _ = m.generate(prompt, 8)
+    for rest in (64, 128):
+        for i in range(rest):
+            assert m.decode_form_at(0) == LAUNCHES
+            if i % 2:
+                m.forward_logits(0, 3)
+            else:
+                assert np.array_equal(m.generate(prompt, 8)[0], ref)
+        assert m.decode_form_at(0) == ONE_LAUNCH
+        assert np.array_equal(m.generate(prompt, 8)[0], ref)   # (gives up again)
+    m.destroy(); g.close(); b.close()
