@@ -486,8 +486,9 @@ int handoff_check(slai_ctx *ctx) {
     SLAI_HIP_TRY(ctx, hipMemcpy(&flag, ctx->handoff_counters + (size_t)ctx->handoff_heads * 32, sizeof flag, hipMemcpyDeviceToHost));
     if (flag) {
         // reported once: the slot is cleared so that later, healthy calls are not failed for an old time-out, and so are
-        // the per-head counters, which a launch that gave up may have left anywhere
-        (void)hipMemset(ctx->handoff_counters, 0, ((size_t)ctx->handoff_heads * 32 + 32) * sizeof(uint32_t));
+        // the per-head counters, which a launch that gave up may have left anywhere.  (On the context's stream: it does not wait for
+        // the null stream, and the call may be repeated at once.)
+        SLAI_HIP_TRY(ctx, hipMemsetAsync(ctx->handoff_counters, 0, ((size_t)ctx->handoff_heads * 32 + 32) * sizeof(uint32_t), ctx->stream));
         return set_error(ctx, SLAI_E_HIP, "q/k/v -> attention hand-off timed out inside a launch; results are invalid");
     }
     return SLAI_OK;
