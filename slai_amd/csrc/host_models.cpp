@@ -312,9 +312,9 @@ struct SmallForm {
     // `params` but for the buffers, and the layers' vectors and caches; mats(l): its seven matrices (q, k, v, o, gate, up, down; null: none)
     template <class Mats> int setup(slai_ctx *ctx, std::vector<SmallLayer> &host, bool one_die, Mats &&mats) {
         SmallParams &p = params;
-        if (!ctx->persistent || !ctx->handoff_counters) return SLAI_OK;
+        if (!ctx->persistent) return SLAI_OK;
         if (one_die) {
-            if (!ctx->fuse_qkv_attention || !small_shape_ok(p)) return SLAI_OK;
+            if (!ctx->handoff_counters || !ctx->fuse_qkv_attention || !small_shape_ok(p)) return SLAI_OK;
         } else {
             uint32_t resident = 0;
             if (!mid_shape_ok(p) || mid_capacity(p, ctx->device, &resident) != hipSuccess || resident < MID_WGS) return SLAI_OK;
@@ -330,6 +330,7 @@ struct SmallForm {
             }
         }
         if (!make(ctx)) { drop(ctx); return SLAI_OK; }
+        TRY(handoff_reserve(ctx, p.n_heads));                  // (the flag; models without the form have none to look at)
         for (size_t l = 0; l < host.size(); ++l) {
             const auto &r = rows[l];
             SmallLayer &d = host[l];
@@ -1770,7 +1771,6 @@ int slai_gpt2::load(const slai_gguf *gg) {
 }
 
 int slai_gpt2::small_setup() {
-    TRY(handoff_reserve(ctx, params.n_head));
     if (layers.empty()) return SLAI_OK;
     SmallParams &p = small.params;
     p.n_layers = params.n_layer; p.dim = params.n_embd; p.kvd = params.n_embd; p.hidden = params.ff_len; p.n_heads = params.n_head; p.kv_mul = 1; p.head_size = params.n_embd / params.n_head;
@@ -2034,7 +2034,7 @@ SLAI_EXPORT int slai_gpt2_forward_logits(slai_gpt2 *m, uint32_t pos, uint32_t to
     TRY(slai_write_buffer(ctx, m->loop.state, 0, &ds, sizeof ds));
     TRY(m->enqueue_fused(0, m->form_at(pos)));
     TRY(slai_synchronize(ctx));
-    if (const int rc = handoff_check(ctx)) {
+    if (const int rc = m->form_at(pos) ? handoff_check(ctx) : SLAI_OK) {
         if (!m->small.gave_up()) return rc;
         return slai_gpt2_forward_logits(m, pos, token, logits_out);
     }
