@@ -310,14 +310,18 @@ struct SmallForm {
         return true;
     }
     // `params` but for the buffers, and the layers' vectors and caches; mats(l): its seven matrices (q, k, v, o, gate, up, down; null: none)
-    template <class Mats> int setup(slai_ctx *ctx, std::vector<SmallLayer> &host, bool one_die, Mats &&mats) {
+    // (a model that does not get the form, for its shape or for want of memory, does without)
+    template <class Mats> void setup(slai_ctx *ctx, std::vector<SmallLayer> &host, bool one_die, Mats &&mats) {
+        if (!build(ctx, host, one_die, mats)) drop(ctx);
+    }
+    template <class Mats> bool build(slai_ctx *ctx, std::vector<SmallLayer> &host, bool one_die, Mats &&mats) {
         SmallParams &p = params;
-        if (!ctx->persistent) return SLAI_OK;
+        if (!ctx->persistent) return false;
         if (one_die) {
-            if (!ctx->handoff_counters || !ctx->fuse_qkv_attention || !small_shape_ok(p)) return SLAI_OK;
+            if (!ctx->handoff_counters || !ctx->fuse_qkv_attention || !small_shape_ok(p)) return false;
         } else {
             uint32_t resident = 0;
-            if (!mid_shape_ok(p) || mid_capacity(p, ctx->device, &resident) != hipSuccess || resident < MID_WGS) return SLAI_OK;
+            if (!mid_shape_ok(p) || mid_capacity(p, ctx->device, &resident) != hipSuccess || resident < MID_WGS) return false;
         }
         p.stride_e = (uint32_t)device_row_stride(p.type, p.dim); p.stride_h = (uint32_t)device_row_stride(p.type, p.hidden);
         std::vector<std::array<slai_qmat *, 7>> rows(host.size());
@@ -325,12 +329,11 @@ struct SmallForm {
             rows[l] = mats(l);
             for (slai_qmat *&m : rows[l]) {
                 if (!m) continue;
-                if (m->type != p.type) { drop(ctx); return SLAI_OK; }
+                if (m->type != p.type) return false;
                 m = take(m);
             }
         }
-        if (!make(ctx)) { drop(ctx); return SLAI_OK; }
-        TRY(handoff_reserve(ctx, p.n_heads));                  // (the flag; models without the form have none to look at)
+        if (!make(ctx) || handoff_reserve(ctx, p.n_heads)) return false;     // (the flag; models without the form have none to look at)
         for (size_t l = 0; l < host.size(); ++l) {
             const auto &r = rows[l];
             SmallLayer &d = host[l];
@@ -338,10 +341,10 @@ struct SmallForm {
             for (int i = 0; i < 7; ++i) *at[i] = r[i] ? r[i]->dptr : nullptr;
         }
         p.work_stride = small_pad(p.dim + 2 * p.kvd) + 3 * small_pad(p.dim) + small_pad(p.hidden);
-        TRY(slai_buffer_create(ctx, host.size() * sizeof(SmallLayer), SLAI_DT_U8, STORAGE | COPY_DST, &layers));
-        TRY(slai_write_buffer(ctx, layers, 0, host.data(), host.size() * sizeof(SmallLayer)));
-        TRY(slai_buffer_create(ctx, host.size() * p.work_stride * sizeof(float), SLAI_DT_F32, STORAGE, &work));
-        TRY(slai_buffer_create(ctx, (size_t)counter_words() * 4, SLAI_DT_U8, STORAGE, &counters));
+        if (slai_buffer_create(ctx, host.size() * sizeof(SmallLayer), SLAI_DT_U8, STORAGE | COPY_DST, &layers) ||
+            slai_write_buffer(ctx, layers, 0, host.data(), host.size() * sizeof(SmallLayer)) ||
+            slai_buffer_create(ctx, host.size() * p.work_stride * sizeof(float), SLAI_DT_F32, STORAGE, &work) ||
+            slai_buffer_create(ctx, (size_t)counter_words() * 4, SLAI_DT_U8, STORAGE, &counters)) return false;
         p.layers = (const SmallLayer *)layers->dptr; p.work = (float *)work->dptr; p.counters = (uint32_t *)counters->dptr;
         p.abort_flag = ctx->handoff_counters + (size_t)ctx->handoff_heads * 32;
         // (contexts that run at the same time take different dies: a die keeps the workgroups of one launch resident)
@@ -351,7 +354,7 @@ struct SmallForm {
         p.absent = std::min(ctx->small_absent, SMALL_WGS - 1);
         max_pos = ctx->small_max_pos >= 0 ? (uint32_t)ctx->small_max_pos : one_die ? small_positions(p) : mid_positions(p);
         ready = true;
-        return SLAI_OK;
+        return true;
     }
     void drop(slai_ctx *ctx) {
         ready = false;
@@ -432,7 +435,7 @@ struct slai_llama2 {
         size_t flow_bytes = 0;
     } persistent;
     SmallForm small;                              // form 3
-    int small_setup();
+    void small_setup();
     int enqueue_small(int sampler);
     int enqueue_output(const float *prepared, int sampler);   // the output matrix and the pick
     bool persistent_supported() const;
@@ -597,7 +600,7 @@ int slai_llama2::load(const slai_gguf *gg) {
     TRY(ensure_attn_scratch(ctx, attention_scratch_floats(config.n_q_heads, head_size(), attn_splits)));
     TRY(loop_init(ctx, loop, config.seq_len + 1));
     TRY(persistent_setup());
-    TRY(small_setup());
+    small_setup();
     wide_setup();
     // (said only to a caller who asked for the form by name: most models simply have other shapes)
     const char *asked = getenv("SLAI_PERSISTENT");
@@ -761,8 +764,8 @@ int slai_llama2::form_at(uint32_t pos) const {
     return pos > resident_far_from(kv_dtype == SLAI_KV_F16) ? 2 : 1;
 }
 
-int slai_llama2::small_setup() {
-    if (persistent.ready || weights.layers.empty()) return SLAI_OK;
+void slai_llama2::small_setup() {
+    if (persistent.ready || weights.layers.empty()) return;
     SmallParams &p = small.params;
     p.n_layers = config.n_layers; p.dim = config.dim; p.kvd = kv_dim(); p.hidden = config.hidden_dim; p.n_heads = config.n_q_heads; p.kv_mul = config.n_q_heads / config.n_kv_heads;
     p.head_size = head_size(); p.seq_len = config.seq_len; p.type = weights.layers[0].attn_q->type; p.kv_f16 = kv_dtype == SLAI_KV_F16;
@@ -776,7 +779,7 @@ int slai_llama2::small_setup() {
         d.norm1 = vec(w.attn_norm); d.norm2 = vec(w.ffn_norm); d.qb = vec(w.attn_q_bias); d.kb = vec(w.attn_k_bias); d.vb = vec(w.attn_v_bias);
         d.kcache = state.key_cache[l].buf->dptr; d.vcache = state.value_cache[l].buf->dptr;
     }
-    return small.setup(ctx, host, true, [&](size_t l) {
+    small.setup(ctx, host, true, [&](size_t l) {
         const Llama2LayerWeights &w = weights.layers[l];
         return std::array<slai_qmat *, 7>{w.attn_q, w.attn_k, w.attn_v, w.attn_output, w.ffn_gate, w.ffn_up, w.ffn_down};
     });
@@ -1644,7 +1647,7 @@ struct slai_gpt2 {
     int enqueue_fused(int sampler, int form = 0);   // 0: stop at the logits, 1: greedy pick + loop state, 2: temperature / top-p pick + loop state, 3: the same without a top-p cut (form 3: the layers as one launch)
     int form_at(uint32_t pos) const { return small.at(pos) ? 3 : 0; }
     SmallForm small;                              // form 3
-    int small_setup();
+    void small_setup();
 
     // Prompt tokens in chunks of up to 32 on the matrix cores (see slai_llama2::enqueue_chunk_gemm); row-major x and qkv,
     // quad-major xn (normalised rows, then the attention output) and h.
@@ -1766,12 +1769,12 @@ int slai_gpt2::load(const slai_gguf *gg) {
     attn_splits = pick_attn_splits(ctx, params.n_head, params.n_seq);
     TRY(ensure_attn_scratch(ctx, attention_scratch_floats(params.n_head, E / params.n_head, attn_splits)));
     TRY(loop_init(ctx, loop, params.n_seq + 1));
-    TRY(small_setup());
+    small_setup();
     return slai_synchronize(ctx);
 }
 
-int slai_gpt2::small_setup() {
-    if (layers.empty()) return SLAI_OK;
+void slai_gpt2::small_setup() {
+    if (layers.empty()) return;
     SmallParams &p = small.params;
     p.n_layers = params.n_layer; p.dim = params.n_embd; p.kvd = params.n_embd; p.hidden = params.ff_len; p.n_heads = params.n_head; p.kv_mul = 1; p.head_size = params.n_embd / params.n_head;
     p.seq_len = params.n_seq; p.type = layers[0].c_attn_attn_w->type; p.kv_f16 = kv_dtype == SLAI_KV_F16; p.rope_variant = -1; p.eps = 1.0e-5f;
@@ -1785,7 +1788,7 @@ int slai_gpt2::small_setup() {
         d.qb = vec(w.c_attn_attn_b); d.ob = vec(w.c_attn_proj_b); d.upb = vec(w.c_mlp_fc_b); d.downb = vec(w.c_mlp_proj_b);
         d.kcache = w.key_cache.buf->dptr; d.vcache = w.value_cache.buf->dptr;
     }
-    return small.setup(ctx, host, false, [&](size_t l) {
+    small.setup(ctx, host, false, [&](size_t l) {
         const Gpt2Layer &w = layers[l];
         return std::array<slai_qmat *, 7>{w.c_attn_attn_w, nullptr, nullptr, w.c_attn_proj_w, nullptr, w.c_mlp_fc_w, w.c_mlp_proj_w};
     });

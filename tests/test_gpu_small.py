@@ -273,3 +273,11 @@ def test_the_form_comes_back(monkeypatch, which):
         assert m.decode_form_at(0) == ONE_LAUNCH
         assert np.array_equal(m.generate(prompt, 8)[0], ref)   # (gives up again)
     m.destroy(); g.close(); b.close()
+
+
+def test_without_memory_for_row_copies(monkeypatch):
+    """A GPT-2 model in tiles whose row copies are not allowed the memory loads all the same and takes launches."""
+    monkeypatch.setenv("SLAI_PROMPT_COPY_MB", "0")
+    b = Backend(0)
+    check_gpt2(b, gw.gpt2_gguf(n_embd=768, n_layer=2, n_head=12, ff_len=3072, vocab=700, n_seq=64, wtype=8, seed=61, std=0.05), False, 7, 20, 700, LAUNCHES)
+    b.close()
