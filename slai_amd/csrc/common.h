@@ -502,12 +502,13 @@ struct SmallParams {
 bool small_shape_ok(const SmallParams &p);
 uint32_t small_positions(const SmallParams &p);                // where a token in launches becomes the faster one
 hipError_t launch_decode_small(hipStream_t s, const SmallParams &p);
+hipError_t small_capacity(const SmallParams &p, int device, uint32_t *resident);      // workgroups that a die keeps resident
 // The same for GPT-2 over the whole device (kernels_decode_mid.hip); `work` holds FLOW_EMPTY at the start of a launch, no counters
 constexpr uint32_t MID_WGS = 256;
 bool mid_shape_ok(const SmallParams &p);
 uint32_t mid_positions(const SmallParams &p);
 hipError_t launch_decode_mid(hipStream_t s, const SmallParams &p);
-hipError_t mid_capacity(const SmallParams &p, int device, uint32_t *resident);
+hipError_t mid_capacity(const SmallParams &p, int device, uint32_t *resident);        // that the device keeps resident
 
 // ---- the whole layer stack of a Llama-2 token in one resident launch (kernels_decode_persistent.hip) ----------------------
 // A matrix, vector or cache as the kernel sees it: address and size in bytes.  Every access of the kernel to it goes

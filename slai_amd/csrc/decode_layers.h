@@ -28,6 +28,15 @@ __device__ __forceinline__ float max64(float v) {
                  fmaxf(__builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 32)), __builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 48))));
 }
 
+// Workgroups of `kernel` that a device keeps resident
+inline hipError_t resident_workgroups(const void *kernel, int device, uint32_t *resident) {
+    int per_cu = 0, cus = 0;
+    if (const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, (int)NT, 0)) return e;
+    if (const hipError_t e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device)) return e;
+    *resident = (uint32_t)per_cu * (uint32_t)cus;
+    return hipSuccess;
+}
+
 // The flag of a launch that gave up (the host clears it once it has seen it).  A launch looks at it once, as it starts: a call that cannot have its
 // compute units then pays one time limit and not one for every token queued.  (Looking every 64 rounds of a wait as well was 1 us a
 // token of 92, for the instructions around its rounds.)

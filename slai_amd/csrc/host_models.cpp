@@ -317,10 +317,10 @@ struct SmallForm {
     template <class Mats> bool build(slai_ctx *ctx, std::vector<SmallLayer> &host, bool one_die, Mats &&mats) {
         SmallParams &p = params;
         if (!ctx->persistent) return false;
+        uint32_t resident = 0;
         if (one_die) {
-            if (!ctx->handoff_counters || !ctx->fuse_qkv_attention || !small_shape_ok(p)) return false;
+            if (!ctx->handoff_counters || !ctx->fuse_qkv_attention || !small_shape_ok(p) || small_capacity(p, ctx->device, &resident) != hipSuccess || resident < SMALL_WGS) return false;
         } else {
-            uint32_t resident = 0;
             if (!mid_shape_ok(p) || mid_capacity(p, ctx->device, &resident) != hipSuccess || resident < MID_WGS) return false;
         }
         p.stride_e = (uint32_t)device_row_stride(p.type, p.dim); p.stride_h = (uint32_t)device_row_stride(p.type, p.hidden);

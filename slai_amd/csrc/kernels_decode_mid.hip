@@ -254,15 +254,7 @@ bool mid_shape_ok(const SmallParams &p) {
 //   640, 1100: 189 / 191;  768, 900: 188 / 174, 1100: 188 / 192;  1024, 1000: 178 / 182, Q8_0 181 / 172
 uint32_t mid_positions(const SmallParams &p) { return min(p.dim * 8 / 5, p.type == T_Q4_0 ? 960u : 1024u); }
 
-// Workgroups of the launch that the device keeps resident
-hipError_t mid_capacity(const SmallParams &p, int device, uint32_t *resident) {
-    int per_cu = 0;
-    hipDeviceProp_t prop;
-    if (const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel_of(p), (int)NT, 0)) return e;
-    if (const hipError_t e = hipGetDeviceProperties(&prop, device)) return e;
-    *resident = (uint32_t)per_cu * (uint32_t)prop.multiProcessorCount;
-    return hipSuccess;
-}
+hipError_t mid_capacity(const SmallParams &p, int device, uint32_t *resident) { return resident_workgroups(kernel_of(p), device, resident); }
 
 hipError_t launch_decode_mid(hipStream_t s, const SmallParams &p) {
     if (!mid_shape_ok(p) || p.absent >= NWG || !p.layers || !p.work || !p.abort_flag || !p.x || !p.pos_ptr || p.rope_variant >= 0) return hipErrorInvalidValue;

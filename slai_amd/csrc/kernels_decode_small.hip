@@ -280,6 +280,14 @@ bool small_shape_ok(const SmallParams &p) {
 //   288 wide 154 / 137, 156 / 153, 156 / 166;  480 wide 151 / 135, 151 / 151, 151 / 164;  128 wide 123 / 126, 123 / 140;  64 wide 122 / 126, 123 / 141
 uint32_t small_positions(const SmallParams &p) { return p.dim < 256 ? 448 : 672; }
 
+hipError_t small_capacity(const SmallParams &p, int device, uint32_t *resident) {
+    const void *kernel = p.type == T_Q8_0 ? (p.kv_f16 ? (const void *)decode_small_kernel<T_Q8_0, true> : (const void *)decode_small_kernel<T_Q8_0, false>)
+                                          : (p.kv_f16 ? (const void *)decode_small_kernel<T_Q4_0, true> : (const void *)decode_small_kernel<T_Q4_0, false>);
+    if (const hipError_t e = layers::resident_workgroups(kernel, device, resident)) return e;
+    *resident /= 8;                                            // (eight dies)
+    return hipSuccess;
+}
+
 hipError_t launch_decode_small(hipStream_t s, const SmallParams &p) {
     if (!small_shape_ok(p) || p.die > 7 || p.absent >= NWG || !p.layers || !p.work || !p.counters || !p.abort_flag || !p.x || !p.pos_ptr || (p.rope_variant >= 0 && !p.rope_theta)) return hipErrorInvalidValue;
     const dim3 grid((NWG - p.absent) * 8);
