@@ -175,7 +175,6 @@ struct GemvTiledSeg {
     const float *bias = nullptr;
     uint32_t flags = 0;
 };
-constexpr uint32_t GEMV_TILED_LAUNCH_GROUPS = 32;            // column groups of one launch, at most: sixteen waves, two groups each
 struct GemvTiledParams {
     GemvTiledSeg seg[3];
     int nseg = 1;

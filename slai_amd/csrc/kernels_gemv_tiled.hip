@@ -248,25 +248,26 @@ __global__ void __launch_bounds__(MAXT) gemv_tiled_batch_kernel(const GemvTiledP
 template <int T, bool DUAL, int G>
 hipError_t go(hipStream_t s, const GemvTiledParams &p, dim3 grid, int NT, size_t smem, const GemvBatch *bt) {
     // the bound decides the register budget: 256/512 threads leave 256, 768 leave 168, 1024 leave 128 per lane (two groups per wave: nine waves or more)
+    constexpr bool FULL = G == 1 || gemv_tiled_launch_groups(T) > 24;    // sixteen waves are possible
     if (bt && bt->n > 1) {
         const uint32_t total = grid.x;
         const dim3 g((total + 7) / 8 * 8 * bt->n);
         if (G == 1 && NT <= 256) gemv_tiled_batch_kernel<T, DUAL, G == 1 ? 256 : 768, G><<<g, NT, smem, s>>>(p, *bt, total);
         else if (G == 1 && NT <= 512) gemv_tiled_batch_kernel<T, DUAL, G == 1 ? 512 : 768, G><<<g, NT, smem, s>>>(p, *bt, total);
         else if (NT <= 768) gemv_tiled_batch_kernel<T, DUAL, 768, G><<<g, NT, smem, s>>>(p, *bt, total);
-        else gemv_tiled_batch_kernel<T, DUAL, 1024, G><<<g, NT, smem, s>>>(p, *bt, total);
+        else if constexpr (FULL) gemv_tiled_batch_kernel<T, DUAL, 1024, G><<<g, NT, smem, s>>>(p, *bt, total);
         return hipGetLastError();
     }
     if (G == 1 && NT <= 256) gemv_tiled_kernel<T, DUAL, G == 1 ? 256 : 768, G><<<grid, NT, smem, s>>>(p);
     else if (G == 1 && NT <= 512) gemv_tiled_kernel<T, DUAL, G == 1 ? 512 : 768, G><<<grid, NT, smem, s>>>(p);
     else if (NT <= 768) gemv_tiled_kernel<T, DUAL, 768, G><<<grid, NT, smem, s>>>(p);
-    else gemv_tiled_kernel<T, DUAL, 1024, G><<<grid, NT, smem, s>>>(p);
+    else if constexpr (FULL) gemv_tiled_kernel<T, DUAL, 1024, G><<<grid, NT, smem, s>>>(p);
     return hipGetLastError();
 }
 
 template <int T> hipError_t launch_t(slai_ctx *ctx, GemvTiledParams &p, const GemvBatch *bt) {
     if (p.launch_groups == 0) p.launch_groups = p.ngroups;
-    if (p.ngroups == 0 || p.launch_groups > GEMV_TILED_LAUNCH_GROUPS || p.group0 + p.launch_groups > p.ngroups) return hipErrorInvalidValue;
+    if (p.ngroups == 0 || p.launch_groups > gemv_tiled_launch_groups(T) || p.group0 + p.launch_groups > p.ngroups) return hipErrorInvalidValue;
     // a partial launch cannot normalise its input (that needs every column) or apply a non-linear epilogue
     if (p.launch_groups != p.ngroups && p.prologue != PRO_NONE) return hipErrorInvalidValue;
     for (int i = 0; i < p.nseg; ++i)

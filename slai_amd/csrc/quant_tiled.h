@@ -31,6 +31,10 @@
 
 namespace slai {
 
+// Column groups of one launch, at most: sixteen waves, two groups each; Q6_K twelve, whose two groups need more than the 128 registers a lane of sixteen has
+// (8192 rows x 28672 columns: 57.3 us with sixteen waves and spills, 39.6 as two launches of one group per wave)
+constexpr uint32_t gemv_tiled_launch_groups(int type) { return type == T_Q6_K ? 24 : 32; }
+
 struct TiledGeom {
     int type = 0;
     uint32_t nrows = 0, ncols = 0;

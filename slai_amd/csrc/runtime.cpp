@@ -582,7 +582,7 @@ static int gemv_call_impl(slai_ctx *ctx, const GemvCall &c, const char *who, con
             if (c.prologue != PRO_NONE) return set_error(ctx, SLAI_E_SHAPE, std::string(who) + ": no normalisation prologue over more than 16384 columns in 16-row tiles");
             for (int i = 0; i < c.nseg; ++i)
                 if (c.flags[i] & (GEMV_GELU | GEMV_SILU_GATE)) return set_error(ctx, SLAI_E_SHAPE, std::string(who) + ": no non-linear epilogue over more than 16384 columns in 16-row tiles");
-            const uint32_t nchunks = (m0->ngroups + GEMV_TILED_LAUNCH_GROUPS - 1) / GEMV_TILED_LAUNCH_GROUPS, per = (m0->ngroups + nchunks - 1) / nchunks;
+            const uint32_t most = gemv_tiled_launch_groups(m0->type), nchunks = (m0->ngroups + most - 1) / most, per = (m0->ngroups + nchunks - 1) / nchunks;
             e = hipSuccess;
             for (uint32_t k = 0; k < nchunks && e == hipSuccess; ++k) {
                 GemvTiledParams q = p;

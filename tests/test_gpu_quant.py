@@ -284,16 +284,19 @@ def test_prepared_activations_chain(backend, oracle_lib, t):
         o.destroy()
 
 
-@pytest.mark.parametrize("t", [12, 14, 8], ids=lambda t: NAMES[t])
-def test_wide_matrix_in_16_row_tiles_takes_several_launches(backend, oracle_lib, t):
-    """More than 16384 columns in 16-row tiles (a feed-forward width like 18944): the GEMV runs as several launches over
+# columns: 19 column groups in one launch, two a wave (a feed-forward width like 18944); 28: fourteen waves, Q6_K two launches of one a wave; 34: two
+# launches of 17, the second adding to the first; 50: the same, Q6_K three
+@pytest.mark.parametrize("ncols", [18944, 28672, 34048, 50176])
+@pytest.mark.parametrize("t", [12, 13, 14, 8, 2], ids=lambda t: NAMES[t])
+def test_wide_matrix_in_16_row_tiles_takes_several_launches(backend, oracle_lib, t, ncols):
+    """More than 16384 columns in 16-row tiles: two column groups per wave, and beyond what a launch holds several launches over
     column slices.  Plain product, residual accumulate with the prepared copy emitted by the last slice, and bit-exact
     dequantisation of the layout."""
     import os
     if os.environ.get("SLAI_TILED") == "0":
         pytest.skip("needs the tiled layouts")
     from slai_amd.runtime import GpuQuantMatrix, GpuTensor, LlmContext
-    nrows, ncols = 272, 18944                                  # 74 super-blocks -> 19 column groups -> two launches
+    nrows = 272
     ctxt = LlmContext(backend)
     raw = synth.normal_quantized(900 + t, t, nrows, ncols, 0.02)
     w = oracle_deq(oracle_lib, t, raw, nrows * ncols).reshape(nrows, ncols)
@@ -317,6 +320,32 @@ def test_wide_matrix_in_16_row_tiles_takes_several_launches(backend, oracle_lib,
     assert rel_err(prep[nrows:], (got * nw).reshape(-1, 16).sum(axis=1)) < 1e-5
     for o in (m, gh, out, gx, gnw, gprep):
         o.destroy()
+
+
+def test_wide_q6_k_takes_about_its_bytes(backend):
+    """8192 rows x 28672 columns of Q6_K against Q5_K, which has 0.84 of the bytes: 1.24 times its time (1.78 with sixteen waves of two groups)."""
+    import ctypes as C
+    import time
+    from slai_amd.runtime import GpuQuantMatrix, GpuTensor, LlmContext
+    ctxt = LlmContext(backend)
+    nrows, ncols, best = 8192, 28672, {}
+    x, out = GpuTensor.vector(backend, np.ones(ncols, np.float32)), GpuTensor(backend, nrows)
+    for t in (13, 14):
+        m = GpuQuantMatrix(backend, t, nrows, ncols, synth.normal_quantized(1, t, nrows, ncols, 0.05), layout=2)
+        backend.graph_begin_capture()
+        for _ in range(20):
+            ctxt.matmul_quant_assign(out, m, x)
+        g = backend.graph_end_capture()
+        for _ in range(10):
+            backend.synchronize()
+            t0 = time.perf_counter()
+            backend.graph_launch(g)
+            backend.synchronize()
+            best[t] = min(best.get(t, 1e9), time.perf_counter() - t0)
+        backend.graph_destroy(g)
+        m.destroy()
+    assert best[14] < 1.5 * best[13], best
+    x.destroy(); out.destroy()
 
 
 @pytest.mark.parametrize("t", [12, 13, 14, 8, 2], ids=lambda t: NAMES[t])
