@@ -789,7 +789,9 @@ void slai_llama2::small_setup() {
 int slai_llama2::enqueue_small(int sampler) {
     DecodeState *ds = (DecodeState *)loop.state->dptr;
     SLAI_HIP_TRY(ctx, launch_embed(ctx->stream, weights.token_embd, &ds->token, nullptr, nullptr, config.dim, (float *)state.x.buf->dptr, small.params.counters, small.counter_words()));
+    TRY(step_mark(ctx, "embedding row"));
     SLAI_HIP_TRY(ctx, launch_decode_small(ctx->stream, small.params));
+    TRY(step_mark(ctx, "llama2 layers"));
     return enqueue_output(nullptr, sampler);
 }
 
@@ -1328,8 +1330,9 @@ SLAI_EXPORT int slai_llama2_trace_token(slai_llama2 *m, uint32_t pos, uint32_t t
 }
 
 // One token, launched from the host `reps` times at the same position, with an event after every launch (the resident
-// form: the embedding row, the emptying of the hand-off buffers and the one launch of the layer stack): mean time from the end of the launch before to the end of each launch, by step name in order of
-// first appearance (`names`: newline separated), and how often the step occurs per token.
+// form: the embedding row, the emptying of the hand-off buffers and the one launch of the layer stack; a small model's: the
+// embedding row, the one launch of its layers and the output matrix): mean time from the end of the launch before to the end of
+// each launch, by step name in order of first appearance (`names`: newline separated), and how often the step occurs per token.
 SLAI_EXPORT int slai_llama2_time_steps(slai_llama2 *m, uint32_t pos, uint32_t token, uint32_t reps, char *names, size_t names_len, float *mean_us,
                                        float *alone_us, uint32_t *per_token, uint32_t capacity, uint32_t *n_steps) {
     if (!m || !names || !mean_us || !alone_us || !per_token || !n_steps || reps == 0) return SLAI_E_ARG;
@@ -1338,7 +1341,8 @@ SLAI_EXPORT int slai_llama2_time_steps(slai_llama2 *m, uint32_t pos, uint32_t to
     if (ctx->capturing) return set_error(ctx, SLAI_E_STATE, "slai_llama2_time_steps: not during graph capture");
     DecodeState ds{(int)pos, (int)token, 0, 0};
     TRY(slai_write_buffer(ctx, m->loop.state, 0, &ds, sizeof ds));
-    const auto enqueue = [&]() { return m->enqueue_fused(0, m->persistent.ready ? (pos > resident_far_from(m->kv_dtype == SLAI_KV_F16) ? 2 : 1) : 0); };
+    const bool small = m->small.at(pos);
+    const auto enqueue = [&]() { return m->enqueue_fused(0, small ? 3 : m->persistent.ready ? (pos > resident_far_from(m->kv_dtype == SLAI_KV_F16) ? 2 : 1) : 0); };
     TRY(enqueue());                                             // untimed: sizes scratch, warms the caches
     TRY(slai_synchronize(ctx));
     std::vector<std::pair<const char *, hipEvent_t>> marks;
@@ -1365,6 +1369,7 @@ SLAI_EXPORT int slai_llama2_time_steps(slai_llama2 *m, uint32_t pos, uint32_t to
         total[k] += ms; ++count[k];
     }
     for (auto &mk : marks) (void)hipEventDestroy(mk.second);
+    if (rc && small && m->small.gave_up()) return slai_llama2_time_steps(m, pos, token, reps, names, names_len, mean_us, alone_us, per_token, capacity, n_steps);
     if (rc) return rc;
     if (order.size() > capacity) return set_error(ctx, SLAI_E_SHAPE, "slai_llama2_time_steps: more steps than room for them");
     std::string joined;
@@ -1383,7 +1388,7 @@ SLAI_EXPORT int slai_llama2_time_steps(slai_llama2 *m, uint32_t pos, uint32_t to
     SLAI_HIP_TRY(ctx, hipEventCreate(&e0));
     SLAI_HIP_TRY(ctx, hipEventCreate(&e1));
     for (size_t k = 0; k < order.size() && !rc; ++k) {
-        if (m->persistent.ready) { alone_us[k] = mean_us[k]; continue; }     // (a resident launch needs the buffers emptied before it: never alone)
+        if (m->persistent.ready || small) { alone_us[k] = mean_us[k]; continue; }     // (a resident launch needs the buffers emptied before it: never alone)
         ctx->only_step = order[k];
         rc = m->enqueue_fused(0, 0);                            // untimed
         if (!rc && hipEventRecord(e0, ctx->stream) != hipSuccess) rc = SLAI_E_HIP;
@@ -1400,6 +1405,7 @@ SLAI_EXPORT int slai_llama2_time_steps(slai_llama2 *m, uint32_t pos, uint32_t to
     if (rc == SLAI_E_HIP) return set_error(ctx, SLAI_E_HIP, "slai_llama2_time_steps: event");
     if (rc) return rc;
     // leave the state a whole forward at this position leaves
+    if (small) return SLAI_OK;                                  // (nothing ran alone)
     TRY(enqueue());
     TRY(slai_synchronize(ctx));
     return handoff_check(ctx);

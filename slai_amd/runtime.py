@@ -552,7 +552,7 @@ class Llama2:
 
     def time_steps(self, pos, token, reps=8):
         """[(step name, microseconds per launch inside a token with an event after every launch, launches per token,
-        microseconds per launch of the step alone)] of the launch-per-step form (see slai_llama2_time_steps)."""
+        microseconds per launch of the step alone)] of the form that the model takes at `pos` (see slai_llama2_time_steps)."""
         cap = 32
         names = C.create_string_buffer(4096)
         us = np.zeros(cap, np.float32)

@@ -281,3 +281,19 @@ def test_without_memory_for_row_copies(monkeypatch):
     b = Backend(0)
     check_gpt2(b, gw.gpt2_gguf(n_embd=768, n_layer=2, n_head=12, ff_len=3072, vocab=700, n_seq=64, wtype=8, seed=61, std=0.05), False, 7, 20, 700, LAUNCHES)
     b.close()
+
+
+def test_time_steps_of_the_form_that_runs(monkeypatch):
+    """slai_llama2_time_steps names the launches that generate makes at that position, and those of a model that rests after it gave up."""
+    for env, names in ((None, ["embedding row", "llama2 layers", "llama2 output"]), ("SLAI_SMALL_SPINS", None)):
+        if env:
+            monkeypatch.setenv(env, "1")
+        b = Backend(0)
+        g = Gguf(model("15 M parameters", 8, 1024))
+        m = Llama2(b, g, _ffi.MODEL_LLAMA, _ffi.KV_F32)
+        steps = m.time_steps(8, 5, reps=3)
+        if names:
+            assert [s[0] for s in steps] == names and all(s[2] == 1 and s[1] > 0.0 and s[3] == s[1] for s in steps)
+            steps = m.time_steps(900, 5, reps=3)
+        assert {"llama2 qkv", "llama2 ffn_down"} <= {s[0] for s in steps}, steps
+        m.destroy(); g.close(); b.close()
