@@ -437,8 +437,8 @@ struct AttnLaunch {
     uint32_t n_splits;
     // When set (n_splits > 1, fast form only): one zeroed 128-byte line of counters per head.  The workgroup of a head's
     // split that finishes last merges the head's partial results itself and no combine launch follows.  Only for callers
-    // who have verified that workgroup i of a launch runs on die i mod 8 (slai_ctx::fuse_qkv_attention): the partial
-    // results of a head's splits then meet in that die's L2.
+    // who have verified that workgroup i of a launch runs on die i mod 8 (slai_ctx::fuse_qkv_attention): where all splits of a
+    // head then run on one die, their partial results meet in its L2; otherwise they go through memory (combine_far).
     uint32_t *combine_counters;
     int combine_far;         // (launch_attention) the splits of a head run on several dies: the partial results and the count go through memory
 };
@@ -490,10 +490,10 @@ struct SmallParams {
     float *x = nullptr;                                        // the embedding row in, the last layer's residual out
     const uint32_t *pos_ptr = nullptr;
     const float *rope_theta = nullptr;
-    uint32_t work_stride = 0, n_layers = 0, dim = 0, kvd = 0, hidden = 0, n_heads = 0, kv_mul = 1, head_size = 0, seq_len = 0;
+    uint32_t work_stride = 0, n_layers = 0, dim = 0, kvd = 0, hidden = 0, n_heads = 0, kv_mul = 1, head_size = 0;
     uint32_t stride_e = 0, stride_h = 0;                       // bytes of a packed row of dim / hidden columns
     int type = 0, kv_f16 = 0, rope_variant = -1;
-    float eps = 0.0f, rope_base = 0.0f;
+    float eps = 0.0f;
     uint32_t die = 0;                                          // workgroups i with i mod 8 == die
     uint32_t spin_limit = 1u << 17;                            // looks at a counter before a workgroup gives up (about 0.1 s)
     uint32_t absent = 0;                                       // workgroups left out of the launch, which then gives up (for tests)

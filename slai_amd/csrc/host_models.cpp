@@ -768,8 +768,8 @@ void slai_llama2::small_setup() {
     if (persistent.ready || weights.layers.empty()) return;
     SmallParams &p = small.params;
     p.n_layers = config.n_layers; p.dim = config.dim; p.kvd = kv_dim(); p.hidden = config.hidden_dim; p.n_heads = config.n_q_heads; p.kv_mul = config.n_q_heads / config.n_kv_heads;
-    p.head_size = head_size(); p.seq_len = config.seq_len; p.type = weights.layers[0].attn_q->type; p.kv_f16 = kv_dtype == SLAI_KV_F16;
-    p.rope_variant = rope_variant(); p.rope_base = config.rope_base_freq; p.rope_theta = (const float *)state.rope_theta.buf->dptr; p.eps = config.rms_norm_eps;
+    p.head_size = head_size(); p.type = weights.layers[0].attn_q->type; p.kv_f16 = kv_dtype == SLAI_KV_F16;
+    p.rope_variant = rope_variant(); p.rope_theta = (const float *)state.rope_theta.buf->dptr; p.eps = config.rms_norm_eps;
     p.x = (float *)state.x.buf->dptr; p.pos_ptr = (const uint32_t *)&((DecodeState *)loop.state->dptr)->pos;
     std::vector<SmallLayer> host(config.n_layers);
     const auto vec = [](const GpuTensor &t) { return t.buf ? (const float *)t.buf->dptr : nullptr; };
@@ -1783,7 +1783,7 @@ void slai_gpt2::small_setup() {
     if (layers.empty()) return;
     SmallParams &p = small.params;
     p.n_layers = params.n_layer; p.dim = params.n_embd; p.kvd = params.n_embd; p.hidden = params.ff_len; p.n_heads = params.n_head; p.kv_mul = 1; p.head_size = params.n_embd / params.n_head;
-    p.seq_len = params.n_seq; p.type = layers[0].c_attn_attn_w->type; p.kv_f16 = kv_dtype == SLAI_KV_F16; p.rope_variant = -1; p.eps = 1.0e-5f;
+    p.type = layers[0].c_attn_attn_w->type; p.kv_f16 = kv_dtype == SLAI_KV_F16; p.rope_variant = -1; p.eps = 1.0e-5f;
     p.x = (float *)layer_input.buf->dptr; p.pos_ptr = (const uint32_t *)&((DecodeState *)loop.state->dptr)->pos;
     std::vector<SmallLayer> host(params.n_layer);
     const auto vec = [](const GpuTensor &t) { return (const float *)t.buf->dptr; };

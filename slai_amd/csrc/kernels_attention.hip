@@ -196,8 +196,9 @@ __global__ void __launch_bounds__(NT) attn_fast_kernel(AttnLaunch a, uint32_t ma
     else attn_fast_body<F16, NT, HS, SINGLE, false, 4, false, false, PADDED>(a, h, split, threadIdx.x, []() {});
     if constexpr (!SINGLE) {
         // The last of a head's splits merges them: every workgroup waits until its partial result is in the die's L2
-        // (all splits of the head run on this die: the launcher has checked), then counts itself in with an atomic that
+        // (where all splits of the head run on this die), then counts itself in with an atomic that
         // executes there and returns the count; the one that completes it finds every partial result in that L2.
+        // combine_far, splits on several dies: results, count and the reads of the merge at agent scope, through memory.
         if (a.combine_counters) {
             __shared__ uint32_t last;
             __shared__ float sw[64];
@@ -360,9 +361,9 @@ hipError_t launch_attention(hipStream_t s, const AttnLaunch &a_in) {
     // (SLAI_GQA_ON_DIE=0: one workgroup per (query head, split) in plain order, for comparisons)
     static const bool on_die = [] { const char *e = getenv("SLAI_GQA_ON_DIE"); return !(e && e[0] == '0'); }();
     const uint32_t grouped = fast && on_die && a.kv_mul > 1 && a.n_heads % a.kv_mul == 0 ? 1u : 0u;
-    // The splits of a head merge themselves only in the fast form, and only when all of them run on one die: workgroup
+    // The splits of a head merge themselves in the fast form, in their die's L2 when all of them run on one: workgroup
     // (head, split) of the two-dimensional grid has index head + n_heads * split, a (kv head, split) key of the grouped
-    // grid lands on die (kv head + n_kv_heads * split) mod 8.
+    // grid lands on die (kv head + n_kv_heads * split) mod 8.  Otherwise through memory.
     const uint32_t per_die = grouped ? a.n_heads / a.kv_mul : a.n_heads;
     if (a.n_splits <= 1 || !fast) a.combine_counters = nullptr;
     a.combine_far = a.combine_counters && per_die % 8 != 0 ? 1 : 0;
