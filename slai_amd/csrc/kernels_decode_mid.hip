@@ -11,7 +11,8 @@
 //     weights as soon as they have; wave 0 finishes and writes the results;
 //   * one workgroup per head takes the attention (decode_layers.h).
 // us a token in the loop, launches / this: Q8_0, f32 cache, position 16: 329 / 195, 100: 330 / 201, 900: 429 / 307; Q4_0, f16 cache, 100: 322 / 218.
-// A layer takes about 13 us: five hand-overs through memory of 1.5 us and their instructions; on one die (kernels_decode_small.hip) a token took 321 us,
+// A layer takes 12 us (time stamps, position 100): five hand-overs through memory, 0.4 to 1.1 us from the last result to the first workgroup's whole input and 0.8 to
+// 1.6 to the last's (the FFN's, four times as wide: 1.6 and 2.2), and 0.6 to 1.1 us from input to result, the attention's 1.7 (10.7 at position 900); on one die (kernels_decode_small.hip) a token took 321 us,
 // bound by instructions.  Copies of the matrices as rows are 90 MB of memory.
 // Every wait is bounded: a workgroup that gives up sets a flag and waits no more, nor does any of a launch that finds the flag set; the host then
 // repeats the call with launches.
