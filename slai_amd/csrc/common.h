@@ -91,7 +91,7 @@ struct slai_ctx {
     hipEvent_t timer0 = nullptr, timer1 = nullptr;
     // the one-launch-per-token form of the Llama-2 layer stack where a model's shapes allow it (SLAI_PERSISTENT=0 switches it off)
     bool persistent = true;
-    uint32_t small_spins = 1u << 17;        // SLAI_SMALL_SPINS: see SmallParams::spin_limit
+    uint32_t small_spins = 1u << 12;        // SLAI_SMALL_SPINS: see SmallParams::spin_limit
     int small_max_pos = -1;                 // SLAI_SMALL_MAX_POS: tokens at positions below this take a small model's one launch; -1: small_positions, mid_positions
     uint32_t small_absent = 0;              // SLAI_SMALL_ABSENT: see SmallParams::absent
     uint32_t resident_max_pos = 2048;   // tokens at positions below this take the resident launch (where the model has one): SLAI_RESIDENT_MAX_POS
@@ -495,7 +495,9 @@ struct SmallParams {
     int type = 0, kv_f16 = 0, rope_variant = -1;
     float eps = 0.0f;
     uint32_t die = 0;                                          // workgroups i with i mod 8 == die
-    uint32_t spin_limit = 1u << 17;                            // looks at a counter before a workgroup gives up (about 0.1 s)
+    // looks at a counter or vector before a workgroup gives up: 1 to 4 ms, well below the 20 ms of the 7B resident launch.  Where two such launches each hold some of
+    // the compute units that the other waits for, this one has to give up first: its host repeats the call, the other's reports an error.
+    uint32_t spin_limit = 1u << 12;
     uint32_t absent = 0;                                       // workgroups left out of the launch, which then gives up (for tests)
 };
 bool small_shape_ok(const SmallParams &p);

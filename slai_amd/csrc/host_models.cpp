@@ -269,7 +269,7 @@ struct SmallForm {
     uint8_t *block = nullptr;
 
     // After a launch that did not get its compute units (another process or context had them) the form rests for 64 calls, twice as many after each further one
-    // up to 65536: a limit of 0.1 s then costs a program that keeps colliding less and less, and one that collided once next to nothing.
+    // up to 65536: a limit of a few ms then costs a program that keeps colliding less and less, and one that collided once next to nothing.
     uint32_t resting = 0, next_rest = 64;
     struct Call {                                              // one of generate, forward_logits
         SmallForm &form;

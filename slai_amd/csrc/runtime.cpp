@@ -92,7 +92,7 @@ SLAI_EXPORT int slai_ctx_create(int device, slai_ctx **out) {
     ctx->rowtile_gemv = env_int("SLAI_ROWTILE", 1) != 0;
     ctx->fuse_qkv_attention = env_int("SLAI_FUSE_QKV_ATTN", 1) != 0;
     ctx->persistent = env_int("SLAI_PERSISTENT", 1) != 0;
-    ctx->small_spins = (uint32_t)std::max(1, env_int("SLAI_SMALL_SPINS", 1 << 17));
+    ctx->small_spins = (uint32_t)std::max(1, env_int("SLAI_SMALL_SPINS", 1 << 12));
     ctx->small_max_pos = env_int("SLAI_SMALL_MAX_POS", -1);
     ctx->small_absent = (uint32_t)std::max(0, env_int("SLAI_SMALL_ABSENT", 0));
     ctx->resident_max_pos = (uint32_t)std::max(0, env_int("SLAI_RESIDENT_MAX_POS", 2048));

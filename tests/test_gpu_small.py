@@ -1,6 +1,7 @@
 """The layers of a small model's token as one launch, on one die (kernels_decode_small.hip) or over the device (kernels_decode_mid.hip): shapes at the edges of what it covers (two
 rows per wave, heads of 8 to 64, grouped queries, biases and NeoX pairs), both formats and cache types, positions past one and two passes of
 its attention (120 positions each), against the oracle; a launch that gives up; several models taking turns on one context."""
+import threading
 import time
 
 import numpy as np
@@ -80,7 +81,7 @@ def test_small_gives_up_and_the_call_is_repeated(monkeypatch):
     data = model("15 M parameters", 8, 64)
     prompt = np.array([3, 77, 410, 8], np.int32)
     results = []
-    for spins in ("131072", "1"):
+    for spins in ("4096", "1"):
         monkeypatch.setenv("SLAI_SMALL_SPINS", spins)
         b = Backend(0)
         g = Gguf(data)
@@ -170,7 +171,7 @@ def test_gpt2_in_one_launch_single_layer(backend):
 def test_gpt2_gives_up_and_the_call_is_repeated(monkeypatch):
     data = gw.gpt2_gguf(n_embd=768, n_layer=2, n_head=12, ff_len=3072, vocab=700, n_seq=64, wtype=8, seed=63, std=0.05)
     results = []
-    for spins in ("131072", "1"):
+    for spins in ("4096", "1"):
         monkeypatch.setenv("SLAI_SMALL_SPINS", spins)
         b = Backend(0)
         g = Gguf(data)
@@ -297,3 +298,46 @@ def test_time_steps_of_the_form_that_runs(monkeypatch):
             steps = m.time_steps(900, 5, reps=3)
         assert {"llama2 qkv", "llama2 ffn_down"} <= {s[0] for s in steps}, steps
         m.destroy(); g.close(); b.close()
+
+
+@pytest.mark.parametrize("which", [0, 1], ids=["llama", "gpt2"])
+def test_gives_up_before_the_resident_launch(monkeypatch, which):
+    """The time limit, with what two tokens take besides, is below the 20 ms after which the resident launch of the 7B shape reports an error."""
+    monkeypatch.setenv("SLAI_SMALL_ABSENT", "1")
+    make, data = small_and_gpt2()[which]
+    b = Backend(0)
+    g = Gguf(data)
+    m = make(b, g)
+    _, ms = m.generate(np.array([3, 77], np.int32), 2)
+    assert m.decode_form_at(0) == LAUNCHES and ms < 15.0, ms
+    m.destroy(); g.close(); b.close()
+
+
+def test_beside_a_resident_launch():
+    """A program that decodes with the resident launch, whose workgroups take every compute unit, beside one with a small model: neither sees an error."""
+    g = [Gguf(gw.llama_gguf(dim=4096, hidden_dim=11008, n_layers=2, n_heads=32, n_kv_heads=32, vocab=1024, seq_len=128, wtype=12, v_type=14, out_type=14, embd_type=12, seed=71,
+                            std=0.02, distinct_layers=1)), Gguf(model("15 M parameters", 8, 128))]
+    prompt = np.array([3, 77, 5], np.int32)
+    got = [[], []]
+
+    def work(i):
+        b = Backend(0)
+        for _ in range(1 if i == 0 else 12):                   # (a new small model each time: one that gave up rests)
+            m = Llama2(b, g[i], _ffi.MODEL_LLAMA, _ffi.KV_F16)
+            assert m.decode_form_at(0) == (1 if i == 0 else ONE_LAUNCH)
+            for _ in range(30 if i == 0 else 2):
+                got[i].append(m.generate(prompt, 48)[0].tolist())
+            m.destroy()
+        b.close()
+    for i in (0, 1):
+        work(i)
+    alone = [x[0] for x in got]
+    threads = [threading.Thread(target=work, args=(i,)) for i in (0, 1)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(got[0]) == 60 and len(got[1]) == 48
+    assert all(x == alone[i] for i in (0, 1) for x in got[i])
+    for x in g:
+        x.close()
