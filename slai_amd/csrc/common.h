@@ -350,6 +350,9 @@ struct AttnLaunch;
 int gemv_call(slai_ctx *ctx, const GemvCall &c, const char *who, const AttnLaunch *fused_attn = nullptr);
 int step_mark(slai_ctx *ctx, const char *name);        // records an event under `name` when step timing is on
 bool qkv_attention_fusable(const slai_ctx *ctx, const slai_qmat *v, const slai_qmat *k, const slai_qmat *q, const AttnLaunch &a);
+// A word of device memory, once everything enqueued on the context's stream is done.  (Nothing in this library uses the legacy stream: while a thread
+// captures, another one's operation on it fails, and takes the capture with it.)
+int read_word(slai_ctx *ctx, const void *from, uint32_t *word);
 int handoff_reserve(slai_ctx *ctx, uint32_t n_heads);   // not during graph capture
 int handoff_check(slai_ctx *ctx);                        // after a synchronize: error if a hand-off ever timed out
 // Makes sure the row-tile GEMV's scratch holds `floats` floats (call outside graph capture).

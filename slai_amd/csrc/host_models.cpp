@@ -1593,8 +1593,8 @@ SLAI_EXPORT int slai_llama2_prefill(slai_llama2 *m, const int32_t *tokens, uint3
         SLAI_HIP_TRY(ctx, hipEventRecord(m->loop.ev1, ctx->stream));
         TRY(slai_synchronize(ctx));
         if (!split) break;
-        int beyond = 0;
-        SLAI_HIP_TRY(ctx, hipMemcpy(&beyond, ctx->split_flag, sizeof(int), hipMemcpyDeviceToHost));
+        uint32_t beyond = 0;
+        TRY(read_word(ctx, ctx->split_flag, &beyond));
         if (!beyond) break;
         ++m->prefill_fp32_repeats;
         split = false;
@@ -2108,8 +2108,8 @@ SLAI_EXPORT int slai_gpt2_prefill(slai_gpt2 *m, const int32_t *tokens, uint32_t 
         SLAI_HIP_TRY(ctx, hipEventRecord(m->loop.ev1, ctx->stream));
         TRY(slai_synchronize(ctx));
         if (!split) break;
-        int beyond = 0;
-        SLAI_HIP_TRY(ctx, hipMemcpy(&beyond, ctx->split_flag, sizeof(int), hipMemcpyDeviceToHost));
+        uint32_t beyond = 0;
+        TRY(read_word(ctx, ctx->split_flag, &beyond));
         if (!beyond) break;
         ++m->prefill_fp32_repeats;
         split = false;

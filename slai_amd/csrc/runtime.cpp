@@ -83,7 +83,7 @@ SLAI_EXPORT int slai_ctx_create(int device, slai_ctx **out) {
     ctx->use_graph = env_int("SLAI_NO_GRAPH", 0) == 0;
     ctx->prompt_gemm = env_int("SLAI_PROMPT_GEMM", 1) != 0;
     ctx->prompt_split_f16 = env_int("SLAI_PROMPT_SPLIT_F16", 1);
-    if (hipMalloc((void **)&ctx->split_flag, sizeof(int)) != hipSuccess || hipMemset(ctx->split_flag, 0, sizeof(int)) != hipSuccess) {
+    if (hipMalloc((void **)&ctx->split_flag, sizeof(int)) != hipSuccess || hipMemsetAsync(ctx->split_flag, 0, sizeof(int), ctx->stream) != hipSuccess) {
         (void)hipStreamDestroy(ctx->stream); delete ctx; return SLAI_E_HIP;
     }
     ctx->gemv_max_wgs = env_int("SLAI_GEMV_MAX_WGS", 512);
@@ -459,6 +459,11 @@ bool qkv_attention_fusable(const slai_ctx *ctx, const slai_qmat *v, const slai_q
     }
     return true;
 }
+int read_word(slai_ctx *ctx, const void *from, uint32_t *word) {
+    SLAI_HIP_TRY(ctx, hipMemcpyAsync(word, from, sizeof *word, hipMemcpyDeviceToHost, ctx->stream));
+    SLAI_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    return SLAI_OK;
+}
 // Allocated once per context and never moved (captured graphs hold the address): models with more heads than the
 // first reservation allows simply keep separate launches.
 int handoff_reserve(slai_ctx *ctx, uint32_t n_heads) {
@@ -483,7 +488,7 @@ int handoff_reserve(slai_ctx *ctx, uint32_t n_heads) {
 int handoff_check(slai_ctx *ctx) {
     if (!ctx->handoff_counters) return SLAI_OK;
     uint32_t flag = 0;
-    SLAI_HIP_TRY(ctx, hipMemcpy(&flag, ctx->handoff_counters + (size_t)ctx->handoff_heads * 32, sizeof flag, hipMemcpyDeviceToHost));
+    if (const int rc = read_word(ctx, ctx->handoff_counters + (size_t)ctx->handoff_heads * 32, &flag)) return rc;
     if (flag) {
         // reported once: the slot is cleared so that later, healthy calls are not failed for an old time-out, and so are
         // the per-head counters, which a launch that gave up may have left anywhere.  (On the context's stream: it does not wait for

@@ -349,3 +349,39 @@ def test_what_the_caches_held_before_does_not_matter(backend, heads, kv_f16):
         m.destroy()
     assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
     gg.close()
+
+
+def test_beside_a_capture_in_another_thread(backend):
+    """Contexts are independent: one thread captures over and over while another makes contexts, loads, reads prompts (whose pass ends with a look at a
+    flag on the device) and decodes."""
+    import threading
+    from slai_amd.runtime import Backend, Gguf, GpuTensor, Gpt2, Llama2, LlmContext
+    files = [gw.tiny_llama_gguf(seed=72, vocab=1000, n_layers=2, seq_len=64), gw.gpt2_gguf(n_layer=1, seed=72, vocab=1000, n_seq=64)]
+    errors, done = [], threading.Event()
+
+    def capture():
+        try:
+            ctxt, x, y = LlmContext(backend), GpuTensor(backend, 512), GpuTensor(backend, 512)
+            while not done.is_set():
+                backend.graph_begin_capture()
+                for _ in range(50):
+                    ctxt.add_assign(x, y)
+                backend.graph_destroy(backend.graph_end_capture())
+            x.destroy(); y.destroy()
+        except Exception as e:
+            errors.append(e)
+    t = threading.Thread(target=capture)
+    t.start()
+    try:
+        for i in range(10):
+            b = Backend(0)
+            g = Gguf(files[i % 2])
+            m = Llama2(b, g, _ffi.MODEL_LLAMA, _ffi.KV_F16) if i % 2 == 0 else Gpt2(b, g, _ffi.KV_F16)
+            m.prefill(np.arange(12, dtype=np.int32), 0)
+            m.generate(np.array([1, 2, 3], np.int32), 4)
+            m.forward_logits(0, 3)
+            m.destroy(); g.close(); b.close()
+    finally:
+        done.set()
+        t.join()
+    assert not errors, errors
