@@ -75,6 +75,7 @@ struct slai_ctx {
     bool fuse_qkv_attention = true;     // SLAI_FUSE_QKV_ATTN=0: always separate launches
     int prompt_split_f16 = 1;           // SLAI_PROMPT_SPLIT_F16: 0 = prompt-chunk GEMMs in fp32 MFMA, 1 = the models' on the f16 matrix cores (f16 head + remainder), 2 = slai_matmul_quant_columns too
     int *split_flag = nullptr;          // device word the kernels that write split activations set when a value is beyond f16
+    uint32_t *host_word = nullptr;      // pinned: where read_word's copy arrives
     bool prompt_gemm = true;            // SLAI_PROMPT_GEMM=0: prompt chunks never take the matrix-core kernels
     size_t prompt_copy_bytes = (size_t)1 << 30;   // SLAI_PROMPT_COPY_MB (1024): most a model's padded copies for the wide prompt pass may take
     // tuning knobs (environment overridable, see runtime.cpp)
@@ -351,7 +352,8 @@ int gemv_call(slai_ctx *ctx, const GemvCall &c, const char *who, const AttnLaunc
 int step_mark(slai_ctx *ctx, const char *name);        // records an event under `name` when step timing is on
 bool qkv_attention_fusable(const slai_ctx *ctx, const slai_qmat *v, const slai_qmat *k, const slai_qmat *q, const AttnLaunch &a);
 // A word of device memory, once everything enqueued on the context's stream is done.  (Nothing in this library uses the legacy stream: while a thread
-// captures, another one's operation on it fails, and takes the capture with it.)
+// captures, another one's operation on it fails, and takes the capture with it.  By way of pinned memory: 12 us; with a copy to pageable memory 20, a
+// twentieth of a prompt of 37 tokens for the 15 M parameter Llama.)
 int read_word(slai_ctx *ctx, const void *from, uint32_t *word);
 int handoff_reserve(slai_ctx *ctx, uint32_t n_heads);   // not during graph capture
 int handoff_check(slai_ctx *ctx);                        // after a synchronize: error if a hand-off ever timed out

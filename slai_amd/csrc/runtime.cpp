@@ -86,6 +86,9 @@ SLAI_EXPORT int slai_ctx_create(int device, slai_ctx **out) {
     if (hipMalloc((void **)&ctx->split_flag, sizeof(int)) != hipSuccess || hipMemsetAsync(ctx->split_flag, 0, sizeof(int), ctx->stream) != hipSuccess) {
         (void)hipStreamDestroy(ctx->stream); delete ctx; return SLAI_E_HIP;
     }
+    if (hipHostMalloc((void **)&ctx->host_word, sizeof(uint32_t), hipHostMallocDefault) != hipSuccess) {
+        (void)hipFree(ctx->split_flag); (void)hipStreamDestroy(ctx->stream); delete ctx; return SLAI_E_HIP;
+    }
     ctx->gemv_max_wgs = env_int("SLAI_GEMV_MAX_WGS", 512);
     ctx->tiled_layout = env_int("SLAI_TILED", 1) != 0;
     ctx->prompt_copy_bytes = (size_t)std::max(0, env_int("SLAI_PROMPT_COPY_MB", 1024)) << 20;
@@ -113,6 +116,7 @@ SLAI_EXPORT void slai_ctx_destroy(slai_ctx *ctx) {
     if (ctx->attn_scratch) (void)hipFree(ctx->attn_scratch);
     if (ctx->gemv_scratch) (void)hipFree(ctx->gemv_scratch);
     if (ctx->split_flag) (void)hipFree(ctx->split_flag);
+    if (ctx->host_word) (void)hipHostFree(ctx->host_word);
     if (ctx->sampler_scratch) (void)hipFree(ctx->sampler_scratch);
     if (ctx->handoff_counters) (void)hipFree(ctx->handoff_counters);
     for (void *p : ctx->retired_scratch) (void)hipFree(p);
@@ -460,8 +464,9 @@ bool qkv_attention_fusable(const slai_ctx *ctx, const slai_qmat *v, const slai_q
     return true;
 }
 int read_word(slai_ctx *ctx, const void *from, uint32_t *word) {
-    SLAI_HIP_TRY(ctx, hipMemcpyAsync(word, from, sizeof *word, hipMemcpyDeviceToHost, ctx->stream));
+    SLAI_HIP_TRY(ctx, hipMemcpyAsync(ctx->host_word, from, sizeof *word, hipMemcpyDeviceToHost, ctx->stream));
     SLAI_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    *word = *ctx->host_word;
     return SLAI_OK;
 }
 // Allocated once per context and never moved (captured graphs hold the address): models with more heads than the
