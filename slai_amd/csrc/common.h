@@ -506,13 +506,13 @@ struct SmallParams {
     uint32_t absent = 0;                                       // workgroups left out of the launch, which then gives up (for tests)
 };
 bool small_shape_ok(const SmallParams &p);
-uint32_t small_positions(const SmallParams &p);                // where a token in launches becomes the faster one
+uint32_t small_positions(const SmallParams &p, bool split);    // where a token in launches becomes the faster one (split: their attention is)
 hipError_t launch_decode_small(hipStream_t s, const SmallParams &p);
 hipError_t small_capacity(const SmallParams &p, int device, uint32_t *resident);      // workgroups that a die keeps resident
 // The same for GPT-2 over the whole device (kernels_decode_mid.hip); `work` holds FLOW_EMPTY at the start of a launch, no counters
 constexpr uint32_t MID_WGS = 256;
 bool mid_shape_ok(const SmallParams &p);
-uint32_t mid_positions(const SmallParams &p);
+uint32_t mid_positions(const SmallParams &p, bool split);
 hipError_t launch_decode_mid(hipStream_t s, const SmallParams &p);
 hipError_t mid_capacity(const SmallParams &p, int device, uint32_t *resident);        // that the device keeps resident
 

@@ -311,10 +311,10 @@ struct SmallForm {
     }
     // `params` but for the buffers, and the layers' vectors and caches; mats(l): its seven matrices (q, k, v, o, gate, up, down; null: none)
     // (a model that does not get the form, for its shape or for want of memory, does without)
-    template <class Mats> void setup(slai_ctx *ctx, std::vector<SmallLayer> &host, bool one_die, Mats &&mats) {
-        if (!build(ctx, host, one_die, mats)) drop(ctx);
+    template <class Mats> void setup(slai_ctx *ctx, std::vector<SmallLayer> &host, bool one_die, bool split, Mats &&mats) {
+        if (!build(ctx, host, one_die, split, mats)) drop(ctx);
     }
-    template <class Mats> bool build(slai_ctx *ctx, std::vector<SmallLayer> &host, bool one_die, Mats &&mats) {
+    template <class Mats> bool build(slai_ctx *ctx, std::vector<SmallLayer> &host, bool one_die, bool split, Mats &&mats) {
         SmallParams &p = params;
         if (!ctx->persistent) return false;
         uint32_t resident = 0;
@@ -352,7 +352,7 @@ struct SmallForm {
         p.die = next_die.fetch_add(1) & 7u;
         p.spin_limit = ctx->small_spins;
         p.absent = std::min(ctx->small_absent, SMALL_WGS - 1);
-        max_pos = ctx->small_max_pos >= 0 ? (uint32_t)ctx->small_max_pos : one_die ? small_positions(p) : mid_positions(p);
+        max_pos = ctx->small_max_pos >= 0 ? (uint32_t)ctx->small_max_pos : one_die ? small_positions(p, split) : mid_positions(p, split);
         ready = true;
         return true;
     }
@@ -779,7 +779,7 @@ void slai_llama2::small_setup() {
         d.norm1 = vec(w.attn_norm); d.norm2 = vec(w.ffn_norm); d.qb = vec(w.attn_q_bias); d.kb = vec(w.attn_k_bias); d.vb = vec(w.attn_v_bias);
         d.kcache = state.key_cache[l].buf->dptr; d.vcache = state.value_cache[l].buf->dptr;
     }
-    small.setup(ctx, host, true, [&](size_t l) {
+    small.setup(ctx, host, true, attn_splits > 1, [&](size_t l) {
         const Llama2LayerWeights &w = weights.layers[l];
         return std::array<slai_qmat *, 7>{w.attn_q, w.attn_k, w.attn_v, w.attn_output, w.ffn_gate, w.ffn_up, w.ffn_down};
     });
@@ -1794,7 +1794,7 @@ void slai_gpt2::small_setup() {
         d.qb = vec(w.c_attn_attn_b); d.ob = vec(w.c_attn_proj_b); d.upb = vec(w.c_mlp_fc_b); d.downb = vec(w.c_mlp_proj_b);
         d.kcache = w.key_cache.buf->dptr; d.vcache = w.value_cache.buf->dptr;
     }
-    small.setup(ctx, host, false, [&](size_t l) {
+    small.setup(ctx, host, false, attn_splits > 1, [&](size_t l) {
         const Gpt2Layer &w = layers[l];
         return std::array<slai_qmat *, 7>{w.c_attn_attn_w, nullptr, nullptr, w.c_attn_proj_w, nullptr, w.c_mlp_fc_w, w.c_mlp_proj_w};
     });

@@ -253,7 +253,12 @@ bool mid_shape_ok(const SmallParams &p) {
 // layers, launches / this (Q4_0, f16 cache, the slowest):
 //   96 wide, position 250: 132 / 130, 400: 132 / 139;  320, 500: 154 / 151, 700: 155 / 166;  384, 700: 164 / 162;  512, 900: 166 / 172;
 //   640, 1100: 189 / 191;  768, 900: 188 / 174, 1100: 188 / 192;  1024, 1000: 178 / 182, Q8_0 181 / 172
-uint32_t mid_positions(const SmallParams &p) { return min(p.dim * 8 / 5, p.type == T_Q4_0 ? 960u : 1024u); }
+// and where contexts of up to 1024 leave the launches' attention whole, two layers at positions 2 and 100: 64 wide 50.3 / 49.1, 50.5 / 50.4; 96 in 12 heads 48.8 / 50.1,
+// 48.7 / 51.4, in 3 heads 48.3 / 48.8, 48.5 / 50.0; 128 wide 50.1 / 48.6, 50.1 / 49.9; one layer of 64 34.3 / 34.6, 34.6 / 35.3
+uint32_t mid_positions(const SmallParams &p, bool split) {
+    if (!split && p.dim < 128 && (p.dim > 64 || p.n_layers == 1)) return 0;
+    return min(p.dim * 8 / 5, p.type == T_Q4_0 ? 960u : 1024u);
+}
 
 hipError_t mid_capacity(const SmallParams &p, int device, uint32_t *resident) { return resident_workgroups(kernel_of(p), device, resident); }
 

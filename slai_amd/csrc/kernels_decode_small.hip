@@ -278,7 +278,12 @@ bool small_shape_ok(const SmallParams &p) {
 // One workgroup per head walks the cache at 11 ns (f32) or 12 (f16) a position and layer; launches split a head over the device and grow by less than one.
 // us a token of six layers, launches / this, at positions 500, 700, 900 (the slowest format and cache type of each shape; Q4_0 with an f16 cache):
 //   288 wide 154 / 137, 156 / 153, 156 / 166;  480 wide 151 / 135, 151 / 151, 151 / 164;  128 wide 123 / 126, 123 / 140;  64 wide 122 / 126, 123 / 141
-uint32_t small_positions(const SmallParams &p) { return p.dim < 256 ? 448 : 672; }
+// A single layer of up to 128 columns has little to save.  At positions 2, 200, 400: 64 wide 32.5 / 32.3, 33.4 / 34.0, 34.9 / 36.2; with split
+// attention (contexts beyond 1024) 34.6 / 32.4, 34.6 / 34.2, 34.6 / 36.4; 128 wide the same; 192 wide 35.5 / 31.9, 36.7 / 34.0, 38.0 / 36.0
+uint32_t small_positions(const SmallParams &p, bool split) {
+    if (p.dim >= 256) return 672;
+    return p.n_layers > 1 || p.dim > 128 ? 448 : split ? 256 : 0;
+}
 
 hipError_t small_capacity(const SmallParams &p, int device, uint32_t *resident) {
     const void *kernel = p.type == T_Q8_0 ? (p.kv_f16 ? (const void *)decode_small_kernel<T_Q8_0, true> : (const void *)decode_small_kernel<T_Q8_0, false>)

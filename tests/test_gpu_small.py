@@ -148,11 +148,14 @@ def check_gpt2(backend, data, kv_f16, n_prompt, steps, vocab, form=ONE_LAUNCH):
 @pytest.mark.parametrize("kv_f16", [False, True])
 @pytest.mark.parametrize("wtype", [8, 2], ids=["q8_0", "q4_0"])
 @pytest.mark.parametrize("shape", sorted(GPT2))
-def test_gpt2_in_one_launch(backend, shape, wtype, kv_f16):
+def test_gpt2_in_one_launch(monkeypatch, shape, wtype, kv_f16):
+    monkeypatch.setenv("SLAI_SMALL_MAX_POS", "1024")           # (also where launches are the faster form)
+    b = Backend(0)
     dim, hidden, heads, seq = GPT2[shape]
     data = gw.gpt2_gguf(n_embd=dim, n_layer=2, n_head=heads, ff_len=hidden, vocab=700, n_seq=seq, wtype=wtype, seed=61, std=0.05)
     # ("small": positions past two passes of the attention)
-    check_gpt2(backend, data, kv_f16, seq - 30 if shape == "small" else 7, seq - 4 if shape == "small" else 30, 700)
+    check_gpt2(b, data, kv_f16, seq - 30 if shape == "small" else 7, seq - 4 if shape == "small" else 30, 700)
+    b.close()
 
 
 @pytest.mark.parametrize("wtype", [8, 2], ids=["q8_0", "q4_0"])
@@ -163,9 +166,12 @@ def test_gpt2_in_launches(monkeypatch, wtype):
     b.close()
 
 
-def test_gpt2_in_one_launch_single_layer(backend):
+def test_gpt2_in_one_launch_single_layer(monkeypatch):
+    monkeypatch.setenv("SLAI_SMALL_MAX_POS", "1024")
+    b = Backend(0)
     data = gw.gpt2_gguf(n_embd=64, n_layer=1, n_head=2, ff_len=128, vocab=700, n_seq=32, wtype=8, seed=62, std=0.08)
-    check_gpt2(backend, data, False, 4, 20, 700)
+    check_gpt2(b, data, False, 4, 20, 700)
+    b.close()
 
 
 def test_gpt2_gives_up_and_the_call_is_repeated(monkeypatch):
@@ -227,12 +233,29 @@ def test_form_by_position(backend):
         m.destroy(); g.close()
 
 
+# columns, layers, context, line (0: launches at every position)
+@pytest.mark.parametrize("dim,layers,seq,line", [(96, 2, 1024, 0), (96, 6, 64, 0), (64, 1, 512, 0), (64, 2, 1024, 102), (128, 1, 1024, 204), (96, 1, 2048, 153)])
+def test_form_of_narrow_gpt2(backend, dim, layers, seq, line):
+    g = Gguf(gw.gpt2_gguf(n_embd=dim, n_layer=layers, n_head=4, ff_len=2 * dim, vocab=700, n_seq=seq, wtype=8, seed=65, std=0.05))
+    m = Gpt2(backend, g, _ffi.KV_F32)
+    assert [m.decode_form_at(p) for p in (0, max(line, 1) - 1, line)] == [ONE_LAUNCH if line else LAUNCHES] * 2 + [LAUNCHES]
+    m.destroy(); g.close()
+
+
+@pytest.mark.parametrize("dim,layers,seq,line", [(64, 1, 1024, 0), (128, 1, 512, 0), (192, 1, 512, 448), (64, 1, 2048, 256), (64, 2, 1024, 448), (256, 1, 1024, 672)])
+def test_form_of_narrow_llama(backend, dim, layers, seq, line):
+    g = Gguf(gw.llama_gguf(dim=dim, hidden_dim=2 * dim, n_layers=layers, n_heads=4, n_kv_heads=4, vocab=500, seq_len=seq, wtype=8, seed=64, std=0.08))
+    m = Llama2(backend, g, _ffi.MODEL_LLAMA, _ffi.KV_F16)
+    assert [m.decode_form_at(p) for p in (0, max(line, 1) - 1, line)] == [ONE_LAUNCH if line else LAUNCHES] * 2 + [LAUNCHES]
+    m.destroy(); g.close()
+
+
 def test_tokens_across_the_line(backend):
     """The caches are the same in both forms: a call that passes from one to the other, and one that begins beyond."""
     prompt = np.random.Generator(np.random.PCG64(5)).integers(0, 500, 440)
     check_llama(backend, gw.llama_gguf(dim=64, hidden_dim=96, n_layers=2, n_heads=8, n_kv_heads=2, vocab=500, seq_len=512, wtype=8, seed=66, std=0.08, norm_random=True),
                 prompt, 470, check_logit_steps=460)
-    check_gpt2(backend, gw.gpt2_gguf(n_embd=96, n_layer=2, n_head=12, ff_len=160, vocab=700, n_seq=192, wtype=8, seed=67, std=0.05), True, 140, 180, 700, None)
+    check_gpt2(backend, gw.gpt2_gguf(n_embd=64, n_layer=2, n_head=8, ff_len=160, vocab=700, n_seq=192, wtype=8, seed=67, std=0.05), True, 90, 130, 700, None)
 
 
 @pytest.mark.parametrize("which", [0, 1], ids=["llama", "gpt2"])
