@@ -294,10 +294,12 @@ struct WideGemmParams {
 };
 bool wide_gemm_supports(const slai_qmat *m);
 bool wide_reads_sums(const slai_qmat *m);   // whether its input needs the sums of 32 (offsets per sub-block)
-// Form and number of column ranges for nseg matrices over one input (splits: ranges are possible, WIDE_ROWS)
+// Form and number of column ranges for nseg matrices over one input.  WIDE_WHOLE: no ranges; WIDE_SUMMED: partial results are summed by the next norm;
+// WIDE_READ: by each of their readers
 enum { WIDE_LARGE = 0, WIDE_SMALL, WIDE_SLIM4, WIDE_SLIM8 };
+enum WideSplits { WIDE_WHOLE, WIDE_SUMMED, WIDE_READ };
 struct WidePlan { int form; uint32_t ksplit; };
-WidePlan wide_plan(const uint32_t *nrows, int nseg, uint32_t ntokens, uint32_t ncb, bool splits);
+WidePlan wide_plan(const uint32_t *nrows, int nseg, uint32_t ntokens, uint32_t ncb, WideSplits splits);
 hipError_t launch_wide_gemm(hipStream_t st, WideGemmParams p, int mode);
 // x += its nparts partial results (parts + s * part_stride, rows of n), then RMSNorm (b null) or LayerNorm as pairs (with
 // `sums` also their sums of 32)

@@ -1203,15 +1203,17 @@ int slai_llama2::enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev) 
     const uint32_t dim = config.dim, kvd = kv_dim(), hid = config.hidden_dim, hs = head_size(), ncb = (dim + 255) / 256, hcb = (hid + 255) / 256;
     if (n == 0 || n > wide::MAX_TOKENS || pos0 + n > config.seq_len) return set_error(ctx, SLAI_E_ARG, "prompt pass out of range");
     const uint32_t r_qkv[3] = {kvd, kvd, dim}, r_ffn[2] = {hid, hid};
-    const WidePlan p_qkv = wide_plan(r_qkv, 3, n, ncb, true), p_o = wide_plan(&dim, 1, n, ncb, true), p_d = wide_plan(&dim, 1, n, hcb, true);
+    const WidePlan p_qkv = wide_plan(r_qkv, 3, n, ncb, WIDE_READ), p_o = wide_plan(&dim, 1, n, ncb, WIDE_SUMMED), p_d = wide_plan(&dim, 1, n, hcb, WIDE_SUMMED);
+    // the last layer's keys and values: few rows in large workgroups leave most of the device idle (Qwen2-7B shape, 900 tokens: 70 us for 1024 rows)
+    const WidePlan p_kv = p_qkv.form == WIDE_LARGE || p_qkv.form == WIDE_SMALL ? wide_plan(r_qkv, 2, n, ncb, WIDE_READ) : p_qkv;
     const uint32_t ks_qkv = p_qkv.ksplit, ks_o = p_o.ksplit, ks_d = p_d.ksplit;
     const size_t rows = (size_t)n * sizeof(float);
     TRY(WidePass::grow(ctx, wide.x, rows * dim));
     TRY(WidePass::grow(ctx, wide.pairs, wide::activation_bytes(dim, n)));
     TRY(WidePass::grow(ctx, wide.hidden, wide::activation_bytes(hid, n)));
     TRY(WidePass::grow(ctx, wide.q, rows * dim * ks_qkv));
-    TRY(WidePass::grow(ctx, wide.k, rows * kvd * ks_qkv));
-    TRY(WidePass::grow(ctx, wide.v, rows * kvd * ks_qkv));
+    TRY(WidePass::grow(ctx, wide.k, rows * kvd * std::max(ks_qkv, p_kv.ksplit)));
+    TRY(WidePass::grow(ctx, wide.v, rows * kvd * std::max(ks_qkv, p_kv.ksplit)));
     TRY(WidePass::grow(ctx, wide.parts, rows * dim * std::max(ks_o, ks_d)));
     float *x = (float *)wide.x->dptr, *q = (float *)wide.q->dptr, *k = (float *)wide.k->dptr, *v = (float *)wide.v->dptr, *parts = (float *)wide.parts->dptr;
     uint8_t *pairs = (uint8_t *)wide.pairs->dptr, *hidden = (uint8_t *)wide.hidden->dptr;
@@ -1225,7 +1227,7 @@ int slai_llama2::enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev) 
         SLAI_HIP_TRY(ctx, launch_norm_pairs(ctx->stream, pairs, x, parts, nparts, n * dim, (const float *)wl.attn_norm.buf->dptr, nullptr, dim, n, config.rms_norm_eps,
                                              wide_reads_sums(wm.q) || wide_reads_sums(wm.k) || wide_reads_sums(wm.v), flag));
         const WideGemmSeg qkv[3] = {wide_seg(wm.v, v, kvd, n * kvd), wide_seg(wm.k, k, kvd, n * kvd), wide_seg(wm.q, q, dim, n * dim)};
-        TRY(wide_rows(ctx, last ? 2 : 3, qkv, pairs, ncb, n, p_qkv, "llama2 qkv (prompt)"));
+        TRY(wide_rows(ctx, last ? 2 : 3, qkv, pairs, ncb, n, last ? p_kv : p_qkv, "llama2 qkv (prompt)"));
         AttnLaunch a{};
         a.kcache = state.key_cache[l].buf->dptr; a.vcache = state.value_cache[l].buf->dptr; a.kv_f16 = kv_dtype == SLAI_KV_F16;
         a.n_heads = config.n_q_heads; a.kv_mul = config.n_q_heads / config.n_kv_heads; a.head_size = hs; a.kv_dim = kvd; a.seq_len = config.seq_len;
@@ -1234,7 +1236,7 @@ int slai_llama2::enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev) 
         a.kbias = wl.attn_k_bias.buf ? (const float *)wl.attn_k_bias.buf->dptr : nullptr;
         a.vbias = wl.attn_v_bias.buf ? (const float *)wl.attn_v_bias.buf->dptr : nullptr;
         a.rope_variant = rope_variant(); a.rope_base = config.rope_base_freq; a.rope_theta = (const float *)state.rope_theta.buf->dptr;
-        SLAI_HIP_TRY(ctx, launch_rope_store_batch(ctx->stream, a, last ? nullptr : q, k, v, n, dim, kvd, ks_qkv, n * dim, n * kvd));
+        SLAI_HIP_TRY(ctx, launch_rope_store_batch(ctx->stream, a, last ? nullptr : q, k, v, n, dim, kvd, last ? p_kv.ksplit : ks_qkv, n * dim, n * kvd));
         if (last) break;
         PromptAttention pa;
         pa.q = q; pa.q_stride = dim; pa.kcache = a.kcache; pa.vcache = a.vcache; pa.kv_dim = kvd; pa.n_heads = a.n_heads; pa.kv_mul = a.kv_mul;
@@ -1246,7 +1248,7 @@ int slai_llama2::enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev) 
                                              wide_reads_sums(wm.gate), flag));
         WideGemmParams g;
         g.nseg = 2; g.seg[0] = wide_seg(wm.gate, nullptr, 0, 0); g.seg[1] = wide_seg(wm.up, nullptr, 0, 0);
-        g.x = pairs; g.ncb = ncb; g.ntokens = n; g.pairs_out = hidden; g.out_ncb = hcb; g.out_sums = wide_reads_sums(wm.down); g.up = wm.hidden_up; g.flag = flag; g.form = wide_plan(r_ffn, 2, n, ncb, false).form;
+        g.x = pairs; g.ncb = ncb; g.ntokens = n; g.pairs_out = hidden; g.out_ncb = hcb; g.out_sums = wide_reads_sums(wm.down); g.up = wm.hidden_up; g.flag = flag; g.form = wide_plan(r_ffn, 2, n, ncb, WIDE_WHOLE).form;
         TRY(wide_call(ctx, g, WIDE_GATED, "llama2 ffn gate/up (prompt)"));
         WideGemmSeg d = wide_seg(wm.down, parts, dim, n * dim);
         d.down = 1.0f / wm.hidden_up;
@@ -1948,7 +1950,7 @@ int slai_gpt2::enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev) {
     const uint32_t E = params.n_embd, F = params.ff_len, hs = E / params.n_head, ncb = E / 256, fcb = F / 256;
     if (n == 0 || n > wide::MAX_TOKENS || pos0 + n > params.n_seq) return set_error(ctx, SLAI_E_ARG, "prompt pass out of range");
     const uint32_t r_qkv = 3 * E;
-    const WidePlan p_qkv = wide_plan(&r_qkv, 1, n, ncb, true), p_o = wide_plan(&E, 1, n, ncb, true), p_d = wide_plan(&E, 1, n, fcb, true);
+    const WidePlan p_qkv = wide_plan(&r_qkv, 1, n, ncb, WIDE_READ), p_o = wide_plan(&E, 1, n, ncb, WIDE_SUMMED), p_d = wide_plan(&E, 1, n, fcb, WIDE_SUMMED);
     const uint32_t ks_qkv = p_qkv.ksplit, ks_o = p_o.ksplit, ks_d = p_d.ksplit;
     const size_t rows = (size_t)n * sizeof(float);
     TRY(WidePass::grow(ctx, wide.x, rows * E));
@@ -1987,7 +1989,7 @@ int slai_gpt2::enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev) {
                                              wide_reads_sums(w.c_mlp_fc_w), flag));
         WideGemmParams g;
         g.nseg = 1; g.seg[0] = wide_seg(w.c_mlp_fc_w, nullptr, 0, 0, &w.c_mlp_fc_b);
-        g.x = pairs; g.ncb = ncb; g.ntokens = n; g.pairs_out = hidden; g.out_ncb = fcb; g.out_sums = wide_reads_sums(w.c_mlp_proj_w); g.flag = flag; g.form = wide_plan(&F, 1, n, ncb, false).form;
+        g.x = pairs; g.ncb = ncb; g.ntokens = n; g.pairs_out = hidden; g.out_ncb = fcb; g.out_sums = wide_reads_sums(w.c_mlp_proj_w); g.flag = flag; g.form = wide_plan(&F, 1, n, ncb, WIDE_WHOLE).form;
         TRY(wide_call(ctx, g, WIDE_GELU, "gpt2 mlp fc (prompt)"));
         const WideGemmSeg sd = wide_seg(w.c_mlp_proj_w, parts, E, n * E, &w.c_mlp_proj_b);
         TRY(wide_rows(ctx, 1, &sd, hidden, fcb, n, p_d, "gpt2 mlp proj (prompt)"));
