@@ -72,6 +72,8 @@ struct slai_ctx {
     size_t sampler_scratch_floats = 0;
     uint32_t *handoff_counters = nullptr;   // q/k/v + attention in one launch: one 128-byte line per head, then a timeout flag
     uint32_t handoff_heads = 0;
+    float *spread_sums = nullptr;           // row tiles that several workgroups share (gemv_spread_kernel): their sums, and a count per workgroup
+    uint32_t *spread_counters = nullptr;
     bool fuse_qkv_attention = true;     // SLAI_FUSE_QKV_ATTN=0: always separate launches
     int prompt_split_f16 = 1;           // SLAI_PROMPT_SPLIT_F16: 0 = prompt-chunk GEMMs in fp32 MFMA, 1 = the models' on the f16 matrix cores (f16 head + remainder), 2 = slai_matmul_quant_columns too
     int *split_flag = nullptr;          // device word the kernels that write split activations set when a value is beyond f16
@@ -218,6 +220,8 @@ struct GemvRowtileParams {
     float *scratch = nullptr;         // one slot of ncols + ncols/16 floats per workgroup (= per tile); unused with `prepared`
     uint32_t scratch_stride = 0;      // filled by the launcher
 };
+size_t gemv_spread_floats();             // of slai_ctx::spread_sums
+size_t gemv_spread_counter_words();      // of slai_ctx::spread_counters
 size_t gemv_rowtile_scratch_floats(const GemvRowtileParams &p);
 // With a batch of more than one vector the input must come `prepared`.
 hipError_t launch_gemv_rowtile(slai_ctx *ctx, GemvRowtileParams p, const GemvBatch *batch = nullptr);

@@ -16,6 +16,9 @@
 //
 // One workgroup = one tile = 64 complete output rows; wave w owns super-blocks w, w+NW, ...; partial
 // sums meet in LDS once.  Segments of one launch may differ in block format (Q4_K q/k with a Q6_K v).
+#include <algorithm>
+#include <type_traits>
+
 #include "common.h"
 #include "attention_fast.h"
 #include "device_util.h"
@@ -212,6 +215,163 @@ __global__ void __launch_bounds__(1024) gemv_rowtile_kernel(const GemvRowtilePar
     }
 }
 
+// The same tiles spread evenly over the device (prepared input only).  A launch of one workgroup per tile leaves compute units idle
+// where the tiles are no multiple of them: gate + up of the Qwen2-7B shape are 296 tiles on 256 compute units, a second round of 40, its
+// q/k/v 72 tiles.  Here the tiles of a die (workgroup i runs on die i mod 8) are cut into (tile, super-block) units and its 32 workgroups
+// take equal runs of them, a wave one or two units.  A tile that several workgroups share meets in the die's L2: each leaves its
+// sums, waits until they are there and counts itself in with an atomic that executes there; the one that completes the count adds
+// them up in the order of the workgroups (so results do not depend on who comes last) and finishes the rows.  Nobody waits for anybody.
+// What bounds it: memory (gate + up of the Qwen2-7B shape, Q4_K: 76 MB in 17.2 us, 4.4 TB/s, 21.5 with a workgroup per tile; q/k/v 9.1 -> 7.4 us),
+// of which about 4 us start the launch and 1 us merges the tiles.  64 workgroups of half as many waves per die: 17.2 to 17.4.
+constexpr uint32_t SPREAD_DIES = 8, SPREAD_RUNS = 32, SPREAD_UNITS = 32;       // runs of a die; most units of a run
+
+template <int TT, bool DUAL>
+__global__ void __launch_bounds__(1024) gemv_spread_kernel(const GemvRowtileParams p, float *shared_sums, uint32_t *counters, uint32_t total_tiles) {
+    const uint32_t waves = blockDim.x >> 6;
+    __shared__ float partial[(DUAL ? 2 : 1) * SPREAD_UNITS * 64];
+    __shared__ float red[16];
+    touch_kernel_arguments<((sizeof(GemvRowtileParams) + 24 + 63) / 64) * 64>();
+    const int NT = blockDim.x;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t die = blockIdx.x % SPREAD_DIES, run = blockIdx.x / SPREAD_DIES, ncb = p.ncb;
+    const uint32_t tiles = (total_tiles + SPREAD_DIES - 1 - die) / SPREAD_DIES, units = tiles * ncb;      // of this die: tiles die, die + 8, ...
+    const uint32_t u0 = units * run / SPREAD_RUNS, u1 = units * (run + 1) / SPREAD_RUNS;
+    const uint32_t n0 = p.seg[0].ntiles, n1 = p.seg[1].ntiles;           // unused segments have ntiles = 0
+    const auto segment = [&](uint32_t tile) { return tile < n0 ? 0 : (tile - n0 < n1 ? 1 : 2); };
+    const auto pick = [](int s, auto a, auto b, auto c) { return s == 0 ? a : (s == 1 ? b : c); };
+
+    constexpr int XMAX = 4, NM = DUAL ? 2 : 1;                // float4 of x per thread: ncols <= 16 * NT
+    float4 xv[XMAX];
+    const bool norm = p.prologue == PRO_RMSNORM;
+    const auto request_x = [&]() {
+        if (!norm) return;
+#pragma unroll
+        for (int j = 0; j < XMAX; ++j) xv[j] = *(const float4 *)(p.x + min((uint32_t)(j * NT + tid) * 4, p.ncols - 4));
+    };
+    const auto sum_squares = [&]() {                          // while the first weights travel
+        if (!norm) return;
+        float ss = 0.0f;
+#pragma unroll
+        for (int j = 0; j < XMAX; ++j) {
+            const float4 q = xv[j];
+            const float live = (uint32_t)(j * NT + tid) * 4 < p.ncols ? 1.0f : 0.0f;
+            ss = fmaf(live * q.x, q.x, ss); ss = fmaf(live * q.y, q.y, ss); ss = fmaf(live * q.z, q.z, ss); ss = fmaf(live * q.w, q.w, ss);
+        }
+        ss = wave_sum(ss);
+        if (lane == 0) red[wave] = ss;
+    };
+    cfloat *const xs = (cfloat *)(uintptr_t)p.prepared;
+    const auto unit = [&](auto type, uint32_t u, auto first_of_wave) __attribute__((always_inline)) {
+        constexpr bool first = decltype(first_of_wave)::value;
+        constexpr int T = decltype(type)::value;
+        using F = Tiled<T>;
+        const uint32_t tile_all = die + SPREAD_DIES * (u / ncb), cb = u % ncb;
+        const int s = segment(tile_all);
+        const uint32_t tile = tile_all - (s == 0 ? 0u : (s == 1 ? n0 : n0 + n1));
+        const uint32_t unit_bytes = F::PT * 1024 + (F::TAIL ? 128 : 0);
+        const uint8_t *W = pick(s, p.seg[0].W, p.seg[1].W, p.seg[2].W);
+        typename F::Data d, e;
+        uint16_t dt = 0, et = 0;
+        UnitLoader<T, NM, ROWTILE_LD> ld;
+        const size_t off = ((size_t)tile * ncb + cb) * unit_bytes;
+        ld.unit[0] = W + off + lane * 16; ld.tailp[0] = W + off + (size_t)F::PT * 1024 + lane * 2; ld.d[0] = &d; ld.t[0] = &dt;
+        if constexpr (DUAL) {
+            const uint8_t *W2 = pick(s, p.seg[0].W2, p.seg[1].W2, p.seg[2].W2);
+            ld.unit[1] = W2 + off + lane * 16; ld.tailp[1] = W2 + off + (size_t)F::PT * 1024 + lane * 2; ld.d[1] = &e; ld.t[1] = &et;
+        }
+        F::lead(ld);
+        if constexpr (first) request_x();
+        {   // the cache lines of this super-block's activations, touched at once (see tile_body)
+            typedef const uint32_t __attribute__((address_space(4))) cu32;
+            cu32 *wx = (cu32 *)(xs + (size_t)cb * 256), *ws = (cu32 *)(xs + p.ncols + (size_t)cb * 16);
+            uint32_t warm = ws[0];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) warm |= wx[16 * i];
+            asm volatile("" : : "s"(warm));
+        }
+        if constexpr (first) sum_squares();
+        ScalarX X{xs + (size_t)cb * 256, xs + p.ncols + (size_t)cb * 16};
+        const typename F::Data *dp[NM];
+        uint16_t tails[NM];
+        float o2[NM];
+        dp[0] = &d; tails[0] = dt;
+        if constexpr (DUAL) { dp[1] = &e; tails[1] = et; }
+        F::template dotn<NM>(dp, tails, X, o2, ld);
+        partial[(u - u0) * 64 + lane] = o2[0];
+        if constexpr (DUAL) partial[(SPREAD_UNITS + u - u0) * 64 + lane] = o2[1];
+    };
+    const auto any_unit = [&](uint32_t u, auto first) __attribute__((always_inline)) {
+        if constexpr (TT != 0) {
+            unit(std::integral_constant<int, TT>(), u, first);
+        } else {
+            const int s = segment(die + SPREAD_DIES * (u / ncb));
+            switch (pick(s, p.seg[0].type, p.seg[1].type, p.seg[2].type)) {          // uniform over the wave
+            case T_Q4_K: unit(std::integral_constant<int, T_Q4_K>(), u, first); break;
+            case T_Q6_K: unit(std::integral_constant<int, T_Q6_K>(), u, first); break;
+            case T_Q5_K: if constexpr (!DUAL) unit(std::integral_constant<int, T_Q5_K>(), u, first); break;
+            default: break;                                    // the launcher sends the other formats to their own kernels
+            }
+        }
+    };
+    if (u0 + wave < u1) any_unit(u0 + wave, std::true_type());
+    else { request_x(); sum_squares(); }
+    if (u0 + wave + waves < u1) any_unit(u0 + wave + waves, std::false_type());
+    lds_barrier();
+
+    // ---- the tiles of this workgroup, one per wave in turn
+    for (uint32_t j = (u0 / ncb) + wave; j * ncb < u1 && u0 < u1; j += waves) {
+        const uint32_t a = max(u0, j * ncb), b = min(u1, (j + 1) * ncb);
+        float o = 0.0f, up = 0.0f;
+        for (uint32_t u = a; u < b; ++u) {
+            o += partial[(u - u0) * 64 + lane];
+            if constexpr (DUAL) up += partial[(SPREAD_UNITS + u - u0) * 64 + lane];
+        }
+        if (b - a < ncb) {                                     // shared with the workgroups next to this one
+            const auto owner = [&](uint32_t u) { return (SPREAD_RUNS * (u + 1) - 1) / units; };
+            const uint32_t r0 = owner(j * ncb), r1 = owner((j + 1) * ncb - 1);
+            // a workgroup's place: 0 for a tile that begins before its run, 1 for one that begins in it
+            const auto place = [&](uint32_t r) { return shared_sums + (size_t)((r * SPREAD_DIES + die) * 2 + (r == r0 ? 1 : 0)) * 128; };
+            float *mine = place(run);
+            mine[lane] = o;
+            if constexpr (DUAL) mine[64 + lane] = up;
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            uint32_t *counter = counters + (size_t)(r0 * SPREAD_DIES + die) * 32;
+            uint32_t seen = 0;
+            if (lane == 0) {
+                const uint32_t one = 1;
+                asm volatile("global_atomic_add %0, %1, %2, off sc0\n\ts_waitcnt vmcnt(0)" : "=&v"(seen) : "v"(counter), "v"(one) : "memory");
+            }
+            seen = __builtin_amdgcn_readfirstlane(seen);
+            if (seen != r1 - r0) continue;
+            if (lane == 0) *counter = 0u;                      // for the next launch; nobody else touches it any more
+            o = 0.0f; up = 0.0f;
+            for (uint32_t r = r0; r <= r1; ++r) {
+                const float *q = place(r);
+                o += q[lane];
+                if constexpr (DUAL) up += q[64 + lane];
+            }
+        }
+        const uint32_t tile_all = die + SPREAD_DIES * j;
+        const int s = segment(tile_all);
+        const uint32_t row = (tile_all - (s == 0 ? 0u : (s == 1 ? n0 : n0 + n1))) * 64 + lane;
+        const uint32_t flags = pick(s, p.seg[0].flags, p.seg[1].flags, p.seg[2].flags);
+        if (row >= pick(s, p.seg[0].nrows, p.seg[1].nrows, p.seg[2].nrows)) continue;
+        float *out = pick(s, p.seg[0].out, p.seg[1].out, p.seg[2].out) + row;
+        if (norm) {
+            float t = 0.0f;
+            for (uint32_t w = 0; w < waves; ++w) t += red[w];
+            const float scale = 1.0f / sqrtf(t / (float)p.ncols + p.eps);     // (applied to the finished dot product, as in tile_body)
+            o *= scale; up *= scale;
+        }
+        if constexpr (DUAL) o = up * (o / (1.0f + expf(-o)));  // silu.slang:8-26
+        if (flags & GEMV_BIAS) o += pick(s, p.seg[0].bias, p.seg[1].bias, p.seg[2].bias)[row];
+        if (flags & GEMV_GELU) o = gelu_f(o);
+        if (flags & GEMV_ACCUM) o = *out + o;
+        *out = o;
+    }
+}
+
 // The same tiles for several input vectors (a chunk of prompt tokens; prepared input only).  Workgroup i runs on XCD
 // i % 8, and workgroups are dispatched in index order: the bt.n workgroups of one tile get consecutive indices on ONE
 // XCD, i = ((tile / 8) * bt.n + b) * 8 + tile % 8, so they run at the same time on neighbouring compute units, the
@@ -314,11 +474,41 @@ __global__ void __launch_bounds__(1024) qkv_attention_kernel(const GemvRowtilePa
     });
 }
 
+// Units of the longest run
+uint32_t spread_units(uint32_t tiles, uint32_t ncb) { return ((tiles + SPREAD_DIES - 1) / SPREAD_DIES * ncb + SPREAD_RUNS - 1) / SPREAD_RUNS; }
+
+// Where the even spread is the faster form: tiles a little beyond a round of the compute units, and few tiles of long rows.  us a launch, one
+// workgroup per tile / spread (gated pairs, then single matrices; 256-column groups x format):
+//   tiles      16 x Q4_K pair  16 x Q8_0 pair   8 x Q4_K pair   10 x Q4_K pair   16 x Q4_K      12 x Q4_K      12 x Q6_K
+//   40 to 48   10.3 / 7.8      13.7 / 8.7                        8.7 / 7.4       6.1 / 5.7      5.3 / 5.6      6.7 / 6.3
+//   64 to 72   10.5 / 8.0      14.4 / 10.1                       8.8 / 7.5       6.2 / 5.7      5.4 / 5.5      6.8 / 6.3
+//   88 to 96   11.0 / 9.3      15.5 / 12.7     7.3 / 7.5         9.0 / 7.8       6.3 / 6.3      5.5 / 5.9      7.1 / 7.0
+//   128        11.8 / 10.1     16.4 / 15.0     7.5 / 7.8                         6.6 / 6.6      5.6 / 6.1      7.3 / 7.3
+//   172        12.2 / 12.4     18.2 / 20.0                                       6.9 / 7.9
+//   272        22.1 / 17.5     35.1 / 27.1                                      12.5 / 10.7
+//   320        22.8 / 19.5     37.0 / 31.3    12.6 / 11.6                       12.8 / 11.3
+//   384        23.5 / 21.9     37.6 / 37.1    13.2 / 12.8                       13.0 / 12.5
+//   432        24.4 / 24.8     41.6 / 41.2    (448: 13.7 / 15.2)                13.6 / 14.2
+// (tile: 147 KB of a Q4_K row tile of 16 groups, twice that of a pair)
+bool spread_pays(const GemvRowtileParams &p, uint32_t tiles) {
+    uint64_t bytes = 0;
+    for (int i = 0; i < p.nseg; ++i) bytes += (uint64_t)p.seg[i].ntiles * (p.seg[i].W2 ? 2 : 1) * p.ncb * (tiled_pieces(p.seg[i].type) * 1024 + tiled_tail(p.seg[i].type));
+    const uint64_t tile = bytes / tiles;
+    if (tiles * p.ncb < SPREAD_DIES * SPREAD_RUNS + SPREAD_DIES * p.ncb || spread_units(tiles, p.ncb) > SPREAD_UNITS) return false;   // (no run may be empty)
+    if (tiles > 256) return tiles <= 352 && tile >= 140000;
+    return p.ncb >= 10 && ((tiles <= 96 && tile >= 124000) || (tiles <= 128 && tile >= 180000));
+}
+
 template <int TT, bool DUAL>
-hipError_t go(const GemvRowtileParams &p, uint32_t tiles, int NT, size_t smem, hipStream_t s, const GemvBatch *bt) {
+hipError_t go(const GemvRowtileParams &p, uint32_t tiles, int NT, size_t smem, hipStream_t s, const GemvBatch *bt, float *spread_sums, uint32_t *spread_counters) {
     if (bt && bt->n > 1) {
         if (!p.prepared) return hipErrorInvalidValue;
         gemv_rowtile_batch_kernel<TT, DUAL><<<(tiles + 7) / 8 * 8 * bt->n, NT, smem, s>>>(p, *bt, tiles);
+        return hipGetLastError();
+    }
+    if (p.prepared && spread_sums) {
+        const uint32_t most = spread_units(tiles, p.ncb), waves = std::min(16u, std::max(std::max(most, 4u), (p.ncols + 1023) / 1024));     // (x: four float4 per thread)
+        gemv_spread_kernel<TT, DUAL><<<SPREAD_DIES * SPREAD_RUNS, waves * 64, 0, s>>>(p, spread_sums, spread_counters, tiles);
         return hipGetLastError();
     }
     if (p.prepared) gemv_rowtile_kernel<TT, DUAL, true><<<tiles, NT, smem, s>>>(p);
@@ -327,6 +517,9 @@ hipError_t go(const GemvRowtileParams &p, uint32_t tiles, int NT, size_t smem, h
 }
 
 }  // namespace
+
+size_t gemv_spread_floats() { return (size_t)SPREAD_DIES * SPREAD_RUNS * 2 * 128; }
+size_t gemv_spread_counter_words() { return (size_t)SPREAD_DIES * SPREAD_RUNS * 32; }
 
 size_t gemv_rowtile_scratch_floats(const GemvRowtileParams &p) {
     uint32_t tiles = 0;
@@ -362,13 +555,14 @@ hipError_t launch_gemv_rowtile(slai_ctx *ctx, GemvRowtileParams p, const GemvBat
     }
     const int NT = NW * 64;
     hipStream_t st = ctx->stream;
+    float *spread = ctx->fuse_qkv_attention && spread_pays(p, tiles) ? ctx->spread_sums : nullptr;
     switch (tt) {
-    case T_Q4_K: return dual ? go<T_Q4_K, true>(p, tiles, NT, smem, st, bt) : go<T_Q4_K, false>(p, tiles, NT, smem, st, bt);
-    case T_Q6_K: return dual ? go<T_Q6_K, true>(p, tiles, NT, smem, st, bt) : go<T_Q6_K, false>(p, tiles, NT, smem, st, bt);
-    case T_Q8_0: return dual ? go<T_Q8_0, true>(p, tiles, NT, smem, st, bt) : go<T_Q8_0, false>(p, tiles, NT, smem, st, bt);
-    case T_Q4_0: return dual ? go<T_Q4_0, true>(p, tiles, NT, smem, st, bt) : go<T_Q4_0, false>(p, tiles, NT, smem, st, bt);
-    case T_Q5_K: return dual ? go<T_Q5_K, true>(p, tiles, NT, smem, st, bt) : go<T_Q5_K, false>(p, tiles, NT, smem, st, bt);
-    default: return dual ? go<0, true>(p, tiles, NT, smem, st, bt) : go<0, false>(p, tiles, NT, smem, st, bt);
+    case T_Q4_K: return dual ? go<T_Q4_K, true>(p, tiles, NT, smem, st, bt, spread, ctx->spread_counters) : go<T_Q4_K, false>(p, tiles, NT, smem, st, bt, spread, ctx->spread_counters);
+    case T_Q6_K: return dual ? go<T_Q6_K, true>(p, tiles, NT, smem, st, bt, spread, ctx->spread_counters) : go<T_Q6_K, false>(p, tiles, NT, smem, st, bt, spread, ctx->spread_counters);
+    case T_Q8_0: return dual ? go<T_Q8_0, true>(p, tiles, NT, smem, st, bt, spread, ctx->spread_counters) : go<T_Q8_0, false>(p, tiles, NT, smem, st, bt, spread, ctx->spread_counters);
+    case T_Q4_0: return dual ? go<T_Q4_0, true>(p, tiles, NT, smem, st, bt, spread, ctx->spread_counters) : go<T_Q4_0, false>(p, tiles, NT, smem, st, bt, spread, ctx->spread_counters);
+    case T_Q5_K: return dual ? go<T_Q5_K, true>(p, tiles, NT, smem, st, bt, spread, ctx->spread_counters) : go<T_Q5_K, false>(p, tiles, NT, smem, st, bt, spread, ctx->spread_counters);
+    default: return dual ? go<0, true>(p, tiles, NT, smem, st, bt, spread, ctx->spread_counters) : go<0, false>(p, tiles, NT, smem, st, bt, spread, ctx->spread_counters);
     }
 }
 

@@ -119,6 +119,8 @@ SLAI_EXPORT void slai_ctx_destroy(slai_ctx *ctx) {
     if (ctx->host_word) (void)hipHostFree(ctx->host_word);
     if (ctx->sampler_scratch) (void)hipFree(ctx->sampler_scratch);
     if (ctx->handoff_counters) (void)hipFree(ctx->handoff_counters);
+    if (ctx->spread_sums) (void)hipFree(ctx->spread_sums);
+    if (ctx->spread_counters) (void)hipFree(ctx->spread_counters);
     for (void *p : ctx->retired_scratch) (void)hipFree(p);
     for (slai_buffer *b : ctx->retired_buffers) buffer_free(b);
     if (ctx->timer0) (void)hipEventDestroy(ctx->timer0);
@@ -486,6 +488,9 @@ int handoff_reserve(slai_ctx *ctx, uint32_t n_heads) {
     for (uint32_t i = 8; i < 256; ++i)
         if (where[i] != where[i % 8]) ctx->fuse_qkv_attention = false;
     SLAI_HIP_TRY(ctx, hipMemsetAsync(ctx->handoff_counters, 0, bytes, ctx->stream));
+    SLAI_HIP_TRY(ctx, hipMalloc((void **)&ctx->spread_counters, gemv_spread_counter_words() * sizeof(uint32_t)));
+    SLAI_HIP_TRY(ctx, hipMemsetAsync(ctx->spread_counters, 0, gemv_spread_counter_words() * sizeof(uint32_t), ctx->stream));
+    SLAI_HIP_TRY(ctx, hipMalloc((void **)&ctx->spread_sums, gemv_spread_floats() * sizeof(float)));
     SLAI_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
     ctx->handoff_heads = n_heads;
     return SLAI_OK;

@@ -1,0 +1,57 @@
+"""Row tiles spread evenly over the device (gemv_spread_kernel): where its tiles and runs meet."""
+import numpy as np
+import pytest
+
+from gpu_common import backend  # noqa: F401
+from slai_amd import synth
+
+pytestmark = pytest.mark.gpu
+NAMES = {2: "q4_0", 8: "q8_0", 12: "q4_k", 13: "q5_k", 14: "q6_k"}
+
+
+@pytest.fixture(scope="module")
+def model(backend):
+    # a context whose models have looked where its workgroups run takes the spread form
+    from slai_amd import _ffi
+    from slai_amd import gguf_writer as gw
+    from slai_amd.runtime import Gguf, Llama2
+    g = Gguf(gw.llama_gguf(256, 512, 1, 2, 2, 512, 64, 12, v_type=14, out_type=14, embd_type=12))
+    m = Llama2(backend, g, _ffi.MODEL_LLAMA, _ffi.KV_F16)
+    yield m
+    m.destroy()
+    g.close()
+
+
+# rows: the last tile whole, one row of it, tiles of a die beyond the others'; columns: the fewest groups, runs that end inside
+# tiles and at their ends, two units per wave
+@pytest.mark.parametrize("t,rows,cols,gated", [(12, 2048, 2560, True), (8, 1985, 3584, True), (13, 4609, 3584, True), (12, 6144, 2560, True), (2, 6100, 4096, True), (14, 3072, 2560, False),
+                                               (12, 8192, 5120, False), (8, 16385, 2048, True), (12, 22528, 4096, True), (14, 18944, 3584, False), (12, 22465, 2560, False)],
+                         ids=lambda v: NAMES.get(v, str(v)))
+def test_spread_against_float64(backend, model, t, rows, cols, gated):
+    from slai_amd import _ffi
+    from slai_amd.runtime import GpuQuantMatrix, GpuTensor, LlmContext
+    print("case", NAMES[t], rows, cols, gated, flush=True)
+    mats = [GpuQuantMatrix(backend, t, rows, cols, synth.normal_quantized(5 + i, t, rows, cols, 0.02), layout=_ffi.LAYOUT_TILE64) for i in range(2 if gated else 1)]
+    x, w = synth.normal(7, cols, 1.0), 1 + synth.normal(8, cols, 0.1)
+    xd, wd, prep, out = GpuTensor.vector(backend, x), GpuTensor.vector(backend, w if gated else np.ones(cols, np.float32)), GpuTensor(backend, cols + cols // 16), GpuTensor(backend, rows)
+    c = LlmContext(backend)
+    c.rms_norm_prepare(prep, xd, wd)
+    results = []
+    for _ in range(3):                                         # the counts are back at zero after each launch
+        if gated:
+            c.ffn_gate_up_silu_prepared(out, mats[0], mats[1], xd, prep, 1e-5)
+        else:
+            c.matmul_quant_assign_prepared(out, mats[0], prep)
+        results.append(out.read())
+    assert all(np.array_equal(results[0], r) for r in results[1:])
+    x64 = x.astype(np.float64)
+    if gated:
+        n = x64 * w / np.sqrt(np.mean(x64 * x64) + 1e-5)
+        g, u = (np.array([np.dot(row, n) for row in m.dequantize().astype(np.float64)]) for m in mats)
+        ref = u * g / (1 + np.exp(-g))
+    else:
+        ref = mats[0].dequantize().astype(np.float64) @ x64
+    # sums of at most 5120 products in 32 bits, taken in lanes and blocks: a few 2^-24 of their norm, twice in a gated product
+    assert np.linalg.norm(results[0] - ref) / np.linalg.norm(ref) < 1.5e-6
+    for o in mats + [xd, wd, prep, out]:
+        o.destroy()
