@@ -294,16 +294,20 @@ struct WideGemmParams {
     bool out_sums = false;        // their sums of 32 too
     float up = 1.0f;              // WIDE_GATED: factor of the output, a power of two
     int *flag = nullptr;          // set when an output is beyond f16
+    uint8_t *shared = nullptr;    // WIDE_SHARE: tiles that several workgroups share, and a count for each workgroup (zero between launches)
+    uint32_t *counters = nullptr;
     uint32_t token_blocks = 0, row_units = 0, out_c8 = 0;   // filled by the launcher
 };
 bool wide_gemm_supports(const slai_qmat *m);
 bool wide_reads_sums(const slai_qmat *m);   // whether its input needs the sums of 32 (offsets per sub-block)
 // Form and number of column ranges for nseg matrices over one input.  WIDE_WHOLE: no ranges; WIDE_SUMMED: partial results are summed by the next norm;
 // WIDE_READ: by each of their readers
-enum { WIDE_LARGE = 0, WIDE_SMALL, WIDE_SLIM4, WIDE_SLIM8 };
+enum { WIDE_LARGE = 0, WIDE_SMALL, WIDE_SLIM4, WIDE_SLIM8, WIDE_SHARE };
 enum WideSplits { WIDE_WHOLE, WIDE_SUMMED, WIDE_READ };
 struct WidePlan { int form; uint32_t ksplit; };
-WidePlan wide_plan(const uint32_t *nrows, int nseg, uint32_t ntokens, uint32_t ncb, WideSplits splits);
+WidePlan wide_plan(const uint32_t *nrows, int nseg, uint32_t ntokens, uint32_t ncb, WideSplits splits, bool may_share);
+size_t wide_share_bytes();                   // of WideGemmParams::shared
+size_t wide_share_counter_words();           // of WideGemmParams::counters
 hipError_t launch_wide_gemm(hipStream_t st, WideGemmParams p, int mode);
 // x += its nparts partial results (parts + s * part_stride, rows of n), then RMSNorm (b null) or LayerNorm as pairs (with
 // `sums` also their sums of 32)

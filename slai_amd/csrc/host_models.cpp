@@ -150,6 +150,7 @@ struct WidePass {
     slai_buffer *x = nullptr, *pairs = nullptr, *hidden = nullptr;   // residual rows; normalised rows / attention results and the hidden layer as pairs
     slai_buffer *q = nullptr, *k = nullptr, *v = nullptr;            // projections (k, v: Llama; GPT-2's are columns of q), possibly in partial results
     slai_buffer *parts = nullptr;                                    // partial results of the projection into the residual
+    slai_buffer *shared = nullptr;                                   // of tiles that workgroups share (WIDE_SHARE)
 
     static int grow(slai_ctx *ctx, slai_buffer *&b, size_t bytes) {
         if (b && b->bytes >= bytes) return SLAI_OK;
@@ -158,7 +159,7 @@ struct WidePass {
         return slai_buffer_create(ctx, bytes, SLAI_DT_F32, STORAGE, &b);
     }
     void destroy(slai_ctx *ctx) {
-        for (slai_buffer **b : {&x, &pairs, &hidden, &q, &k, &v, &parts})
+        for (slai_buffer **b : {&x, &pairs, &hidden, &q, &k, &v, &parts, &shared})
             if (*b) { slai_buffer_destroy(ctx, *b); *b = nullptr; }
     }
 };
@@ -234,13 +235,20 @@ WideGemmSeg wide_seg(const slai_qmat *m, float *out, uint32_t out_stride, uint32
     s.bias = bias && bias->buf ? (const float *)bias->buf->dptr : nullptr;
     return s;
 }
-int wide_call(slai_ctx *ctx, const WideGemmParams &p, int mode, const char *who) {
+// Whether workgroups may share a tile through their die's L2: their placement has been looked at (handoff_reserve)
+bool wide_may_share(const slai_ctx *ctx) { return ctx->fuse_qkv_attention && ctx->spread_counters; }
+int wide_call(slai_ctx *ctx, WidePass &pass, WideGemmParams p, int mode, const char *who) {
+    if (p.form == WIDE_SHARE) {
+        TRY(WidePass::grow(ctx, pass.shared, wide_share_bytes()));
+        p.shared = (uint8_t *)pass.shared->dptr;
+        p.counters = ctx->spread_counters;
+    }
     const hipError_t e = launch_wide_gemm(ctx->stream, p, mode);
     if (e == hipErrorInvalidValue) return set_error(ctx, SLAI_E_SHAPE, std::string(who) + ": unsupported shape for the wide prompt GEMM");
     return e == hipSuccess ? SLAI_OK : hip_fail(ctx, e, who);
 }
 // Segments over one input as rows: formats that can share a launch do (any K-quants, otherwise equal ones)
-int wide_rows(slai_ctx *ctx, int nseg, const WideGemmSeg *segs, const uint8_t *x, uint32_t ncb, uint32_t ntokens, const WidePlan &plan, const char *who) {
+int wide_rows(slai_ctx *ctx, WidePass &pass, int nseg, const WideGemmSeg *segs, const uint8_t *x, uint32_t ncb, uint32_t ntokens, const WidePlan &plan, const char *who) {
     bool done[3] = {false, false, false};
     const auto kq = [](int t) { return t == T_Q4_K || t == T_Q5_K || t == T_Q6_K; };
     for (int i = 0; i < nseg; ++i) {
@@ -252,7 +260,7 @@ int wide_rows(slai_ctx *ctx, int nseg, const WideGemmSeg *segs, const uint8_t *x
             p.seg[p.nseg++] = segs[j];
             done[j] = true;
         }
-        TRY(wide_call(ctx, p, WIDE_ROWS, who));
+        TRY(wide_call(ctx, pass, p, WIDE_ROWS, who));
     }
     return SLAI_OK;
 }
@@ -453,6 +461,7 @@ struct slai_llama2 {
     int enqueue_chunk_gemm(uint32_t pos0, uint32_t n, const int *tokens_dev, bool split_f16);   // the same on the matrix cores, n <= 32
     WidePass wide;
     struct WideLayer { slai_qmat *q, *k, *v, *o, *gate, *up, *down; float hidden_up; };   // hidden_up: see wide_hidden_up
+    bool wide_one_format = true;         // q, k and v of every layer (launches of several formats share no tiles)
     std::vector<WideLayer> wide_layers;  // empty: the model has no wide pass (kernels_prompt_wide.hip)
     WideMats wide_mats;
     void wide_setup();
@@ -1190,6 +1199,7 @@ void slai_llama2::wide_setup() {
         for (const slai_qmat *m : {l.q, l.k, l.v, l.o, l.gate, l.up, l.down}) ok = ok && m && m->wbound < 255.0f;
         if (!ok) break;
         ok = l.gate->type == l.up->type && l.gate->rows_log2 == l.up->rows_log2 && !(hs == 48 && (l.o->type == T_Q4_K || l.o->type == T_Q5_K));
+        wide_one_format = wide_one_format && ok && l.q->type == l.k->type && l.q->type == l.v->type;
         layers.push_back(l);
     }
     if (ok && wide_mats.make(ctx)) wide_layers = std::move(layers);
@@ -1203,9 +1213,10 @@ int slai_llama2::enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev) 
     const uint32_t dim = config.dim, kvd = kv_dim(), hid = config.hidden_dim, hs = head_size(), ncb = (dim + 255) / 256, hcb = (hid + 255) / 256;
     if (n == 0 || n > wide::MAX_TOKENS || pos0 + n > config.seq_len) return set_error(ctx, SLAI_E_ARG, "prompt pass out of range");
     const uint32_t r_qkv[3] = {kvd, kvd, dim}, r_ffn[2] = {hid, hid};
-    const WidePlan p_qkv = wide_plan(r_qkv, 3, n, ncb, WIDE_READ), p_o = wide_plan(&dim, 1, n, ncb, WIDE_SUMMED), p_d = wide_plan(&dim, 1, n, hcb, WIDE_SUMMED);
+    const bool share = wide_may_share(ctx), share_qkv = share && wide_one_format;
+    const WidePlan p_qkv = wide_plan(r_qkv, 3, n, ncb, WIDE_READ, share_qkv), p_o = wide_plan(&dim, 1, n, ncb, WIDE_SUMMED, share), p_d = wide_plan(&dim, 1, n, hcb, WIDE_SUMMED, share);
     // the last layer's keys and values: few rows in large workgroups leave most of the device idle (Qwen2-7B shape, 900 tokens: 70 us for 1024 rows)
-    const WidePlan p_kv = p_qkv.form == WIDE_LARGE || p_qkv.form == WIDE_SMALL ? wide_plan(r_qkv, 2, n, ncb, WIDE_READ) : p_qkv;
+    const WidePlan p_kv = p_qkv.form == WIDE_LARGE || p_qkv.form == WIDE_SMALL || p_qkv.form == WIDE_SHARE ? wide_plan(r_qkv, 2, n, ncb, WIDE_READ, share_qkv) : p_qkv;
     const uint32_t ks_qkv = p_qkv.ksplit, ks_o = p_o.ksplit, ks_d = p_d.ksplit;
     const size_t rows = (size_t)n * sizeof(float);
     TRY(WidePass::grow(ctx, wide.x, rows * dim));
@@ -1227,7 +1238,7 @@ int slai_llama2::enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev) 
         SLAI_HIP_TRY(ctx, launch_norm_pairs(ctx->stream, pairs, x, parts, nparts, n * dim, (const float *)wl.attn_norm.buf->dptr, nullptr, dim, n, config.rms_norm_eps,
                                              wide_reads_sums(wm.q) || wide_reads_sums(wm.k) || wide_reads_sums(wm.v), flag));
         const WideGemmSeg qkv[3] = {wide_seg(wm.v, v, kvd, n * kvd), wide_seg(wm.k, k, kvd, n * kvd), wide_seg(wm.q, q, dim, n * dim)};
-        TRY(wide_rows(ctx, last ? 2 : 3, qkv, pairs, ncb, n, last ? p_kv : p_qkv, "llama2 qkv (prompt)"));
+        TRY(wide_rows(ctx, wide, last ? 2 : 3, qkv, pairs, ncb, n, last ? p_kv : p_qkv, "llama2 qkv (prompt)"));
         AttnLaunch a{};
         a.kcache = state.key_cache[l].buf->dptr; a.vcache = state.value_cache[l].buf->dptr; a.kv_f16 = kv_dtype == SLAI_KV_F16;
         a.n_heads = config.n_q_heads; a.kv_mul = config.n_q_heads / config.n_kv_heads; a.head_size = hs; a.kv_dim = kvd; a.seq_len = config.seq_len;
@@ -1243,16 +1254,16 @@ int slai_llama2::enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev) 
         pa.pos0 = pos0; pa.n = n; pa.out = pairs; pa.out_ncb = ncb; pa.sums = wide_reads_sums(wm.o); pa.flag = flag;
         SLAI_HIP_TRY(ctx, launch_prompt_attention(ctx->stream, pa, hs, a.kv_f16 != 0));
         const WideGemmSeg o = wide_seg(wm.o, parts, dim, n * dim);
-        TRY(wide_rows(ctx, 1, &o, pairs, ncb, n, p_o, "llama2 attn_output (prompt)"));
+        TRY(wide_rows(ctx, wide, 1, &o, pairs, ncb, n, p_o, "llama2 attn_output (prompt)"));
         SLAI_HIP_TRY(ctx, launch_norm_pairs(ctx->stream, pairs, x, parts, ks_o, n * dim, (const float *)wl.ffn_norm.buf->dptr, nullptr, dim, n, config.rms_norm_eps,
                                              wide_reads_sums(wm.gate), flag));
         WideGemmParams g;
         g.nseg = 2; g.seg[0] = wide_seg(wm.gate, nullptr, 0, 0); g.seg[1] = wide_seg(wm.up, nullptr, 0, 0);
-        g.x = pairs; g.ncb = ncb; g.ntokens = n; g.pairs_out = hidden; g.out_ncb = hcb; g.out_sums = wide_reads_sums(wm.down); g.up = wm.hidden_up; g.flag = flag; g.form = wide_plan(r_ffn, 2, n, ncb, WIDE_WHOLE).form;
-        TRY(wide_call(ctx, g, WIDE_GATED, "llama2 ffn gate/up (prompt)"));
+        g.x = pairs; g.ncb = ncb; g.ntokens = n; g.pairs_out = hidden; g.out_ncb = hcb; g.out_sums = wide_reads_sums(wm.down); g.up = wm.hidden_up; g.flag = flag; g.form = wide_plan(r_ffn, 2, n, ncb, WIDE_WHOLE, share).form;
+        TRY(wide_call(ctx, wide, g, WIDE_GATED, "llama2 ffn gate/up (prompt)"));
         WideGemmSeg d = wide_seg(wm.down, parts, dim, n * dim);
         d.down = 1.0f / wm.hidden_up;
-        TRY(wide_rows(ctx, 1, &d, hidden, hcb, n, p_d, "llama2 ffn_down (prompt)"));
+        TRY(wide_rows(ctx, wide, 1, &d, hidden, hcb, n, p_d, "llama2 ffn_down (prompt)"));
         nparts = ks_d;
     }
     return SLAI_OK;
@@ -1950,7 +1961,8 @@ int slai_gpt2::enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev) {
     const uint32_t E = params.n_embd, F = params.ff_len, hs = E / params.n_head, ncb = E / 256, fcb = F / 256;
     if (n == 0 || n > wide::MAX_TOKENS || pos0 + n > params.n_seq) return set_error(ctx, SLAI_E_ARG, "prompt pass out of range");
     const uint32_t r_qkv = 3 * E;
-    const WidePlan p_qkv = wide_plan(&r_qkv, 1, n, ncb, WIDE_READ), p_o = wide_plan(&E, 1, n, ncb, WIDE_SUMMED), p_d = wide_plan(&E, 1, n, fcb, WIDE_SUMMED);
+    const bool share = wide_may_share(ctx);
+    const WidePlan p_qkv = wide_plan(&r_qkv, 1, n, ncb, WIDE_READ, share), p_o = wide_plan(&E, 1, n, ncb, WIDE_SUMMED, share), p_d = wide_plan(&E, 1, n, fcb, WIDE_SUMMED, share);
     const uint32_t ks_qkv = p_qkv.ksplit, ks_o = p_o.ksplit, ks_d = p_d.ksplit;
     const size_t rows = (size_t)n * sizeof(float);
     TRY(WidePass::grow(ctx, wide.x, rows * E));
@@ -1971,7 +1983,7 @@ int slai_gpt2::enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev) {
         SLAI_HIP_TRY(ctx, launch_norm_pairs(ctx->stream, pairs, x, parts, nparts, n * E, (const float *)w.ln_1_g.buf->dptr, (const float *)w.ln_1_b.buf->dptr, E, n, eps,
                                              wide_reads_sums(w.c_attn_attn_w), flag));
         const WideGemmSeg sq = wide_seg(w.c_attn_attn_w, qkv, 3 * E, n * 3 * E, &w.c_attn_attn_b);
-        TRY(wide_rows(ctx, 1, &sq, pairs, ncb, n, p_qkv, "gpt2 qkv (prompt)"));
+        TRY(wide_rows(ctx, wide, 1, &sq, pairs, ncb, n, p_qkv, "gpt2 qkv (prompt)"));
         AttnLaunch a{};
         a.kcache = w.key_cache.buf->dptr; a.vcache = w.value_cache.buf->dptr; a.kv_f16 = kv_dtype == SLAI_KV_F16;
         a.n_heads = params.n_head; a.kv_mul = 1; a.head_size = hs; a.kv_dim = E; a.seq_len = params.n_seq;
@@ -1984,15 +1996,15 @@ int slai_gpt2::enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev) {
         pa.pos0 = pos0; pa.n = n; pa.out = pairs; pa.out_ncb = ncb; pa.sums = wide_reads_sums(w.c_attn_proj_w); pa.flag = flag;
         SLAI_HIP_TRY(ctx, launch_prompt_attention(ctx->stream, pa, hs, a.kv_f16 != 0));
         const WideGemmSeg so = wide_seg(w.c_attn_proj_w, parts, E, n * E, &w.c_attn_proj_b);
-        TRY(wide_rows(ctx, 1, &so, pairs, ncb, n, p_o, "gpt2 attn proj (prompt)"));
+        TRY(wide_rows(ctx, wide, 1, &so, pairs, ncb, n, p_o, "gpt2 attn proj (prompt)"));
         SLAI_HIP_TRY(ctx, launch_norm_pairs(ctx->stream, pairs, x, parts, ks_o, n * E, (const float *)w.ln_2_g.buf->dptr, (const float *)w.ln_2_b.buf->dptr, E, n, eps,
                                              wide_reads_sums(w.c_mlp_fc_w), flag));
         WideGemmParams g;
         g.nseg = 1; g.seg[0] = wide_seg(w.c_mlp_fc_w, nullptr, 0, 0, &w.c_mlp_fc_b);
-        g.x = pairs; g.ncb = ncb; g.ntokens = n; g.pairs_out = hidden; g.out_ncb = fcb; g.out_sums = wide_reads_sums(w.c_mlp_proj_w); g.flag = flag; g.form = wide_plan(&F, 1, n, ncb, WIDE_WHOLE).form;
-        TRY(wide_call(ctx, g, WIDE_GELU, "gpt2 mlp fc (prompt)"));
+        g.x = pairs; g.ncb = ncb; g.ntokens = n; g.pairs_out = hidden; g.out_ncb = fcb; g.out_sums = wide_reads_sums(w.c_mlp_proj_w); g.flag = flag; g.form = wide_plan(&F, 1, n, ncb, WIDE_WHOLE, share).form;
+        TRY(wide_call(ctx, wide, g, WIDE_GELU, "gpt2 mlp fc (prompt)"));
         const WideGemmSeg sd = wide_seg(w.c_mlp_proj_w, parts, E, n * E, &w.c_mlp_proj_b);
-        TRY(wide_rows(ctx, 1, &sd, hidden, fcb, n, p_d, "gpt2 mlp proj (prompt)"));
+        TRY(wide_rows(ctx, wide, 1, &sd, hidden, fcb, n, p_d, "gpt2 mlp proj (prompt)"));
         nparts = ks_d;
     }
     return SLAI_OK;

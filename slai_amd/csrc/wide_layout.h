@@ -31,5 +31,44 @@ WIDE_HD size_t sums_offset(uint32_t ncb, uint32_t t, uint32_t cb) { return (size
 WIDE_HD uint32_t wide_pos(uint32_t i) { return (i & 4u) | ((i & 1u) << 1) | ((i >> 1) & 1u); }
 WIDE_HD size_t activation_bytes(uint32_t ncols, uint32_t ntokens) { return (size_t)((ntokens + 31) / 32) * ((ncols + 255) / 256) * SUPER_BYTES; }
 
+// How tiles (512 rows x 64 tokens) that are no multiple of the compute units are shared out.  Workgroup i runs on die i mod 8; a die's 32
+// workgroups take an eighth of the tiles in whole rounds, and of the last, incomplete round each group of mains + 1 workgroups
+// takes `mains` tiles: one of it super-blocks 0 .. cut of each, the last one the rest of all of them.  Everybody begins a tile at super-block 0
+// or at cut, so that the workgroups of a die still read the same weights and activations at about the same time.  (Runs of equal length that begin
+// anywhere read them each for itself: gate + up of the 7B shape at 255 tokens 238 us, 124 in plain rounds.)
+constexpr uint32_t SHARE_DIES = 8, SHARE_RUNS = 32;
+struct TileShare {
+    uint32_t units, blocks, ncb, per_die, rounds, rest, mains, cut;
+    WIDE_HD TileShare(uint32_t row_units, uint32_t token_blocks, uint32_t ncb_) : units(row_units), blocks(token_blocks), ncb(ncb_) {
+        per_die = (units * blocks + SHARE_DIES - 1) / SHARE_DIES;
+        rounds = per_die / SHARE_RUNS; rest = per_die % SHARE_RUNS;
+        mains = (rest + SHARE_RUNS - rest - 1) / (SHARE_RUNS - rest);        // (0: no incomplete round)
+        cut = (ncb * mains + mains) / (mains + 1);                           // at least as long as the rests of `mains` tiles
+    }
+    struct Part { uint32_t tile, c0, c1, place; bool any; };                 // place: of a shared tile among those of its die
+    // part i of a workgroup; parts past the last are not `any`
+    WIDE_HD Part part(uint32_t die, uint32_t run, uint32_t i) const {
+        uint32_t j = i * SHARE_RUNS + run, c0 = 0, c1 = ncb;
+        if (i >= rounds) {
+            const uint32_t group = run / (mains + 1), at = run % (mains + 1);
+            i -= rounds;
+            j = rounds * SHARE_RUNS + group * mains + (at < mains ? at : i);
+            if (at < mains ? i > 0 : i >= mains) return Part{0, 0, 0, 0, false};
+            if (at < mains) c1 = cut;
+            else c0 = cut;
+        }
+        const uint32_t tile = die * per_die + j;
+        return Part{tile, c0, c1, j - rounds * SHARE_RUNS, j < per_die && tile < units * blocks && c0 < c1};
+    }
+    WIDE_HD uint32_t token_block(uint32_t tile) const { return tile % blocks; }
+    // the row unit of a tile: units 0, 8, 16 .. first (formats differ between the first units and the last, and every die is to have some of each)
+    WIDE_HD uint32_t unit(uint32_t tile) const {
+        const uint32_t p = tile / blocks, per = units / SHARE_DIES, more = units % SHARE_DIES, edge = more * (per + 1);
+        return p < edge ? p / (per + 1) + SHARE_DIES * (p % (per + 1)) : more + (p - edge) / (per ? per : 1u) + SHARE_DIES * ((p - edge) % (per ? per : 1u));
+    }
+    // super-blocks of the workgroup with the most
+    WIDE_HD uint32_t longest() const { return rounds * ncb + (rest ? cut : 0u); }
+};
+
 }  // namespace wide
 }  // namespace slai
