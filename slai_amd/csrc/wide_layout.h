@@ -32,8 +32,8 @@ WIDE_HD uint32_t wide_pos(uint32_t i) { return (i & 4u) | ((i & 1u) << 1) | ((i 
 WIDE_HD size_t activation_bytes(uint32_t ncols, uint32_t ntokens) { return (size_t)((ntokens + 31) / 32) * ((ncols + 255) / 256) * SUPER_BYTES; }
 
 // How tiles (512 rows x 64 tokens) that are no multiple of the compute units are shared out.  Workgroup i runs on die i mod 8; a die's 32
-// workgroups take an eighth of the tiles in whole rounds, and of the last, incomplete round each group of mains + 1 workgroups
-// takes `mains` tiles: one of it super-blocks 0 .. cut of each, the last one the rest of all of them.  Everybody begins a tile at super-block 0
+// workgroups take an eighth of the tiles in whole rounds, and of the `rest` tiles of the last, incomplete round one workgroup each takes super-blocks
+// 0 .. cut and every other one the rests of `mains` of them (the last such may have fewer).  Everybody begins a tile at super-block 0
 // or at cut, so that the workgroups of a die still read the same weights and activations at about the same time.  (Runs of equal length that begin
 // anywhere read them each for itself: gate + up of the 7B shape at 255 tokens 238 us, 124 in plain rounds.)
 constexpr uint32_t SHARE_DIES = 8, SHARE_RUNS = 32;
@@ -50,11 +50,12 @@ struct TileShare {
     WIDE_HD Part part(uint32_t die, uint32_t run, uint32_t i) const {
         uint32_t j = i * SHARE_RUNS + run, c0 = 0, c1 = ncb;
         if (i >= rounds) {
-            const uint32_t group = run / (mains + 1), at = run % (mains + 1);
             i -= rounds;
-            j = rounds * SHARE_RUNS + group * mains + (at < mains ? at : i);
-            if (at < mains ? i > 0 : i >= mains) return Part{0, 0, 0, 0, false};
-            if (at < mains) c1 = cut;
+            const bool main = run < rest;
+            const uint32_t at = main ? run : (run - rest) * mains + i;
+            if (main ? i > 0 : i >= mains || at >= rest) return Part{0, 0, 0, 0, false};
+            j = rounds * SHARE_RUNS + at;
+            if (main) c1 = cut;
             else c0 = cut;
         }
         const uint32_t tile = die * per_die + j;

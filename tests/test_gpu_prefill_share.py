@@ -32,6 +32,20 @@ def test_shared_tiles_llama(backend, t, hidden, n):
     g.close()
 
 
+# 43 row units at 5 token blocks are 27 tiles a die, whose rests are dealt out to five workgroups, the last of them with fewer; 24 units at 7: 21 and eleven
+@pytest.mark.parametrize("hidden,n", [(11008, 301), (6144, 449)])
+def test_last_rests(backend, hidden, n):
+    from slai_amd.runtime import Gguf, Llama2
+    t = 12
+    print("case", hidden, n, flush=True)
+    g = Gguf(gw.llama_gguf(4096, hidden, 2, 32, 32, 512, 512, t, v_type=t, out_type=t, embd_type=t, std=0.02, norm_random=True, distinct_layers=1))
+    prompt = np.random.Generator(np.random.PCG64(n)).integers(0, 512, n).astype(np.int32)
+    got, again, ref = (logits_of(Llama2(backend, g, _ffi.MODEL_LLAMA, _ffi.KV_F32), prompt, chunk) for chunk in (0, 0, 32))
+    assert np.array_equal(got, again)
+    assert rel_err(got, ref) < SELF_TOL
+    g.close()
+
+
 def test_shared_tiles_gpt2(backend):
     from slai_amd.runtime import Gguf, Gpt2
     g = Gguf(gw.gpt2_gguf(2048, 2, 32, 8192, 512, 1024, 8, std=0.02))
