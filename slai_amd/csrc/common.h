@@ -56,6 +56,7 @@ struct slai_graph {
     hipGraphExec_t exec = nullptr;
 };
 
+constexpr uint32_t HOST_WORDS = 256;
 struct slai_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -72,12 +73,13 @@ struct slai_ctx {
     size_t sampler_scratch_floats = 0;
     uint32_t *handoff_counters = nullptr;   // q/k/v + attention in one launch: one 128-byte line per head, then a timeout flag
     uint32_t handoff_heads = 0;
-    float *spread_sums = nullptr;           // row tiles that several workgroups share (gemv_spread_kernel): their sums, and a count per workgroup
+    // row tiles that several workgroups of a die share (gemv_spread_kernel, wide_share_kernel): their sums, and a count per workgroup; null: none are shared
+    float *spread_sums = nullptr;
     uint32_t *spread_counters = nullptr;
     bool fuse_qkv_attention = true;     // SLAI_FUSE_QKV_ATTN=0: always separate launches
     int prompt_split_f16 = 1;           // SLAI_PROMPT_SPLIT_F16: 0 = prompt-chunk GEMMs in fp32 MFMA, 1 = the models' on the f16 matrix cores (f16 head + remainder), 2 = slai_matmul_quant_columns too
     int *split_flag = nullptr;          // device word the kernels that write split activations set when a value is beyond f16
-    uint32_t *host_word = nullptr;      // pinned: where read_word's copy arrives
+    uint32_t *host_words = nullptr;     // pinned, HOST_WORDS of them: where read_word's copy arrives
     bool prompt_gemm = true;            // SLAI_PROMPT_GEMM=0: prompt chunks never take the matrix-core kernels
     size_t prompt_copy_bytes = (size_t)1 << 30;   // SLAI_PROMPT_COPY_MB (1024): most a model's padded copies for the wide prompt pass may take
     // tuning knobs (environment overridable, see runtime.cpp)

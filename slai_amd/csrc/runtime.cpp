@@ -67,6 +67,26 @@ static bool as_view4(const slai_view &v, View4 *out) {
 using namespace slai;
 
 // ---- context ------------------------------------------------------------------
+// Workgroups that meet in a die's L2 (hand-offs, tiles that several of them share) rely on workgroup i running on XCD i mod 8: look
+// before relying on it, and keep separate launches and a workgroup per tile on a device that places workgroups differently.  Done
+// with the context, not with the first model that asks for it: what a call computes, to the last bit, is not to depend on what else was loaded.
+// Without memory for it the context does without.
+static void spread_setup(slai_ctx *ctx) {
+    const size_t words = gemv_spread_counter_words();
+    bool placed = hipMalloc((void **)&ctx->spread_counters, std::max(words, (size_t)HOST_WORDS) * sizeof(uint32_t)) == hipSuccess &&
+                  launch_xcd_of_workgroup(ctx->stream, ctx->spread_counters, HOST_WORDS) == hipSuccess &&
+                  hipMemcpyAsync(ctx->host_words, ctx->spread_counters, HOST_WORDS * sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream) == hipSuccess &&
+                  hipStreamSynchronize(ctx->stream) == hipSuccess;
+    for (uint32_t i = 8; placed && i < HOST_WORDS; ++i) placed = ctx->host_words[i] == ctx->host_words[i % 8];
+    if (!placed) ctx->fuse_qkv_attention = false;
+    if (placed && hipMalloc((void **)&ctx->spread_sums, gemv_spread_floats() * sizeof(float)) == hipSuccess &&
+        hipMemsetAsync(ctx->spread_counters, 0, words * sizeof(uint32_t), ctx->stream) == hipSuccess) return;
+    (void)hipGetLastError();                                   // (an allocation that failed is not the next launch's error)
+    if (ctx->spread_sums) (void)hipFree(ctx->spread_sums);
+    if (ctx->spread_counters) (void)hipFree(ctx->spread_counters);
+    ctx->spread_sums = nullptr; ctx->spread_counters = nullptr;
+}
+
 SLAI_EXPORT int slai_ctx_create(int device, slai_ctx **out) {
     if (!out) return SLAI_E_ARG;
     *out = nullptr;
@@ -86,7 +106,7 @@ SLAI_EXPORT int slai_ctx_create(int device, slai_ctx **out) {
     if (hipMalloc((void **)&ctx->split_flag, sizeof(int)) != hipSuccess || hipMemsetAsync(ctx->split_flag, 0, sizeof(int), ctx->stream) != hipSuccess) {
         (void)hipStreamDestroy(ctx->stream); delete ctx; return SLAI_E_HIP;
     }
-    if (hipHostMalloc((void **)&ctx->host_word, sizeof(uint32_t), hipHostMallocDefault) != hipSuccess) {
+    if (hipHostMalloc((void **)&ctx->host_words, HOST_WORDS * sizeof(uint32_t), hipHostMallocDefault) != hipSuccess) {
         (void)hipFree(ctx->split_flag); (void)hipStreamDestroy(ctx->stream); delete ctx; return SLAI_E_HIP;
     }
     ctx->gemv_max_wgs = env_int("SLAI_GEMV_MAX_WGS", 512);
@@ -99,6 +119,7 @@ SLAI_EXPORT int slai_ctx_create(int device, slai_ctx **out) {
     ctx->small_max_pos = env_int("SLAI_SMALL_MAX_POS", -1);
     ctx->small_absent = (uint32_t)std::max(0, env_int("SLAI_SMALL_ABSENT", 0));
     ctx->resident_max_pos = (uint32_t)std::max(0, env_int("SLAI_RESIDENT_MAX_POS", 2048));
+    spread_setup(ctx);
     *out = ctx;
     return SLAI_OK;
 }
@@ -116,7 +137,7 @@ SLAI_EXPORT void slai_ctx_destroy(slai_ctx *ctx) {
     if (ctx->attn_scratch) (void)hipFree(ctx->attn_scratch);
     if (ctx->gemv_scratch) (void)hipFree(ctx->gemv_scratch);
     if (ctx->split_flag) (void)hipFree(ctx->split_flag);
-    if (ctx->host_word) (void)hipHostFree(ctx->host_word);
+    if (ctx->host_words) (void)hipHostFree(ctx->host_words);
     if (ctx->sampler_scratch) (void)hipFree(ctx->sampler_scratch);
     if (ctx->handoff_counters) (void)hipFree(ctx->handoff_counters);
     if (ctx->spread_sums) (void)hipFree(ctx->spread_sums);
@@ -466,9 +487,9 @@ bool qkv_attention_fusable(const slai_ctx *ctx, const slai_qmat *v, const slai_q
     return true;
 }
 int read_word(slai_ctx *ctx, const void *from, uint32_t *word) {
-    SLAI_HIP_TRY(ctx, hipMemcpyAsync(ctx->host_word, from, sizeof *word, hipMemcpyDeviceToHost, ctx->stream));
+    SLAI_HIP_TRY(ctx, hipMemcpyAsync(ctx->host_words, from, sizeof *word, hipMemcpyDeviceToHost, ctx->stream));
     SLAI_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-    *word = *ctx->host_word;
+    *word = *ctx->host_words;
     return SLAI_OK;
 }
 // Allocated once per context and never moved (captured graphs hold the address): models with more heads than the
@@ -478,20 +499,10 @@ int handoff_reserve(slai_ctx *ctx, uint32_t n_heads) {
     if (ctx->capturing) return set_error(ctx, SLAI_E_STATE, "hand-off counters must be reserved before graph capture");
     if (n_heads < 256) n_heads = 256;
     const size_t bytes = ((size_t)n_heads * 32 + 32) * sizeof(uint32_t);
-    SLAI_HIP_TRY(ctx, hipMalloc((void **)&ctx->handoff_counters, bytes));
-    // The hand-off relies on workgroup i running on XCD i mod 8 (workgroups with equal i mod 8 then share an L2):
-    // look before relying on it, and keep separate launches on a device that places workgroups differently.
-    uint32_t where[256];
-    SLAI_HIP_TRY(ctx, launch_xcd_of_workgroup(ctx->stream, ctx->handoff_counters, 256));
-    SLAI_HIP_TRY(ctx, hipMemcpyAsync(where, ctx->handoff_counters, sizeof where, hipMemcpyDeviceToHost, ctx->stream));
-    SLAI_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-    for (uint32_t i = 8; i < 256; ++i)
-        if (where[i] != where[i % 8]) ctx->fuse_qkv_attention = false;
-    SLAI_HIP_TRY(ctx, hipMemsetAsync(ctx->handoff_counters, 0, bytes, ctx->stream));
-    SLAI_HIP_TRY(ctx, hipMalloc((void **)&ctx->spread_counters, gemv_spread_counter_words() * sizeof(uint32_t)));
-    SLAI_HIP_TRY(ctx, hipMemsetAsync(ctx->spread_counters, 0, gemv_spread_counter_words() * sizeof(uint32_t), ctx->stream));
-    SLAI_HIP_TRY(ctx, hipMalloc((void **)&ctx->spread_sums, gemv_spread_floats() * sizeof(float)));
-    SLAI_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    uint32_t *counters = nullptr;
+    SLAI_HIP_TRY(ctx, hipMalloc((void **)&counters, bytes));
+    if (const hipError_t e = hipMemsetAsync(counters, 0, bytes, ctx->stream)) { (void)hipFree(counters); return hip_fail(ctx, e, "hand-off counters"); }
+    ctx->handoff_counters = counters;
     ctx->handoff_heads = n_heads;
     return SLAI_OK;
 }

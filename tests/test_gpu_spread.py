@@ -55,3 +55,34 @@ def test_spread_against_float64(backend, model, t, rows, cols, gated):
     assert np.linalg.norm(results[0] - ref) / np.linalg.norm(ref) < 1.5e-6
     for o in mats + [xd, wd, prep, out]:
         o.destroy()
+
+
+def test_whatever_was_loaded_before():
+    """A call's last bits are those of a context of its own also where a model was loaded in between: a prepared operator call and a GPT-2 that has no one-launch form."""
+    from slai_amd import _ffi
+    from slai_amd import gguf_writer as gw
+    from slai_amd.runtime import Backend, Gguf, GpuQuantMatrix, GpuTensor, Gpt2, Llama2, LlmContext
+    b = Backend(0)
+    rows, cols, t = 2048, 4096, 8
+    mat = GpuQuantMatrix(b, t, rows, cols, synth.normal_quantized(5, t, rows, cols, 0.02), layout=_ffi.LAYOUT_TILE64)
+    xd, wd, prep, out = GpuTensor.vector(b, synth.normal(7, cols, 1.0)), GpuTensor.vector(b, np.ones(cols, np.float32)), GpuTensor(b, cols + cols // 16), GpuTensor(b, rows)
+    c = LlmContext(b)
+    c.rms_norm_prepare(prep, xd, wd)
+    wide = Gguf(gw.gpt2_gguf(2048, 2, 32, 8192, 512, 1024, t, std=0.02))
+    prompt = np.random.Generator(np.random.PCG64(3)).integers(0, 512, 490).astype(np.int32)
+
+    def both():
+        c.matmul_quant_assign_prepared(out, mat, prep)
+        m = Gpt2(b, wide, _ffi.KV_F32)
+        m.prefill(prompt[:-1], 0, 0)
+        logits = m.forward_logits(prompt.size - 1, int(prompt[-1]))
+        m.destroy()
+        return out.read(), logits
+
+    before = both()
+    g = Gguf(gw.llama_gguf(256, 512, 1, 2, 2, 512, 64, 12, v_type=14, out_type=14, embd_type=12))
+    Llama2(b, g, _ffi.MODEL_LLAMA, _ffi.KV_F16).destroy()
+    after = both()
+    assert all(np.array_equal(x, y) for x, y in zip(before, after))
+    for o in (mat, xd, wd, prep, out, g, wide, b):
+        o.close() if hasattr(o, "close") else o.destroy()
