@@ -73,10 +73,10 @@ struct slai_ctx {
     size_t sampler_scratch_floats = 0;
     uint32_t *handoff_counters = nullptr;   // q/k/v + attention in one launch: one 128-byte line per head, then a timeout flag
     uint32_t handoff_heads = 0;
-    // row tiles that several workgroups of a die share (gemv_spread_kernel, wide_share_kernel): their sums, and a count per workgroup; null: none are shared
+    // row tiles that several workgroups of a die share (gemv_spread_kernel, wide_share_kernel): their sums, and a count per workgroup; null: none are shared (no memory, or a device that places workgroups differently)
     float *spread_sums = nullptr;
     uint32_t *spread_counters = nullptr;
-    bool fuse_qkv_attention = true;     // SLAI_FUSE_QKV_ATTN=0: always separate launches
+    bool fuse_qkv_attention = true;     // SLAI_FUSE_QKV_ATTN=0: q/k/v and attention as separate launches, attention splits merged by a launch of their own, no resident or one-die launch
     int prompt_split_f16 = 1;           // SLAI_PROMPT_SPLIT_F16: 0 = prompt-chunk GEMMs in fp32 MFMA, 1 = the models' on the f16 matrix cores (f16 head + remainder), 2 = slai_matmul_quant_columns too
     int *split_flag = nullptr;          // device word the kernels that write split activations set when a value is beyond f16
     uint32_t *host_words = nullptr;     // pinned, HOST_WORDS of them: where read_word's copy arrives

@@ -236,7 +236,7 @@ WideGemmSeg wide_seg(const slai_qmat *m, float *out, uint32_t out_stride, uint32
     return s;
 }
 // Whether workgroups may share a tile through their die's L2: their placement has been looked at (spread_setup)
-bool wide_may_share(const slai_ctx *ctx) { return ctx->fuse_qkv_attention && ctx->spread_counters; }
+bool wide_may_share(const slai_ctx *ctx) { return ctx->spread_counters != nullptr; }
 int wide_call(slai_ctx *ctx, WidePass &pass, WideGemmParams p, int mode, const char *who) {
     if (p.form == WIDE_SHARE) {
         TRY(WidePass::grow(ctx, pass.shared, wide_share_bytes()));

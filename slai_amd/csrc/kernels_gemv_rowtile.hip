@@ -555,7 +555,7 @@ hipError_t launch_gemv_rowtile(slai_ctx *ctx, GemvRowtileParams p, const GemvBat
     }
     const int NT = NW * 64;
     hipStream_t st = ctx->stream;
-    float *spread = ctx->fuse_qkv_attention && spread_pays(p, tiles) ? ctx->spread_sums : nullptr;
+    float *spread = spread_pays(p, tiles) ? ctx->spread_sums : nullptr;
     switch (tt) {
     case T_Q4_K: return dual ? go<T_Q4_K, true>(p, tiles, NT, smem, st, bt, spread, ctx->spread_counters) : go<T_Q4_K, false>(p, tiles, NT, smem, st, bt, spread, ctx->spread_counters);
     case T_Q6_K: return dual ? go<T_Q6_K, true>(p, tiles, NT, smem, st, bt, spread, ctx->spread_counters) : go<T_Q6_K, false>(p, tiles, NT, smem, st, bt, spread, ctx->spread_counters);

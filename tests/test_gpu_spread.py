@@ -86,3 +86,31 @@ def test_whatever_was_loaded_before():
     assert all(np.array_equal(x, y) for x, y in zip(before, after))
     for o in (mat, xd, wd, prep, out, g, wide, b):
         o.close() if hasattr(o, "close") else o.destroy()
+
+
+def test_the_attention_switch_leaves_them_alone(monkeypatch):
+    """SLAI_FUSE_QKV_ATTN=0 is about q/k/v and attention: what a comparison by it measures is not also the sharing of tiles."""
+    from slai_amd import _ffi
+    from slai_amd import gguf_writer as gw
+    from slai_amd.runtime import Backend, Gguf, GpuQuantMatrix, GpuTensor, Gpt2, LlmContext
+    rows, cols, t = 2048, 4096, 8
+    wide = Gguf(gw.gpt2_gguf(2048, 2, 32, 8192, 512, 1024, t, std=0.02))
+    prompt = np.random.Generator(np.random.PCG64(3)).integers(0, 512, 490).astype(np.int32)
+    results = []
+    for switch in ("1", "0"):
+        monkeypatch.setenv("SLAI_FUSE_QKV_ATTN", switch)
+        b = Backend(0)
+        mat = GpuQuantMatrix(b, t, rows, cols, synth.normal_quantized(5, t, rows, cols, 0.02), layout=_ffi.LAYOUT_TILE64)
+        xd, wd, prep, out = GpuTensor.vector(b, synth.normal(7, cols, 1.0)), GpuTensor.vector(b, np.ones(cols, np.float32)), GpuTensor(b, cols + cols // 16), GpuTensor(b, rows)
+        c = LlmContext(b)
+        c.rms_norm_prepare(prep, xd, wd)
+        c.matmul_quant_assign_prepared(out, mat, prep)
+        m = Gpt2(b, wide, _ffi.KV_F32)
+        m.prefill(prompt[:-1], 0, 0)
+        results.append((out.read(), m.forward_logits(prompt.size - 1, int(prompt[-1]))))
+        for o in (mat, xd, wd, prep, out, m):
+            o.destroy()
+        b.close()
+    wide.close()
+    assert np.array_equal(results[0][0], results[1][0])
+    assert np.array_equal(results[0][1], results[1][1])
