@@ -289,7 +289,7 @@ struct WideGemmParams {
     int nseg = 1;
     const uint8_t *x = nullptr;
     uint32_t ncb = 0, ntokens = 0;
-    int form = 0;                 // wide_plan
+    int form = 0;                 // wide_plan (wide_plan.h)
     uint32_t ksplit = 1;          // WIDE_ROWS: the columns in ranges of whole super-blocks, each its own workgroups and result
     uint8_t *pairs_out = nullptr; // WIDE_GATED, WIDE_GELU: super-blocks per token out_ncb
     uint32_t out_ncb = 0;
@@ -302,12 +302,6 @@ struct WideGemmParams {
 };
 bool wide_gemm_supports(const slai_qmat *m);
 bool wide_reads_sums(const slai_qmat *m);   // whether its input needs the sums of 32 (offsets per sub-block)
-// Form and number of column ranges for nseg matrices over one input.  WIDE_WHOLE: no ranges; WIDE_SUMMED: partial results are summed by the next norm;
-// WIDE_READ: by each of their readers
-enum { WIDE_LARGE = 0, WIDE_SMALL, WIDE_SLIM4, WIDE_SLIM8, WIDE_SHARE };
-enum WideSplits { WIDE_WHOLE, WIDE_SUMMED, WIDE_READ };
-struct WidePlan { int form; uint32_t ksplit; };
-WidePlan wide_plan(const uint32_t *nrows, int nseg, uint32_t ntokens, uint32_t ncb, WideSplits splits, bool may_share);
 size_t wide_share_bytes();                   // of WideGemmParams::shared
 size_t wide_share_counter_words();           // of WideGemmParams::counters
 hipError_t launch_wide_gemm(hipStream_t st, WideGemmParams p, int mode);

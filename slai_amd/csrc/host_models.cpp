@@ -10,6 +10,7 @@
 #include "quant_tiled.h"
 #include "resident_plan.h"
 #include "wide_layout.h"
+#include "wide_plan.h"
 
 #include <algorithm>
 #include <array>
