@@ -1213,11 +1213,11 @@ void slai_llama2::wide_setup() {
 int slai_llama2::enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev) {
     const uint32_t dim = config.dim, kvd = kv_dim(), hid = config.hidden_dim, hs = head_size(), ncb = (dim + 255) / 256, hcb = (hid + 255) / 256;
     if (n == 0 || n > wide::MAX_TOKENS || pos0 + n > config.seq_len) return set_error(ctx, SLAI_E_ARG, "prompt pass out of range");
-    const uint32_t r_qkv[3] = {kvd, kvd, dim}, r_ffn[2] = {hid, hid};
+    const uint32_t r_qkv[3] = {kvd, kvd, dim};
     const bool share = wide_may_share(ctx), share_qkv = share && wide_one_format;
-    const WidePlan p_qkv = wide_plan(r_qkv, 3, n, ncb, WIDE_READ, share_qkv), p_o = wide_plan(&dim, 1, n, ncb, WIDE_SUMMED, share), p_d = wide_plan(&dim, 1, n, hcb, WIDE_SUMMED, share);
+    const WidePlan p_qkv = wide_plan(r_qkv, 3, n, ncb, WIDE_READ, false, share_qkv), p_o = wide_plan(&dim, 1, n, ncb, WIDE_SUMMED, false, share), p_d = wide_plan(&dim, 1, n, hcb, WIDE_SUMMED, false, share);
     // the last layer's keys and values: few rows in large workgroups leave most of the device idle (Qwen2-7B shape, 900 tokens: 70 us for 1024 rows)
-    const WidePlan p_kv = p_qkv.form == WIDE_LARGE || p_qkv.form == WIDE_SMALL || p_qkv.form == WIDE_SHARE ? wide_plan(r_qkv, 2, n, ncb, WIDE_READ, share_qkv) : p_qkv;
+    const WidePlan p_kv = p_qkv.form == WIDE_LARGE || p_qkv.form == WIDE_SMALL || p_qkv.form == WIDE_SHARE ? wide_plan(r_qkv, 2, n, ncb, WIDE_READ, false, share_qkv) : p_qkv;
     const uint32_t ks_qkv = p_qkv.ksplit, ks_o = p_o.ksplit, ks_d = p_d.ksplit;
     const size_t rows = (size_t)n * sizeof(float);
     TRY(WidePass::grow(ctx, wide.x, rows * dim));
@@ -1260,7 +1260,7 @@ int slai_llama2::enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev) 
                                              wide_reads_sums(wm.gate), flag));
         WideGemmParams g;
         g.nseg = 2; g.seg[0] = wide_seg(wm.gate, nullptr, 0, 0); g.seg[1] = wide_seg(wm.up, nullptr, 0, 0);
-        g.x = pairs; g.ncb = ncb; g.ntokens = n; g.pairs_out = hidden; g.out_ncb = hcb; g.out_sums = wide_reads_sums(wm.down); g.up = wm.hidden_up; g.flag = flag; g.form = wide_plan(r_ffn, 2, n, ncb, WIDE_WHOLE, share).form;
+        g.x = pairs; g.ncb = ncb; g.ntokens = n; g.pairs_out = hidden; g.out_ncb = hcb; g.out_sums = wide_reads_sums(wm.down); g.up = wm.hidden_up; g.flag = flag; g.form = wide_plan(&hid, 1, n, ncb, WIDE_WHOLE, true, share).form;
         TRY(wide_call(ctx, wide, g, WIDE_GATED, "llama2 ffn gate/up (prompt)"));
         WideGemmSeg d = wide_seg(wm.down, parts, dim, n * dim);
         d.down = 1.0f / wm.hidden_up;
@@ -1963,7 +1963,7 @@ int slai_gpt2::enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev) {
     if (n == 0 || n > wide::MAX_TOKENS || pos0 + n > params.n_seq) return set_error(ctx, SLAI_E_ARG, "prompt pass out of range");
     const uint32_t r_qkv = 3 * E;
     const bool share = wide_may_share(ctx);
-    const WidePlan p_qkv = wide_plan(&r_qkv, 1, n, ncb, WIDE_READ, share), p_o = wide_plan(&E, 1, n, ncb, WIDE_SUMMED, share), p_d = wide_plan(&E, 1, n, fcb, WIDE_SUMMED, share);
+    const WidePlan p_qkv = wide_plan(&r_qkv, 1, n, ncb, WIDE_READ, false, share), p_o = wide_plan(&E, 1, n, ncb, WIDE_SUMMED, false, share), p_d = wide_plan(&E, 1, n, fcb, WIDE_SUMMED, false, share);
     const uint32_t ks_qkv = p_qkv.ksplit, ks_o = p_o.ksplit, ks_d = p_d.ksplit;
     const size_t rows = (size_t)n * sizeof(float);
     TRY(WidePass::grow(ctx, wide.x, rows * E));
@@ -2002,7 +2002,7 @@ int slai_gpt2::enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev) {
                                              wide_reads_sums(w.c_mlp_fc_w), flag));
         WideGemmParams g;
         g.nseg = 1; g.seg[0] = wide_seg(w.c_mlp_fc_w, nullptr, 0, 0, &w.c_mlp_fc_b);
-        g.x = pairs; g.ncb = ncb; g.ntokens = n; g.pairs_out = hidden; g.out_ncb = fcb; g.out_sums = wide_reads_sums(w.c_mlp_proj_w); g.flag = flag; g.form = wide_plan(&F, 1, n, ncb, WIDE_WHOLE, share).form;
+        g.x = pairs; g.ncb = ncb; g.ntokens = n; g.pairs_out = hidden; g.out_ncb = fcb; g.out_sums = wide_reads_sums(w.c_mlp_proj_w); g.flag = flag; g.form = wide_plan(&F, 1, n, ncb, WIDE_WHOLE, false, share).form;
         TRY(wide_call(ctx, wide, g, WIDE_GELU, "gpt2 mlp fc (prompt)"));
         const WideGemmSeg sd = wide_seg(w.c_mlp_proj_w, parts, E, n * E, &w.c_mlp_proj_b);
         TRY(wide_rows(ctx, wide, 1, &sd, hidden, fcb, n, p_d, "gpt2 mlp proj (prompt)"));

@@ -9,11 +9,16 @@
 
 namespace slai {
 
-// Form and number of column ranges for nseg matrices over one input.  WIDE_WHOLE: no ranges; WIDE_SUMMED: partial results are summed by the next norm;
+// Form and number of column ranges for nseg matrices over one input (a gated pair is one, of the rows of either).  WIDE_WHOLE: no ranges; WIDE_SUMMED: partial results are summed by the next norm;
 // WIDE_READ: by each of their readers
 enum { WIDE_LARGE = 0, WIDE_SMALL, WIDE_SLIM4, WIDE_SLIM8, WIDE_SHARE };
 enum WideSplits { WIDE_WHOLE, WIDE_SUMMED, WIDE_READ };
 struct WidePlan { int form; uint32_t ksplit; };
+
+// Rows of a matrix that a workgroup of a form has (gated: of the gate matrix and of the up matrix each), and row units of a matrix: what a launch is made of and
+// what the choice has to count
+inline uint32_t wide_unit_rows(int form, bool gated) { return (gated ? 32u : 64u) * (form == WIDE_SLIM4 || form == WIDE_SLIM8 ? 1u : form == WIDE_SMALL ? 4u : 8u); }
+inline uint32_t wide_row_units(uint32_t nrows, int form, bool gated) { return (nrows + wide_unit_rows(form, gated) - 1) / wide_unit_rows(form, gated); }
 
 // The forms of a launch: large, 512 rows x 64 tokens (one workgroup fills a compute unit); small, 256 rows x 32 tokens; and slim, 64 rows x
 // 32 tokens with the super-blocks shared out among four waves, or eight where that fills the device no more than once.  The columns are
@@ -38,9 +43,12 @@ struct WidePlan { int form; uint32_t ksplit; };
 // sums partial results (the norm) takes 1 us more and 0.4 us per million of them, what reads each several times (bias + RoPE + cache rows, attention) 2 us per million.
 // Over twelve shapes and formats and 64 to 1024 tokens in steps of 64 the picks cost 0.3 % more than the better form of every launch would (3.2 % without the
 // many tokens, the dies and the readers in the estimate: 7B shape, Q8_0, two layers, 832 tokens 1411 us for 1193).
-inline WidePlan wide_plan(const uint32_t *nrows, int nseg, uint32_t ntokens, uint32_t ncb, WideSplits splits, bool may_share) {
+inline WidePlan wide_plan(const uint32_t *nrows, int nseg, uint32_t ntokens, uint32_t ncb, WideSplits splits, bool gated, bool may_share) {
     uint32_t r8 = 0, r4 = 0, r1 = 0, rows = 0;
-    for (int i = 0; i < nseg; ++i) { r8 += (nrows[i] + 511) / 512; r4 += (nrows[i] + 255) / 256; r1 += (nrows[i] + 63) / 64; rows += nrows[i]; }
+    for (int i = 0; i < nseg; ++i) {
+        r8 += wide_row_units(nrows[i], WIDE_LARGE, gated); r4 += wide_row_units(nrows[i], WIDE_SMALL, gated); r1 += wide_row_units(nrows[i], WIDE_SLIM4, gated);
+        rows += nrows[i];
+    }
     const uint32_t large = r8 * ((ntokens + 63) / 64), small = r4 * ((ntokens + 31) / 32), slim = r1 * ((ntokens + 31) / 32);
     const auto ranges = [&](uint32_t units, uint32_t most) { return splits != WIDE_WHOLE ? std::max(1u, std::min(std::min(units, most), 8u)) : 1u; };
     const uint32_t ks_large = ranges(256u / large, ncb / 2), ks_small = ranges(512u / small, ncb), ks_fill = ranges(256u / slim, (ncb + 3) / 4);
