@@ -352,6 +352,13 @@ int slai_llama2_prefill(slai_llama2 *m, const int32_t *tokens, uint32_t n_tokens
                         float *elapsed_ms);
 int slai_llama2_prefill_supported(const slai_llama2 *m);
 uint32_t slai_llama2_prefill_fp32_repeats(const slai_llama2 *m);
+/* What a pass of n_tokens prompt tokens (at most 1024) in f16 pairs takes for a step of its layers -- 0: q/k/v, 1: attention output, 2: gate / up (GPT-2: the MLP's
+ * first matrix), 3: the projection behind it.  -1: the model has no such pass, or no such step. */
+#define SLAI_PROMPT_LARGE 0  /* workgroups of 512 rows x 64 tokens */
+#define SLAI_PROMPT_SMALL 1  /* 256 rows x 32 tokens */
+#define SLAI_PROMPT_SLIM 2   /* 64 rows x 32 tokens, the columns shared out among waves */
+#define SLAI_PROMPT_SHARED 3 /* 512 rows x 64 tokens, the tiles of the last round each shared by two workgroups */
+int slai_llama2_prompt_form(const slai_llama2 *m, uint32_t n_tokens, int step);
 /* Which form the per-token loop of this model takes: 0 = one launch per step of `Llama2::launch` (transformer.rs:316-381;
  * four to five per layer; or a small model's layers in one launch: slai_llama2_decode_form_at), 1 = the whole layer stack and the output matrix in one resident launch per token (widths of
  * 1024 .. 4096 in steps of 1024, as many cache heads as query heads of size 128, Q4_K / Q5_K / Q6_K mixes, gate / up in
@@ -407,6 +414,7 @@ int slai_gpt2_prefill(slai_gpt2 *m, const int32_t *tokens, uint32_t n_tokens, ui
                       float *elapsed_ms);
 int slai_gpt2_prefill_supported(const slai_gpt2 *m);
 uint32_t slai_gpt2_prefill_fp32_repeats(const slai_gpt2 *m);
+int slai_gpt2_prompt_form(const slai_gpt2 *m, uint32_t n_tokens, int step);
 
 /* ---- Tokenizers (host only) ---------------------------------------------------
  * `AnyTokenizer` (crates/slai-chat/src/llm.rs:100-164) over `LlamaTokenizer`

@@ -143,6 +143,8 @@ SIGNATURES = {
     "slai_llama2_decode_form": (i32, [vp]),
     "slai_llama2_decode_form_at": (i32, [vp, u32]),
     "slai_gpt2_decode_form_at": (i32, [vp, u32]),
+    "slai_llama2_prompt_form": (i32, [vp, u32, i32]),
+    "slai_gpt2_prompt_form": (i32, [vp, u32, i32]),
     "slai_llama2_trace_token": (i32, [vp, u32, u32, vp, sz, P(u32), P(u32)]),
     "slai_llama2_time_steps": (i32, [vp, u32, u32, u32, vp, sz, vp, vp, vp, u32, P(u32)]),
     "slai_llama2_destroy": (None, [vp]),

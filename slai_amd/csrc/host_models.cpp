@@ -238,6 +238,15 @@ WideGemmSeg wide_seg(const slai_qmat *m, float *out, uint32_t out_stride, uint32
 }
 // Whether workgroups may share a tile through their die's L2: their placement has been looked at (spread_setup)
 bool wide_may_share(const slai_ctx *ctx) { return ctx->spread_counters != nullptr; }
+// The forms of a pass's launches (kv: the last layer's keys and values)
+struct WidePlans { WidePlan qkv, kv, o, ffn, down; };
+// the step as slai_llama2_prompt_form counts it, and its form
+int prompt_form(const WidePlans &p, int step) {
+    const WidePlan *const plans[4] = {&p.qkv, &p.o, &p.ffn, &p.down};
+    if (step < 0 || step > 3) return -1;
+    const int form = plans[step]->form;
+    return form == WIDE_SHARE ? SLAI_PROMPT_SHARED : form == WIDE_LARGE ? SLAI_PROMPT_LARGE : form == WIDE_SMALL ? SLAI_PROMPT_SMALL : SLAI_PROMPT_SLIM;
+}
 int wide_call(slai_ctx *ctx, WidePass &pass, WideGemmParams p, int mode, const char *who) {
     if (p.form == WIDE_SHARE) {
         TRY(WidePass::grow(ctx, pass.shared, wide_share_bytes()));
@@ -466,6 +475,7 @@ struct slai_llama2 {
     std::vector<WideLayer> wide_layers;  // empty: the model has no wide pass (kernels_prompt_wide.hip)
     WideMats wide_mats;
     void wide_setup();
+    WidePlans wide_plans(uint32_t n) const;
     int enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev);   // n <= wide::MAX_TOKENS, activations as f16 pairs
     // q / k / v given as nparts partial sums, 32 rows apart; out_quads: the result goes to xn, quad-major, instead of xb
     int chunk_attention(uint32_t l, uint32_t pos0, uint32_t n, uint32_t nparts = 1, bool out_quads = false, int *split_flag = nullptr);
@@ -1207,25 +1217,34 @@ void slai_llama2::wide_setup() {
     else wide_mats.drop();
 }
 
+WidePlans slai_llama2::wide_plans(uint32_t n) const {
+    const uint32_t dim = config.dim, kvd = kv_dim(), hid = config.hidden_dim, ncb = (dim + 255) / 256, hcb = (hid + 255) / 256, r_qkv[3] = {kvd, kvd, dim};
+    const bool share = wide_may_share(ctx), share_qkv = share && wide_one_format;
+    WidePlans p;
+    p.qkv = wide_plan(r_qkv, 3, n, ncb, WIDE_READ, false, share_qkv);
+    // the last layer's keys and values: few rows in large workgroups leave most of the device idle (Qwen2-7B shape, 900 tokens: 70 us for 1024 rows)
+    p.kv = p.qkv.form == WIDE_LARGE || p.qkv.form == WIDE_SMALL || p.qkv.form == WIDE_SHARE ? wide_plan(r_qkv, 2, n, ncb, WIDE_READ, false, share_qkv) : p.qkv;
+    p.o = wide_plan(&dim, 1, n, ncb, WIDE_SUMMED, false, share);
+    p.ffn = wide_plan(&hid, 1, n, ncb, WIDE_WHOLE, true, share);
+    p.down = wide_plan(&dim, 1, n, hcb, WIDE_SUMMED, false, share);
+    return p;
+}
+
 // The layer loop (transformer.rs:316-381) for up to 1024 tokens at once: per layer the residual brought up to date and its
 // norm, q/k/v, bias + RoPE + cache write, attention, output projection, norm, gate/up + SiLU, down projection: eight
 // launches.  The last layer ends with its cache rows: nothing after them reaches the caches, and no logits are computed.
 int slai_llama2::enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev) {
     const uint32_t dim = config.dim, kvd = kv_dim(), hid = config.hidden_dim, hs = head_size(), ncb = (dim + 255) / 256, hcb = (hid + 255) / 256;
     if (n == 0 || n > wide::MAX_TOKENS || pos0 + n > config.seq_len) return set_error(ctx, SLAI_E_ARG, "prompt pass out of range");
-    const uint32_t r_qkv[3] = {kvd, kvd, dim};
-    const bool share = wide_may_share(ctx), share_qkv = share && wide_one_format;
-    const WidePlan p_qkv = wide_plan(r_qkv, 3, n, ncb, WIDE_READ, false, share_qkv), p_o = wide_plan(&dim, 1, n, ncb, WIDE_SUMMED, false, share), p_d = wide_plan(&dim, 1, n, hcb, WIDE_SUMMED, false, share);
-    // the last layer's keys and values: few rows in large workgroups leave most of the device idle (Qwen2-7B shape, 900 tokens: 70 us for 1024 rows)
-    const WidePlan p_kv = p_qkv.form == WIDE_LARGE || p_qkv.form == WIDE_SMALL || p_qkv.form == WIDE_SHARE ? wide_plan(r_qkv, 2, n, ncb, WIDE_READ, false, share_qkv) : p_qkv;
-    const uint32_t ks_qkv = p_qkv.ksplit, ks_o = p_o.ksplit, ks_d = p_d.ksplit;
+    const WidePlans plan = wide_plans(n);
+    const uint32_t ks_qkv = plan.qkv.ksplit, ks_kv = plan.kv.ksplit, ks_o = plan.o.ksplit, ks_d = plan.down.ksplit;
     const size_t rows = (size_t)n * sizeof(float);
     TRY(WidePass::grow(ctx, wide.x, rows * dim));
     TRY(WidePass::grow(ctx, wide.pairs, wide::activation_bytes(dim, n)));
     TRY(WidePass::grow(ctx, wide.hidden, wide::activation_bytes(hid, n)));
     TRY(WidePass::grow(ctx, wide.q, rows * dim * ks_qkv));
-    TRY(WidePass::grow(ctx, wide.k, rows * kvd * std::max(ks_qkv, p_kv.ksplit)));
-    TRY(WidePass::grow(ctx, wide.v, rows * kvd * std::max(ks_qkv, p_kv.ksplit)));
+    TRY(WidePass::grow(ctx, wide.k, rows * kvd * std::max(ks_qkv, ks_kv)));
+    TRY(WidePass::grow(ctx, wide.v, rows * kvd * std::max(ks_qkv, ks_kv)));
     TRY(WidePass::grow(ctx, wide.parts, rows * dim * std::max(ks_o, ks_d)));
     float *x = (float *)wide.x->dptr, *q = (float *)wide.q->dptr, *k = (float *)wide.k->dptr, *v = (float *)wide.v->dptr, *parts = (float *)wide.parts->dptr;
     uint8_t *pairs = (uint8_t *)wide.pairs->dptr, *hidden = (uint8_t *)wide.hidden->dptr;
@@ -1239,7 +1258,7 @@ int slai_llama2::enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev) 
         SLAI_HIP_TRY(ctx, launch_norm_pairs(ctx->stream, pairs, x, parts, nparts, n * dim, (const float *)wl.attn_norm.buf->dptr, nullptr, dim, n, config.rms_norm_eps,
                                              wide_reads_sums(wm.q) || wide_reads_sums(wm.k) || wide_reads_sums(wm.v), flag));
         const WideGemmSeg qkv[3] = {wide_seg(wm.v, v, kvd, n * kvd), wide_seg(wm.k, k, kvd, n * kvd), wide_seg(wm.q, q, dim, n * dim)};
-        TRY(wide_rows(ctx, wide, last ? 2 : 3, qkv, pairs, ncb, n, last ? p_kv : p_qkv, "llama2 qkv (prompt)"));
+        TRY(wide_rows(ctx, wide, last ? 2 : 3, qkv, pairs, ncb, n, last ? plan.kv : plan.qkv, "llama2 qkv (prompt)"));
         AttnLaunch a{};
         a.kcache = state.key_cache[l].buf->dptr; a.vcache = state.value_cache[l].buf->dptr; a.kv_f16 = kv_dtype == SLAI_KV_F16;
         a.n_heads = config.n_q_heads; a.kv_mul = config.n_q_heads / config.n_kv_heads; a.head_size = hs; a.kv_dim = kvd; a.seq_len = config.seq_len;
@@ -1248,23 +1267,23 @@ int slai_llama2::enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev) 
         a.kbias = wl.attn_k_bias.buf ? (const float *)wl.attn_k_bias.buf->dptr : nullptr;
         a.vbias = wl.attn_v_bias.buf ? (const float *)wl.attn_v_bias.buf->dptr : nullptr;
         a.rope_variant = rope_variant(); a.rope_base = config.rope_base_freq; a.rope_theta = (const float *)state.rope_theta.buf->dptr;
-        SLAI_HIP_TRY(ctx, launch_rope_store_batch(ctx->stream, a, last ? nullptr : q, k, v, n, dim, kvd, last ? p_kv.ksplit : ks_qkv, n * dim, n * kvd));
+        SLAI_HIP_TRY(ctx, launch_rope_store_batch(ctx->stream, a, last ? nullptr : q, k, v, n, dim, kvd, last ? ks_kv : ks_qkv, n * dim, n * kvd));
         if (last) break;
         PromptAttention pa;
         pa.q = q; pa.q_stride = dim; pa.kcache = a.kcache; pa.vcache = a.vcache; pa.kv_dim = kvd; pa.n_heads = a.n_heads; pa.kv_mul = a.kv_mul;
         pa.pos0 = pos0; pa.n = n; pa.out = pairs; pa.out_ncb = ncb; pa.sums = wide_reads_sums(wm.o); pa.flag = flag;
         SLAI_HIP_TRY(ctx, launch_prompt_attention(ctx->stream, pa, hs, a.kv_f16 != 0));
         const WideGemmSeg o = wide_seg(wm.o, parts, dim, n * dim);
-        TRY(wide_rows(ctx, wide, 1, &o, pairs, ncb, n, p_o, "llama2 attn_output (prompt)"));
+        TRY(wide_rows(ctx, wide, 1, &o, pairs, ncb, n, plan.o, "llama2 attn_output (prompt)"));
         SLAI_HIP_TRY(ctx, launch_norm_pairs(ctx->stream, pairs, x, parts, ks_o, n * dim, (const float *)wl.ffn_norm.buf->dptr, nullptr, dim, n, config.rms_norm_eps,
                                              wide_reads_sums(wm.gate), flag));
         WideGemmParams g;
         g.nseg = 2; g.seg[0] = wide_seg(wm.gate, nullptr, 0, 0); g.seg[1] = wide_seg(wm.up, nullptr, 0, 0);
-        g.x = pairs; g.ncb = ncb; g.ntokens = n; g.pairs_out = hidden; g.out_ncb = hcb; g.out_sums = wide_reads_sums(wm.down); g.up = wm.hidden_up; g.flag = flag; g.form = wide_plan(&hid, 1, n, ncb, WIDE_WHOLE, true, share).form;
+        g.x = pairs; g.ncb = ncb; g.ntokens = n; g.pairs_out = hidden; g.out_ncb = hcb; g.out_sums = wide_reads_sums(wm.down); g.up = wm.hidden_up; g.flag = flag; g.form = plan.ffn.form;
         TRY(wide_call(ctx, wide, g, WIDE_GATED, "llama2 ffn gate/up (prompt)"));
         WideGemmSeg d = wide_seg(wm.down, parts, dim, n * dim);
         d.down = 1.0f / wm.hidden_up;
-        TRY(wide_rows(ctx, wide, 1, &d, hidden, hcb, n, p_d, "llama2 ffn_down (prompt)"));
+        TRY(wide_rows(ctx, wide, 1, &d, hidden, hcb, n, plan.down, "llama2 ffn_down (prompt)"));
         nparts = ks_d;
     }
     return SLAI_OK;
@@ -1315,6 +1334,10 @@ SLAI_EXPORT int slai_llama2_decode_form(const slai_llama2 *m) { return m && m->p
 // the forms of form_at as the header counts them (the resident launch for far positions is one of the two kernels of form 1)
 static int form_for_callers(int form) { return form == 3 ? 2 : form == 0 ? 0 : 1; }
 SLAI_EXPORT int slai_llama2_decode_form_at(const slai_llama2 *m, uint32_t pos) { return m ? form_for_callers(m->form_at(pos)) : 0; }
+
+SLAI_EXPORT int slai_llama2_prompt_form(const slai_llama2 *m, uint32_t n_tokens, int step) {
+    return m && !m->wide_layers.empty() && n_tokens && n_tokens <= wide::MAX_TOKENS ? prompt_form(m->wide_plans(n_tokens), step) : -1;
+}
 
 // One token at (pos, token) through the resident launch with its time stamps switched on: per workgroup 16 stamps per
 // layer (four per phase: entered, input staged, multiplied, reduced) and 8 for the output matrix, in ticks of the
@@ -1679,6 +1702,7 @@ struct slai_gpt2 {
     int enqueue_chunk_gemm(uint32_t pos0, uint32_t n, const int *tokens_dev, bool split_f16);
     WidePass wide;                                             // see slai_llama2::enqueue_wide
     bool wide_supported() const;
+    WidePlans wide_plans(uint32_t n) const;
     int enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev);
 };
 
@@ -1957,14 +1981,23 @@ bool slai_gpt2::wide_supported() const {
     return chunk_split_ok();
 }
 
+WidePlans slai_gpt2::wide_plans(uint32_t n) const {
+    const uint32_t E = params.n_embd, F = params.ff_len, r_qkv = 3 * E;
+    const bool share = wide_may_share(ctx);
+    WidePlans p;
+    p.qkv = p.kv = wide_plan(&r_qkv, 1, n, E / 256, WIDE_READ, false, share);
+    p.o = wide_plan(&E, 1, n, E / 256, WIDE_SUMMED, false, share);
+    p.ffn = wide_plan(&F, 1, n, E / 256, WIDE_WHOLE, false, share);
+    p.down = wide_plan(&E, 1, n, F / 256, WIDE_SUMMED, false, share);
+    return p;
+}
+
 // gpt2/cpu.rs:225-383 for up to 1024 tokens at once (see slai_llama2::enqueue_wide)
 int slai_gpt2::enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev) {
     const uint32_t E = params.n_embd, F = params.ff_len, hs = E / params.n_head, ncb = E / 256, fcb = F / 256;
     if (n == 0 || n > wide::MAX_TOKENS || pos0 + n > params.n_seq) return set_error(ctx, SLAI_E_ARG, "prompt pass out of range");
-    const uint32_t r_qkv = 3 * E;
-    const bool share = wide_may_share(ctx);
-    const WidePlan p_qkv = wide_plan(&r_qkv, 1, n, ncb, WIDE_READ, false, share), p_o = wide_plan(&E, 1, n, ncb, WIDE_SUMMED, false, share), p_d = wide_plan(&E, 1, n, fcb, WIDE_SUMMED, false, share);
-    const uint32_t ks_qkv = p_qkv.ksplit, ks_o = p_o.ksplit, ks_d = p_d.ksplit;
+    const WidePlans plan = wide_plans(n);
+    const uint32_t ks_qkv = plan.qkv.ksplit, ks_o = plan.o.ksplit, ks_d = plan.down.ksplit;
     const size_t rows = (size_t)n * sizeof(float);
     TRY(WidePass::grow(ctx, wide.x, rows * E));
     TRY(WidePass::grow(ctx, wide.pairs, wide::activation_bytes(E, n)));
@@ -1984,7 +2017,7 @@ int slai_gpt2::enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev) {
         SLAI_HIP_TRY(ctx, launch_norm_pairs(ctx->stream, pairs, x, parts, nparts, n * E, (const float *)w.ln_1_g.buf->dptr, (const float *)w.ln_1_b.buf->dptr, E, n, eps,
                                              wide_reads_sums(w.c_attn_attn_w), flag));
         const WideGemmSeg sq = wide_seg(w.c_attn_attn_w, qkv, 3 * E, n * 3 * E, &w.c_attn_attn_b);
-        TRY(wide_rows(ctx, wide, 1, &sq, pairs, ncb, n, p_qkv, "gpt2 qkv (prompt)"));
+        TRY(wide_rows(ctx, wide, 1, &sq, pairs, ncb, n, plan.qkv, "gpt2 qkv (prompt)"));
         AttnLaunch a{};
         a.kcache = w.key_cache.buf->dptr; a.vcache = w.value_cache.buf->dptr; a.kv_f16 = kv_dtype == SLAI_KV_F16;
         a.n_heads = params.n_head; a.kv_mul = 1; a.head_size = hs; a.kv_dim = E; a.seq_len = params.n_seq;
@@ -1997,15 +2030,15 @@ int slai_gpt2::enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev) {
         pa.pos0 = pos0; pa.n = n; pa.out = pairs; pa.out_ncb = ncb; pa.sums = wide_reads_sums(w.c_attn_proj_w); pa.flag = flag;
         SLAI_HIP_TRY(ctx, launch_prompt_attention(ctx->stream, pa, hs, a.kv_f16 != 0));
         const WideGemmSeg so = wide_seg(w.c_attn_proj_w, parts, E, n * E, &w.c_attn_proj_b);
-        TRY(wide_rows(ctx, wide, 1, &so, pairs, ncb, n, p_o, "gpt2 attn proj (prompt)"));
+        TRY(wide_rows(ctx, wide, 1, &so, pairs, ncb, n, plan.o, "gpt2 attn proj (prompt)"));
         SLAI_HIP_TRY(ctx, launch_norm_pairs(ctx->stream, pairs, x, parts, ks_o, n * E, (const float *)w.ln_2_g.buf->dptr, (const float *)w.ln_2_b.buf->dptr, E, n, eps,
                                              wide_reads_sums(w.c_mlp_fc_w), flag));
         WideGemmParams g;
         g.nseg = 1; g.seg[0] = wide_seg(w.c_mlp_fc_w, nullptr, 0, 0, &w.c_mlp_fc_b);
-        g.x = pairs; g.ncb = ncb; g.ntokens = n; g.pairs_out = hidden; g.out_ncb = fcb; g.out_sums = wide_reads_sums(w.c_mlp_proj_w); g.flag = flag; g.form = wide_plan(&F, 1, n, ncb, WIDE_WHOLE, false, share).form;
+        g.x = pairs; g.ncb = ncb; g.ntokens = n; g.pairs_out = hidden; g.out_ncb = fcb; g.out_sums = wide_reads_sums(w.c_mlp_proj_w); g.flag = flag; g.form = plan.ffn.form;
         TRY(wide_call(ctx, wide, g, WIDE_GELU, "gpt2 mlp fc (prompt)"));
         const WideGemmSeg sd = wide_seg(w.c_mlp_proj_w, parts, E, n * E, &w.c_mlp_proj_b);
-        TRY(wide_rows(ctx, wide, 1, &sd, hidden, fcb, n, p_d, "gpt2 mlp proj (prompt)"));
+        TRY(wide_rows(ctx, wide, 1, &sd, hidden, fcb, n, plan.down, "gpt2 mlp proj (prompt)"));
         nparts = ks_d;
     }
     return SLAI_OK;
@@ -2134,4 +2167,7 @@ SLAI_EXPORT int slai_gpt2_prefill(slai_gpt2 *m, const int32_t *tokens, uint32_t 
     return SLAI_OK;
 }
 
+SLAI_EXPORT int slai_gpt2_prompt_form(const slai_gpt2 *m, uint32_t n_tokens, int step) {
+    return m && n_tokens && n_tokens <= wide::MAX_TOKENS && m->wide_supported() ? prompt_form(m->wide_plans(n_tokens), step) : -1;
+}
 SLAI_EXPORT uint32_t slai_gpt2_prefill_fp32_repeats(const slai_gpt2 *m) { return m ? m->prefill_fp32_repeats : 0; }

@@ -572,6 +572,11 @@ class Llama2:
         """Prefill calls that were repeated with fp32 MFMA because an activation was beyond the f16 range."""
         return int(self.b.L.slai_llama2_prefill_fp32_repeats(self.h))
 
+    def prompt_form(self, n_tokens, step):
+        """The form of step 0..3 (q/k/v, attention output, gate / up, down) of a prompt pass of n_tokens -- 0: large, 1: small,
+        2: slim, 3: shared tiles, -1: none (see slai_llama2_prompt_form)."""
+        return int(self.b.L.slai_llama2_prompt_form(self.h, n_tokens, step))
+
     def prefill(self, tokens, start_pos=0, chunk=0):
         """Fill the caches for positions start_pos .. start_pos+len(tokens)-1, `chunk` tokens per pass over the
         weights (0 = the library's default); returns the stream time in ms."""
@@ -642,6 +647,11 @@ class Gpt2:
     def prefill_fp32_repeats(self):
         """Prefill calls that were repeated with fp32 MFMA because an activation was beyond the f16 range."""
         return int(self.b.L.slai_gpt2_prefill_fp32_repeats(self.h))
+
+    def prompt_form(self, n_tokens, step):
+        """The form of step 0..3 (q/k/v, attention output, gate / up, down) of a prompt pass of n_tokens -- 0: large, 1: small,
+        2: slim, 3: shared tiles, -1: none (see slai_llama2_prompt_form)."""
+        return int(self.b.L.slai_gpt2_prompt_form(self.h, n_tokens, step))
 
     def prefill(self, tokens, start_pos=0, chunk=0):
         """Fill the caches for positions start_pos .. start_pos+len(tokens)-1; returns the stream time in ms."""
