@@ -76,6 +76,8 @@ struct slai_ctx {
     // row tiles that several workgroups of a die share (gemv_spread_kernel, wide_share_kernel): their sums, and a count per workgroup; null: none are shared (no memory, or a device that places workgroups differently)
     float *spread_sums = nullptr;
     uint32_t *spread_counters = nullptr;
+    uint8_t *share_sums = nullptr;      // wide_share_kernel's sums, wide_share_bytes of them, made when the first launch wants them (share_reserve)
+    size_t share_bytes = (size_t)64 << 20;   // SLAI_PROMPT_SHARE_MB (64): most they may take; fewer: prompt passes share no tiles
     bool fuse_qkv_attention = true;     // SLAI_FUSE_QKV_ATTN=0: q/k/v and attention as separate launches, attention splits merged by a launch of their own, no resident or one-die launch
     int prompt_split_f16 = 1;           // SLAI_PROMPT_SPLIT_F16: 0 = prompt-chunk GEMMs in fp32 MFMA, 1 = the models' on the f16 matrix cores (f16 head + remainder), 2 = slai_matmul_quant_columns too
     int *split_flag = nullptr;          // device word the kernels that write split activations set when a value is beyond f16
@@ -362,6 +364,7 @@ bool qkv_attention_fusable(const slai_ctx *ctx, const slai_qmat *v, const slai_q
 // twentieth of a prompt of 37 tokens for the 15 M parameter Llama.)
 int read_word(slai_ctx *ctx, const void *from, uint32_t *word);
 int handoff_reserve(slai_ctx *ctx, uint32_t n_heads);   // not during graph capture
+bool share_reserve(slai_ctx *ctx);   // slai_ctx::share_sums; false: no memory for them
 int handoff_check(slai_ctx *ctx);                        // after a synchronize: error if a hand-off ever timed out
 // Makes sure the row-tile GEMV's scratch holds `floats` floats (call outside graph capture).
 int gemv_scratch_reserve(slai_ctx *ctx, size_t floats);

@@ -151,7 +151,6 @@ struct WidePass {
     slai_buffer *x = nullptr, *pairs = nullptr, *hidden = nullptr;   // residual rows; normalised rows / attention results and the hidden layer as pairs
     slai_buffer *q = nullptr, *k = nullptr, *v = nullptr;            // projections (k, v: Llama; GPT-2's are columns of q), possibly in partial results
     slai_buffer *parts = nullptr;                                    // partial results of the projection into the residual
-    slai_buffer *shared = nullptr;                                   // of tiles that workgroups share (WIDE_SHARE)
 
     static int grow(slai_ctx *ctx, slai_buffer *&b, size_t bytes) {
         if (b && b->bytes >= bytes) return SLAI_OK;
@@ -160,7 +159,7 @@ struct WidePass {
         return slai_buffer_create(ctx, bytes, SLAI_DT_F32, STORAGE, &b);
     }
     void destroy(slai_ctx *ctx) {
-        for (slai_buffer **b : {&x, &pairs, &hidden, &q, &k, &v, &parts, &shared})
+        for (slai_buffer **b : {&x, &pairs, &hidden, &q, &k, &v, &parts})
             if (*b) { slai_buffer_destroy(ctx, *b); *b = nullptr; }
     }
 };
@@ -236,8 +235,6 @@ WideGemmSeg wide_seg(const slai_qmat *m, float *out, uint32_t out_stride, uint32
     s.bias = bias && bias->buf ? (const float *)bias->buf->dptr : nullptr;
     return s;
 }
-// Whether workgroups may share a tile through their die's L2: their placement has been looked at (spread_setup)
-bool wide_may_share(const slai_ctx *ctx) { return ctx->spread_counters != nullptr; }
 // The forms of a pass's launches (kv: the last layer's keys and values)
 struct WidePlans { WidePlan qkv, kv, o, ffn, down; };
 // the step as slai_llama2_prompt_form counts it, and its form
@@ -247,18 +244,19 @@ int prompt_form(const WidePlans &p, int step) {
     const int form = plans[step]->form;
     return form == WIDE_SHARE ? SLAI_PROMPT_SHARED : form == WIDE_LARGE ? SLAI_PROMPT_LARGE : form == WIDE_SMALL ? SLAI_PROMPT_SMALL : SLAI_PROMPT_SLIM;
 }
-int wide_call(slai_ctx *ctx, WidePass &pass, WideGemmParams p, int mode, const char *who) {
-    if (p.form == WIDE_SHARE) {
-        TRY(WidePass::grow(ctx, pass.shared, wide_share_bytes()));
-        p.shared = (uint8_t *)pass.shared->dptr;
-        p.counters = ctx->spread_counters;
-    }
+// wide_plan with shared tiles where the context can have them
+WidePlan wide_plan_in(slai_ctx *ctx, const uint32_t *nrows, int nseg, uint32_t ntokens, uint32_t ncb, WideSplits splits, bool gated, bool may_share) {
+    const WidePlan p = wide_plan(nrows, nseg, ntokens, ncb, splits, gated, may_share && ctx->spread_counters);
+    return p.form == WIDE_SHARE && !share_reserve(ctx) ? wide_plan(nrows, nseg, ntokens, ncb, splits, gated, false) : p;
+}
+int wide_call(slai_ctx *ctx, WideGemmParams p, int mode, const char *who) {
+    if (p.form == WIDE_SHARE) { p.shared = ctx->share_sums; p.counters = ctx->spread_counters; }
     const hipError_t e = launch_wide_gemm(ctx->stream, p, mode);
     if (e == hipErrorInvalidValue) return set_error(ctx, SLAI_E_SHAPE, std::string(who) + ": unsupported shape for the wide prompt GEMM");
     return e == hipSuccess ? SLAI_OK : hip_fail(ctx, e, who);
 }
 // Segments over one input as rows: formats that can share a launch do (any K-quants, otherwise equal ones)
-int wide_rows(slai_ctx *ctx, WidePass &pass, int nseg, const WideGemmSeg *segs, const uint8_t *x, uint32_t ncb, uint32_t ntokens, const WidePlan &plan, const char *who) {
+int wide_rows(slai_ctx *ctx, int nseg, const WideGemmSeg *segs, const uint8_t *x, uint32_t ncb, uint32_t ntokens, const WidePlan &plan, const char *who) {
     bool done[3] = {false, false, false};
     const auto kq = [](int t) { return t == T_Q4_K || t == T_Q5_K || t == T_Q6_K; };
     for (int i = 0; i < nseg; ++i) {
@@ -270,7 +268,7 @@ int wide_rows(slai_ctx *ctx, WidePass &pass, int nseg, const WideGemmSeg *segs, 
             p.seg[p.nseg++] = segs[j];
             done[j] = true;
         }
-        TRY(wide_call(ctx, pass, p, WIDE_ROWS, who));
+        TRY(wide_call(ctx, p, WIDE_ROWS, who));
     }
     return SLAI_OK;
 }
@@ -1219,14 +1217,13 @@ void slai_llama2::wide_setup() {
 
 WidePlans slai_llama2::wide_plans(uint32_t n) const {
     const uint32_t dim = config.dim, kvd = kv_dim(), hid = config.hidden_dim, ncb = (dim + 255) / 256, hcb = (hid + 255) / 256, r_qkv[3] = {kvd, kvd, dim};
-    const bool share = wide_may_share(ctx), share_qkv = share && wide_one_format;
     WidePlans p;
-    p.qkv = wide_plan(r_qkv, 3, n, ncb, WIDE_READ, false, share_qkv);
+    p.qkv = wide_plan_in(ctx, r_qkv, 3, n, ncb, WIDE_READ, false, wide_one_format);
     // the last layer's keys and values: few rows in large workgroups leave most of the device idle (Qwen2-7B shape, 900 tokens: 70 us for 1024 rows)
-    p.kv = p.qkv.form == WIDE_LARGE || p.qkv.form == WIDE_SMALL || p.qkv.form == WIDE_SHARE ? wide_plan(r_qkv, 2, n, ncb, WIDE_READ, false, share_qkv) : p.qkv;
-    p.o = wide_plan(&dim, 1, n, ncb, WIDE_SUMMED, false, share);
-    p.ffn = wide_plan(&hid, 1, n, ncb, WIDE_WHOLE, true, share);
-    p.down = wide_plan(&dim, 1, n, hcb, WIDE_SUMMED, false, share);
+    p.kv = p.qkv.form == WIDE_LARGE || p.qkv.form == WIDE_SMALL || p.qkv.form == WIDE_SHARE ? wide_plan_in(ctx, r_qkv, 2, n, ncb, WIDE_READ, false, wide_one_format) : p.qkv;
+    p.o = wide_plan_in(ctx, &dim, 1, n, ncb, WIDE_SUMMED, false, true);
+    p.ffn = wide_plan_in(ctx, &hid, 1, n, ncb, WIDE_WHOLE, true, true);
+    p.down = wide_plan_in(ctx, &dim, 1, n, hcb, WIDE_SUMMED, false, true);
     return p;
 }
 
@@ -1258,7 +1255,7 @@ int slai_llama2::enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev) 
         SLAI_HIP_TRY(ctx, launch_norm_pairs(ctx->stream, pairs, x, parts, nparts, n * dim, (const float *)wl.attn_norm.buf->dptr, nullptr, dim, n, config.rms_norm_eps,
                                              wide_reads_sums(wm.q) || wide_reads_sums(wm.k) || wide_reads_sums(wm.v), flag));
         const WideGemmSeg qkv[3] = {wide_seg(wm.v, v, kvd, n * kvd), wide_seg(wm.k, k, kvd, n * kvd), wide_seg(wm.q, q, dim, n * dim)};
-        TRY(wide_rows(ctx, wide, last ? 2 : 3, qkv, pairs, ncb, n, last ? plan.kv : plan.qkv, "llama2 qkv (prompt)"));
+        TRY(wide_rows(ctx, last ? 2 : 3, qkv, pairs, ncb, n, last ? plan.kv : plan.qkv, "llama2 qkv (prompt)"));
         AttnLaunch a{};
         a.kcache = state.key_cache[l].buf->dptr; a.vcache = state.value_cache[l].buf->dptr; a.kv_f16 = kv_dtype == SLAI_KV_F16;
         a.n_heads = config.n_q_heads; a.kv_mul = config.n_q_heads / config.n_kv_heads; a.head_size = hs; a.kv_dim = kvd; a.seq_len = config.seq_len;
@@ -1274,16 +1271,16 @@ int slai_llama2::enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev) 
         pa.pos0 = pos0; pa.n = n; pa.out = pairs; pa.out_ncb = ncb; pa.sums = wide_reads_sums(wm.o); pa.flag = flag;
         SLAI_HIP_TRY(ctx, launch_prompt_attention(ctx->stream, pa, hs, a.kv_f16 != 0));
         const WideGemmSeg o = wide_seg(wm.o, parts, dim, n * dim);
-        TRY(wide_rows(ctx, wide, 1, &o, pairs, ncb, n, plan.o, "llama2 attn_output (prompt)"));
+        TRY(wide_rows(ctx, 1, &o, pairs, ncb, n, plan.o, "llama2 attn_output (prompt)"));
         SLAI_HIP_TRY(ctx, launch_norm_pairs(ctx->stream, pairs, x, parts, ks_o, n * dim, (const float *)wl.ffn_norm.buf->dptr, nullptr, dim, n, config.rms_norm_eps,
                                              wide_reads_sums(wm.gate), flag));
         WideGemmParams g;
         g.nseg = 2; g.seg[0] = wide_seg(wm.gate, nullptr, 0, 0); g.seg[1] = wide_seg(wm.up, nullptr, 0, 0);
         g.x = pairs; g.ncb = ncb; g.ntokens = n; g.pairs_out = hidden; g.out_ncb = hcb; g.out_sums = wide_reads_sums(wm.down); g.up = wm.hidden_up; g.flag = flag; g.form = plan.ffn.form;
-        TRY(wide_call(ctx, wide, g, WIDE_GATED, "llama2 ffn gate/up (prompt)"));
+        TRY(wide_call(ctx, g, WIDE_GATED, "llama2 ffn gate/up (prompt)"));
         WideGemmSeg d = wide_seg(wm.down, parts, dim, n * dim);
         d.down = 1.0f / wm.hidden_up;
-        TRY(wide_rows(ctx, wide, 1, &d, hidden, hcb, n, plan.down, "llama2 ffn_down (prompt)"));
+        TRY(wide_rows(ctx, 1, &d, hidden, hcb, n, plan.down, "llama2 ffn_down (prompt)"));
         nparts = ks_d;
     }
     return SLAI_OK;
@@ -1983,12 +1980,11 @@ bool slai_gpt2::wide_supported() const {
 
 WidePlans slai_gpt2::wide_plans(uint32_t n) const {
     const uint32_t E = params.n_embd, F = params.ff_len, r_qkv = 3 * E;
-    const bool share = wide_may_share(ctx);
     WidePlans p;
-    p.qkv = p.kv = wide_plan(&r_qkv, 1, n, E / 256, WIDE_READ, false, share);
-    p.o = wide_plan(&E, 1, n, E / 256, WIDE_SUMMED, false, share);
-    p.ffn = wide_plan(&F, 1, n, E / 256, WIDE_WHOLE, false, share);
-    p.down = wide_plan(&E, 1, n, F / 256, WIDE_SUMMED, false, share);
+    p.qkv = p.kv = wide_plan_in(ctx, &r_qkv, 1, n, E / 256, WIDE_READ, false, true);
+    p.o = wide_plan_in(ctx, &E, 1, n, E / 256, WIDE_SUMMED, false, true);
+    p.ffn = wide_plan_in(ctx, &F, 1, n, E / 256, WIDE_WHOLE, false, true);
+    p.down = wide_plan_in(ctx, &E, 1, n, F / 256, WIDE_SUMMED, false, true);
     return p;
 }
 
@@ -2017,7 +2013,7 @@ int slai_gpt2::enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev) {
         SLAI_HIP_TRY(ctx, launch_norm_pairs(ctx->stream, pairs, x, parts, nparts, n * E, (const float *)w.ln_1_g.buf->dptr, (const float *)w.ln_1_b.buf->dptr, E, n, eps,
                                              wide_reads_sums(w.c_attn_attn_w), flag));
         const WideGemmSeg sq = wide_seg(w.c_attn_attn_w, qkv, 3 * E, n * 3 * E, &w.c_attn_attn_b);
-        TRY(wide_rows(ctx, wide, 1, &sq, pairs, ncb, n, plan.qkv, "gpt2 qkv (prompt)"));
+        TRY(wide_rows(ctx, 1, &sq, pairs, ncb, n, plan.qkv, "gpt2 qkv (prompt)"));
         AttnLaunch a{};
         a.kcache = w.key_cache.buf->dptr; a.vcache = w.value_cache.buf->dptr; a.kv_f16 = kv_dtype == SLAI_KV_F16;
         a.n_heads = params.n_head; a.kv_mul = 1; a.head_size = hs; a.kv_dim = E; a.seq_len = params.n_seq;
@@ -2030,15 +2026,15 @@ int slai_gpt2::enqueue_wide(uint32_t pos0, uint32_t n, const int *tokens_dev) {
         pa.pos0 = pos0; pa.n = n; pa.out = pairs; pa.out_ncb = ncb; pa.sums = wide_reads_sums(w.c_attn_proj_w); pa.flag = flag;
         SLAI_HIP_TRY(ctx, launch_prompt_attention(ctx->stream, pa, hs, a.kv_f16 != 0));
         const WideGemmSeg so = wide_seg(w.c_attn_proj_w, parts, E, n * E, &w.c_attn_proj_b);
-        TRY(wide_rows(ctx, wide, 1, &so, pairs, ncb, n, plan.o, "gpt2 attn proj (prompt)"));
+        TRY(wide_rows(ctx, 1, &so, pairs, ncb, n, plan.o, "gpt2 attn proj (prompt)"));
         SLAI_HIP_TRY(ctx, launch_norm_pairs(ctx->stream, pairs, x, parts, ks_o, n * E, (const float *)w.ln_2_g.buf->dptr, (const float *)w.ln_2_b.buf->dptr, E, n, eps,
                                              wide_reads_sums(w.c_mlp_fc_w), flag));
         WideGemmParams g;
         g.nseg = 1; g.seg[0] = wide_seg(w.c_mlp_fc_w, nullptr, 0, 0, &w.c_mlp_fc_b);
         g.x = pairs; g.ncb = ncb; g.ntokens = n; g.pairs_out = hidden; g.out_ncb = fcb; g.out_sums = wide_reads_sums(w.c_mlp_proj_w); g.flag = flag; g.form = plan.ffn.form;
-        TRY(wide_call(ctx, wide, g, WIDE_GELU, "gpt2 mlp fc (prompt)"));
+        TRY(wide_call(ctx, g, WIDE_GELU, "gpt2 mlp fc (prompt)"));
         const WideGemmSeg sd = wide_seg(w.c_mlp_proj_w, parts, E, n * E, &w.c_mlp_proj_b);
-        TRY(wide_rows(ctx, wide, 1, &sd, hidden, fcb, n, plan.down, "gpt2 mlp proj (prompt)"));
+        TRY(wide_rows(ctx, 1, &sd, hidden, fcb, n, plan.down, "gpt2 mlp proj (prompt)"));
         nparts = ks_d;
     }
     return SLAI_OK;

@@ -72,7 +72,7 @@ using namespace slai;
 // with the context, not with the first model that asks for it: what a call computes, to the last bit, is not to depend on what else was loaded.
 // Without memory for it the context does without.
 static void spread_setup(slai_ctx *ctx) {
-    const size_t words = gemv_spread_counter_words();
+    const size_t words = std::max(gemv_spread_counter_words(), wide_share_counter_words());
     bool placed = hipMalloc((void **)&ctx->spread_counters, std::max(words, (size_t)HOST_WORDS) * sizeof(uint32_t)) == hipSuccess &&
                   launch_xcd_of_workgroup(ctx->stream, ctx->spread_counters, HOST_WORDS) == hipSuccess &&
                   hipMemcpyAsync(ctx->host_words, ctx->spread_counters, HOST_WORDS * sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream) == hipSuccess &&
@@ -111,6 +111,7 @@ SLAI_EXPORT int slai_ctx_create(int device, slai_ctx **out) {
     }
     ctx->gemv_max_wgs = env_int("SLAI_GEMV_MAX_WGS", 512);
     ctx->tiled_layout = env_int("SLAI_TILED", 1) != 0;
+    ctx->share_bytes = (size_t)std::max(0, env_int("SLAI_PROMPT_SHARE_MB", 64)) << 20;
     ctx->prompt_copy_bytes = (size_t)std::max(0, env_int("SLAI_PROMPT_COPY_MB", 1024)) << 20;
     ctx->rowtile_gemv = env_int("SLAI_ROWTILE", 1) != 0;
     ctx->fuse_qkv_attention = env_int("SLAI_FUSE_QKV_ATTN", 1) != 0;
@@ -142,6 +143,7 @@ SLAI_EXPORT void slai_ctx_destroy(slai_ctx *ctx) {
     if (ctx->handoff_counters) (void)hipFree(ctx->handoff_counters);
     if (ctx->spread_sums) (void)hipFree(ctx->spread_sums);
     if (ctx->spread_counters) (void)hipFree(ctx->spread_counters);
+    if (ctx->share_sums) (void)hipFree(ctx->share_sums);
     for (void *p : ctx->retired_scratch) (void)hipFree(p);
     for (slai_buffer *b : ctx->retired_buffers) buffer_free(b);
     if (ctx->timer0) (void)hipEventDestroy(ctx->timer0);
@@ -505,6 +507,15 @@ int handoff_reserve(slai_ctx *ctx, uint32_t n_heads) {
     ctx->handoff_counters = counters;
     ctx->handoff_heads = n_heads;
     return SLAI_OK;
+}
+// The prompt passes that would share tiles take plain forms without this memory, so its absence is nobody's error.
+bool share_reserve(slai_ctx *ctx) {
+    if (ctx->share_sums) return true;
+    if (ctx->capturing || wide_share_bytes() > ctx->share_bytes) return false;
+    if (hipMalloc((void **)&ctx->share_sums, wide_share_bytes()) == hipSuccess) return true;
+    ctx->share_sums = nullptr;
+    (void)hipGetLastError();                                   // (not the next launch's error)
+    return false;
 }
 int handoff_check(slai_ctx *ctx) {
     if (!ctx->handoff_counters) return SLAI_OK;

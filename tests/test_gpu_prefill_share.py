@@ -53,3 +53,21 @@ def test_shared_tiles_gpt2(backend):
     got, ref = (logits_of(Gpt2(backend, g, _ffi.KV_F32), prompt, chunk) for chunk in (0, 32))
     assert rel_err(got, ref) < SELF_TOL
     g.close()
+
+
+def test_without_memory_for_shared_tiles(monkeypatch):
+    """A prompt whose launches would share tiles is read all the same, in the plain forms, where the sums of shared tiles are not allowed their 64 MB."""
+    from slai_amd.runtime import Backend, Gguf, Llama2
+    t, n = 8, 513
+    g = Gguf(gw.llama_gguf(2048, 5632, 2, 16, 16, 512, 1024, t, v_type=t, out_type=t, embd_type=t, std=0.03, norm_random=True))
+    prompt = np.random.Generator(np.random.PCG64(n)).integers(0, 512, n).astype(np.int32)
+    logits = []
+    for mb, form in ((64, 3), (63, 0)):
+        monkeypatch.setenv("SLAI_PROMPT_SHARE_MB", str(mb))
+        b = Backend(0)
+        m = Llama2(b, g, _ffi.MODEL_LLAMA, _ffi.KV_F32)
+        assert m.prompt_form(n - 1, 2) == form
+        logits.append(logits_of(m, prompt, 0))
+        b.close()
+    assert rel_err(logits[1], logits[0]) < SELF_TOL
+    g.close()
