@@ -89,6 +89,9 @@ void slai_ctx_destroy(slai_ctx *ctx);
 const char *slai_last_error(slai_ctx *ctx);
 /* The HIP stream every launch of this context goes to (as a `hipStream_t`). */
 void *slai_ctx_stream(slai_ctx *ctx);
+/* Inspection: how many GEMV launches of this context so far had their 64-row tiles spread evenly over the device, several workgroups to a tile (inside a graph they count
+ * when it is captured). */
+uint32_t slai_ctx_spread_launches(const slai_ctx *ctx);
 
 /* `LlmContext::begin_submission` / `submit` (crates/slai/src/context.rs:79-95) and
  * `Backend::synchronize` (crates/slai-chat/src/chat_llama2.rs:219). */

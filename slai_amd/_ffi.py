@@ -54,6 +54,7 @@ SIGNATURES = {
     "slai_ctx_destroy": (None, [vp]),
     "slai_last_error": (C.c_char_p, [vp]),
     "slai_ctx_stream": (vp, [vp]),
+    "slai_ctx_spread_launches": (u32, [vp]),
     "slai_begin_submission": (i32, [vp]),
     "slai_submit": (i32, [vp]),
     "slai_synchronize": (i32, [vp]),

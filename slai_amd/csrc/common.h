@@ -76,6 +76,7 @@ struct slai_ctx {
     // row tiles that several workgroups of a die share (gemv_spread_kernel, wide_share_kernel): their sums, and a count per workgroup; null: none are shared (no memory, or a device that places workgroups differently)
     float *spread_sums = nullptr;
     uint32_t *spread_counters = nullptr;
+    uint32_t spread_launches = 0;       // GEMV launches that were spread evenly
     uint8_t *share_sums = nullptr;      // wide_share_kernel's sums, wide_share_bytes of them, made when the first launch wants them (share_reserve)
     size_t share_bytes = (size_t)64 << 20;   // SLAI_PROMPT_SHARE_MB (64): most they may take; fewer: prompt passes share no tiles
     bool fuse_qkv_attention = true;     // SLAI_FUSE_QKV_ATTN=0: q/k/v and attention as separate launches, attention splits merged by a launch of their own, no resident or one-die launch

@@ -506,7 +506,7 @@ hipError_t go(const GemvRowtileParams &p, uint32_t tiles, int NT, size_t smem, h
         gemv_rowtile_batch_kernel<TT, DUAL><<<(tiles + 7) / 8 * 8 * bt->n, NT, smem, s>>>(p, *bt, tiles);
         return hipGetLastError();
     }
-    if (p.prepared && spread_sums) {
+    if (spread_sums) {
         const uint32_t most = spread_units(tiles, p.ncb), waves = std::min(16u, std::max(std::max(most, 4u), (p.ncols + 1023) / 1024));     // (x: four float4 per thread)
         gemv_spread_kernel<TT, DUAL><<<SPREAD_DIES * SPREAD_RUNS, waves * 64, 0, s>>>(p, spread_sums, spread_counters, tiles);
         return hipGetLastError();
@@ -555,7 +555,8 @@ hipError_t launch_gemv_rowtile(slai_ctx *ctx, GemvRowtileParams p, const GemvBat
     }
     const int NT = NW * 64;
     hipStream_t st = ctx->stream;
-    float *spread = spread_pays(p, tiles) ? ctx->spread_sums : nullptr;
+    float *spread = p.prepared && !(bt && bt->n > 1) && spread_pays(p, tiles) ? ctx->spread_sums : nullptr;
+    if (spread) ++ctx->spread_launches;
     switch (tt) {
     case T_Q4_K: return dual ? go<T_Q4_K, true>(p, tiles, NT, smem, st, bt, spread, ctx->spread_counters) : go<T_Q4_K, false>(p, tiles, NT, smem, st, bt, spread, ctx->spread_counters);
     case T_Q6_K: return dual ? go<T_Q6_K, true>(p, tiles, NT, smem, st, bt, spread, ctx->spread_counters) : go<T_Q6_K, false>(p, tiles, NT, smem, st, bt, spread, ctx->spread_counters);

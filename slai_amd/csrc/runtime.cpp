@@ -154,6 +154,7 @@ SLAI_EXPORT void slai_ctx_destroy(slai_ctx *ctx) {
 
 SLAI_EXPORT const char *slai_last_error(slai_ctx *ctx) { return ctx ? ctx->err.c_str() : "null context"; }
 SLAI_EXPORT void *slai_ctx_stream(slai_ctx *ctx) { return ctx ? (void *)ctx->stream : nullptr; }
+SLAI_EXPORT uint32_t slai_ctx_spread_launches(const slai_ctx *ctx) { return ctx ? ctx->spread_launches : 0; }
 
 // context.rs:79-95.  The reference records launches into an encoder and hands it to the queue on submit; here every
 // launch goes to the context's stream at once, so the pair only keeps the reference's state rules: beginning while a

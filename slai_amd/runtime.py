@@ -42,6 +42,10 @@ class Backend:
     def synchronize(self):
         self.check(self.L.slai_synchronize(self.h))
 
+    def spread_launches(self):
+        """GEMV launches so far whose 64-row tiles were spread evenly over the device (see slai_ctx_spread_launches)."""
+        return int(self.L.slai_ctx_spread_launches(self.h))
+
     def graph_begin_capture(self):
         self.check(self.L.slai_graph_begin_capture(self.h))
 
