@@ -11,6 +11,15 @@ pytestmark = pytest.mark.gpu
 NAMES = {2: "q4_0", 8: "q8_0", 12: "q4_k", 13: "q5_k", 14: "q6_k"}
 
 
+QKV, OUTPUT, FFN, DOWN = range(4)                              # prompt_form's steps
+PLAIN, SHARED = 0, 3                                           # its forms: large workgroups alone, with shared tiles
+# format, hidden columns of a model 2048 wide, tokens (one fewer is read); how gate + up are dealt out: whole rounds, most rests a workgroup has to finish (None: in plain
+# rounds, q/k/v share).  Row units of 256 rows of both matrices, token blocks of 64: a last unit with 32 rows (5664), last blocks with 1, 32, 33 and 64 tokens, one to
+# four rests, workgroups with fewer than the others (22, 23 and 25 tiles), a whole round in front.
+DEALS = [(12, 5632, 450, 0, 3), (12, 5888, 482, 0, 3), (8, 5632, 513, 0, 3), (13, 5632, 513, 0, 3), (2, 5632, 450, 0, 3), (14, 5632, 513, 0, 3), (8, 5664, 481, 0, 3), (12, 8192, 257, 0, 1),
+         (12, 4608, 642, 0, 4), (8, 11008, 641, 1, 3), (12, 9216, 705, 1, 2), (8, 11008, 705, None, None)]
+
+
 def logits_of(m, prompt, chunk):
     m.prefill(prompt[:-1], 0, chunk)
     out = m.forward_logits(prompt.size - 1, int(prompt[-1]))
@@ -18,41 +27,52 @@ def logits_of(m, prompt, chunk):
     return out
 
 
-# gate + up of 22 or 23 row units (the last a quarter full) at 7 and 8 token blocks (the last with 1, 33 and 64 tokens): one main per group and three; and an incomplete second round
-@pytest.mark.parametrize("t,hidden,n", [(12, 5632, 450), (12, 5888, 482), (8, 5632, 513), (13, 5632, 513), (2, 5632, 450), (14, 5632, 513), (8, 11008, 705)],
-                         ids=lambda v: NAMES.get(v, str(v)))
-def test_shared_tiles_llama(backend, t, hidden, n):
+@pytest.mark.parametrize("t,hidden,n,rounds,rests", DEALS, ids=["%s-%d-%d" % (NAMES[d[0]], d[1], d[2]) for d in DEALS])
+def test_shared_tiles_llama(backend, t, hidden, n, rounds, rests):
     from slai_amd.runtime import Gguf, Llama2
     print("case", NAMES[t], hidden, n, flush=True)
     g = Gguf(gw.llama_gguf(2048, hidden, 2, 16, 16, 512, 1024, t, v_type=t, out_type=t, embd_type=t, std=0.03, norm_random=True))
     prompt = np.random.Generator(np.random.PCG64(n)).integers(0, 512, n).astype(np.int32)
+    m = Llama2(backend, g, _ffi.MODEL_LLAMA, _ffi.KV_F32)
+    assert m.prompt_form(n - 1, FFN) == (PLAIN if rounds is None else SHARED) and SHARED in [m.prompt_form(n - 1, step) for step in range(4)]
+    m.destroy()
     got, again, ref = (logits_of(Llama2(backend, g, _ffi.MODEL_LLAMA, _ffi.KV_F32), prompt, chunk) for chunk in (0, 0, 32))
     assert np.array_equal(got, again)                          # whoever of a tile's two workgroups comes last
     assert rel_err(got, ref) < SELF_TOL
     g.close()
 
 
-# 43 row units at 5 token blocks are 27 tiles a die, whose rests are dealt out to five workgroups, the last of them with fewer; 24 units at 7: 21 and eleven
-@pytest.mark.parametrize("hidden,n", [(11008, 301), (6144, 449)])
-def test_last_rests(backend, hidden, n):
+# 24 row units at 7 token blocks are 21 tiles a die, whose rests are dealt out to eleven workgroups, the last of them with fewer; 43 at 5 are 27, which would leave six rests to
+# each of five workgroups: gate + up in plain rounds, q/k/v (24 units, 15 tiles a die) shared
+@pytest.mark.parametrize("hidden,n,forms", [(11008, 301, (SHARED, PLAIN)), (6144, 449, (SHARED, SHARED))])
+def test_last_rests(backend, hidden, n, forms):
     from slai_amd.runtime import Gguf, Llama2
     t = 12
     print("case", hidden, n, flush=True)
     g = Gguf(gw.llama_gguf(4096, hidden, 2, 32, 32, 512, 512, t, v_type=t, out_type=t, embd_type=t, std=0.02, norm_random=True, distinct_layers=1))
     prompt = np.random.Generator(np.random.PCG64(n)).integers(0, 512, n).astype(np.int32)
+    m = Llama2(backend, g, _ffi.MODEL_LLAMA, _ffi.KV_F32)
+    assert (m.prompt_form(n - 1, QKV), m.prompt_form(n - 1, FFN)) == forms
+    m.destroy()
     got, again, ref = (logits_of(Llama2(backend, g, _ffi.MODEL_LLAMA, _ffi.KV_F32), prompt, chunk) for chunk in (0, 0, 32))
     assert np.array_equal(got, again)
     assert rel_err(got, ref) < SELF_TOL
     g.close()
 
 
-def test_shared_tiles_gpt2(backend):
-    from slai_amd.runtime import Gguf, Gpt2
+# the MLP's first matrix (its GELU as pairs); that and q/k/v with their bias
+@pytest.mark.parametrize("n,steps", [(490, [FFN]), (701, [QKV, FFN])])
+def test_shared_tiles_gpt2(n, steps):
+    from slai_amd.runtime import Backend, Gguf, Gpt2
+    b = Backend(0)                                             # (a context that has held no other model)
     g = Gguf(gw.gpt2_gguf(2048, 2, 32, 8192, 512, 1024, 8, std=0.02))
-    prompt = np.random.Generator(np.random.PCG64(3)).integers(0, 512, 490).astype(np.int32)
-    got, ref = (logits_of(Gpt2(backend, g, _ffi.KV_F32), prompt, chunk) for chunk in (0, 32))
+    prompt = np.random.Generator(np.random.PCG64(3)).integers(0, 512, n).astype(np.int32)
+    m = Gpt2(b, g, _ffi.KV_F32)
+    assert [step for step in range(4) if m.prompt_form(n - 1, step) == SHARED] == steps
+    m.destroy()
+    got, ref = (logits_of(Gpt2(b, g, _ffi.KV_F32), prompt, chunk) for chunk in (0, 32))
     assert rel_err(got, ref) < SELF_TOL
-    g.close()
+    g.close(); b.close()
 
 
 def test_without_memory_for_shared_tiles(monkeypatch):
@@ -62,11 +82,11 @@ def test_without_memory_for_shared_tiles(monkeypatch):
     g = Gguf(gw.llama_gguf(2048, 5632, 2, 16, 16, 512, 1024, t, v_type=t, out_type=t, embd_type=t, std=0.03, norm_random=True))
     prompt = np.random.Generator(np.random.PCG64(n)).integers(0, 512, n).astype(np.int32)
     logits = []
-    for mb, form in ((64, 3), (63, 0)):
+    for mb, form in ((64, SHARED), (63, PLAIN)):
         monkeypatch.setenv("SLAI_PROMPT_SHARE_MB", str(mb))
         b = Backend(0)
         m = Llama2(b, g, _ffi.MODEL_LLAMA, _ffi.KV_F32)
-        assert m.prompt_form(n - 1, 2) == form
+        assert m.prompt_form(n - 1, FFN) == form
         logits.append(logits_of(m, prompt, 0))
         b.close()
     assert rel_err(logits[1], logits[0]) < SELF_TOL

@@ -157,9 +157,10 @@ def test_wide_gpt2_values_beyond_f16_repeat_in_fp32(backend, scale, repeats):
 
 
 @pytest.mark.parametrize("wtype", [12, 13, 14, 8, 2], ids=["q4_k", "q5_k", "q6_k", "q8_0", "q4_0"])
-@pytest.mark.parametrize("hidden,n", [(16640, 1000), (2816, 640)], ids=["large workgroups", "small workgroups"])
-def test_wide_many_tokens_against_passes_of_32(backend, wtype, hidden, n):
-    """Passes whose gate + up (and down, 16640 columns) run in the large workgroups, or whose gate + up runs in the small ones, against the kernels for up to 32
+@pytest.mark.parametrize("hidden,n,form", [(16640, 1000, 3), (2816, 640, 2), (4096, 1000, 0), (3072, 640, 1)],
+                         ids=["whole rounds, then shared tiles", "slim workgroups", "large workgroups", "small workgroups"])
+def test_wide_many_tokens_against_passes_of_32(backend, wtype, hidden, n, form):
+    """Gate + up in each form that many tokens take (down in large workgroups for 1000 tokens, in slim ones for 640), against the kernels for up to 32
     tokens.  Either is within 1.3e-6 of exact sums (2-norm, values of a second layer); the largest element of a million is five times that of each."""
     from slai_amd.runtime import Gguf, Llama2
     import ctypes as C
@@ -167,6 +168,7 @@ def test_wide_many_tokens_against_passes_of_32(backend, wtype, hidden, n):
     rows = []
     for chunk in (0, 32):
         m = Llama2(backend, g, _ffi.MODEL_LLAMA, _ffi.KV_F32)
+        assert m.prompt_form(n, 2) == form
         m.prefill(prompt_of(n, 512), 0, chunk)
         out = []
         for b in m.kv_buffers(1):

@@ -5,6 +5,8 @@ import subprocess
 
 import pytest
 
+from test_gpu_prefill_share import DEALS
+
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 LARGE, SMALL, SLIM4, SLIM8, SHARE = range(5)
@@ -49,3 +51,25 @@ def test_what_is_shared_is_what_was_planned(plan, dim, gated):
 def test_nothing_is_shared_where_it_may_not(plan, rows):
     for tokens in range(9, 1025, 13):
         assert plan(rows, tokens, 4096, READ, may_share=False).form != SHARE
+
+
+@pytest.mark.parametrize("deal", DEALS, ids=str)
+def test_deals_of_the_gpu_tests(plan, deal):
+    """The prompts that the GPU tests read reach the rounds and rests that they name."""
+    _, hidden, n, rounds, rests = deal
+    p = plan([hidden], n - 1, 2048, WHOLE, True)
+    if rounds is None:
+        assert p.form == LARGE and plan([2048, 2048, 2048], n - 1, 2048, READ).form == SHARE
+    else:
+        assert (p.form, p.rounds, p.mains) == (SHARE, rounds, rests)
+
+
+@pytest.mark.parametrize("tokens,output,down", [(256, 1, 1), (257, 2, 4), (320, 2, 4), (321, 2, 2), (384, 2, 2), (385, 1, None)])
+def test_ranges_of_the_gpu_tests(plan, tokens, output, down):
+    """Slim launches of a model 2048 wide with 8704 hidden columns: the ranges of columns at the edges that test_gpu_prefill_ranges reads (with 8192, two)."""
+    slim = (SLIM4, SLIM8)
+    p = plan([2048], tokens, 2048, SUMMED)
+    assert p.form in slim and p.ksplit == output
+    for hidden, ranges in ((8704, down), (8192, down and min(down, 2))):
+        p = plan([2048], tokens, hidden, SUMMED)
+        assert (p.form in slim and p.ksplit == ranges) if ranges else p.ksplit != 2
