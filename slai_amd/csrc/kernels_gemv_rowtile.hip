@@ -489,7 +489,8 @@ uint32_t spread_units(uint32_t tiles, uint32_t ncb) { return ((tiles + SPREAD_DI
 //   320        22.8 / 19.5     37.0 / 31.3    12.6 / 11.6                       12.8 / 11.3
 //   384        23.5 / 21.9     37.6 / 37.1    13.2 / 12.8                       13.0 / 12.5
 //   432        24.4 / 24.8     41.6 / 41.2    (448: 13.7 / 15.2)                13.6 / 14.2
-// (tile: 147 KB of a Q4_K row tile of 16 groups, twice that of a pair)
+// (tile: 147 KB of a Q4_K row tile of 16 groups, twice that of a pair.  The two columns measured at 384 tiles still gain 4 to 7 % there, Q8_0 1 %; nothing between 320 and
+// 384 was measured, so the line is at 352)
 bool spread_pays(const GemvRowtileParams &p, uint32_t tiles) {
     uint64_t bytes = 0;
     for (int i = 0; i < p.nseg; ++i) bytes += (uint64_t)p.seg[i].ntiles * (p.seg[i].W2 ? 2 : 1) * p.ncb * (tiled_pieces(p.seg[i].type) * 1024 + tiled_tail(p.seg[i].type));
