@@ -76,17 +76,21 @@ inline WidePlan wide_plan(const uint32_t *nrows, int nseg, uint32_t ntokens, uin
     const uint32_t tile_tokens = (ntokens + 31) / 32 * 32;
     const float many = tile_tokens > 576 && ncb > 2 ? 1.0f + 0.0003f * (float)(tile_tokens - 576) * (float)(std::min(ncb, 8u) - 2) : 1.0f;
     const float t_slim = std::max(6.0f + (uneven ? 0.0026f : 0.0029f) * (float)slim * (float)ncb * many, turns > 4 ? 5.2f * (float)turns : 0.0f) + parts(ks_slim);
-    // Shared tiles, where the longest share is at most nine tenths of whole rounds and nobody has the rests of more than four tiles to finish (320 tokens: six): 7.6 us per super-block, and 20 us.  us a launch, large or slim / shared, gate + up of
+    // Shared tiles, where the longest share is at most nine tenths of whole rounds and nobody has the rests of more than four tiles to finish (320 tokens: six): 7.6 us per super-block, and 21 us (with 20, which the launches below take, the 21 picks nearest to the other forms were no faster than those, and 1024 x 4096 of GPT-2 at 993 tokens 6 us slower).  us a launch, large or slim / shared, gate + up of
     // the 7B shape (43 row units):
     //   tokens      192        256        320        384        448        512        576        640        768        896       1024
     //   Q4_K     112 / 90   130 / 111  132 / 131  214 / 192  235 / 198  247 / 207  255 / 229  264 / 245  367 / 326  383 / 344  404 / 390
     //   Q8_0     126 / 101  144 / 123  138 / 142  243 / 209  264 / 221  271 / 234  281 / 257  293 / 273  394 / 362  414 / 386  (968: 428 / 434)
     // (with every compute unit busy each is slower, 8.3 us per super-block at 1024 tokens, by its clock and not by waits: requests in flight over a
     // super-block's end instead of waiting for them there changed 1.5 %)
+    // Not where large workgroups in column ranges are the other choice and fill one round: they cut every tile in two as well, and nobody meets anybody.  q/k/v, us
+    // of the prompt that sharing took more: 7B shape, 257 to 320 tokens, Q4_K 14 to 17, Q5_K 11 to 18, Q4_0 8, Q8_0 3; 8192 x 4096 + 2 x 1024, 545: 20; 5120 wide, 193: 12
+    // (of 450 shared launches in 26 shapes and formats, those were 33 of the 49 that sharing made slower; in two rounds of ranges it takes 45 to 63 less)
+    const bool in_ranges = ks_large > 1 && rounds == 1 && t_wide <= t_slim;
     const wide::TileShare sh(r8, (ntokens + 63) / 64, ncb);
     const uint32_t longest = sh.longest(), whole = (sh.rounds + (sh.rest ? 1u : 0u)) * ncb;
-    const float t_share = 20.0f + 7.6f * (float)longest;
-    if (may_share && sh.mains <= 4 && 10 * longest <= 9 * whole && t_share < t_wide && t_share < t_slim) return WidePlan{WIDE_SHARE, 1};
+    const float t_share = 21.0f + 7.6f * (float)longest;
+    if (may_share && !in_ranges && sh.mains <= 4 && 10 * longest <= 9 * whole && t_share < t_wide && t_share < t_slim) return WidePlan{WIDE_SHARE, 1};
     if (t_slim < t_wide) return WidePlan{eight ? WIDE_SLIM8 : WIDE_SLIM4, ks_slim};
     return wide ? WidePlan{WIDE_LARGE, ks_large} : WidePlan{WIDE_SMALL, ks_small};
 }

@@ -15,9 +15,9 @@ QKV, OUTPUT, FFN, DOWN = range(4)                              # prompt_form's s
 PLAIN, SHARED = 0, 3                                           # its forms: large workgroups alone, with shared tiles
 # format, hidden columns of a model 2048 wide, tokens (one fewer is read); how gate + up are dealt out: whole rounds, most rests a workgroup has to finish (None: in plain
 # rounds, q/k/v share).  Row units of 256 rows of both matrices, token blocks of 64: a last unit with 32 rows (5664), last blocks with 1, 32, 33 and 64 tokens, one to
-# four rests, workgroups with fewer than the others (22, 23 and 25 tiles), a whole round in front.
+# four rests, workgroups with fewer than the others (22, 23 and 25 tiles), a whole round in front, two and then a single tile.
 DEALS = [(12, 5632, 450, 0, 3), (12, 5888, 482, 0, 3), (8, 5632, 513, 0, 3), (13, 5632, 513, 0, 3), (2, 5632, 450, 0, 3), (14, 5632, 513, 0, 3), (8, 5664, 481, 0, 3), (12, 8192, 257, 0, 1),
-         (12, 4608, 642, 0, 4), (8, 11008, 641, 1, 3), (12, 9216, 705, 1, 2), (8, 11008, 705, None, None)]
+         (12, 4608, 642, 0, 4), (8, 11008, 641, 1, 3), (12, 9216, 705, 1, 2), (8, 11008, 706, 2, 1), (8, 11008, 898, None, None)]
 
 
 def logits_of(m, prompt, chunk):
@@ -43,8 +43,8 @@ def test_shared_tiles_llama(backend, t, hidden, n, rounds, rests):
 
 
 # 24 row units at 7 token blocks are 21 tiles a die, whose rests are dealt out to eleven workgroups, the last of them with fewer; 43 at 5 are 27, which would leave six rests to
-# each of five workgroups: gate + up in plain rounds, q/k/v (24 units, 15 tiles a die) shared
-@pytest.mark.parametrize("hidden,n,forms", [(11008, 301, (SHARED, PLAIN)), (6144, 449, (SHARED, SHARED))])
+# each of five workgroups: gate + up in plain rounds, q/k/v (24 units, 15 tiles a die) in two ranges of columns
+@pytest.mark.parametrize("hidden,n,forms", [(11008, 301, (PLAIN, PLAIN)), (6144, 449, (SHARED, SHARED))])
 def test_last_rests(backend, hidden, n, forms):
     from slai_amd.runtime import Gguf, Llama2
     t = 12
@@ -61,7 +61,7 @@ def test_last_rests(backend, hidden, n, forms):
 
 
 # the MLP's first matrix (its GELU as pairs); that and q/k/v with their bias
-@pytest.mark.parametrize("n,steps", [(490, [FFN]), (701, [QKV, FFN])])
+@pytest.mark.parametrize("n,steps", [(490, [FFN]), (706, [QKV, FFN])])
 def test_shared_tiles_gpt2(n, steps):
     from slai_amd.runtime import Backend, Gguf, Gpt2
     b = Backend(0)                                             # (a context that has held no other model)

@@ -73,3 +73,11 @@ def test_ranges_of_the_gpu_tests(plan, tokens, output, down):
     for hidden, ranges in ((8704, down), (8192, down and min(down, 2))):
         p = plan([2048], tokens, hidden, SUMMED)
         assert (p.form in slim and p.ksplit == ranges) if ranges else p.ksplit != 2
+
+
+# q/k/v of one format: large workgroups in two ranges fill the device once, three of 7B's 512-row units more tokens and they no longer do; ranges in two rounds
+@pytest.mark.parametrize("rows,ncols,tokens,form,ranges", [([4096] * 3, 4096, 257, LARGE, 2), ([4096] * 3, 4096, 320, LARGE, 2), ([1024, 1024, 4096], 4096, 576, LARGE, 2), ([5120] * 3, 5120, 256, LARGE, 2),
+                                                           ([4096] * 3, 4096, 353, SHARE, 1), ([512, 512, 3584], 3584, 801, SHARE, 1)])
+def test_no_meeting_where_ranges_fill_the_device(plan, rows, ncols, tokens, form, ranges):
+    p = plan(rows, tokens, ncols, READ)
+    assert (p.form, p.ksplit) == (form, ranges)
